@@ -1,13 +1,12 @@
 // gemm_i8.hip -- launchers of the int8 GEMM: the gfx950 MFMA tile kernel
-// (gemm_i8_kernel.hpp), the decode kernel for m <= 64 (gemm_i8_decode_kernel.hpp),
-// the packed-weight tile kernel (gemm_i8_pb_kernel.hpp), a generic strided
+// (gemm_i8_kernel.hpp) over row-major or packed weights (gemm_i8_pack.hpp), the
+// decode kernels for m <= 64 (gemm_i8_decode_kernel.hpp), a generic strided
 // kernel for shapes the tile kernels do not take (k % 16 != 0, unaligned
 // operands) and the repack used for the reference sample's A col-major /
 // B [K,N] layout.
 #include "gemm_i8_decode_kernel.hpp"
 #include "gemm_i8_decode_wide_kernel.hpp"
 #include "gemm_i8_kernel.hpp"
-#include "gemm_i8_pb_kernel.hpp"
 #include "gemm_i8_persist_kernel.hpp"
 #include "gemm_i8_streamk_kernel.hpp"
 #include "w8a8_internal.hpp"
@@ -29,22 +28,24 @@ using gemm::KArgs;
 // 16 x 16 x 64 MFMA (gemm::Cfg): against the 32 x 32 x 32 form, GEMM-only,
 // cold weights, cfg3 projections: M = 8192 1448 -> 1389 µs, M = 2048 411 ->
 // 398 µs, M = 512 144 -> 132 µs (sum of the four).
-using GemmMain  = gemm::Cfg<256, 256, 128, 2, 2, 4, 4, 16>;
-// 3 LDS stages: these launches have few tiles per CU and read their panels
-// from HBM, where a third k-tile in flight hides the latency (cold weights,
-// M = 512: 128 x 128 o_proj 32 -> 22 µs, down 100 -> 66 µs; M = 2048,
-// 128 x 256: o_proj 47 -> 40 µs, down 146 -> 116 µs).
-using GemmMidM  = gemm::Cfg<128, 256, 128, 3, 2, 4, 4, 16>; // 8 waves of 64 x 64, 144 KiB LDS
-using GemmSmall = gemm::Cfg<128, 128, 128, 3, 2, 4, 4, 16>; // 8 waves of 64 x 32, 96 KiB LDS
-// m <= 64 over row-major weights (tiles_beat_decode): 4 waves of 64 x 32,
-// 4 stages (96 KiB LDS), one tile row.
-using GemmDecTile = gemm::Cfg<64, 128, 128, 4, 1, 4, 1, 16>;
-// Packed-weight tile configurations (m > kDecodeMaxM): 256 x 256 blocks, and
-// 128 / 64-row blocks for launches that would leave most CUs idle with them
-// (pick_packed_cfg).
-using GemmPacked    = gemm::PbCfg<256, 4, 2, 4>;
-using GemmPacked128 = gemm::PbCfg<128, 4, 2, 4>;
-using GemmPacked64  = gemm::PbCfg<64, 4, 2, 4>;
+// PB: over packed weights.
+// 3 LDS stages in the smaller two: these launches have few tiles per CU and
+// read their panels from HBM, where a third k-tile in flight hides the latency
+// (cold weights, M = 512: 128 x 128 o_proj 32 -> 22 µs, down 100 -> 66 µs;
+// M = 2048, 128 x 256: o_proj 47 -> 40 µs, down 146 -> 116 µs).
+template <bool PB>
+struct Tiles {
+    using Main  = gemm::Cfg<256, 256, 128, 2, 2, 4, 4, 16, PB>;
+    using MidM  = gemm::Cfg<128, 256, 128, 3, 2, 4, 4, 16, PB>; // 8 waves of 64 x 64, 144 KiB LDS
+    using Small = gemm::Cfg<128, 128, 128, 3, 2, 4, 4, 16, PB>; // 8 waves of 64 x 32, 96 KiB LDS
+    // m <= 64 (row-major weights: tiles_beat_decode): 4 waves of 64 x 32,
+    // 4 stages (96 KiB LDS), one tile row.
+    using Dec   = gemm::Cfg<64, 128, 128, 4, 1, 4, 1, 16, PB>;
+};
+using GemmMain    = Tiles<false>::Main;
+using GemmMidM    = Tiles<false>::MidM;
+using GemmSmall   = Tiles<false>::Small;
+using GemmDecTile = Tiles<false>::Dec;
 // Decode configurations: <32-row m tiles, 32-row weight tiles, waves, ring>.
 using DecSmall   = gemm::DecCfg<1, 1, 4, 3>; // m <= 32, or <= 16 packed
 using DecSmallW  = gemm::DecCfg<1, 2, 8, 3>; // packed, 8 <= m <= 32, many slabs
@@ -141,6 +142,36 @@ __global__ void __launch_bounds__(256) transpose_i8_kernel(const int8_t* src, ui
     }
 }
 
+// One thread per 16-byte packed chunk.
+__global__ void __launch_bounds__(256) pack_weights_kernel(const int8_t* __restrict__ w,
+                                                           uint32_t n, uint32_t k, uint32_t ldw,
+                                                           int8_t* __restrict__ out,
+                                                           size_t nchunks)
+{
+    const size_t idx = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
+    if(idx >= nchunks) return;
+    const uint32_t nkt   = gemm::packed_ktiles(k);
+    const uint32_t lane  = idx % 64;
+    const uint32_t frag  = (idx / 64) % gemm::kPackFrags;
+    const size_t   blk   = idx / (64 * gemm::kPackFrags); // slab * nkt + ktile
+    const uint32_t kt    = blk % nkt;
+    const uint32_t slab  = blk / nkt;
+    const uint32_t row   = slab * gemm::kSlab + (frag / 4) * 32 + lane % 32;
+    const uint32_t k0    = kt * gemm::kPackK + (frag % 4) * 32 + (lane / 32) * 16;
+    int4           v     = make_int4(0, 0, 0, 0);
+    if(row < n) {
+        const int8_t* src = w + (size_t)row * ldw + k0;
+        if(k0 + 16 <= k && (reinterpret_cast<uintptr_t>(src) % 16) == 0) {
+            v = *reinterpret_cast<const int4*>(src);
+        } else {
+            int8_t tmp[16];
+            for(int e = 0; e < 16; ++e) tmp[e] = (k0 + e < k) ? src[e] : 0;
+            v = *reinterpret_cast<const int4*>(tmp);
+        }
+    }
+    reinterpret_cast<int4*>(out)[idx] = v;
+}
+
 KArgs make_kargs(const GemmArgs& g)
 {
     return KArgs{g.a,   g.b,   g.c,   g.scale_a, g.scale_b, g.m,   g.n,
@@ -212,18 +243,6 @@ TileCfg pick_tile_cfg(uint32_t m, uint32_t n)
     if(tiles(GemmMain::kBM, GemmMain::kBN) >= enough) return TileCfg::kMain;
     if(tiles(GemmMidM::kBM, GemmMidM::kBN) >= enough) return TileCfg::kMidM;
     return TileCfg::kSmall;
-}
-
-// Block height of a packed-weight launch (blocks are always 256 weight
-// columns): the tallest of 256 / 128 / 64 rows that gives at least 3/4 of a
-// round of blocks, else 64.
-int pick_packed_cfg(uint32_t m, uint32_t n)
-{
-    const uint64_t cols   = (n + GemmPacked::kBN - 1) / GemmPacked::kBN;
-    const uint64_t enough = (uint64_t)device_cus() * 3 / 4;
-    if((m + 255) / 256 * cols >= enough) return 256;
-    if((m + 127) / 128 * cols >= enough) return 128;
-    return 64;
 }
 
 // K split of a dense launch (one panel): when the chosen tiles fill at most
@@ -386,43 +405,15 @@ hipError_t launch_gemm_decode(const GemmArgs& g, bool packed, void* ws, size_t w
     return hipSuccess;
 }
 
-hipError_t launch_gemm_packed(const GemmArgs& g, void* ws, size_t ws_bytes, hipStream_t stream)
-{
-    if(g.m == 0 || g.n == 0) return hipSuccess;
-    if(gemm_decode_ok(g)) return launch_gemm_decode(g, true, ws, ws_bytes, stream);
-    const size_t   esz    = g.out_type == W8A8_OUT_I32 ? 4 : 2;
-    const int      vec_ok = out_vec_ok(g);
-    constexpr size_t kLimit = 0x7FFFFFFFull;
-    const uint32_t mstep  = (uint32_t)std::min<size_t>(
-        g.m, std::max<size_t>(GemmPacked::kBM, kLimit / g.lda / GemmPacked::kBM * GemmPacked::kBM));
-    // the packed tile kernel's blocks cover 256 weight rows: keep panels aligned to that
-    const uint32_t nstep = std::max<uint32_t>(
-        GemmPacked::kBN, weight_panel_rows(g, true) / GemmPacked::kBN * GemmPacked::kBN);
-    for(uint32_t m0 = 0; m0 < g.m; m0 += mstep) {
-        for(uint32_t n0 = 0; n0 < g.n; n0 += nstep) {
-            KArgs p = n_panel(g, n0, std::min(nstep, g.n - n0), true);
-            p.m     = std::min(mstep, g.m - m0);
-            p.a     = g.a + (size_t)m0 * g.lda;
-            p.c     = static_cast<int8_t*>(p.c) + (size_t)m0 * g.ldc * esz;
-            p.sa    = g.scale_a ? g.scale_a + m0 : nullptr;
-            hipError_t e;
-            switch(pick_packed_cfg(p.m, p.n)) {
-            case 256: e = gemm::launch_pb<GemmPacked>(p, g.out_type, vec_ok, stream); break;
-            case 128: e = gemm::launch_pb<GemmPacked128>(p, g.out_type, vec_ok, stream); break;
-            default: e = gemm::launch_pb<GemmPacked64>(p, g.out_type, vec_ok, stream); break;
-            }
-            if(e != hipSuccess) return e;
-        }
-    }
-    return hipSuccess;
-}
-
 size_t packed_weight_bytes(uint32_t n, uint32_t k) { return gemm::packed_bytes(n, k); }
 
 hipError_t launch_pack_weights(const int8_t* w, uint32_t n, uint32_t k, uint32_t ldw,
                                int8_t* packed, hipStream_t stream)
 {
-    return gemm::launch_pack_weights(w, n, k, ldw, packed, stream);
+    const size_t chunks = gemm::packed_bytes(n, k) / 16;
+    hipLaunchKernelGGL(pack_weights_kernel, dim3((chunks + 255) / 256), dim3(256), 0, stream, w, n,
+                       k, ldw, packed, chunks);
+    return hipGetLastError();
 }
 
 bool gemm_fast_path_ok(const GemmArgs& g)
@@ -442,7 +433,7 @@ bool gemm_packed_ok(const GemmArgs& g)
     if(reinterpret_cast<uintptr_t>(g.a) % 16 != 0 || g.lda % 16 != 0 || g.k % 16 != 0) return false;
     // one packed k-row of a 64-row slab must fit in 2 GiB
     if((uint64_t)gemm::packed_ktiles(g.k) * gemm::kPackFrags * 1024 > kLimit) return false;
-    return g.m <= kDecodeMaxM ? gemm_decode_ok(g) : (uint64_t)g.lda * GemmPacked::kBM <= kLimit;
+    return g.m <= kDecodeMaxM ? gemm_decode_ok(g) : (uint64_t)g.lda * GemmMain::kBM <= kLimit;
 }
 
 // Row-major weights at m <= 64: the decode kernel streams 32-row weight
@@ -465,16 +456,25 @@ bool tiles_beat_decode(const GemmArgs& g, void* ws, size_t ws_bytes)
 // per tile (workgroup launch, cold prologue, store burst), which pays where
 // tiles are short: 2-4% at M=8192 K=4096 N=28672, 10-20% at K <= 1024,
 // nothing measurable at K=14336 with two tiles per CU.
+template <class C>
 bool persist_pays(const KArgs& p, int out_type, int vec_ok)
 {
-    return out_type == W8A8_OUT_F16 && (p.k + GemmMain::kBK - 1) / GemmMain::kBK <= 32
-           && gemm::persist_ok<GemmMain>(p, vec_ok, device_cus());
+    return out_type == W8A8_OUT_F16 && (p.k + C::kBK - 1) / C::kBK <= 32
+           && gemm::persist_ok<C>(p, vec_ok, device_cus());
 }
 
 size_t gemm_nk_workspace_bytes(const GemmArgs& g)
 {
     if(g.m == 0 || g.n == 0 || g.k == 0) return 0;
     return dense_split(g.m, g.n, g.k).bytes;
+}
+
+// The weights of rows [n0, ...) of a panel (packed: n0 a multiple of the slab).
+template <bool PB>
+const int8_t* weight_rows(const KArgs& p, uint32_t n0)
+{
+    return PB ? p.b + (size_t)(n0 / gemm::kSlab) * gemm::packed_ktiles(p.k) * gemm::kPackFrags * 1024
+              : p.b + (size_t)n0 * p.ldb;
 }
 
 // One 256 x 256 launch (a panel).  When its tiles make whole rounds over the
@@ -485,41 +485,47 @@ size_t gemm_nk_workspace_bytes(const GemmArgs& g)
 // 8 x 112 tiles = 3 rounds + 128 tiles; the last 16 columns become one
 // round of 256 tiles of 128 x 256).  The same k-order per output, so the
 // result is bit-identical to the single launch.
+template <bool PB>
 hipError_t launch_main(const KArgs& p, int out_type, int vec_ok, hipStream_t stream)
 {
+    using Main           = typename Tiles<PB>::Main;
+    using MidM           = typename Tiles<PB>::MidM;
     const uint32_t cus   = device_cus();
-    const uint32_t tm    = (p.m + GemmMain::kBM - 1) / GemmMain::kBM;
-    const uint32_t tiles = tm * ((p.n + GemmMain::kBN - 1) / GemmMain::kBN);
+    const uint32_t tm    = (p.m + Main::kBM - 1) / Main::kBM;
+    const uint32_t tiles = tm * ((p.n + Main::kBN - 1) / Main::kBN);
     const uint32_t full = tiles / cus, rest = tiles % cus;
-    const uint32_t mid_rows = (p.m + GemmMidM::kBM - 1) / GemmMidM::kBM;
+    const uint32_t mid_rows = (p.m + MidM::kBM - 1) / MidM::kBM;
+    auto whole = [&](const KArgs& q) {
+        return persist_pays<Main>(q, out_type, vec_ok)
+                   ? gemm::launch_cfg_persist<Main>(q, vec_ok, cus, stream)
+                   : gemm::launch_cfg<Main>(q, out_type, vec_ok, stream);
+    };
     if(full >= 1 && rest > 0 && rest * 2 <= cus && (full * cus) % tm == 0) {
-        const uint32_t n1   = full * cus / tm * GemmMain::kBN; // < p.n: rest > 0
+        const uint32_t n1   = full * cus / tm * Main::kBN; // < p.n: rest > 0
         const uint32_t n2   = p.n - n1;
         const size_t   esz  = out_type == W8A8_OUT_I32 ? 4 : 2;
-        if((uint64_t)mid_rows * ((n2 + GemmMidM::kBN - 1) / GemmMidM::kBN) <= cus) {
+        if((uint64_t)mid_rows * ((n2 + MidM::kBN - 1) / MidM::kBN) <= cus) {
             KArgs head = p, tail = p;
             head.n     = n1;
             tail.n     = n2;
-            tail.b     = p.b + (size_t)n1 * p.ldb;
+            tail.b     = weight_rows<PB>(p, n1);
             tail.c     = static_cast<int8_t*>(p.c) + (size_t)n1 * esz;
             tail.sb    = p.sb ? p.sb + n1 : nullptr;
-            hipError_t e = persist_pays(head, out_type, vec_ok)
-                               ? gemm::launch_cfg_persist<GemmMain>(head, vec_ok, cus, stream)
-                               : gemm::launch_cfg<GemmMain>(head, out_type, vec_ok, stream);
+            hipError_t e = whole(head);
             if(e != hipSuccess) return e;
-            return gemm::launch_cfg<GemmMidM>(tail, out_type, vec_ok, stream);
+            return gemm::launch_cfg<MidM>(tail, out_type, vec_ok, stream);
         }
     }
-    return persist_pays(p, out_type, vec_ok)
-               ? gemm::launch_cfg_persist<GemmMain>(p, vec_ok, cus, stream)
-               : gemm::launch_cfg<GemmMain>(p, out_type, vec_ok, stream);
+    return whole(p);
 }
 
-hipError_t launch_gemm_nk(const GemmArgs& g, void* ws, size_t ws_bytes, hipStream_t stream)
+// The tile kernels over a whole problem, row-major (PB = false) or packed
+// weights: one K-split launch where dense_split says so and the workspace
+// holds it, else row and column panels.
+template <bool PB>
+hipError_t launch_tiles(const GemmArgs& g, void* ws, size_t ws_bytes, hipStream_t stream)
 {
-    if(g.m == 0 || g.n == 0) return hipSuccess;
-    if(gemm_decode_ok(g) && !tiles_beat_decode(g, ws, ws_bytes))
-        return launch_gemm_decode(g, false, nullptr, 0, stream);
+    using T             = Tiles<PB>;
     const size_t esz    = g.out_type == W8A8_OUT_I32 ? 4 : 2;
     const int    vec_ok = out_vec_ok(g);
     // The tile kernel addresses each operand through a buffer resource whose
@@ -528,8 +534,10 @@ hipError_t launch_gemm_nk(const GemmArgs& g, void* ws, size_t ws_bytes, hipStrea
     constexpr size_t kLimit = 0x7FFFFFFFull;
     const uint32_t   mstep  = (uint32_t)std::min<size_t>(
         g.m, std::max<size_t>(GemmMain::kBM, kLimit / g.lda / GemmMain::kBM * GemmMain::kBM));
+    // weight rows under 2 GiB: ldb bytes a row, or packed rows of whole k-tiles
+    const size_t   row   = PB ? (size_t)gemm::packed_ktiles(g.k) * gemm::kPackK : g.ldb;
     const uint32_t nstep = (uint32_t)std::min<size_t>(
-        g.n, std::max<size_t>(GemmMain::kBN, kLimit / g.ldb / GemmMain::kBN * GemmMain::kBN));
+        g.n, std::max<size_t>(GemmMain::kBN, kLimit / row / GemmMain::kBN * GemmMain::kBN));
     if(ws != nullptr && mstep == g.m && nstep == g.n) {
         const DenseSplit d = dense_split(g.m, g.n, g.k);
         if(d.parts > 1 && ws_bytes >= d.bytes) {
@@ -537,14 +545,14 @@ hipError_t launch_gemm_nk(const GemmArgs& g, void* ws, size_t ws_bytes, hipStrea
             int32_t*    pw = static_cast<int32_t*>(ws);
             switch(d.cfg) {
             case TileCfg::kMain:
-                return gemm::launch_cfg_split<GemmMain>(p, g.out_type, vec_ok, pw, d.parts, stream);
+                return gemm::launch_cfg_split<typename T::Main>(p, g.out_type, vec_ok, pw, d.parts, stream);
             case TileCfg::kMidM:
-                return gemm::launch_cfg_split<GemmMidM>(p, g.out_type, vec_ok, pw, d.parts, stream);
+                return gemm::launch_cfg_split<typename T::MidM>(p, g.out_type, vec_ok, pw, d.parts, stream);
             case TileCfg::kSmall:
-                return gemm::launch_cfg_split<GemmSmall>(p, g.out_type, vec_ok, pw, d.parts, stream);
+                return gemm::launch_cfg_split<typename T::Small>(p, g.out_type, vec_ok, pw, d.parts, stream);
             default:
-                return gemm::launch_cfg_split<GemmDecTile>(p, g.out_type, vec_ok, pw, d.parts,
-                                                           stream);
+                return gemm::launch_cfg_split<typename T::Dec>(p, g.out_type, vec_ok, pw, d.parts,
+                                                               stream);
             }
         }
     }
@@ -554,21 +562,46 @@ hipError_t launch_gemm_nk(const GemmArgs& g, void* ws, size_t ws_bytes, hipStrea
             p.m     = std::min(mstep, g.m - m0);
             p.n     = std::min(nstep, g.n - n0);
             p.a     = g.a + (size_t)m0 * g.lda;
-            p.b     = g.b + (size_t)n0 * g.ldb;
+            p.b     = weight_rows<PB>(p, n0);
             p.c     = static_cast<int8_t*>(g.c) + ((size_t)m0 * g.ldc + n0) * esz;
             p.sa    = g.scale_a ? g.scale_a + m0 : nullptr;
             p.sb    = g.scale_b ? g.scale_b + n0 : nullptr;
             hipError_t e;
             switch(pick_tile_cfg(p.m, p.n)) {
-            case TileCfg::kMain: e = launch_main(p, g.out_type, vec_ok, stream); break;
-            case TileCfg::kMidM: e = gemm::launch_cfg<GemmMidM>(p, g.out_type, vec_ok, stream); break;
-            case TileCfg::kSmall: e = gemm::launch_cfg<GemmSmall>(p, g.out_type, vec_ok, stream); break;
-            default: e = gemm::launch_cfg<GemmDecTile>(p, g.out_type, vec_ok, stream); break;
+            case TileCfg::kMain: e = launch_main<PB>(p, g.out_type, vec_ok, stream); break;
+            case TileCfg::kMidM:
+                e = gemm::launch_cfg<typename T::MidM>(p, g.out_type, vec_ok, stream);
+                break;
+            case TileCfg::kSmall:
+                e = gemm::launch_cfg<typename T::Small>(p, g.out_type, vec_ok, stream);
+                break;
+            default: e = gemm::launch_cfg<typename T::Dec>(p, g.out_type, vec_ok, stream); break;
             }
             if(e != hipSuccess) return e;
         }
     }
     return hipSuccess;
+}
+
+hipError_t launch_gemm_nk(const GemmArgs& g, void* ws, size_t ws_bytes, hipStream_t stream)
+{
+    if(g.m == 0 || g.n == 0) return hipSuccess;
+    if(gemm_decode_ok(g) && !tiles_beat_decode(g, ws, ws_bytes))
+        return launch_gemm_decode(g, false, nullptr, 0, stream);
+    return launch_tiles<false>(g, ws, ws_bytes, stream);
+}
+
+// Packed weights: m <= 64 streams them through the decode kernels; larger m
+// runs the row-major GEMM's tile kernels and rules over the packed layout.
+// (A kernel that loaded B fragments straight to registers, 32 x 32 x 32 MFMA,
+// no K split, was 5-10% slower at M = 8192 and far behind below: 300 x 6144 x
+// 4096 24.0 -> 18.5 us, 1000 x 1024 x 26576 120 -> 94 us, 322 x 566 x 3936
+// 50 -> 20 us, where it also cut N into two launches.)
+hipError_t launch_gemm_packed(const GemmArgs& g, void* ws, size_t ws_bytes, hipStream_t stream)
+{
+    if(g.m == 0 || g.n == 0) return hipSuccess;
+    if(gemm_decode_ok(g)) return launch_gemm_decode(g, true, ws, ws_bytes, stream);
+    return launch_tiles<true>(g, ws, ws_bytes, stream);
 }
 
 namespace {

@@ -1,6 +1,6 @@
 // gemm_i8_decode_kernel.hpp -- skinny (decode) int8 GEMM for gfx950:
 // M <= 64 tokens, HBM-bound weight streaming, over plain [N, K] weights or
-// weights packed in MFMA register order (gemm_i8_pb_kernel.hpp).
+// weights packed in MFMA register order (gemm_i8_pack.hpp).
 //
 // Computation: acc[m,n] = sum_k A[m,k] * W[n,k]; C = half((acc * sa[m]) * sb[n])
 // (the split-K decode role of gemm_splitk_stage1 + gemm_splitk_reduce,
@@ -23,7 +23,7 @@
 //     wave w then sums fragments w, w+KW, ... and runs the dequant epilogue.
 #pragma once
 
-#include "gemm_i8_pb_kernel.hpp"
+#include "gemm_i8_kernel.hpp"
 
 namespace w8a8 {
 namespace gemm {

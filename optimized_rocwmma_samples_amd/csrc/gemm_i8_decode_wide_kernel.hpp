@@ -20,7 +20,7 @@
 // wave has finished reading stage t-1, which the refill then overwrites.
 #pragma once
 
-#include "gemm_i8_pb_kernel.hpp"
+#include "gemm_i8_kernel.hpp"
 
 namespace w8a8 {
 namespace gemm {

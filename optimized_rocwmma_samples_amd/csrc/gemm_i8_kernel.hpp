@@ -41,6 +41,7 @@
 #pragma once
 
 #include "../../include/w8a8.h"
+#include "gemm_i8_pack.hpp"
 #include "w8a8_device.hpp"
 
 #include <mutex>
@@ -57,8 +58,13 @@ namespace gemm {
 // operands (3.60 against 3.16 POP/s in a loop fed from LDS like the tile
 // body; plausibly because it reads and writes half the accumulator bytes per
 // op).
+// PACKB_: B is the packed weight buffer (gemm_i8_pack.hpp; KArgs::ldb unused)
+// instead of rows of K bytes.  Its 8 KiB (slab, k-tile) blocks go to LDS as
+// they are, 1 KiB contiguous per wave-load, and the fragments are read from
+// that order (FragReader); everything else of the tile is the same, and so
+// are the sums.
 template <int BM_, int BN_, int BK_, int STAGES_, int WAVES_M_, int WAVES_N_, int GROUP_M_ = 8,
-          int MFMA_ = 32>
+          int MFMA_ = 32, bool PACKB_ = false>
 struct Cfg {
     static constexpr int kBM      = BM_;
     static constexpr int kBN      = BN_;
@@ -72,6 +78,7 @@ struct Cfg {
     static constexpr int kWaveM   = kBM / kWavesM;
     static constexpr int kWaveN   = kBN / kWavesN;
     static constexpr int kMfma    = MFMA_;
+    static constexpr bool kPackB  = PACKB_;
     static constexpr int kTilesM  = kWaveM / kMfma;      // MFMA blocks per wave tile
     static constexpr int kTilesN  = kWaveN / kMfma;
     static constexpr int kChunks  = kBK / 16;           // 16-byte chunks per LDS row
@@ -94,6 +101,8 @@ struct Cfg {
     static_assert(kLoadsA * kWaves * 1024 == kABytes && kLoadsB * kWaves * 1024 == kBBytes,
                   "tile bytes must split evenly into 1 KiB wave-loads");
     static_assert(kMfma == 32 || kMfma == 16, "32x32x32 or 16x16x64 MFMA");
+    static_assert(!kPackB || (kMfma == 16 && kBK == kPackK && kBN % kSlab == 0),
+                  "packed B: the 16x16x64 form over whole slabs and packed k-tiles");
     static_assert(kBK % kMfmaK == 0, "whole MFMA k-groups per tile");
     static_assert(kWaveM % 32 == 0 && kWaveN % 32 == 0, "wave tile of whole 32-row passes");
     static_assert(kStages >= 2, "at least double buffering");
@@ -285,6 +294,25 @@ struct Acc {
     }
 };
 
+// The global -> LDS loads of the packed B operand: wave-load j of a tile's B
+// stage copies fragment j % 8 of slab n0 / 64 + j / 8, lane l its bytes
+// [16 l, 16 l + 16).  k-tile kt adds kt * 8 KiB (the uniform soffset).  A slab
+// past N gets kOob; the packed padding makes a K tail zeros.
+__device__ __forceinline__ uint32_t packed_b_offset(const KArgs& p, uint32_t n0, int j, int lane)
+{
+    const uint32_t slab = n0 / kSlab + j / kPackFrags;
+    return slab < packed_slabs(p.n)
+               ? (slab * packed_ktiles(p.k) * kPackFrags + j % kPackFrags) * 1024u + lane * 16
+               : kOob;
+}
+
+// Bytes of the B operand a buffer resource covers.
+template <class C>
+__device__ __forceinline__ int b_bytes(const KArgs& p)
+{
+    return C::kPackB ? (int)packed_bytes(p.n, p.k) : (int)(p.n * p.ldb);
+}
+
 // LDS -> register fragments of one k-group.  Fragment t of A covers wave-tile
 // rows [t kMfma, (t + 1) kMfma): lane l reads row t kMfma + l % kMfma, 16
 // bytes at k-chunk (kMfmaK / 16) g + l / kMfma of the k-tile, i.e. the
@@ -298,6 +326,7 @@ struct FragReader {
     using FragB = v4i[C::kTilesN];
     int offa, offb;       // byte offsets of fragment 0 within a stage
     int cofs[C::kSubK];   // byte offset of each k-group's chunk
+    int cofb;             // packed B: byte offset of k-group 0's chunk
 
     __device__ __forceinline__ FragReader(int wm, int wn, int lane)
     {
@@ -305,6 +334,9 @@ struct FragReader {
         const int fswz = (frow >> C::kSwzShift) & (C::kChunks - 1);
         offa           = (wm * C::kWaveM + frow) * C::kBK;
         offb           = C::kABytes + (wn * C::kWaveN + frow) * C::kBK;
+        // packed B: half slabs of 32 rows x 128 k as [chunk][row] (4 KiB)
+        if constexpr(C::kPackB) offb = C::kABytes + wn * C::kWaveN * C::kBK + frow * 16;
+        cofb = lane / C::kMfma * 512;
         constexpr int kPerG = C::kMfmaK / 16; // 16-byte k-chunks per lane group and k-group
 #pragma unroll
         for(int g = 0; g < C::kSubK; ++g)
@@ -316,6 +348,9 @@ struct FragReader {
     }
     __device__ __forceinline__ v4i b(const int8_t* sbase, int g, int t) const
     {
+        if constexpr(C::kPackB)
+            return *reinterpret_cast<const v4i*>(sbase + offb + (t / 2) * 4096 + (t % 2) * 256
+                                                 + g * (C::kMfmaK / 16 * 512) + cofb);
         return *reinterpret_cast<const v4i*>(sbase + offb + t * C::kMfma * C::kBK + cofs[g]);
     }
     __device__ __forceinline__ void load(const int8_t* sbase, int g, FragA& af, FragB& bf) const
@@ -737,11 +772,12 @@ __device__ __forceinline__ void gemm_tile_acc(const KArgs& p, uint32_t m0, uint3
         const uint32_t r = (wave * C::kLoadsB + i) * C::kRowsPerLoad + lrow;
         chb[i]           = (lane % C::kChunks) ^ ((r >> C::kSwzShift) & (C::kChunks - 1));
         vb[i]            = (n0 + r) < p.n ? (n0 + r) * p.ldb + chb[i] * 16 : kOob;
+        if constexpr(C::kPackB) vb[i] = packed_b_offset(p, n0, wave * C::kLoadsB + i, lane);
     }
     const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<int8_t*>(p.a), 0, (int)(p.m * p.lda), kBufferFlags);
     const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<int8_t*>(p.b), 0, (int)(p.n * p.ldb), kBufferFlags);
+        const_cast<int8_t*>(p.b), 0, b_bytes<C>(p), kBufferFlags);
     const uint32_t lds0 = (uint32_t)(uintptr_t)lds; // LDS byte address of the ring
 
     auto issue_stage = [&](int stage, uint32_t kt) {
@@ -758,9 +794,12 @@ __device__ __forceinline__ void gemm_tile_acc(const KArgs& p, uint32_t m0, uint3
         }
 #pragma unroll
         for(int i = 0; i < C::kLoadsB; ++i) {
-            const uint32_t v = (full_k || k0 + chb[i] * 16 < p.k) ? vb[i] : kOob;
+            // packed: whole k-tiles (zero padded), 8 KiB apart
+            const bool     live = C::kPackB ? k0 < p.k : (full_k || k0 + chb[i] * 16 < p.k);
+            const uint32_t so   = C::kPackB ? (live ? k0 * (kPackFrags * 1024 / kPackK) : 0u) : k0;
+            const uint32_t v    = live ? vb[i] : kOob;
             __builtin_amdgcn_raw_ptr_buffer_load_lds(
-                rb, (lds_void_t*)(uintptr_t)(sbaseb + i * 1024), 16, v, k0, 0, 0);
+                rb, (lds_void_t*)(uintptr_t)(sbaseb + i * 1024), 16, v, so, 0, 0);
         }
     };
 

@@ -176,7 +176,7 @@ __global__ void __launch_bounds__(C::kThreads, 1) gemm_i8_persist_kernel(KArgs p
     const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<int8_t*>(p.a), 0, (int)(p.m * p.lda), kBufferFlags);
     const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<int8_t*>(p.b), 0, (int)(p.n * p.ldb), kBufferFlags);
+        const_cast<int8_t*>(p.b), 0, b_bytes<C>(p), kBufferFlags);
     const __amdgpu_buffer_rsrc_t rc = __builtin_amdgcn_make_buffer_rsrc(
         p.c, 0, (int)(((p.m - 1) * p.ldc + p.n) * 2), kBufferFlags);
     const uint32_t lds0 = (uint32_t)(uintptr_t)lds;
@@ -200,6 +200,8 @@ __global__ void __launch_bounds__(C::kThreads, 1) gemm_i8_persist_kernel(KArgs p
         for(int i = 0; i < C::kLoadsB; ++i) {
             const uint32_t r = rowB(i);
             vb[i] = (live && n0 + r < p.n) ? (n0 + r) * p.ldb + chunk_of(r) * 16 : kOob;
+            if constexpr(C::kPackB)
+                vb[i] = live ? packed_b_offset(p, n0, wave * C::kLoadsB + i, lane) : kOob;
         }
     };
     set_load_tile(0);
@@ -217,9 +219,12 @@ __global__ void __launch_bounds__(C::kThreads, 1) gemm_i8_persist_kernel(KArgs p
         }
 #pragma unroll
         for(int i = 0; i < C::kLoadsB; ++i) {
-            const uint32_t v = (full_k || k0 + chunk_of(rowB(i)) * 16 < p.k) ? vb[i] : kOob;
+            // packed: whole k-tiles (zero padded), 8 KiB apart
+            const bool     live = C::kPackB || full_k || k0 + chunk_of(rowB(i)) * 16 < p.k;
+            const uint32_t so   = C::kPackB ? lkt * (kPackFrags * 1024) : k0;
+            const uint32_t v    = live ? vb[i] : kOob;
             __builtin_amdgcn_raw_ptr_buffer_load_lds(
-                rb, (lds_void_t*)(uintptr_t)(sbaseb + i * 1024), 16, v, k0, 0, 0);
+                rb, (lds_void_t*)(uintptr_t)(sbaseb + i * 1024), 16, v, so, 0, 0);
         }
         if(++lkt == nk) {
             lkt = 0;

@@ -102,6 +102,26 @@ def test_packed_block_heights_exact(w8a8, gpu, m, n, k):
     assert_f16_bitexact(host(c), O.dequant_f16(acc, sa, sb))
 
 
+# The tile kernels over packed weights: the persistent kernel (17 x 33 tiles,
+# partial last slab, K tail of 32), the last round's columns as 128 x 256 tiles,
+# one k-tile, and the K split with a partial last slab and K tail.
+@pytest.mark.parametrize("m,n,k", [(4100, 8200, 160), (2048, 11000, 144), (4100, 8200, 16),
+                                   (300, 600, 8208)])
+def test_packed_tile_kernels_match_row_major(w8a8, gpu, m, n, k):
+    import torch
+    a, b, sa, sb = inputs(m, n, k, 5 * m + n + k)
+    ad, bd, sad, sbd = dev(a, gpu), dev(b, gpu), dev(sa, gpu), dev(sb, gpu)
+    pw = w8a8.pack_weights(bd)
+    ws = torch.empty(w8a8.gemm_workspace_size(m, n, k), dtype=torch.uint8, device=gpu)
+    for w in (ws, None):
+        c = w8a8.gemm_packed(ad, pw, sad, sbd, workspace=w)
+        assert np.array_equal(host(c).view(np.uint16),
+                              host(w8a8.gemm(ad, bd, sad, sbd)).view(np.uint16))
+    rows = np.unique(np.r_[0:8, m - 8:m, m // 2:m // 2 + 8])
+    acc = O.gemm_i32(a[rows], b)
+    assert_f16_bitexact(host(c)[rows], O.dequant_f16(acc, sa[rows], sb))
+
+
 @pytest.mark.parametrize("packed", [False, True])
 @pytest.mark.parametrize("m", [1, 24, 64])
 def test_decode_f16_modes(w8a8, gpu, packed, m):
