@@ -320,7 +320,9 @@ int w8a8_gemm_noalloc(uint32_t m, uint32_t n, uint32_t k, const int8_t* a, const
     const char* fn = "w8a8_gemm_noalloc";
     int         rc = validate_gemm(fn, m, n, k, a, b, c, lda, ldb, ldc, out_type, layout);
     if(rc != W8A8_SUCCESS) return rc;
-    const size_t need = w8a8_gemm_workspace_size(m, n, k, layout);
+    // the repack needs its room; the primary layout's K split takes a plan that fits
+    const size_t need
+        = layout == W8A8_LAYOUT_A_ROW_B_NK ? 0 : w8a8_gemm_workspace_size(m, n, k, layout);
     if(need > W8A8_NOALLOC_SCRATCH_BYTES)
         return fail(W8A8_ERROR_INVALID_VALUE,
                     "%s: m=%u n=%u k=%u needs %zu bytes of scratch, the library holds %zu per GPU "

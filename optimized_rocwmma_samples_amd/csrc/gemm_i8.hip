@@ -29,23 +29,25 @@ using gemm::KArgs;
 // cold weights, cfg3 projections: M = 8192 1448 -> 1389 µs, M = 2048 411 ->
 // 398 µs, M = 512 144 -> 132 µs (sum of the four).
 // PB: over packed weights.
-// 3 LDS stages in the smaller two: these launches have few tiles per CU and
+// 3 LDS stages in the next two: these launches have few tiles per CU and
 // read their panels from HBM, where a third k-tile in flight hides the latency
 // (cold weights, M = 512: 128 x 128 o_proj 32 -> 22 µs, down 100 -> 66 µs;
 // M = 2048, 128 x 256: o_proj 47 -> 40 µs, down 146 -> 116 µs).
+// The last three are short enough that a CU holds two or three blocks, whose
+// barriers and waits then overlap: what a launch of few or short tiles lacks
+// (plan_tiles says where each wins).
 template <bool PB>
 struct Tiles {
-    using Main  = gemm::Cfg<256, 256, 128, 2, 2, 4, 4, 16, PB>;
-    using MidM  = gemm::Cfg<128, 256, 128, 3, 2, 4, 4, 16, PB>; // 8 waves of 64 x 64, 144 KiB LDS
-    using Small = gemm::Cfg<128, 128, 128, 3, 2, 4, 4, 16, PB>; // 8 waves of 64 x 32, 96 KiB LDS
-    // m <= 64 (row-major weights: tiles_beat_decode): 4 waves of 64 x 32,
-    // 4 stages (96 KiB LDS), one tile row.
-    using Dec   = gemm::Cfg<64, 128, 128, 4, 1, 4, 1, 16, PB>;
+    using Main   = gemm::Cfg<256, 256, 128, 2, 2, 4, 4, 16, PB>;
+    using MidM   = gemm::Cfg<128, 256, 128, 3, 2, 4, 4, 16, PB>; // 8 waves of 64 x 64, 144 KiB LDS
+    using Small  = gemm::Cfg<128, 128, 128, 3, 2, 4, 4, 16, PB>; // 8 waves of 64 x 32, 96 KiB LDS
+    using Narrow = gemm::Cfg<64, 128, 128, 3, 2, 4, 4, 16, PB>;  // 8 waves of 32 x 32, 72 KiB LDS
+    using Tiny   = gemm::Cfg<64, 64, 128, 4, 2, 2, 4, 16, PB>;   // 4 waves of 32 x 32, 64 KiB LDS
+    using Row    = gemm::Cfg<32, 64, 128, 4, 1, 2, 4, 16, PB>;   // 2 waves of 32 x 32, 48 KiB LDS
 };
 using GemmMain    = Tiles<false>::Main;
 using GemmMidM    = Tiles<false>::MidM;
 using GemmSmall   = Tiles<false>::Small;
-using GemmDecTile = Tiles<false>::Dec;
 // Decode configurations: <32-row m tiles, 32-row weight tiles, waves, ring>.
 using DecSmall   = gemm::DecCfg<1, 1, 4, 3>; // m <= 32, or <= 16 packed
 using DecSmallW  = gemm::DecCfg<1, 2, 8, 3>; // packed, 8 <= m <= 32, many slabs
@@ -224,58 +226,155 @@ uint32_t device_cus()
     return cus;
 }
 
-// Tile configuration of one launch.  256 x 256 tiles have the best per-op
-// rate once they fill the chip; a launch with fewer than 3/4 of a round of
-// them leaves most CUs idle, and smaller tiles finish it sooner (measured
-// on MI355X, cfg3 shapes: M = 512 qkv 46 -> 25 µs, o_proj 45 -> 22 µs,
-// down 140 -> 71 µs with 128 x 128; M = 2048 o_proj 59 -> 42 µs, down
-// 164 -> 119 µs with 128 x 256; the shapes with enough 256 x 256 tiles, e.g.
-// M = 2048 qkv or gate_up, are slower with smaller ones).
-enum class TileCfg { kMain, kMidM, kSmall, kDecode };
+// ---------------------------------------------------------------------------
+// Plan of one tile launch: the configuration and the number of K pieces.
+// ---------------------------------------------------------------------------
+enum class TileCfg { kMain, kMidM, kSmall, kNarrow, kTiny, kRow, kDecode };
 
-TileCfg pick_tile_cfg(uint32_t m, uint32_t n)
-{
-    if(m <= kDecodeMaxM) return TileCfg::kDecode;
-    auto tiles = [&](uint32_t bm, uint32_t bn) {
-        return (uint64_t)((m + bm - 1) / bm) * ((n + bn - 1) / bn);
-    };
-    const uint64_t enough = (uint64_t)device_cus() * 3 / 4;
-    if(tiles(GemmMain::kBM, GemmMain::kBN) >= enough) return TileCfg::kMain;
-    if(tiles(GemmMidM::kBM, GemmMidM::kBN) >= enough) return TileCfg::kMidM;
-    return TileCfg::kSmall;
-}
-
-// K split of a dense launch (one panel): when the chosen tiles fill at most
-// half of the CUs, each tile runs as `parts` K pieces on otherwise idle CUs
-// (gemm_i8_split_kernel + fixup).  parts = 1: no split.
-struct DenseSplit {
-    TileCfg  cfg;
-    uint32_t tiles, parts;
-    size_t   bytes; // workspace the split needs
+struct TilePlan {
+    TileCfg cfg;
+    uint32_t parts; // K pieces per tile (gemm_i8_split_kernel + fixup when > 1)
+    size_t   bytes; // int32 partials of the pieces
 };
 
-DenseSplit dense_split(uint32_t m, uint32_t n, uint32_t k)
+// Time of a launch in µs, fitted per configuration to 1000-odd launches of
+// random sizes (m 1-4096, n 64-28672, k 512-28672, weights cold or in the
+// MALL; median error 3-6%):
+//   fixed + sum over a CU's blocks of k-tiles x step[blocks resident together]
+//   + out_mb x output MB + w_mb x weight MB
+//   + (pieces > 1) (split + split_mb x partial MB)
+// with step x cross where row-major operands' rows cross 128-byte lines (K no
+// multiple of 128: every 128-byte row piece of a k-tile is then two requests).
+struct CfgCost {
+    TileCfg  cfg;
+    uint32_t bm, bn, resident; // resident: blocks a CU holds (LDS)
+    double   fixed, step[3], split, split_mb, out_mb, w_mb, cross;
+};
+constexpr CfgCost kCosts[] = {
+    {TileCfg::kMain, 256, 256, 1, 6.2, {1.19}, 6.5, 0.45, 0.27, 0.044, 1.06},
+    {TileCfg::kMidM, 128, 256, 1, 4.9, {0.71}, 4.7, 0.38, 0.34, 0.043, 1.25},
+    {TileCfg::kSmall, 128, 128, 1, 3.6, {0.42}, 3.8, 0.40, 0.40, 0.023, 1.25},
+    {TileCfg::kNarrow, 64, 128, 2, 3.2, {0.30, 0.63}, 3.7, 0.32, 0.23, 0.061, 1.40},
+    {TileCfg::kTiny, 64, 64, 2, 3.3, {0.24, 0.42}, 3.3, 0.47, 0.37, 0.030, 1.10},
+    {TileCfg::kRow, 32, 64, 3, 3.4, {0.23, 0.36, 0.59}, 3.0, 0.41, 0.0, 0.048, 1.02},
+};
+constexpr uint32_t kMinKtPlan    = 6;        // k-tiles of a K piece, at least
+constexpr size_t   kMaxPlanBytes = 64 << 20; // partials of a plan, at most
+// A split call launches twice, and the host needs about 3.5 µs a launch and
+// 4 µs around it: a GPU time below that is not seen (25 x 784 x 2944, split
+// 15.0 -> 19.8 µs a layer although its kernels take 2 µs less).
+constexpr double kSplitHostUs = 11.0;
+
+uint32_t ceil_div(uint32_t a, uint32_t b) { return (a + b - 1) / b; }
+
+double plan_cost(const CfgCost& c, uint32_t m, uint32_t n, uint32_t k, uint32_t parts, bool packed)
 {
-    DenseSplit d{pick_tile_cfg(m, n), 0, 1, 0};
-    uint32_t   bm = GemmMain::kBM, bn = GemmMain::kBN;
-    size_t     part_bytes = gemm::Partial<GemmMain>::kBytes;
-    if(d.cfg == TileCfg::kMidM) {
-        bm = GemmMidM::kBM, bn = GemmMidM::kBN, part_bytes = gemm::Partial<GemmMidM>::kBytes;
-    } else if(d.cfg == TileCfg::kSmall) {
-        bm = GemmSmall::kBM, bn = GemmSmall::kBN, part_bytes = gemm::Partial<GemmSmall>::kBytes;
-    } else if(d.cfg == TileCfg::kDecode) {
-        bm = GemmDecTile::kBM, bn = GemmDecTile::kBN,
-        part_bytes = gemm::Partial<GemmDecTile>::kBytes;
+    const uint32_t cus    = device_cus();
+    const uint32_t tm     = ceil_div(m, c.bm);
+    const uint64_t blocks = (uint64_t)tm * ceil_div(n, c.bn) * parts;
+    const double   steps  = ceil_div(ceil_div(k, 128), parts) * (packed || k % 128 == 0 ? 1.0 : c.cross);
+    uint64_t       per_cu = (blocks + cus - 1) / cus;
+    double         t      = c.fixed + 2e-6 * m * n * c.out_mb + 1e-6 * n * (double)k * c.w_mb;
+    // launch_main runs a last round of at most half the CUs as smaller tiles
+    if(c.cfg == TileCfg::kMain && per_cu > 1 && blocks % cus * 2 <= cus
+       && blocks / cus * cus % tm == 0) {
+        t += steps * kCosts[1].step[0];
+        --per_cu;
     }
-    d.tiles             = ((m + bm - 1) / bm) * ((n + bn - 1) / bn);
-    const uint32_t cus  = device_cus();
-    const uint32_t nk   = (k + 127) / 128;
-    if((uint64_t)d.tiles * 2 > cus) return d;
-    const uint32_t parts = std::min({cus / d.tiles, nk / gemm::kMinKtPerPart, gemm::kMaxParts});
-    if(parts < 2) return d;
-    d.parts = parts;
-    d.bytes = (size_t)d.tiles * parts * part_bytes;
-    return d;
+    t += steps * (per_cu / c.resident * c.step[c.resident - 1]
+                  + (per_cu % c.resident ? c.step[per_cu % c.resident - 1] : 0.0));
+    if(parts == 1) return t;
+    return std::max(t + c.split + 4e-6 * blocks * c.bm * c.bn * c.split_mb, kSplitHostUs);
+}
+
+// The row-major decode kernel (32 weight rows a block, its waves splitting K
+// inside the block): the fewest microseconds where the whole launch is a few
+// k-tiles per wave, e.g. 2 x 784 x 1472 5.3 µs against 6.2 for the best tiles.
+double decode_cost(uint32_t m, uint32_t n, uint32_t k)
+{
+    const double nk = ceil_div(k, 128), blocks = ceil_div(n, 32);
+    return 2.1 + nk * (0.29 * std::ceil(blocks / device_cus())
+                       + 0.11 * (m <= 32 ? 1 : 2) * blocks / device_cus());
+}
+
+// The plan of least estimated time among those whose partials fit ws_bytes.
+// 256 x 256 tiles where the persistent kernel may run them (two whole rounds,
+// K <= 4096) and from four rounds on; below that, what the launch lacks
+// decides: blocks, k-tiles per block or both.  m <= 64: row-major weights also have
+// the decode kernel.  Against the fixed rules this replaced (largest tile
+// that fills 3/4 of the CUs, K split when half of them idle): 128 x 4096 x
+// 4096 15.0 -> 11.4 µs, 512 x 4096 x 4096 20.0 -> 14.7, 226 x 384 x 12224
+// 17.3 -> 13.6, 24 x 16480 x 12672 113 -> 49, 1 x 19584 x 7680 71 -> 33; the
+// plan's time is within 2% of the best plan's on average.
+TilePlan search_plan(uint32_t m, uint32_t n, uint32_t k, size_t ws_bytes, bool decode, bool packed)
+{
+    TilePlan best{TileCfg::kMain, 1, 0};
+    if((uint64_t)ceil_div(m, 256) * ceil_div(n, 256) >= (k <= 4096 ? 2ull : 4ull) * device_cus())
+        return best;
+    double         cost = decode ? decode_cost(m, n, k) : 1e300;
+    const uint32_t most = std::min(gemm::kMaxParts, ceil_div(k, 128) / kMinKtPlan);
+    if(decode) best.cfg = TileCfg::kDecode;
+    for(const CfgCost& c : kCosts) {
+        // m <= 64 never fills taller tiles, larger m never needs shorter ones
+        if(m <= kDecodeMaxM ? c.bm > 64 : c.bm < 64) continue;
+        const uint64_t tiles = (uint64_t)ceil_div(m, c.bm) * ceil_div(n, c.bn);
+        for(uint32_t p = 1; p <= std::max(1u, most); ++p) {
+            const uint64_t bytes = p == 1 ? 0 : tiles * p * c.bm * c.bn * 4;
+            if(bytes > std::min(ws_bytes, kMaxPlanBytes)
+               || (p > 1 && tiles * p > (uint64_t)device_cus() * c.resident))
+                break;
+            const double t = plan_cost(c, m, n, k, p, packed);
+            if(t < cost) {
+                cost = t;
+                best = TilePlan{c.cfg, p, (size_t)bytes};
+            }
+        }
+    }
+    return best;
+}
+
+// search_plan, with the last plans of each host thread kept: a call asks for
+// its plan two or three times (the workspace size, the route, the launch) and
+// the search takes half a microsecond of a 4 µs call.
+TilePlan plan_tiles(uint32_t m, uint32_t n, uint32_t k, size_t ws_bytes, bool decode, bool packed)
+{
+    struct Entry {
+        uint32_t m = 0, n = 0, k = 0; // m = 0: empty
+        bool     decode = false, packed = false;
+        size_t   ws     = 0;
+        TilePlan plan{};
+    };
+    constexpr uint32_t        kEntries = 64;
+    static thread_local Entry seen[kEntries];
+    ws_bytes = std::min(ws_bytes, kMaxPlanBytes);
+    Entry& e = seen[(m * 31 + n * 17 + k * 7 + (ws_bytes != 0) * 4 + decode * 2 + packed)
+                    % kEntries];
+    if(e.m != m || e.n != n || e.k != k || e.decode != decode || e.packed != packed
+       || e.ws != ws_bytes)
+        e = Entry{m,      n,        k, decode, packed,
+                  ws_bytes, search_plan(m, n, k, ws_bytes, decode, packed)};
+    return e.plan;
+}
+
+// Bytes reported to callers at the least where a K split may run: the pieces
+// of 128-row tiles (64 x 128 below 65 rows) on the CUs that half a round of
+// them leaves idle.  A bound from the sizes alone, so that a workspace sized
+// once does not depend on the plan's fitted constants.
+size_t half_round_bytes(uint32_t m, uint32_t n, uint32_t k)
+{
+    const uint32_t cus = device_cus();
+    uint32_t       bm = 64, bn = 128;
+    if(m > kDecodeMaxM) {
+        auto few = [&] { return (uint64_t)ceil_div(m, bm) * ceil_div(n, bn) < cus * 3ull / 4; };
+        bm = bn = 256;
+        if(few()) bm = 128;
+        if(few()) bn = 128;
+    }
+    const uint64_t tiles = (uint64_t)ceil_div(m, bm) * ceil_div(n, bn);
+    if(tiles * 2 > cus) return 0;
+    const uint32_t parts = std::min({cus / (uint32_t)tiles,
+                                     ceil_div(k, 128) / gemm::kMinKtPerPart, gemm::kMaxParts});
+    return parts < 2 ? 0 : (size_t)tiles * parts * bm * bn * 4;
 }
 
 // K splits of the wide decode kernel for one weight panel: the count that
@@ -307,6 +406,7 @@ bool decode_wide_shape(const GemmArgs& g) { return g.m > 32 && g.m <= kDecodeMax
 
 size_t packed_workspace_bytes(const GemmArgs& g)
 {
+    if(g.m > kDecodeMaxM) return plan_tiles(g.m, g.n, g.k, kMaxPlanBytes, false, true).bytes;
     if(!decode_wide_shape(g) || !gemm_decode_ok(g)) return 0;
     const uint32_t step = weight_panel_rows(g, true);
     size_t         most = 0;
@@ -436,21 +536,6 @@ bool gemm_packed_ok(const GemmArgs& g)
     return g.m <= kDecodeMaxM ? gemm_decode_ok(g) : (uint64_t)g.lda * GemmMain::kBM <= kLimit;
 }
 
-// Row-major weights at m <= 64: the decode kernel streams 32-row weight
-// panels with 32-byte pieces per lane and re-reads all of A for every panel
-// (at m = 64 twice the weight bytes from L2); 64 x 128 tiles load each
-// weight tile once as whole 128-byte rows.  They take over when they fill
-// the chip by themselves, or with a K split when the caller gave the
-// workspace.  Cold weights, W [28672, 8192]: m = 1 61 -> 51 µs, m = 16
-// 72 -> 54 µs, m = 32 83 -> 54 µs, m = 64 96 -> 53 µs; W [8192, 28672]
-// has 64 tiles and needs the split.
-bool tiles_beat_decode(const GemmArgs& g, void* ws, size_t ws_bytes)
-{
-    const DenseSplit d = dense_split(g.m, g.n, g.k);
-    if(d.parts == 1) return d.tiles >= (uint64_t)device_cus() * 3 / 4;
-    return ws != nullptr && ws_bytes >= d.bytes;
-}
-
 // The persistent tile kernel for a 256 x 256 launch: fp16 output, at least
 // two tiles per CU and at most 32 k-tiles per tile.  It saves a fixed cost
 // per tile (workgroup launch, cold prologue, store burst), which pays where
@@ -466,7 +551,8 @@ bool persist_pays(const KArgs& p, int out_type, int vec_ok)
 size_t gemm_nk_workspace_bytes(const GemmArgs& g)
 {
     if(g.m == 0 || g.n == 0 || g.k == 0) return 0;
-    return dense_split(g.m, g.n, g.k).bytes;
+    const TilePlan p = plan_tiles(g.m, g.n, g.k, kMaxPlanBytes, g.m <= kDecodeMaxM, false);
+    return std::max(p.bytes, half_round_bytes(g.m, g.n, g.k));
 }
 
 // The weights of rows [n0, ...) of a panel (packed: n0 a multiple of the slab).
@@ -519,13 +605,36 @@ hipError_t launch_main(const KArgs& p, int out_type, int vec_ok, hipStream_t str
     return whole(p);
 }
 
+// One planned launch of a panel.
+template <bool PB>
+hipError_t launch_plan(const KArgs& p, const TilePlan& d, int out_type, int vec_ok, void* ws,
+                       hipStream_t stream)
+{
+    using T = Tiles<PB>;
+    auto go = [&](auto c) {
+        using C = decltype(c);
+        if(d.parts > 1)
+            return gemm::launch_cfg_split<C>(p, out_type, vec_ok, static_cast<int32_t*>(ws),
+                                             d.parts, stream);
+        return gemm::launch_cfg<C>(p, out_type, vec_ok, stream);
+    };
+    switch(d.cfg) {
+    case TileCfg::kMain:
+        return d.parts > 1 ? go(typename T::Main{})
+                           : launch_main<PB>(p, out_type, vec_ok, stream);
+    case TileCfg::kMidM: return go(typename T::MidM{});
+    case TileCfg::kSmall: return go(typename T::Small{});
+    case TileCfg::kNarrow: return go(typename T::Narrow{});
+    case TileCfg::kTiny: return go(typename T::Tiny{});
+    default: return go(typename T::Row{});
+    }
+}
+
 // The tile kernels over a whole problem, row-major (PB = false) or packed
-// weights: one K-split launch where dense_split says so and the workspace
-// holds it, else row and column panels.
+// weights, in row and column panels where an operand exceeds 2 GiB.
 template <bool PB>
 hipError_t launch_tiles(const GemmArgs& g, void* ws, size_t ws_bytes, hipStream_t stream)
 {
-    using T             = Tiles<PB>;
     const size_t esz    = g.out_type == W8A8_OUT_I32 ? 4 : 2;
     const int    vec_ok = out_vec_ok(g);
     // The tile kernel addresses each operand through a buffer resource whose
@@ -538,24 +647,6 @@ hipError_t launch_tiles(const GemmArgs& g, void* ws, size_t ws_bytes, hipStream_
     const size_t   row   = PB ? (size_t)gemm::packed_ktiles(g.k) * gemm::kPackK : g.ldb;
     const uint32_t nstep = (uint32_t)std::min<size_t>(
         g.n, std::max<size_t>(GemmMain::kBN, kLimit / row / GemmMain::kBN * GemmMain::kBN));
-    if(ws != nullptr && mstep == g.m && nstep == g.n) {
-        const DenseSplit d = dense_split(g.m, g.n, g.k);
-        if(d.parts > 1 && ws_bytes >= d.bytes) {
-            const KArgs p  = make_kargs(g);
-            int32_t*    pw = static_cast<int32_t*>(ws);
-            switch(d.cfg) {
-            case TileCfg::kMain:
-                return gemm::launch_cfg_split<typename T::Main>(p, g.out_type, vec_ok, pw, d.parts, stream);
-            case TileCfg::kMidM:
-                return gemm::launch_cfg_split<typename T::MidM>(p, g.out_type, vec_ok, pw, d.parts, stream);
-            case TileCfg::kSmall:
-                return gemm::launch_cfg_split<typename T::Small>(p, g.out_type, vec_ok, pw, d.parts, stream);
-            default:
-                return gemm::launch_cfg_split<typename T::Dec>(p, g.out_type, vec_ok, pw, d.parts,
-                                                               stream);
-            }
-        }
-    }
     for(uint32_t m0 = 0; m0 < g.m; m0 += mstep) {
         for(uint32_t n0 = 0; n0 < g.n; n0 += nstep) {
             KArgs p = make_kargs(g);
@@ -566,17 +657,9 @@ hipError_t launch_tiles(const GemmArgs& g, void* ws, size_t ws_bytes, hipStream_
             p.c     = static_cast<int8_t*>(g.c) + ((size_t)m0 * g.ldc + n0) * esz;
             p.sa    = g.scale_a ? g.scale_a + m0 : nullptr;
             p.sb    = g.scale_b ? g.scale_b + n0 : nullptr;
-            hipError_t e;
-            switch(pick_tile_cfg(p.m, p.n)) {
-            case TileCfg::kMain: e = launch_main<PB>(p, g.out_type, vec_ok, stream); break;
-            case TileCfg::kMidM:
-                e = gemm::launch_cfg<typename T::MidM>(p, g.out_type, vec_ok, stream);
-                break;
-            case TileCfg::kSmall:
-                e = gemm::launch_cfg<typename T::Small>(p, g.out_type, vec_ok, stream);
-                break;
-            default: e = gemm::launch_cfg<typename T::Dec>(p, g.out_type, vec_ok, stream); break;
-            }
+            // panels run in stream order, so they share the workspace
+            const TilePlan   d = plan_tiles(p.m, p.n, p.k, ws ? ws_bytes : 0, false, PB);
+            const hipError_t e = launch_plan<PB>(p, d, g.out_type, vec_ok, ws, stream);
             if(e != hipSuccess) return e;
         }
     }
@@ -586,7 +669,8 @@ hipError_t launch_tiles(const GemmArgs& g, void* ws, size_t ws_bytes, hipStream_
 hipError_t launch_gemm_nk(const GemmArgs& g, void* ws, size_t ws_bytes, hipStream_t stream)
 {
     if(g.m == 0 || g.n == 0) return hipSuccess;
-    if(gemm_decode_ok(g) && !tiles_beat_decode(g, ws, ws_bytes))
+    if(gemm_decode_ok(g)
+       && plan_tiles(g.m, g.n, g.k, ws ? ws_bytes : 0, true, false).cfg == TileCfg::kDecode)
         return launch_gemm_decode(g, false, nullptr, 0, stream);
     return launch_tiles<false>(g, ws, ws_bytes, stream);
 }

@@ -151,6 +151,33 @@ def test_k_split_exact(w8a8, gpu, m, n, k):
     assert_f16_bitexact(cf[rows], O.dequant_f16(acc, sa[rows], sb))
 
 
+# The short tiles (several blocks a CU) and their K pieces, row-major and packed
+# weights: edges of 32 / 64 rows and 64 / 128 columns, K tails, one k-tile.
+SHORT_TILE_SHAPES = [
+    (1, 5000, 4096), (33, 4104, 2064),          # 32 x 64 tiles
+    (31, 520, 17152), (64, 1000, 8208),         # ... in K pieces
+    (65, 4096, 16), (191, 1001, 1040),          # 64 x 64
+    (70, 512, 17072), (226, 380, 12224),        # ... in K pieces
+    (513, 4100, 272), (512, 4096, 2048),        # 64 x 128
+]
+
+
+@pytest.mark.parametrize("m,n,k", SHORT_TILE_SHAPES)
+def test_short_tiles_exact(w8a8, gpu, m, n, k):
+    import torch
+    a, b, sa, sb = inputs(m, n, k, 11 * m + n + k)
+    ad, bd, sad, sbd = dev(a, gpu), dev(b, gpu), dev(sa, gpu), dev(sb, gpu)
+    pw = w8a8.pack_weights(bd)
+    none = torch.empty(0, dtype=torch.uint8, device=gpu)
+    acc = O.gemm_i32(a, b)
+    want = O.dequant_f16(acc, sa, sb)
+    assert_i32_equal(host(w8a8.gemm(ad, bd, out_dtype=torch.int32)), acc)
+    assert_i32_equal(host(w8a8.gemm(ad, bd, out_dtype=torch.int32, workspace=none)), acc)
+    assert_i32_equal(host(w8a8.gemm_packed(ad, pw, out_dtype=torch.int32)), acc)
+    assert_f16_bitexact(host(w8a8.gemm(ad, bd, sad, sbd)), want)
+    assert_f16_bitexact(host(w8a8.gemm_packed(ad, pw, sad, sbd)), want)
+
+
 def test_k_split_strided(w8a8, gpu):
     # split path with row strides on A, B and C (16 tiles x 2 pieces)
     import torch
