@@ -216,7 +216,20 @@ int w8a8_quantize_weights(const void* w, uint32_t n, uint32_t k, uint32_t ldw,
         w8a8::launch_quantize_weights(p, fold == W8A8_FOLD_DIVIDE, packed == 1, stream), fn);
 }
 
-static uint32_t round_up16(uint32_t v) { return (v + 15u) & ~15u; }
+static uint32_t round_up(uint32_t v, uint32_t step) { return (v + step - 1) / step * step; }
+
+static size_t align256(size_t v) { return (v + 255) / 256 * 256; }
+
+// The sample layout's repacked A [m, kp] and B [n, kp], each 256-byte aligned.
+// kp is k rounded up to 128 where the workspace has that room (every row then
+// starts on a 128-byte line: a k-tile's row piece that crosses one is two
+// requests, 6-40% of a k-step over the tile sizes), else to 16, the least that the tile kernels take.
+constexpr uint32_t kRepackStep = 128, kRepackStepLeast = 16;
+static size_t repack_bytes(uint32_t m, uint32_t n, uint32_t k, uint32_t step)
+{
+    const size_t kp = round_up(k, step);
+    return align256(m * kp) + align256(n * kp);
+}
 
 size_t w8a8_gemm_workspace_size(uint32_t m, uint32_t n, uint32_t k, int layout)
 {
@@ -227,9 +240,11 @@ size_t w8a8_gemm_workspace_size(uint32_t m, uint32_t n, uint32_t k, int layout)
         return w8a8::gemm_nk_workspace_bytes(g);
     }
     if(layout != W8A8_LAYOUT_A_COL_B_KN) return 0;
-    const size_t kp = round_up16(k);
-    // repacked A [m, kp] and B [n, kp], each 256-byte aligned
-    return ((size_t)m * kp + 255) / 256 * 256 + ((size_t)n * kp + 255) / 256 * 256;
+    // the repacked operands, then the K split of the GEMM over them
+    const uint32_t kp = round_up(k, kRepackStep);
+    w8a8::GemmArgs g{m, n, kp, nullptr, nullptr, nullptr, kp, kp, n, nullptr, nullptr, 1.f, 1.f,
+                     W8A8_OUT_F16};
+    return repack_bytes(m, n, k, kRepackStep) + align256(w8a8::gemm_nk_workspace_bytes(g));
 }
 
 static int validate_gemm(const char* fn, uint32_t m, uint32_t n, uint32_t k, const int8_t* a,
@@ -271,31 +286,34 @@ static int gemm_entry(const char* fn, uint32_t m, uint32_t n, uint32_t k, const 
                      tensor_scale_a, tensor_scale_b, out_type};
 
     if(layout == W8A8_LAYOUT_A_COL_B_KN) {
-        const size_t need = w8a8_gemm_workspace_size(m, n, k, layout);
-        if(workspace == nullptr || workspace_bytes < need) {
-            // No room to repack: strided generic kernel over the sample layout.
-            return hip_status(w8a8::launch_gemm_generic(g, 1, lda, 1, ldb, stream), fn);
-        }
-        if(reinterpret_cast<uintptr_t>(workspace) % 256 != 0)
+        const bool room = workspace != nullptr
+                          && workspace_bytes >= repack_bytes(m, n, k, kRepackStepLeast);
+        if(room && reinterpret_cast<uintptr_t>(workspace) % 256 != 0)
             return fail(W8A8_ERROR_INVALID_VALUE, "%s: workspace must be 256-byte aligned", fn);
-        const uint32_t kp  = round_up16(k);
-        int8_t*        at  = static_cast<int8_t*>(workspace);
-        int8_t*        bt  = at + ((size_t)m * kp + 255) / 256 * 256;
-        hipError_t     e   = w8a8::launch_transpose_i8(a, lda, at, kp, m, k, stream);
-        if(e == hipSuccess) e = w8a8::launch_transpose_i8(b, ldb, bt, kp, n, k, stream);
+        if(w8a8::direct_kn_pays(g) || (!room && w8a8::gemm_direct_kn_ok(g)))
+            return hip_status(w8a8::launch_gemm_direct(g, true, stream), fn);
+        if(!room) return hip_status(w8a8::launch_gemm_generic(g, 1, lda, 1, ldb, stream), fn);
+        const uint32_t step = workspace_bytes >= repack_bytes(m, n, k, kRepackStep)
+                                  ? kRepackStep
+                                  : kRepackStepLeast;
+        const uint32_t kp   = round_up(k, step);
+        const size_t   need = repack_bytes(m, n, k, step);
+        int8_t*        at = static_cast<int8_t*>(workspace);
+        int8_t*        bt = at + align256((size_t)m * kp);
+        hipError_t     e  = w8a8::launch_repack_kn(g, at, bt, kp, stream);
         if(e != hipSuccess) return hip_status(e, fn);
         g.a   = at;
         g.b   = bt;
         g.lda = kp;
         g.ldb = kp;
         g.k   = kp; // zero padding contributes nothing
-        return hip_status(w8a8::launch_gemm_nk(g, nullptr, 0, stream), fn);
+        return hip_status(w8a8::launch_gemm_nk(g, at + need, workspace_bytes - need, stream), fn);
     }
 
     if(workspace && reinterpret_cast<uintptr_t>(workspace) % 16 != 0)
         return fail(W8A8_ERROR_INVALID_VALUE, "%s: workspace must be 16-byte aligned", fn);
     if(!w8a8::gemm_fast_path_ok(g))
-        return hip_status(w8a8::launch_gemm_generic(g, lda, 1, ldb, 1, stream), fn);
+        return hip_status(w8a8::launch_gemm_direct(g, false, stream), fn);
     return hip_status(w8a8::launch_gemm_nk(g, workspace, workspace ? workspace_bytes : 0, stream),
                       fn);
 }
@@ -322,7 +340,7 @@ int w8a8_gemm_noalloc(uint32_t m, uint32_t n, uint32_t k, const int8_t* a, const
     if(rc != W8A8_SUCCESS) return rc;
     // the repack needs its room; the primary layout's K split takes a plan that fits
     const size_t need
-        = layout == W8A8_LAYOUT_A_ROW_B_NK ? 0 : w8a8_gemm_workspace_size(m, n, k, layout);
+        = layout == W8A8_LAYOUT_A_ROW_B_NK ? 0 : repack_bytes(m, n, k, kRepackStepLeast);
     if(need > W8A8_NOALLOC_SCRATCH_BYTES)
         return fail(W8A8_ERROR_INVALID_VALUE,
                     "%s: m=%u n=%u k=%u needs %zu bytes of scratch, the library holds %zu per GPU "

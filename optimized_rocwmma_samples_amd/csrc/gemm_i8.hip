@@ -6,6 +6,7 @@
 // B [K,N] layout.
 #include "gemm_i8_decode_kernel.hpp"
 #include "gemm_i8_decode_wide_kernel.hpp"
+#include "gemm_i8_direct_kernel.hpp"
 #include "gemm_i8_kernel.hpp"
 #include "gemm_i8_persist_kernel.hpp"
 #include "gemm_i8_streamk_kernel.hpp"
@@ -65,7 +66,8 @@ using DecWide4   = gemm::DecWideCfg<4, 4>;
 constexpr uint32_t kWideSlabs = 384;
 
 // ---------------------------------------------------------------------------
-// Generic strided kernel: one thread per output, any layout / alignment.
+// Generic strided kernel: one thread per output (the sample layout with fewer
+// than 4 rows or columns and no workspace to repack into).
 // ---------------------------------------------------------------------------
 template <int OUT>
 __global__ void __launch_bounds__(256) gemm_i8_generic_kernel(KArgs p, size_t sam, size_t sak,
@@ -89,58 +91,73 @@ __global__ void __launch_bounds__(256) gemm_i8_generic_kernel(KArgs p, size_t sa
     }
 }
 
-__global__ void __launch_bounds__(256) transpose_i8_kernel(const int8_t* src, uint32_t lds_src,
-                                                           int8_t* dst, uint32_t ldd,
-                                                           uint32_t rows, uint32_t cols, int vec)
+// Repack of the sample layout: dst[r, c] = src[c * ld + r] for both operands in
+// one launch, 0 for c in [cols, ldd) (the K padding).  A block moves a tile of
+// 128 rows r x 128 columns c: each thread loads 4 bytes (4 rows) of 16
+// consecutive source rows, 128 contiguous bytes per half wave, transposes them
+// with v_perm_b32 (gemm::transpose_quad) into 16-byte pieces of 4 destination
+// rows, and the tile goes through LDS (swizzled as the GEMM's tiles, no bank
+// conflicts) so that 8 lanes store 128 contiguous bytes of a row.  HBM-bound;
+// any pointer and ld.  3840 x 4096 x 4096, both operands: 18.4 -> 11.1 us (6 TB/s);
+// 4095^3 67.6 -> 16.4 us (two launches whose edge and unaligned loads went byte by
+// byte).
+struct Repack {
+    const int8_t* src;
+    int8_t*       dst;
+    uint32_t      ld, rows; // source leading dimension; rows of dst
+};
+
+__global__ void __launch_bounds__(256) repack_i8_kernel(Repack a, Repack b, uint32_t blocks_a,
+                                                        uint32_t cols, uint32_t ldd)
 {
-    // dst[r, c] = src[c * lds_src + r] (0 for c >= cols: the K padding), one
-    // 64 x 64 tile per block through LDS.  Each thread moves 16 bytes each
-    // way: a 16-byte run of one source row in, a 16-byte run of one
-    // destination row out (vec: src and lds_src 16-byte aligned; dst and ldd
-    // are, by construction).  Rows of the LDS tile are padded to 68 bytes.
-    constexpr int kPitch = 68;
-    __shared__ __attribute__((aligned(16))) int8_t tile[64 * kPitch];
-    const uint32_t r0 = blockIdx.x * 64, c0 = blockIdx.y * 64;
-    const int      t  = threadIdx.x;
+    __shared__ __attribute__((aligned(16))) int8_t tile[128 * 128];
+    const bool     in_b = blockIdx.x >= blocks_a; // uniform
+    const Repack   p    = in_b ? b : a;
+    const uint32_t id   = blockIdx.x - (in_b ? blocks_a : 0);
+    const uint32_t rt   = (p.rows + 127) / 128;
+    const uint32_t r0 = id % rt * 128, c0 = id / rt * 128;
+    const uint32_t t = threadIdx.x;
     {
-        const int      cl = t / 4, rc = (t % 4) * 16; // source row c0 + cl, bytes r0 + rc ..
-        const uint32_t cc = c0 + cl, rr = r0 + rc;
-        int4           v  = make_int4(0, 0, 0, 0);
-        if(cc < cols) {
-            const int8_t* p = src + (size_t)cc * lds_src + rr;
-            if(vec && rr + 16 <= rows) {
-                v = *reinterpret_cast<const int4*>(p);
-            } else {
-                int8_t b[16];
-                for(int e = 0; e < 16; ++e) b[e] = rr + e < rows ? p[e] : 0;
-                v = *reinterpret_cast<const int4*>(b);
+        const uint32_t row = ((t & 3) | ((t >> 3) % 8) << 2) * 4;
+        const uint32_t ch  = ((t >> 2) & 1) | ((t >> 3) / 8) << 1;
+        const uint32_t in  = p.rows < 4 ? 0 : min(r0 + row, p.rows - 4); // a quad past the end moves inside
+        const uint32_t sh  = min(r0 + row - in, 3u) * 8;
+        uint32_t       x[16];
+        if(p.rows < 4) { // uniform: 1-3 source columns, byte by byte
+            for(int j = 0; j < 16; ++j) {
+                const uint32_t c = c0 + ch * 16 + j;
+                x[j]             = 0;
+                for(uint32_t e = 0; e < p.rows && c < cols; ++e)
+                    x[j] |= (uint32_t)(uint8_t)p.src[(size_t)c * p.ld + e] << (8 * e);
+            }
+        } else if(c0 + 128 <= cols) { // uniform
+            const int8_t* s = p.src + (size_t)(c0 + ch * 16) * p.ld + in;
+#pragma unroll
+            for(int j = 0; j < 16; ++j) __builtin_memcpy(&x[j], s + (size_t)j * p.ld, 4);
+        } else {
+#pragma unroll
+            for(int j = 0; j < 16; ++j) {
+                const uint32_t c = c0 + ch * 16 + j;
+                x[j]             = 0;
+                if(c < cols) __builtin_memcpy(&x[j], p.src + (size_t)c * p.ld + in, 4);
             }
         }
-        int* row = reinterpret_cast<int*>(tile + cl * kPitch + rc);
-        row[0] = v.x;
-        row[1] = v.y;
-        row[2] = v.z;
-        row[3] = v.w;
+        v4i o[4];
+        gemm::transpose_quad(x, sh, o);
+#pragma unroll
+        for(int i = 0; i < 4; ++i) {
+            const uint32_t r = row + i;
+            *reinterpret_cast<v4i*>(tile + r * 128 + (ch ^ ((r >> 1) & 7)) * 16) = o[i];
+        }
     }
     __syncthreads();
-    const int      rl = t / 4, cc0 = (t % 4) * 16; // destination row r0 + rl, columns c0 + cc0 ..
-    const uint32_t rr = r0 + rl;
-    if(rr >= rows) return;
-    uint32_t w[4];
 #pragma unroll
-    for(int q = 0; q < 4; ++q) {
-        uint32_t x = 0;
-#pragma unroll
-        for(int e = 0; e < 4; ++e)
-            x |= (uint32_t)(uint8_t)tile[(cc0 + q * 4 + e) * kPitch + rl] << (8 * e);
-        w[q] = x;
-    }
-    const uint32_t cbase = c0 + cc0;
-    int8_t*        d     = dst + (size_t)rr * ldd + cbase;
-    if(cbase + 16 <= ldd) {
-        *reinterpret_cast<int4*>(d) = make_int4((int)w[0], (int)w[1], (int)w[2], (int)w[3]);
-    } else {
-        for(int e = 0; cbase + e < ldd; ++e) d[e] = (int8_t)(w[e / 4] >> (8 * (e % 4)));
+    for(int i = 0; i < 4; ++i) {
+        const uint32_t r = (i * 256 + t) / 8, ch = t % 8;
+        const v4i      v = *reinterpret_cast<const v4i*>(tile + r * 128 + (ch ^ ((r >> 1) & 7)) * 16);
+        // ldd is a multiple of 16: a chunk is inside the row or past it
+        if(r0 + r < p.rows && c0 + ch * 16 < ldd)
+            *reinterpret_cast<v4i*>(p.dst + (size_t)(r0 + r) * ldd + c0 + ch * 16) = v;
     }
 }
 
@@ -910,14 +927,59 @@ hipError_t launch_gemm_generic(const GemmArgs& g, size_t sam, size_t sak, size_t
     return hipGetLastError();
 }
 
-hipError_t launch_transpose_i8(const int8_t* src, uint32_t lds_src, int8_t* dst, uint32_t ldd,
-                               uint32_t rows, uint32_t cols, hipStream_t stream)
+hipError_t launch_repack_kn(const GemmArgs& g, int8_t* at, int8_t* bt, uint32_t kp,
+                            hipStream_t stream)
 {
-    dim3      grid((rows + 63) / 64, (ldd + 63) / 64);
-    const int vec = reinterpret_cast<uintptr_t>(src) % 16 == 0 && lds_src % 16 == 0;
-    hipLaunchKernelGGL(transpose_i8_kernel, grid, dim3(256), 0, stream, src, lds_src, dst, ldd,
-                       rows, cols, vec);
+    const Repack   a{g.a, at, g.lda, g.m}, b{g.b, bt, g.ldb, g.n};
+    const uint32_t kt = (kp + 127) / 128;
+    const uint64_t na = (uint64_t)ceil_div(g.m, 128) * kt, nb = (uint64_t)ceil_div(g.n, 128) * kt;
+    if(na + nb > 0x7FFFFFFFull) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(repack_i8_kernel, dim3((uint32_t)(na + nb)), dim3(256), 0, stream, a, b,
+                       (uint32_t)na, g.k, kp);
     return hipGetLastError();
+}
+
+// Tiles of the direct kernel: 256 x 256 and 128 x 128 from 5/8 of a round of
+// them on, else 64 x 64.  4000 x 4000 x 4001 (256 / 1024 / 3969 tiles) 84 /
+// 113 / 212 us; 3000^3 (144 of 256 x 256) 65 / 65; 2000^3 (256 of 128 x 128)
+// 45 / 21 / 30; 847 x 2388 x 92 (133 of 128 x 128) 19 / 10.9 / 10.2; 1000^3
+// 22 / 9.5 / 7.9.  The sample layout's lie alike: 4095^3 149 / 221 / 407,
+// 2000^3 53 / 25 / 36, 912 x 563 x 2138 (40 of 128 x 128) 64 / 28 / 21.
+template <bool COLS>
+hipError_t launch_direct_tiles(const GemmArgs& g, hipStream_t stream)
+{
+    if(g.m == 0 || g.n == 0) return hipSuccess;
+    using Big    = gemm::Cfg<256, 256, 128, 2, 2, 4, 4, 16>;
+    using Middle = gemm::Cfg<128, 128, 128, 2, 2, 4, 4, 16>;
+    using Little = gemm::Cfg<64, 64, 128, 2, 2, 2, 4, 16>;
+    constexpr int  kAhead = COLS ? 1 : 2; // k-tiles in registers (a quad unit is 16 VGPRs)
+    const KArgs    p      = make_kargs(g);
+    const int      vec_ok = out_vec_ok(g);
+    const uint64_t enough = (uint64_t)device_cus() * 5 / 8;
+    if((uint64_t)ceil_div(g.m, 64) * ceil_div(g.n, 64) > 0x7FFFFFFFull) return hipErrorInvalidValue;
+    if((uint64_t)ceil_div(g.m, 256) * ceil_div(g.n, 256) >= enough)
+        return gemm::launch_direct<Big, COLS, 1>(p, g.out_type, vec_ok, stream);
+    if((uint64_t)ceil_div(g.m, 128) * ceil_div(g.n, 128) >= enough)
+        return gemm::launch_direct<Middle, COLS, kAhead>(p, g.out_type, vec_ok, stream);
+    return gemm::launch_direct<Little, COLS, kAhead>(p, g.out_type, vec_ok, stream);
+}
+
+hipError_t launch_gemm_direct(const GemmArgs& g, bool kn, hipStream_t stream)
+{
+    return kn ? launch_direct_tiles<true>(g, stream) : launch_direct_tiles<false>(g, stream);
+}
+
+bool gemm_direct_kn_ok(const GemmArgs& g) { return g.m >= 4 && g.n >= 4; }
+
+// The sample layout in place, where it beats the repack and its second
+// launch: a direct k-tile costs about 1 us, so up to 8 of them in one round
+// of 64 x 64 tiles (130 x 2767 x 996: 11.7 us against 17.7 with the repack;
+// 186 x 1044 x 3394, 27 k-tiles: 28.8 against 25.7).
+bool direct_kn_pays(const GemmArgs& g)
+{
+    return gemm_direct_kn_ok(g)
+           && (uint64_t)ceil_div(g.m, 64) * ceil_div(g.n, 64) <= device_cus()
+           && ceil_div(g.k, 128) <= 8;
 }
 
 // ---------------------------------------------------------------------------

@@ -134,15 +134,22 @@ hipError_t launch_gemm_packed(const GemmArgs& g, void* ws, size_t ws_bytes, hipS
 // to the unsplit decode kernel.
 size_t     packed_workspace_bytes(const GemmArgs& g);
 
-// Generic strided GEMM (any layout/alignment): A(m,k) = a[m*sam + k*sak],
-// B(n,k) = b[n*sbn + k*sbk].  Slow; used for odd shapes.
+// Tile GEMM over any pointers, strides and K (gemm_i8_direct_kernel.hpp): the
+// primary layout, or the sample layout in place (kn; gemm_direct_kn_ok: at
+// least 4 rows and columns).  direct_kn_pays: sizes where that beats the repack.
+hipError_t launch_gemm_direct(const GemmArgs& g, bool kn, hipStream_t stream);
+bool       gemm_direct_kn_ok(const GemmArgs& g);
+bool       direct_kn_pays(const GemmArgs& g);
+
+// Generic strided GEMM: A(m,k) = a[m*sam + k*sak], B(n,k) = b[n*sbn + k*sbk].
+// Slow; the sample layout with m < 4 or n < 4 and no workspace.
 hipError_t launch_gemm_generic(const GemmArgs& g, size_t sam, size_t sak, size_t sbn,
                                size_t sbk, hipStream_t stream);
 
-// Transposing repack: dst[r, c] = src[c*lds_src + r] for r < rows, c < cols,
-// dst row-major with leading dimension ldd (zero-padded up to ldd).
-hipError_t launch_transpose_i8(const int8_t* src, uint32_t lds_src, int8_t* dst, uint32_t ldd,
-                               uint32_t rows, uint32_t cols, hipStream_t stream);
+// Repack of the sample layout's operands (A [k, lda], B [k, ldb]) into K-contiguous
+// rows of kp bytes (a multiple of 16, zero past k), one launch.
+hipError_t launch_repack_kn(const GemmArgs& g, int8_t* at, int8_t* bt, uint32_t kp,
+                            hipStream_t stream);
 
 // ---- MoE (moe.hip) ----------------------------------------------------------
 hipError_t launch_topk_softmax(const void* logits, bool f16, float* w, int32_t* ids,

@@ -151,6 +151,54 @@ def test_k_split_exact(w8a8, gpu, m, n, k):
     assert_f16_bitexact(cf[rows], O.dequant_f16(acc, sa[rows], sb))
 
 
+# The direct kernel (any pointer, row stride and K): tails of 1, 15 and 16 bytes
+# either side of a k-tile, single rows and columns, K below 16, each tile size
+# (64, 128 and 256 rows), operands 1-7 bytes off alignment.
+DIRECT_SHAPES = [(1, 1, 1), (3, 5, 15), (65, 63, 17), (64, 129, 127), (130, 66, 129), (200, 100, 255),
+                 (1, 300, 1001), (1700, 1650, 100), (3400, 3330, 33)]
+
+
+def _at_offset(a, ld, off, gpu):
+    import torch
+    buf = torch.full((a.shape[0] * ld + off,), 77, dtype=torch.int8, device=gpu)
+    view = buf[off:].view(a.shape[0], ld)[:, :a.shape[1]]
+    view.copy_(dev(a, gpu))
+    return view
+
+
+@pytest.mark.parametrize("pad,off", [(0, 0), (1, 3), (16, 8)])
+@pytest.mark.parametrize("m,n,k", DIRECT_SHAPES)
+def test_any_alignment_exact(w8a8, gpu, m, n, k, pad, off):
+    import torch
+    a, b, sa, sb = inputs(m, n, k, 3 * m + 5 * n + k)
+    ad, bd = _at_offset(a, k + pad, off, gpu), _at_offset(b, k + pad, off + 4, gpu)
+    acc = O.gemm_i32(a, b)
+    assert_i32_equal(host(w8a8.gemm(ad, bd, out_dtype=torch.int32)), acc)
+    assert_f16_bitexact(host(w8a8.gemm(ad, bd, dev(sa, gpu), dev(sb, gpu))),
+                        O.dequant_f16(acc, sa, sb))
+
+
+# The sample layout: in place (few tiles, short K), repacked (with and without
+# the room for 128-byte rows), in place for want of a workspace, and 1-3 rows
+# or columns, each with ragged sizes and leading dimensions.
+@pytest.mark.parametrize("m,n,k", [(4, 4, 1), (130, 767, 996), (186, 1044, 1394), (2, 300, 200),
+                                   (300, 3, 77), (700, 900, 2051), (1, 1, 5)])
+def test_sample_layout_routes_exact(w8a8, gpu, m, n, k):
+    import torch
+    a, b, _, _ = inputs(m, n, k, m + 7 * n + 3 * k)
+    at = _at_offset(np.ascontiguousarray(a.T), m + 1, 3, gpu)
+    bt = _at_offset(np.ascontiguousarray(b.T), n + 5, 1, gpu)
+    acc = O.gemm_i32(a, b)
+    full = w8a8.gemm_workspace_size(m, n, k, w8a8.LAYOUT_A_COL_B_KN)
+    up = lambda v: (v + 255) // 256 * 256  # noqa: E731
+    kp = (k + 15) // 16 * 16
+    for size in (full, up(m * kp) + up(n * kp), 0):
+        ws = torch.empty(size, dtype=torch.uint8, device=gpu)
+        c = w8a8.gemm(at, bt, layout=w8a8.LAYOUT_A_COL_B_KN, out_dtype=torch.int32, workspace=ws,
+                      m=m, n=n, k=k)
+        assert_i32_equal(host(c), acc)
+
+
 # The short tiles (several blocks a CU) and their K pieces, row-major and packed
 # weights: edges of 32 / 64 rows and 64 / 128 columns, K tails, one k-tile.
 SHORT_TILE_SHAPES = [
