@@ -197,13 +197,6 @@ KArgs make_kargs(const GemmArgs& g)
                  g.k,   g.lda, g.ldb, g.ldc,     g.tsa,     g.tsb};
 }
 
-int out_vec_ok(const GemmArgs& g)
-{
-    const size_t esz = g.out_type == W8A8_OUT_I32 ? 4 : 2;
-    return (reinterpret_cast<uintptr_t>(g.c) % (4 * esz) == 0) && (g.ldc % 4 == 0)
-           && (g.scale_b == nullptr || reinterpret_cast<uintptr_t>(g.scale_b) % 16 == 0);
-}
-
 // Sub-problem of rows [n0, n0 + nn) of the weights.  For packed weights n0 is
 // a multiple of the 64-row slab and b points at the slab's packed block.
 KArgs n_panel(const GemmArgs& g, uint32_t n0, uint32_t nn, bool packed)
@@ -459,11 +452,10 @@ hipError_t launch_gemm_decode_fused(const GemmArgs& g, const FuseArgs& f, hipStr
 {
     const uint32_t    ka = gemm::packed_ktiles(g.k) * gemm::kPackK;
     const gemm::FuseQ fq{f.x, f.s, f.q, f.r, f.ldx, ka, ka + gemm::kFusePad, f.qmax};
-    const int      vec_ok = out_vec_ok(g);
     const uint32_t step   = weight_panel_rows(g, true);
     for(uint32_t n0 = 0; n0 < g.n; n0 += step) {
         const KArgs      p = n_panel(g, n0, std::min(step, g.n - n0), true);
-        const hipError_t e = gemm::launch_decode_fused<DecSmall>(p, fq, vec_ok, stream);
+        const hipError_t e = gemm::launch_decode_fused<DecSmall>(p, fq, stream);
         if(e != hipSuccess) return e;
     }
     return hipSuccess;
@@ -473,7 +465,6 @@ hipError_t launch_gemm_decode(const GemmArgs& g, bool packed, void* ws, size_t w
                               hipStream_t stream)
 {
     if(g.m == 0 || g.n == 0) return hipSuccess;
-    const int      vec_ok = out_vec_ok(g);
     const uint32_t step   = weight_panel_rows(g, packed);
     const bool     wide   = packed && gemm::packed_slabs(g.n) >= kWideSlabs;
     for(uint32_t n0 = 0; n0 < g.n; n0 += step) {
@@ -487,14 +478,14 @@ hipError_t launch_gemm_decode(const GemmArgs& g, bool packed, void* ws, size_t w
             const uint64_t b4 = (uint64_t)(p.n + DecWide4::kRows - 1) / DecWide4::kRows * (splits / 2);
             if(splits % 2 == 0 && b4 * 4 >= (uint64_t)device_cus() * 3 && b4 <= device_cus()
                && gemm::decode_ws_bytes(g.m, p.n, splits / 2) <= ws_bytes) {
-                e = gemm::launch_decode_wide<DecWide4>(p, g.out_type, vec_ok,
+                e = gemm::launch_decode_wide<DecWide4>(p, g.out_type,
                                                        static_cast<int32_t*>(ws), splits / 2,
                                                        stream);
                 if(e != hipSuccess) return e;
                 continue;
             }
             if(gemm::decode_ws_bytes(g.m, p.n, splits) <= ws_bytes) {
-                e = gemm::launch_decode_wide<DecWide>(p, g.out_type, vec_ok,
+                e = gemm::launch_decode_wide<DecWide>(p, g.out_type,
                                                       static_cast<int32_t*>(ws), splits, stream);
                 if(e != hipSuccess) return e;
                 continue;
@@ -504,18 +495,18 @@ hipError_t launch_gemm_decode(const GemmArgs& g, bool packed, void* ws, size_t w
             // 8 <= m <= 16 on many slabs: 64 weight rows per block halve the
             // re-reads of the activation rows (M=16 N=28672: 54 -> 52 us)
             if((g.m <= 16 && (!wide || g.m < 8)) || (g.m <= 32 && !wide))
-                e = gemm::launch_decode<DecSmall, true>(p, g.out_type, vec_ok, stream);
+                e = gemm::launch_decode<DecSmall, true>(p, g.out_type, stream);
             else if(g.m <= 32)
-                e = gemm::launch_decode<DecSmallW, true>(p, g.out_type, vec_ok, stream);
+                e = gemm::launch_decode<DecSmallW, true>(p, g.out_type, stream);
             else if(!wide)
-                e = gemm::launch_decode<DecMid, true>(p, g.out_type, vec_ok, stream);
+                e = gemm::launch_decode<DecMid, true>(p, g.out_type, stream);
             else
-                e = gemm::launch_decode<DecMidW, true>(p, g.out_type, vec_ok, stream);
+                e = gemm::launch_decode<DecMidW, true>(p, g.out_type, stream);
         } else {
             if(g.m <= 32)
-                e = gemm::launch_decode<DecSmall, false>(p, g.out_type, vec_ok, stream);
+                e = gemm::launch_decode<DecSmall, false>(p, g.out_type, stream);
             else
-                e = gemm::launch_decode<DecMid, false>(p, g.out_type, vec_ok, stream);
+                e = gemm::launch_decode<DecMid, false>(p, g.out_type, stream);
         }
         if(e != hipSuccess) return e;
     }
@@ -559,10 +550,10 @@ bool gemm_packed_ok(const GemmArgs& g)
 // tiles are short: 2-4% at M=8192 K=4096 N=28672, 10-20% at K <= 1024,
 // nothing measurable at K=14336 with two tiles per CU.
 template <class C>
-bool persist_pays(const KArgs& p, int out_type, int vec_ok)
+bool persist_pays(const KArgs& p, int out_type)
 {
     return out_type == W8A8_OUT_F16 && (p.k + C::kBK - 1) / C::kBK <= 32
-           && gemm::persist_ok<C>(p, vec_ok, device_cus());
+           && gemm::persist_ok<C>(p, device_cus());
 }
 
 size_t gemm_nk_workspace_bytes(const GemmArgs& g)
@@ -589,7 +580,7 @@ const int8_t* weight_rows(const KArgs& p, uint32_t n0)
 // round of 256 tiles of 128 x 256).  The same k-order per output, so the
 // result is bit-identical to the single launch.
 template <bool PB>
-hipError_t launch_main(const KArgs& p, int out_type, int vec_ok, hipStream_t stream)
+hipError_t launch_main(const KArgs& p, int out_type, hipStream_t stream)
 {
     using Main           = typename Tiles<PB>::Main;
     using MidM           = typename Tiles<PB>::MidM;
@@ -599,9 +590,9 @@ hipError_t launch_main(const KArgs& p, int out_type, int vec_ok, hipStream_t str
     const uint32_t full = tiles / cus, rest = tiles % cus;
     const uint32_t mid_rows = (p.m + MidM::kBM - 1) / MidM::kBM;
     auto whole = [&](const KArgs& q) {
-        return persist_pays<Main>(q, out_type, vec_ok)
-                   ? gemm::launch_cfg_persist<Main>(q, vec_ok, cus, stream)
-                   : gemm::launch_cfg<Main>(q, out_type, vec_ok, stream);
+        return persist_pays<Main>(q, out_type)
+                   ? gemm::launch_cfg_persist<Main>(q, cus, stream)
+                   : gemm::launch_cfg<Main>(q, out_type, stream);
     };
     if(full >= 1 && rest > 0 && rest * 2 <= cus && (full * cus) % tm == 0) {
         const uint32_t n1   = full * cus / tm * Main::kBN; // < p.n: rest > 0
@@ -616,7 +607,7 @@ hipError_t launch_main(const KArgs& p, int out_type, int vec_ok, hipStream_t str
             tail.sb    = p.sb ? p.sb + n1 : nullptr;
             hipError_t e = whole(head);
             if(e != hipSuccess) return e;
-            return gemm::launch_cfg<MidM>(tail, out_type, vec_ok, stream);
+            return gemm::launch_cfg<MidM>(tail, out_type, stream);
         }
     }
     return whole(p);
@@ -624,21 +615,21 @@ hipError_t launch_main(const KArgs& p, int out_type, int vec_ok, hipStream_t str
 
 // One planned launch of a panel.
 template <bool PB>
-hipError_t launch_plan(const KArgs& p, const TilePlan& d, int out_type, int vec_ok, void* ws,
+hipError_t launch_plan(const KArgs& p, const TilePlan& d, int out_type, void* ws,
                        hipStream_t stream)
 {
     using T = Tiles<PB>;
     auto go = [&](auto c) {
         using C = decltype(c);
         if(d.parts > 1)
-            return gemm::launch_cfg_split<C>(p, out_type, vec_ok, static_cast<int32_t*>(ws),
+            return gemm::launch_cfg_split<C>(p, out_type, static_cast<int32_t*>(ws),
                                              d.parts, stream);
-        return gemm::launch_cfg<C>(p, out_type, vec_ok, stream);
+        return gemm::launch_cfg<C>(p, out_type, stream);
     };
     switch(d.cfg) {
     case TileCfg::kMain:
         return d.parts > 1 ? go(typename T::Main{})
-                           : launch_main<PB>(p, out_type, vec_ok, stream);
+                           : launch_main<PB>(p, out_type, stream);
     case TileCfg::kMidM: return go(typename T::MidM{});
     case TileCfg::kSmall: return go(typename T::Small{});
     case TileCfg::kNarrow: return go(typename T::Narrow{});
@@ -653,7 +644,6 @@ template <bool PB>
 hipError_t launch_tiles(const GemmArgs& g, void* ws, size_t ws_bytes, hipStream_t stream)
 {
     const size_t esz    = g.out_type == W8A8_OUT_I32 ? 4 : 2;
-    const int    vec_ok = out_vec_ok(g);
     // The tile kernel addresses each operand through a buffer resource whose
     // out-of-range offsets read as zero; keep every launch's A and B under
     // 2 GiB by splitting M and N into row panels (multiples of the tile).
@@ -676,7 +666,7 @@ hipError_t launch_tiles(const GemmArgs& g, void* ws, size_t ws_bytes, hipStream_
             p.sb    = g.scale_b ? g.scale_b + n0 : nullptr;
             // panels run in stream order, so they share the workspace
             const TilePlan   d = plan_tiles(p.m, p.n, p.k, ws ? ws_bytes : 0, false, PB);
-            const hipError_t e = launch_plan<PB>(p, d, g.out_type, vec_ok, ws, stream);
+            const hipError_t e = launch_plan<PB>(p, d, g.out_type, ws, stream);
             if(e != hipSuccess) return e;
         }
     }
@@ -887,27 +877,26 @@ hipError_t launch_gemm_streamk(const GemmArgs& g, uint32_t blocks, void* ws, hip
     if(err != hipSuccess) return err;
     const ExplicitSk e      = explicit_streamk(g.m, g.n, g.k, blocks);
     const KArgs      p      = make_kargs(g);
-    const int        vec_ok = out_vec_ok(g);
     if(e.plan.blocks == e.plan.ntiles) {
         // one whole tile per block, no pieces: the schedule is the tile
         // kernel's one-block-per-tile grid (the same logical block -> tile
         // order), which runs it without the counters' clear launch and with
         // the epilogue's scales loaded under the last k-tile
         switch(e.cfg) {
-        case TileCfg::kMain: return gemm::launch_cfg<GemmMain>(p, g.out_type, vec_ok, stream);
-        case TileCfg::kMidM: return gemm::launch_cfg<GemmMidM>(p, g.out_type, vec_ok, stream);
-        default: return gemm::launch_cfg<GemmSmall>(p, g.out_type, vec_ok, stream);
+        case TileCfg::kMain: return gemm::launch_cfg<GemmMain>(p, g.out_type, stream);
+        case TileCfg::kMidM: return gemm::launch_cfg<GemmMidM>(p, g.out_type, stream);
+        default: return gemm::launch_cfg<GemmSmall>(p, g.out_type, stream);
         }
     }
     switch(e.cfg) {
     case TileCfg::kMain:
-        return gemm::launch_cfg_streamk<GemmMain>(p, g.out_type, vec_ok, 0, e.plan, ws, watch,
+        return gemm::launch_cfg_streamk<GemmMain>(p, g.out_type, 0, e.plan, ws, watch,
                                                   stream);
     case TileCfg::kMidM:
-        return gemm::launch_cfg_streamk<GemmMidM>(p, g.out_type, vec_ok, 0, e.plan, ws, watch,
+        return gemm::launch_cfg_streamk<GemmMidM>(p, g.out_type, 0, e.plan, ws, watch,
                                                   stream);
     default:
-        return gemm::launch_cfg_streamk<GemmSmall>(p, g.out_type, vec_ok, 0, e.plan, ws, watch,
+        return gemm::launch_cfg_streamk<GemmSmall>(p, g.out_type, 0, e.plan, ws, watch,
                                                    stream);
     }
 }
@@ -954,14 +943,13 @@ hipError_t launch_direct_tiles(const GemmArgs& g, hipStream_t stream)
     using Little = gemm::Cfg<64, 64, 128, 2, 2, 2, 4, 16>;
     constexpr int  kAhead = COLS ? 1 : 2; // k-tiles in registers (a quad unit is 16 VGPRs)
     const KArgs    p      = make_kargs(g);
-    const int      vec_ok = out_vec_ok(g);
     const uint64_t enough = (uint64_t)device_cus() * 5 / 8;
     if((uint64_t)ceil_div(g.m, 64) * ceil_div(g.n, 64) > 0x7FFFFFFFull) return hipErrorInvalidValue;
     if((uint64_t)ceil_div(g.m, 256) * ceil_div(g.n, 256) >= enough)
-        return gemm::launch_direct<Big, COLS, 1>(p, g.out_type, vec_ok, stream);
+        return gemm::launch_direct<Big, COLS, 1>(p, g.out_type, stream);
     if((uint64_t)ceil_div(g.m, 128) * ceil_div(g.n, 128) >= enough)
-        return gemm::launch_direct<Middle, COLS, kAhead>(p, g.out_type, vec_ok, stream);
-    return gemm::launch_direct<Little, COLS, kAhead>(p, g.out_type, vec_ok, stream);
+        return gemm::launch_direct<Middle, COLS, kAhead>(p, g.out_type, stream);
+    return gemm::launch_direct<Little, COLS, kAhead>(p, g.out_type, stream);
 }
 
 hipError_t launch_gemm_direct(const GemmArgs& g, bool kn, hipStream_t stream)

@@ -156,7 +156,7 @@ __device__ __forceinline__ void fuse_quantize(const FuseQ& fq, uint32_t m, uint3
 // PACKED: p.b is the packed weight buffer (p.ldb unused).  Otherwise p.b is
 // W [n, ldb] with K contiguous.
 template <class C, int OUT, bool PACKED, bool FUSE = false>
-__global__ void __launch_bounds__(C::kThreads) gemm_i8_decode_kernel(KArgs p, int vec_ok, FuseQ fq)
+__global__ void __launch_bounds__(C::kThreads) gemm_i8_decode_kernel(KArgs p, FuseQ fq)
 {
     extern __shared__ __attribute__((aligned(1024))) int8_t lds[];
 
@@ -351,18 +351,9 @@ __global__ void __launch_bounds__(C::kThreads) gemm_i8_decode_kernel(KArgs p, in
             sa = p.sa[m];
         }
         float4 sb = make_float4(p.tsb, p.tsb, p.tsb, p.tsb);
-        if(OUT == W8A8_OUT_F16 && p.sb != nullptr) {
-            if(vec_ok && n + 4 <= p.n)
-                sb = *reinterpret_cast<const float4*>(p.sb + n);
-            else {
-                if(n + 0 < p.n) sb.x = p.sb[n + 0];
-                if(n + 1 < p.n) sb.y = p.sb[n + 1];
-                if(n + 2 < p.n) sb.z = p.sb[n + 2];
-                if(n + 3 < p.n) sb.w = p.sb[n + 3];
-            }
-        }
+        if(OUT == W8A8_OUT_F16 && p.sb != nullptr) sb = load_sb4(p, n, p.tsb);
         const int v[4] = {s[0], s[1], s[2], s[3]};
-        store4<OUT>(p, m, n, v, sa, sb, ab, mode1, vec_ok != 0);
+        store4<OUT>(p, m, n, v, sa, sb, ab, mode1);
     }
 }
 
@@ -370,7 +361,7 @@ __global__ void __launch_bounds__(C::kThreads) gemm_i8_decode_kernel(KArgs p, in
 // lda % 16 == 0, ldb % 16 == 0, k % 16 == 0; (m-1)*lda + k < 2^31; the
 // weights under 2^31 bytes (packed_bytes(n, k), or (n-1)*ldb + k).
 template <class C, bool PACKED>
-hipError_t launch_decode(const KArgs& p, int out_type, int vec_ok, hipStream_t stream)
+hipError_t launch_decode(const KArgs& p, int out_type, hipStream_t stream)
 {
     using K32 = decltype(&gemm_i8_decode_kernel<C, W8A8_OUT_I32, PACKED>);
     const K32 kern[2] = {&gemm_i8_decode_kernel<C, W8A8_OUT_I32, PACKED>,
@@ -387,7 +378,7 @@ hipError_t launch_decode(const KArgs& p, int out_type, int vec_ok, hipStream_t s
     }
     const dim3 grid((p.n + C::kNT * 32 - 1) / (C::kNT * 32), (p.m + C::kMT * 32 - 1) / (C::kMT * 32));
     hipLaunchKernelGGL(kern[out_type == W8A8_OUT_I32 ? 0 : 1], grid, dim3(C::kThreads),
-                       C::kLdsBytes, stream, p, vec_ok, FuseQ{});
+                       C::kLdsBytes, stream, p, FuseQ{});
     return hipGetLastError();
 }
 
@@ -395,7 +386,7 @@ hipError_t launch_decode(const KArgs& p, int out_type, int vec_ok, hipStream_t s
 // weights, fp16 output, p.m <= kFuseRows, C::kMT == 1).  p.sa must be fq.r.
 // The host checks C::kLdsBytes + p.m * fq.pitch <= 160 KiB.
 template <class C>
-hipError_t launch_decode_fused(const KArgs& p, const FuseQ& fq, int vec_ok, hipStream_t stream)
+hipError_t launch_decode_fused(const KArgs& p, const FuseQ& fq, hipStream_t stream)
 {
     static_assert(C::kMT == 1, "one 32-row m tile holds the fused rows");
     const void* kern = reinterpret_cast<const void*>(
@@ -407,7 +398,7 @@ hipError_t launch_decode_fused(const KArgs& p, const FuseQ& fq, int vec_ok, hipS
     });
     const dim3 grid((p.n + C::kNT * 32 - 1) / (C::kNT * 32), 1);
     hipLaunchKernelGGL((gemm_i8_decode_kernel<C, W8A8_OUT_F16, true, true>), grid,
-                       dim3(C::kThreads), C::kLdsBytes + p.m * fq.pitch, stream, p, vec_ok, fq);
+                       dim3(C::kThreads), C::kLdsBytes + p.m * fq.pitch, stream, p, fq);
     return hipGetLastError();
 }
 

@@ -48,7 +48,7 @@ struct DecWideCfg {
 constexpr int kOutPartial = 2;
 
 template <class C, int OUT>
-__global__ void __launch_bounds__(C::kThreads) gemm_i8_decode_wide_kernel(KArgs p, int vec_ok,
+__global__ void __launch_bounds__(C::kThreads) gemm_i8_decode_wide_kernel(KArgs p,
                                                                           int32_t* ws,
                                                                           uint32_t ldw,
                                                                           uint32_t per)
@@ -162,17 +162,8 @@ __global__ void __launch_bounds__(C::kThreads) gemm_i8_decode_wide_kernel(KArgs 
                 *reinterpret_cast<int4*>(dst) = make_int4(v[0], v[1], v[2], v[3]);
             } else {
                 float4 sb = make_float4(p.tsb, p.tsb, p.tsb, p.tsb);
-                if(OUT == W8A8_OUT_F16 && p.sb != nullptr) {
-                    if(vec_ok && n + 4 <= p.n)
-                        sb = *reinterpret_cast<const float4*>(p.sb + n);
-                    else {
-                        if(n + 0 < p.n) sb.x = p.sb[n + 0];
-                        if(n + 1 < p.n) sb.y = p.sb[n + 1];
-                        if(n + 2 < p.n) sb.z = p.sb[n + 2];
-                        if(n + 3 < p.n) sb.w = p.sb[n + 3];
-                    }
-                }
-                store4<OUT>(p, m, n, v, sa, sb, ab, mode1, vec_ok != 0);
+                if(OUT == W8A8_OUT_F16 && p.sb != nullptr) sb = load_sb4(p, n, p.tsb);
+                store4<OUT>(p, m, n, v, sa, sb, ab, mode1);
             }
         }
     }
@@ -180,7 +171,7 @@ __global__ void __launch_bounds__(C::kThreads) gemm_i8_decode_wide_kernel(KArgs 
 
 // Sum the splits of each 4-wide run of n (in split order) and run the epilogue.
 template <int OUT>
-__global__ void __launch_bounds__(256) decode_reduce_kernel(KArgs p, int vec_ok,
+__global__ void __launch_bounds__(256) decode_reduce_kernel(KArgs p,
                                                             const int32_t* __restrict__ ws,
                                                             uint32_t ldw, uint32_t splits)
 {
@@ -203,18 +194,9 @@ __global__ void __launch_bounds__(256) decode_reduce_kernel(KArgs p, int vec_ok,
     float       sa    = p.tsa;
     if(OUT == W8A8_OUT_F16 && p.sa != nullptr) sa = p.sa[m];
     float4 sb = make_float4(p.tsb, p.tsb, p.tsb, p.tsb);
-    if(OUT == W8A8_OUT_F16 && p.sb != nullptr) {
-        if(vec_ok && n + 4 <= p.n)
-            sb = *reinterpret_cast<const float4*>(p.sb + n);
-        else {
-            if(n + 0 < p.n) sb.x = p.sb[n + 0];
-            if(n + 1 < p.n) sb.y = p.sb[n + 1];
-            if(n + 2 < p.n) sb.z = p.sb[n + 2];
-            if(n + 3 < p.n) sb.w = p.sb[n + 3];
-        }
-    }
+    if(OUT == W8A8_OUT_F16 && p.sb != nullptr) sb = load_sb4(p, n, p.tsb);
     const int v[4] = {s.x, s.y, s.z, s.w};
-    store4<OUT>(p, m, n, v, sa, sb, ab, mode1, vec_ok != 0);
+    store4<OUT>(p, m, n, v, sa, sb, ab, mode1);
 }
 
 // Workspace row stride (int32) and bytes for `splits` K splits of an m x n GEMM.
@@ -228,7 +210,7 @@ inline size_t   decode_ws_bytes(uint32_t m, uint32_t n, uint32_t splits)
 // 16-byte aligned A with lda % 16 == 0, k % 16 == 0, (m-1)*lda + k < 2^31,
 // packed_bytes(n, k) < 2^31; ws holds decode_ws_bytes(m, n, splits).
 template <class C>
-hipError_t launch_decode_wide(const KArgs& p, int out_type, int vec_ok, int32_t* ws,
+hipError_t launch_decode_wide(const KArgs& p, int out_type, int32_t* ws,
                               uint32_t splits, hipStream_t stream)
 {
     const uint32_t nkt  = packed_ktiles(p.k);
@@ -239,24 +221,22 @@ hipError_t launch_decode_wide(const KArgs& p, int out_type, int vec_ok, int32_t*
     if(splits == 1) {
         if(out_type == W8A8_OUT_I32)
             hipLaunchKernelGGL((gemm_i8_decode_wide_kernel<C, W8A8_OUT_I32>), grid,
-                               dim3(C::kThreads), C::kLdsBytes, stream, p, vec_ok, ws, ldw, per);
+                               dim3(C::kThreads), C::kLdsBytes, stream, p, ws, ldw, per);
         else
             hipLaunchKernelGGL((gemm_i8_decode_wide_kernel<C, W8A8_OUT_F16>), grid,
-                               dim3(C::kThreads), C::kLdsBytes, stream, p, vec_ok, ws, ldw, per);
+                               dim3(C::kThreads), C::kLdsBytes, stream, p, ws, ldw, per);
         return hipGetLastError();
     }
     hipLaunchKernelGGL((gemm_i8_decode_wide_kernel<C, kOutPartial>), grid, dim3(C::kThreads),
-                       C::kLdsBytes, stream, p, vec_ok, ws, ldw, per);
+                       C::kLdsBytes, stream, p, ws, ldw, per);
     hipError_t e = hipGetLastError();
     if(e != hipSuccess) return e;
     const size_t items  = (size_t)p.m * (ldw / 4);
     const dim3   rgrid((uint32_t)((items + 255) / 256));
     if(out_type == W8A8_OUT_I32)
-        hipLaunchKernelGGL((decode_reduce_kernel<W8A8_OUT_I32>), rgrid, dim3(256), 0, stream, p,
-                           vec_ok, ws, ldw, splits);
+        hipLaunchKernelGGL((decode_reduce_kernel<W8A8_OUT_I32>), rgrid, dim3(256), 0, stream, p, ws, ldw, splits);
     else
-        hipLaunchKernelGGL((decode_reduce_kernel<W8A8_OUT_F16>), rgrid, dim3(256), 0, stream, p,
-                           vec_ok, ws, ldw, splits);
+        hipLaunchKernelGGL((decode_reduce_kernel<W8A8_OUT_F16>), rgrid, dim3(256), 0, stream, p, ws, ldw, splits);
     return hipGetLastError();
 }
 

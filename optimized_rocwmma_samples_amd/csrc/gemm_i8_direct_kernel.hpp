@@ -213,7 +213,7 @@ struct ColPair {
 // COLS: both operands K-major (the sample layout), else both K-contiguous.
 // AHEAD: k-tiles held in registers beyond the one in LDS.
 template <class C, int OUT, bool COLS, int AHEAD>
-__global__ void __launch_bounds__(C::kThreads) gemm_i8_direct_kernel(KArgs p, int vec_ok)
+__global__ void __launch_bounds__(C::kThreads) gemm_i8_direct_kernel(KArgs p)
 {
     static_assert(C::kStages == 2 && C::kBK == 128 && C::kSubK == 2, "two stages of 128-deep k-tiles");
     static_assert(AHEAD == 1 || AHEAD == 2, "register ring of one or two k-tiles");
@@ -263,13 +263,13 @@ __global__ void __launch_bounds__(C::kThreads) gemm_i8_direct_kernel(KArgs p, in
         if constexpr(AHEAD == 2)
             if(kt + 1 < nk) step(kt + 1, regs[1]);
     }
-    tile_epilogue<C, OUT>(p, m0, n0, vec_ok, lds, acc);
+    tile_epilogue<C, OUT>(p, m0, n0, lds, acc);
 }
 
 // Preconditions (host): COLS needs m >= 4 and n >= 4; every operand and C of
 // any size and alignment.
 template <class C, bool COLS, int AHEAD>
-hipError_t launch_direct(const KArgs& p, int out_type, int vec_ok, hipStream_t stream)
+hipError_t launch_direct(const KArgs& p, int out_type, hipStream_t stream)
 {
     static_assert(C::kLdsBytes <= 65536 || C::kStages == 2, "dynamic LDS");
     const dim3 grid(((p.m + C::kBM - 1) / C::kBM) * ((p.n + C::kBN - 1) / C::kBN));
@@ -287,10 +287,10 @@ hipError_t launch_direct(const KArgs& p, int out_type, int vec_ok, hipStream_t s
     }
     if(out_type == W8A8_OUT_I32)
         hipLaunchKernelGGL((gemm_i8_direct_kernel<C, W8A8_OUT_I32, COLS, AHEAD>), grid,
-                           dim3(C::kThreads), C::kLdsBytes, stream, p, vec_ok);
+                           dim3(C::kThreads), C::kLdsBytes, stream, p);
     else
         hipLaunchKernelGGL((gemm_i8_direct_kernel<C, W8A8_OUT_F16, COLS, AHEAD>), grid,
-                           dim3(C::kThreads), C::kLdsBytes, stream, p, vec_ok);
+                           dim3(C::kThreads), C::kLdsBytes, stream, p);
     return hipGetLastError();
 }
 

@@ -84,7 +84,7 @@ __device__ __forceinline__ uint32_t problem_tiles(uint32_t m, uint32_t n)
 // Descriptors: KArgs per group (field order of w8a8_group_desc).
 template <class C, int OUT>
 __global__ void __launch_bounds__(C::kThreads, 1)
-    gemm_i8_grouped_kernel(const KArgs* __restrict__ groups, uint32_t ngroups, int vec_ok)
+    gemm_i8_grouped_kernel(const KArgs* __restrict__ groups, uint32_t ngroups)
 {
     extern __shared__ __attribute__((aligned(1024))) int8_t lds[];
     auto tiles = [&](uint32_t i) { return problem_tiles<C>(groups[i].m, groups[i].n); };
@@ -96,7 +96,7 @@ __global__ void __launch_bounds__(C::kThreads, 1)
     const KArgs p = groups[g];
     uint32_t    m0, n0;
     local_tile<C>(lid - first, p.m, p.n, m0, n0);
-    gemm_tile<C, OUT>(p, m0, n0, vec_ok, lds);
+    gemm_tile<C, OUT>(p, m0, n0, lds);
 }
 
 struct MoeArgs {
@@ -386,18 +386,17 @@ __device__ __forceinline__ void epilogue_silu(const KArgs& p, uint32_t m0, uint3
 // One whole MoE tile of shape X (C or W) with its epilogue.
 template <class X, int OUT, bool SILU>
 __device__ __forceinline__ void moe_whole(const KArgs& p, uint32_t m0, uint32_t n0, uint32_t e,
-                                          uint32_t row0, const SiluOut& so, uint32_t nk,
-                                          int vec_ok, int8_t* lds)
+                                          uint32_t row0, const SiluOut& so, uint32_t nk, int8_t* lds)
 {
     if constexpr(SILU) {
         Acc<X>       acc;
         EpiScales<X> sc;
-        gemm_tile_acc<X, true>(p, m0, n0, vec_ok, lds, 0, nk, acc, sc);
+        gemm_tile_acc<X, true>(p, m0, n0, lds, 0, nk, acc, sc);
         epilogue_silu<X>(p, m0, n0, lds, 0, acc, sc, so.h + (size_t)row0 * so.ldh, so.pmax + row0,
                          so.s2 ? so.s2 + (size_t)e * so.inter : nullptr, so.ldh, so.ldp,
                          so.inter);
     } else {
-        gemm_tile<X, OUT>(p, m0, n0, vec_ok, lds);
+        gemm_tile<X, OUT>(p, m0, n0, lds);
     }
 }
 
@@ -406,7 +405,7 @@ __device__ __forceinline__ void moe_whole(const KArgs& p, uint32_t m0, uint32_t 
 template <class X, int OUT, bool SILU>
 __device__ __forceinline__ void moe_fix(const MoeArgs& q, const KArgs& p, uint32_t m0,
                                         uint32_t n0, uint32_t e, uint32_t row0, const SiluOut& so,
-                                        uint32_t slot, uint32_t parts, int wave_base, int vec_ok,
+                                        uint32_t slot, uint32_t parts, int wave_base,
                                         int8_t* lds)
 {
     Acc<X> acc;
@@ -417,13 +416,13 @@ __device__ __forceinline__ void moe_fix(const MoeArgs& q, const KArgs& p, uint32
     if constexpr(SILU) {
         const int    wave = wave_base + __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
         EpiScales<X> sc;
-        sc.load(p, m0, n0, wave / X::kWavesN, wave % X::kWavesN, threadIdx.x % kWave, vec_ok);
+        sc.load(p, m0, n0, wave / X::kWavesN, wave % X::kWavesN, threadIdx.x % kWave);
         epilogue_silu<X>(p, m0, n0, lds, wave_base, acc, sc, so.h + (size_t)row0 * so.ldh,
                          so.pmax + row0,
                          so.s2 ? so.s2 + (size_t)e * so.inter : nullptr, so.ldh, so.ldp,
                          so.inter);
     } else {
-        tile_epilogue<X, OUT>(p, m0, n0, vec_ok, lds, acc, wave_base);
+        tile_epilogue<X, OUT>(p, m0, n0, lds, acc, wave_base);
     }
 }
 
@@ -431,7 +430,7 @@ __device__ __forceinline__ void moe_fix(const MoeArgs& q, const KArgs& p, uint32
 // (MoeShape); W = C: C tiles only.  The two shapes have the same wave tile,
 // so they share the partial slot layout and the fixup blocks.
 template <class C, class W, int OUT, bool SILU = false>
-__global__ void __launch_bounds__(C::kThreads, 1) gemm_i8_moe_kernel(MoeArgs q, int vec_ok,
+__global__ void __launch_bounds__(C::kThreads, 1) gemm_i8_moe_kernel(MoeArgs q,
                                                                       SiluOut so)
 {
     static_assert(Partial<W>::kInts == Partial<C>::kInts
@@ -449,9 +448,9 @@ __global__ void __launch_bounds__(C::kThreads, 1) gemm_i8_moe_kernel(MoeArgs q, 
     if(blockIdx.x < sp.base) {
         moe_tile<C, W, OUT>(q, xcd_remap(blockIdx.x, sp.base), p, m0, n0, e, row0, wide);
         if(kWide && wide)
-            moe_whole<W, OUT, SILU>(p, m0, n0, e, row0, so, nk, vec_ok, lds);
+            moe_whole<W, OUT, SILU>(p, m0, n0, e, row0, so, nk, lds);
         else
-            moe_whole<C, OUT, SILU>(p, m0, n0, e, row0, so, nk, vec_ok, lds);
+            moe_whole<C, OUT, SILU>(p, m0, n0, e, row0, so, nk, lds);
         return;
     }
     const uint32_t x = blockIdx.x - sp.base;
@@ -461,9 +460,9 @@ __global__ void __launch_bounds__(C::kThreads, 1) gemm_i8_moe_kernel(MoeArgs q, 
     moe_tile<C, W, OUT>(q, sp.base + slot, p, m0, n0, e, row0, wide);
     int32_t* const ws = q.ws + (size_t)x * Partial<C>::kInts;
     if(kWide && wide)
-        gemm_tile<W, OUT, true>(p, m0, n0, vec_ok, lds, kt0, kt1 - kt0, ws);
+        gemm_tile<W, OUT, true>(p, m0, n0, lds, kt0, kt1 - kt0, ws);
     else
-        gemm_tile<C, OUT, true>(p, m0, n0, vec_ok, lds, kt0, kt1 - kt0, ws);
+        gemm_tile<C, OUT, true>(p, m0, n0, lds, kt0, kt1 - kt0, ws);
 }
 
 // Split tiles, kPieces blocks each: a block holds kFixupWaves of the tile's
@@ -471,7 +470,7 @@ __global__ void __launch_bounds__(C::kThreads, 1) gemm_i8_moe_kernel(MoeArgs q, 
 // of the tile epilogue.
 template <class C, class W, int OUT, bool SILU = false>
 __global__ void __launch_bounds__(Partial<C>::kFixupWaves * kWave, 1)
-    gemm_i8_moe_fixup_kernel(MoeArgs q, int vec_ok, SiluOut so)
+    gemm_i8_moe_fixup_kernel(MoeArgs q, SiluOut so)
 {
     constexpr bool kWide = MoeShape<C, W>::kWide;
     extern __shared__ __attribute__((aligned(1024))) int8_t lds[];
@@ -486,9 +485,9 @@ __global__ void __launch_bounds__(Partial<C>::kFixupWaves * kWave, 1)
     bool     wide;
     moe_tile<C, W, OUT>(q, sp.base + slot, p, m0, n0, e, row0, wide);
     if(kWide && wide)
-        moe_fix<W, OUT, SILU>(q, p, m0, n0, e, row0, so, slot, sp.parts, wave_base, vec_ok, lds);
+        moe_fix<W, OUT, SILU>(q, p, m0, n0, e, row0, so, slot, sp.parts, wave_base, lds);
     else
-        moe_fix<C, OUT, SILU>(q, p, m0, n0, e, row0, so, slot, sp.parts, wave_base, vec_ok, lds);
+        moe_fix<C, OUT, SILU>(q, p, m0, n0, e, row0, so, slot, sp.parts, wave_base, lds);
 }
 
 // One flag per (configs, output type, kernel kind): the two output types of a
@@ -513,17 +512,17 @@ void raise_lds_once(const void* kern)
 
 template <class C>
 hipError_t launch_grouped(const KArgs* groups_dev, uint32_t ngroups, uint32_t total_tiles,
-                          int out_type, int vec_ok, hipStream_t stream)
+                          int out_type, hipStream_t stream)
 {
     if(total_tiles == 0) return hipSuccess;
     if(out_type == W8A8_OUT_I32) {
         raise_lds_once<C, W8A8_OUT_I32, 0>(reinterpret_cast<const void*>(gemm_i8_grouped_kernel<C, W8A8_OUT_I32>));
         hipLaunchKernelGGL((gemm_i8_grouped_kernel<C, W8A8_OUT_I32>), dim3(total_tiles),
-                           dim3(C::kThreads), C::kLdsBytes, stream, groups_dev, ngroups, vec_ok);
+                           dim3(C::kThreads), C::kLdsBytes, stream, groups_dev, ngroups);
     } else {
         raise_lds_once<C, W8A8_OUT_F16, 0>(reinterpret_cast<const void*>(gemm_i8_grouped_kernel<C, W8A8_OUT_F16>));
         hipLaunchKernelGGL((gemm_i8_grouped_kernel<C, W8A8_OUT_F16>), dim3(total_tiles),
-                           dim3(C::kThreads), C::kLdsBytes, stream, groups_dev, ngroups, vec_ok);
+                           dim3(C::kThreads), C::kLdsBytes, stream, groups_dev, ngroups);
     }
     return hipGetLastError();
 }
@@ -547,7 +546,7 @@ uint64_t moe_grid_bound(const MoeArgs& q)
 }
 
 template <class C, class W, int OUT, bool SILU>
-hipError_t launch_moe_kernels(const MoeArgs& q, const SiluOut& so, int vec_ok, hipStream_t stream)
+hipError_t launch_moe_kernels(const MoeArgs& q, const SiluOut& so, hipStream_t stream)
 {
     const uint64_t bound = moe_grid_bound<C>(q);
     if(bound == 0) return hipSuccess;
@@ -559,33 +558,33 @@ hipError_t launch_moe_kernels(const MoeArgs& q, const SiluOut& so, int vec_ok, h
     raise_lds_once<C, OUT, (SILU ? 2 : 1), W>(
         reinterpret_cast<const void*>(gemm_i8_moe_kernel<C, W, OUT, SILU>));
     hipLaunchKernelGGL((gemm_i8_moe_kernel<C, W, OUT, SILU>), dim3((uint32_t)grid),
-                       dim3(C::kThreads), kLds, stream, q, vec_ok, so);
+                       dim3(C::kThreads), kLds, stream, q, so);
     if(split)
         hipLaunchKernelGGL((gemm_i8_moe_fixup_kernel<C, W, OUT, SILU>), dim3(fixup_blocks),
                            dim3(Partial<C>::kFixupWaves * kWave), Partial<C>::kFixupLds, stream,
-                           q, vec_ok, so);
+                           q, so);
     return hipGetLastError();
 }
 
 // C tiles and, for the experts' rests of at most W::kBM rows, W tiles (W = C:
 // C tiles only).
 template <class C, class W = C>
-hipError_t launch_moe(const MoeArgs& q, int out_type, int vec_ok, hipStream_t stream)
+hipError_t launch_moe(const MoeArgs& q, int out_type, hipStream_t stream)
 {
     return out_type == W8A8_OUT_I32
-               ? launch_moe_kernels<C, W, W8A8_OUT_I32, false>(q, SiluOut{}, vec_ok, stream)
-               : launch_moe_kernels<C, W, W8A8_OUT_F16, false>(q, SiluOut{}, vec_ok, stream);
+               ? launch_moe_kernels<C, W, W8A8_OUT_I32, false>(q, SiluOut{}, stream)
+               : launch_moe_kernels<C, W, W8A8_OUT_F16, false>(q, SiluOut{}, stream);
 }
 
 // The gate_up GEMM with the SiLU epilogue (q.n = 2 * inter interleaved
-// columns, fp16 scales path; the caller checked vec_ok and the alignment of
-// h, ldh and s2).  Both tiles' waves are kWaveN wide, the width of one pmax
+// columns, fp16 scales path; the caller checked the alignment of h,
+// ldh and s2).  Both tiles' waves are kWaveN wide, the width of one pmax
 // group.
 template <class C, class W = C>
-hipError_t launch_moe_silu(const MoeArgs& q, const SiluOut& so, int vec_ok, hipStream_t stream)
+hipError_t launch_moe_silu(const MoeArgs& q, const SiluOut& so, hipStream_t stream)
 {
     static_assert(C::kWaveN == W::kWaveN, "one pmax group per wave column in both tiles");
-    return launch_moe_kernels<C, W, W8A8_OUT_F16, true>(q, so, vec_ok, stream);
+    return launch_moe_kernels<C, W, W8A8_OUT_F16, true>(q, so, stream);
 }
 
 } // namespace gemm

@@ -460,17 +460,33 @@ struct FragPipe {
     }
 };
 
-// Store 4 consecutive-n outputs of one lane.
+// 4 consecutive column scales from column n (4-byte aligned, one 16-byte load);
+// columns past N keep `fill`.
+__device__ __forceinline__ float4 load_sb4(const KArgs& p, uint32_t n, float fill)
+{
+    float4 v = make_float4(fill, fill, fill, fill);
+    if(n + 4 <= p.n) {
+        __builtin_memcpy(&v, p.sb + n, 16);
+    } else {
+        if(n + 0 < p.n) v.x = p.sb[n + 0];
+        if(n + 1 < p.n) v.y = p.sb[n + 1];
+        if(n + 2 < p.n) v.z = p.sb[n + 2];
+    }
+    return v;
+}
+
+// Store 4 consecutive-n outputs of one lane: one 16- or 8-byte store at any
+// alignment of C and ldc (the hardware takes unaligned global accesses), single
+// elements only in a quad that straddles N.
 template <int OUT>
 __device__ __forceinline__ void store4(const KArgs& p, uint32_t m, uint32_t n, const int* v,
-                                       float sa, const float4& sb, float ab, bool mode1,
-                                       bool vec_ok)
+                                       float sa, const float4& sb, float ab, bool mode1)
 {
     if(m >= p.m) return;
     if constexpr(OUT == W8A8_OUT_I32) {
         int32_t* dst = reinterpret_cast<int32_t*>(p.c) + (size_t)m * p.ldc + n;
-        if(vec_ok && n + 4 <= p.n) {
-            *reinterpret_cast<int4*>(dst) = make_int4(v[0], v[1], v[2], v[3]);
+        if(n + 4 <= p.n) {
+            __builtin_memcpy(dst, v, 16);
         } else {
             for(int e = 0; e < 4; ++e)
                 if(n + e < p.n) dst[e] = v[e];
@@ -485,11 +501,8 @@ __device__ __forceinline__ void store4(const KArgs& p, uint32_t m, uint32_t n, c
             h[e]    = float_to_half_bits_2step(f);
         }
         uint16_t* dst = reinterpret_cast<uint16_t*>(p.c) + (size_t)m * p.ldc + n;
-        if(vec_ok && n + 4 <= p.n) {
-            uint2 pk;
-            pk.x = (uint32_t)h[0] | ((uint32_t)h[1] << 16);
-            pk.y = (uint32_t)h[2] | ((uint32_t)h[3] << 16);
-            *reinterpret_cast<uint2*>(dst) = pk;
+        if(n + 4 <= p.n) {
+            __builtin_memcpy(dst, h, 8);
         } else {
             for(int e = 0; e < 4; ++e)
                 if(n + e < p.n) dst[e] = h[e];
@@ -512,7 +525,7 @@ struct EpiScales {
     float4 sb[A::kQuadsN];
 
     __device__ __forceinline__ void load(const KArgs& p, uint32_t m0, uint32_t n0, int wm, int wn,
-                                         int lane, int vec_ok)
+                                         int lane)
     {
         const uint32_t mb = m0 + wm * C::kWaveM;
         const uint32_t nb = n0 + wn * C::kWaveN;
@@ -540,21 +553,13 @@ struct EpiScales {
         if(p.sb == nullptr) {
 #pragma unroll
             for(int j = 0; j < A::kQuadsN; ++j) sb[j] = make_float4(p.tsb, p.tsb, p.tsb, p.tsb);
-        } else if(vec_ok && n0 + C::kBN <= p.n) {
+        } else if(n0 + C::kBN <= p.n) {
 #pragma unroll
             for(int j = 0; j < A::kQuadsN; ++j)
-                sb[j] = *reinterpret_cast<const float4*>(p.sb + nb + A::col(j, lane));
+                __builtin_memcpy(&sb[j], p.sb + nb + A::col(j, lane), 16);
         } else {
 #pragma unroll
-            for(int j = 0; j < A::kQuadsN; ++j) {
-                const uint32_t n = nb + A::col(j, lane);
-                float4         v = make_float4(p.tsb, p.tsb, p.tsb, p.tsb);
-                if(n + 0 < p.n) v.x = p.sb[n + 0];
-                if(n + 1 < p.n) v.y = p.sb[n + 1];
-                if(n + 2 < p.n) v.z = p.sb[n + 2];
-                if(n + 3 < p.n) v.w = p.sb[n + 3];
-                sb[j] = v;
-            }
+            for(int j = 0; j < A::kQuadsN; ++j) sb[j] = load_sb4(p, nb + A::col(j, lane), p.tsb);
         }
     }
 };
@@ -585,8 +590,7 @@ struct StageSwz {
 };
 
 template <class C>
-__device__ __forceinline__ void epilogue_f16_lds(const KArgs& p, uint32_t m0, uint32_t n0,
-                                                 int vec_ok, int8_t* lds, int slot, int lane,
+__device__ __forceinline__ void epilogue_f16_lds(const KArgs& p, uint32_t m0, uint32_t n0, int8_t* lds, int slot, int lane,
                                                  int wm, int wn, const Acc<C>& acc,
                                                  const EpiScales<C>& sc)
 {
@@ -626,11 +630,12 @@ __device__ __forceinline__ void epilogue_f16_lds(const KArgs& p, uint32_t m0, ui
     }
     // a wave reads back only what it wrote itself: LDS returns each wave's
     // accesses in order, so no barrier is needed between the two phases
-    const bool     st16  = vec_ok && (reinterpret_cast<uintptr_t>(p.c) % 16 == 0) && (p.ldc % 8 == 0);
     const int      chunk = lane % kRowChunks;
     const uint32_t n     = n0 + wn * C::kWaveN + chunk * 8;
-    // a tile wholly inside C with 16-byte rows: every store is a whole chunk
-    const bool     inner = st16 && m0 + C::kBM <= p.m && n0 + C::kBN <= p.n;
+    // a tile wholly inside C: every store is a whole chunk.  C and ldc may have
+    // any alignment: the hardware takes unaligned 16-byte stores (4095 x 4095
+    // outputs of K = 4096, odd rows, a layer 86 us with 2-byte stores there, 67 now)
+    const bool     inner = m0 + C::kBM <= p.m && n0 + C::kBN <= p.n;
     constexpr int  kSt   = C::kWaveM / kRowsPerSt; // stores per lane
     constexpr int  kBat  = kSt < 4 ? kSt : 4;
     static_assert(kSt % kBat == 0, "whole batches");
@@ -656,12 +661,12 @@ __device__ __forceinline__ void epilogue_f16_lds(const KArgs& p, uint32_t m0, ui
             const v4i      v   = out[b];
             uint16_t*      dst = reinterpret_cast<uint16_t*>(p.c) + (size_t)m * p.ldc + n;
             if(inner) {
-                *reinterpret_cast<v4i*>(dst) = v;
+                __builtin_memcpy(dst, &v, 16);
                 continue;
             }
             if(m >= p.m || n >= p.n) continue;
-            if(st16 && n + 8 <= p.n) {
-                *reinterpret_cast<v4i*>(dst) = v;
+            if(n + 8 <= p.n) {
+                __builtin_memcpy(dst, &v, 16);
             } else {
                 const uint32_t w[4] = {(uint32_t)v.x, (uint32_t)v.y, (uint32_t)v.z, (uint32_t)v.w};
 #pragma unroll
@@ -730,8 +735,7 @@ __device__ __forceinline__ void add_partial(const int32_t* part, uint32_t tid, A
 }
 
 template <class C, int OUT>
-__device__ __forceinline__ void tile_epilogue_sc(const KArgs& p, uint32_t m0, uint32_t n0,
-                                                 int vec_ok, int8_t* lds,
+__device__ __forceinline__ void tile_epilogue_sc(const KArgs& p, uint32_t m0, uint32_t n0, int8_t* lds,
                                                  const Acc<C>& acc, int wave_base,
                                                  const EpiScales<C>& sc);
 
@@ -741,8 +745,7 @@ __device__ __forceinline__ void tile_epilogue_sc(const KArgs& p, uint32_t m0, ui
 // SCALES: the fp16 epilogue's scales go into `sc` while the last k-tile's
 // MFMAs run.
 template <class C, bool SCALES>
-__device__ __forceinline__ void gemm_tile_acc(const KArgs& p, uint32_t m0, uint32_t n0,
-                                              int vec_ok, int8_t* lds, uint32_t kt0,
+__device__ __forceinline__ void gemm_tile_acc(const KArgs& p, uint32_t m0, uint32_t n0, int8_t* lds, uint32_t kt0,
                                               uint32_t nk, Acc<C>& acc, EpiScales<C>& sc)
 {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave); // wave-uniform
@@ -835,7 +838,7 @@ __device__ __forceinline__ void gemm_tile_acc(const KArgs& p, uint32_t m0, uint3
                                     0);
     }
     // the fp16 epilogue's scales load while the last tile's MFMAs run
-    if constexpr(SCALES) sc.load(p, m0, n0, wm, wn, lane, vec_ok);
+    if constexpr(SCALES) sc.load(p, m0, n0, wm, wn, lane);
     {
         const int8_t* sbase = lds + ((nk - 1) % C::kStages) * C::kStageBytes;
 #pragma unroll
@@ -851,19 +854,19 @@ __device__ __forceinline__ void gemm_tile_acc(const KArgs& p, uint32_t m0, uint3
 // PART: only k-tiles [kt0, kt0 + nkt) are summed and the int32 accumulators
 // go to `part` (store_partial layout) instead of through the epilogue.
 template <class C, int OUT, bool PART = false>
-__device__ __forceinline__ void gemm_tile(const KArgs& p, uint32_t m0, uint32_t n0, int vec_ok,
+__device__ __forceinline__ void gemm_tile(const KArgs& p, uint32_t m0, uint32_t n0,
                                           int8_t* lds, uint32_t kt0 = 0, uint32_t nkt = 0,
                                           int32_t* part = nullptr)
 {
     Acc<C>       acc;
     EpiScales<C> sc;
     if constexpr(PART) {
-        gemm_tile_acc<C, false>(p, m0, n0, vec_ok, lds, kt0, nkt, acc, sc);
+        gemm_tile_acc<C, false>(p, m0, n0, lds, kt0, nkt, acc, sc);
         store_partial<C>(part, acc);
     } else {
-        gemm_tile_acc<C, OUT == W8A8_OUT_F16>(p, m0, n0, vec_ok, lds, 0,
+        gemm_tile_acc<C, OUT == W8A8_OUT_F16>(p, m0, n0, lds, 0,
                                               (p.k + C::kBK - 1) / C::kBK, acc, sc);
-        tile_epilogue_sc<C, OUT>(p, m0, n0, vec_ok, lds, acc, 0, sc);
+        tile_epilogue_sc<C, OUT>(p, m0, n0, lds, acc, 0, sc);
     }
 }
 
@@ -873,8 +876,7 @@ __device__ __forceinline__ void gemm_tile(const KArgs& p, uint32_t m0, uint32_t 
 // split-tile fixup); each wave stages through LDS slice threadIdx.x / 64.
 // sc: the fp16 path's scales, loaded by the caller (unused for int32 output).
 template <class C, int OUT>
-__device__ __forceinline__ void tile_epilogue_sc(const KArgs& p, uint32_t m0, uint32_t n0,
-                                                 int vec_ok, int8_t* lds, const Acc<C>& acc,
+__device__ __forceinline__ void tile_epilogue_sc(const KArgs& p, uint32_t m0, uint32_t n0, int8_t* lds, const Acc<C>& acc,
                                                  int wave_base, const EpiScales<C>& sc)
 {
     const int   slot  = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
@@ -885,7 +887,7 @@ __device__ __forceinline__ void tile_epilogue_sc(const KArgs& p, uint32_t m0, ui
     const bool  mode1 = (p.sa == nullptr && p.sb == nullptr);
     const float ab    = p.tsa * p.tsb;
     if constexpr(OUT == W8A8_OUT_F16) {
-        epilogue_f16_lds<C>(p, m0, n0, vec_ok, lds, slot, lane, wm, wn, acc, sc);
+        epilogue_f16_lds<C>(p, m0, n0, lds, slot, lane, wm, wn, acc, sc);
         return;
     }
     // int32 output: straight from the registers
@@ -898,8 +900,7 @@ __device__ __forceinline__ void tile_epilogue_sc(const KArgs& p, uint32_t m0, ui
             const uint32_t n    = n0 + wn * C::kWaveN + A::col(j, lane);
             const v4i      q    = acc.quad(i, j);
             const int      v[4] = {q.x, q.y, q.z, q.w};
-            store4<OUT>(p, m, n, v, p.tsa, make_float4(p.tsb, p.tsb, p.tsb, p.tsb), ab, mode1,
-                        vec_ok != 0);
+            store4<OUT>(p, m, n, v, p.tsa, make_float4(p.tsb, p.tsb, p.tsb, p.tsb), ab, mode1);
         }
     }
 }
@@ -907,27 +908,26 @@ __device__ __forceinline__ void tile_epilogue_sc(const KArgs& p, uint32_t m0, ui
 // Epilogue of a tile whose scales are not loaded yet (K-split fixups,
 // grouped and MoE fixups): one batch of scale loads, then the epilogue.
 template <class C, int OUT>
-__device__ __forceinline__ void tile_epilogue(const KArgs& p, uint32_t m0, uint32_t n0,
-                                              int vec_ok, int8_t* lds, const Acc<C>& acc,
+__device__ __forceinline__ void tile_epilogue(const KArgs& p, uint32_t m0, uint32_t n0, int8_t* lds, const Acc<C>& acc,
                                               int wave_base = 0)
 {
     EpiScales<C> sc;
     if constexpr(OUT == W8A8_OUT_F16) {
         const int wave = wave_base + __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-        sc.load(p, m0, n0, wave / C::kWavesN, wave % C::kWavesN, threadIdx.x % kWave, vec_ok);
+        sc.load(p, m0, n0, wave / C::kWavesN, wave % C::kWavesN, threadIdx.x % kWave);
     }
-    tile_epilogue_sc<C, OUT>(p, m0, n0, vec_ok, lds, acc, wave_base, sc);
+    tile_epilogue_sc<C, OUT>(p, m0, n0, lds, acc, wave_base, sc);
 }
 
 template <class C, int OUT>
-__global__ void __launch_bounds__(C::kThreads, 1) gemm_i8_tile_kernel(KArgs p, int vec_ok)
+__global__ void __launch_bounds__(C::kThreads, 1) gemm_i8_tile_kernel(KArgs p)
 {
     extern __shared__ __attribute__((aligned(1024))) int8_t lds[];
     const uint32_t tiles_m = (p.m + C::kBM - 1) / C::kBM;
     const uint32_t tiles_n = (p.n + C::kBN - 1) / C::kBN;
     uint32_t       tm, tn;
     tile_coords<C::kGroupM>(xcd_remap(blockIdx.x, tiles_m * tiles_n), tiles_m, tiles_n, tm, tn);
-    gemm_tile<C, OUT>(p, tm * C::kBM, tn * C::kBN, vec_ok, lds);
+    gemm_tile<C, OUT>(p, tm * C::kBM, tn * C::kBN, lds);
 }
 
 // K split of a launch whose tiles fill at most half of the CUs: logical
@@ -942,7 +942,7 @@ __global__ void __launch_bounds__(C::kThreads, 1) gemm_i8_tile_kernel(KArgs p, i
 // the weights four times).
 template <class C, int OUT>
 __global__ void __launch_bounds__(C::kThreads, 1)
-    gemm_i8_split_kernel(KArgs p, int vec_ok, int32_t* ws, uint32_t parts)
+    gemm_i8_split_kernel(KArgs p, int32_t* ws, uint32_t parts)
 {
     extern __shared__ __attribute__((aligned(1024))) int8_t lds[];
     const uint32_t tiles_m = (p.m + C::kBM - 1) / C::kBM;
@@ -953,13 +953,13 @@ __global__ void __launch_bounds__(C::kThreads, 1)
     tile_coords<C::kGroupM>(slot, tiles_m, tiles_n, tm, tn);
     const uint32_t nk  = (p.k + C::kBK - 1) / C::kBK;
     const uint32_t kt0 = part * nk / parts, kt1 = (part + 1) * nk / parts;
-    gemm_tile<C, OUT, true>(p, tm * C::kBM, tn * C::kBN, vec_ok, lds, kt0, kt1 - kt0,
+    gemm_tile<C, OUT, true>(p, tm * C::kBM, tn * C::kBN, lds, kt0, kt1 - kt0,
                             ws + (size_t)lid * Partial<C>::kInts);
 }
 
 template <class C, int OUT>
 __global__ void __launch_bounds__(Partial<C>::kFixupWaves * kWave, 1)
-    gemm_i8_split_fixup_kernel(KArgs p, int vec_ok, const int32_t* ws, uint32_t parts)
+    gemm_i8_split_fixup_kernel(KArgs p, const int32_t* ws, uint32_t parts)
 {
     extern __shared__ __attribute__((aligned(1024))) int8_t lds[];
     const uint32_t tiles_m   = (p.m + C::kBM - 1) / C::kBM;
@@ -973,7 +973,7 @@ __global__ void __launch_bounds__(Partial<C>::kFixupWaves * kWave, 1)
     const uint32_t tid = wave_base * kWave + threadIdx.x;
     for(uint32_t part = 0; part < parts; ++part)
         add_partial<C>(ws + (size_t)(slot * parts + part) * Partial<C>::kInts, tid, acc);
-    tile_epilogue<C, OUT>(p, tm * C::kBM, tn * C::kBN, vec_ok, lds, acc, wave_base);
+    tile_epilogue<C, OUT>(p, tm * C::kBM, tn * C::kBN, lds, acc, wave_base);
 }
 
 template <class C, int OUT>
@@ -1003,24 +1003,24 @@ void raise_split_lds_once()
 // Launch one configuration; the caller has validated the fast-path
 // preconditions (16-byte aligned a/b, lda/ldb/k multiples of 16).
 template <class C>
-hipError_t launch_cfg(const KArgs& p, int out_type, int vec_ok, hipStream_t stream)
+hipError_t launch_cfg(const KArgs& p, int out_type, hipStream_t stream)
 {
     const uint32_t tiles = ((p.m + C::kBM - 1) / C::kBM) * ((p.n + C::kBN - 1) / C::kBN);
     if(out_type == W8A8_OUT_I32) {
         raise_lds_limit_once<C, W8A8_OUT_I32>();
         hipLaunchKernelGGL((gemm_i8_tile_kernel<C, W8A8_OUT_I32>), dim3(tiles), dim3(C::kThreads),
-                           C::kLdsBytes, stream, p, vec_ok);
+                           C::kLdsBytes, stream, p);
     } else {
         raise_lds_limit_once<C, W8A8_OUT_F16>();
         hipLaunchKernelGGL((gemm_i8_tile_kernel<C, W8A8_OUT_F16>), dim3(tiles), dim3(C::kThreads),
-                           C::kLdsBytes, stream, p, vec_ok);
+                           C::kLdsBytes, stream, p);
     }
     return hipGetLastError();
 }
 
 // Split launch (see gemm_i8_split_kernel): ws holds tiles * parts partials.
 template <class C>
-hipError_t launch_cfg_split(const KArgs& p, int out_type, int vec_ok, int32_t* ws,
+hipError_t launch_cfg_split(const KArgs& p, int out_type, int32_t* ws,
                             uint32_t parts, hipStream_t stream)
 {
     const uint32_t tiles  = ((p.m + C::kBM - 1) / C::kBM) * ((p.n + C::kBN - 1) / C::kBN);
@@ -1029,15 +1029,15 @@ hipError_t launch_cfg_split(const KArgs& p, int out_type, int vec_ok, int32_t* w
     if(out_type == W8A8_OUT_I32) {
         raise_split_lds_once<C, W8A8_OUT_I32>();
         hipLaunchKernelGGL((gemm_i8_split_kernel<C, W8A8_OUT_I32>), grid, dim3(C::kThreads),
-                           C::kLdsBytes, stream, p, vec_ok, ws, parts);
+                           C::kLdsBytes, stream, p, ws, parts);
         hipLaunchKernelGGL((gemm_i8_split_fixup_kernel<C, W8A8_OUT_I32>), fgrid, fblock,
-                           Partial<C>::kFixupLds, stream, p, vec_ok, ws, parts);
+                           Partial<C>::kFixupLds, stream, p, ws, parts);
     } else {
         raise_split_lds_once<C, W8A8_OUT_F16>();
         hipLaunchKernelGGL((gemm_i8_split_kernel<C, W8A8_OUT_F16>), grid, dim3(C::kThreads),
-                           C::kLdsBytes, stream, p, vec_ok, ws, parts);
+                           C::kLdsBytes, stream, p, ws, parts);
         hipLaunchKernelGGL((gemm_i8_split_fixup_kernel<C, W8A8_OUT_F16>), fgrid, fblock,
-                           Partial<C>::kFixupLds, stream, p, vec_ok, ws, parts);
+                           Partial<C>::kFixupLds, stream, p, ws, parts);
     }
     return hipGetLastError();
 }

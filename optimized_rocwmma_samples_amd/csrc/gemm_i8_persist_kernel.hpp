@@ -130,7 +130,7 @@ __device__ __forceinline__ void epilogue_f16_persist(const KArgs& p, __amdgpu_bu
 }
 
 template <class C>
-__global__ void __launch_bounds__(C::kThreads, 1) gemm_i8_persist_kernel(KArgs p, int vec_ok, int nt)
+__global__ void __launch_bounds__(C::kThreads, 1) gemm_i8_persist_kernel(KArgs p, int nt)
 {
     using P = Persist<C>;
     static_assert(C::kStages >= 2, "ring");
@@ -289,7 +289,7 @@ __global__ void __launch_bounds__(C::kThreads, 1) gemm_i8_persist_kernel(KArgs p
         int elane = lane;
         asm volatile("" : "+v"(elane));
         EpiScales<C> sc;
-        sc.load(p, m0, n0, wm, wn, elane, vec_ok);
+        sc.load(p, m0, n0, wm, wn, elane);
         kstep(nk == 1 && j > 0, std::true_type{});
         __builtin_amdgcn_sched_barrier(0);
         if(nt)
@@ -319,21 +319,21 @@ void raise_persist_lds_once()
 // (blocks = CUs, a multiple of 8), 8-column chunks that never straddle N,
 // 16-byte aligned rows of C, and C within the 32-bit buffer range.
 template <class C>
-bool persist_ok(const KArgs& p, int vec_ok, uint32_t cus)
+bool persist_ok(const KArgs& p, uint32_t cus)
 {
     const uint64_t tiles = (uint64_t)((p.m + C::kBM - 1) / C::kBM) * ((p.n + C::kBN - 1) / C::kBN);
-    return vec_ok && cus >= 8 && cus % 8 == 0 && tiles >= 2ull * cus && p.n % 8 == 0
+    return cus >= 8 && cus % 8 == 0 && tiles >= 2ull * cus && p.n % 8 == 0
            && p.ldc % 8 == 0 && reinterpret_cast<uintptr_t>(p.c) % 16 == 0
            && ((uint64_t)(p.m - 1) * p.ldc + p.n) * 2 < 0x80000000ull;
 }
 
 template <class C>
-hipError_t launch_cfg_persist(const KArgs& p, int vec_ok, uint32_t cus, hipStream_t stream)
+hipError_t launch_cfg_persist(const KArgs& p, uint32_t cus, hipStream_t stream)
 {
     raise_persist_lds_once<C>();
     const int nt = (uint64_t)p.m * p.ldc * 2 >= kMallBytes / 4;
     hipLaunchKernelGGL((gemm_i8_persist_kernel<C>), dim3(cus), dim3(C::kThreads),
-                       Persist<C>::kLdsBytes, stream, p, vec_ok, nt);
+                       Persist<C>::kLdsBytes, stream, p, nt);
     return hipGetLastError();
 }
 

@@ -166,7 +166,7 @@ __global__ void __launch_bounds__(256) streamk_clear_kernel(uint32_t* sync, uint
 
 template <class C, int OUT>
 __global__ void __launch_bounds__(C::kThreads, 1)
-    gemm_i8_streamk_kernel(KArgs p, int vec_ok, uint32_t t0, SkPlan sk, uint32_t* sync,
+    gemm_i8_streamk_kernel(KArgs p, uint32_t t0, SkPlan sk, uint32_t* sync,
                            int32_t* part, SkWatch watch)
 {
     extern __shared__ __attribute__((aligned(1024))) int8_t lds[];
@@ -187,7 +187,7 @@ __global__ void __launch_bounds__(C::kThreads, 1)
         const uint32_t m0 = tm * C::kBM, n0 = tn * C::kBN;
         Acc<C>         acc;
         EpiScales<C>   unused;
-        gemm_tile_acc<C, false>(p, m0, n0, vec_ok, lds, k0, k1 - k0, acc, unused);
+        gemm_tile_acc<C, false>(p, m0, n0, lds, k0, k1 - k0, acc, unused);
         if(k0 != 0 || k1 != sk.nk) {
             // ---- a piece: arrival order, and this tile's first slot -------
             uint32_t* arrive = sync + 2 * t;
@@ -233,7 +233,7 @@ __global__ void __launch_bounds__(C::kThreads, 1)
             for(uint32_t q = 0; q + 1 < pieces; ++q)
                 add_partial_dev<C>(part + (size_t)(base + q) * Partial<C>::kInts, acc);
         }
-        tile_epilogue<C, OUT>(p, m0, n0, vec_ok, lds, acc);
+        tile_epilogue<C, OUT>(p, m0, n0, lds, acc);
     }
 }
 
@@ -251,7 +251,7 @@ void raise_streamk_lds_once()
 // Stream-K launch over logical tiles [t0, t0 + s.ntiles) with s.blocks blocks;
 // ws holds sk_workspace_bytes<C>(s) bytes (16-byte aligned).
 template <class C>
-hipError_t launch_cfg_streamk(const KArgs& p, int out_type, int vec_ok, uint32_t t0,
+hipError_t launch_cfg_streamk(const KArgs& p, int out_type, uint32_t t0,
                               const SkPlan& s, void* ws, const SkWatch& watch, hipStream_t stream)
 {
     uint32_t*      sync = static_cast<uint32_t*>(ws);
@@ -262,12 +262,12 @@ hipError_t launch_cfg_streamk(const KArgs& p, int out_type, int vec_ok, uint32_t
     if(out_type == W8A8_OUT_I32) {
         raise_streamk_lds_once<C, W8A8_OUT_I32>();
         hipLaunchKernelGGL((gemm_i8_streamk_kernel<C, W8A8_OUT_I32>), dim3(s.blocks),
-                           dim3(C::kThreads), C::kLdsBytes, stream, p, vec_ok, t0, s, sync, part,
+                           dim3(C::kThreads), C::kLdsBytes, stream, p, t0, s, sync, part,
                            watch);
     } else {
         raise_streamk_lds_once<C, W8A8_OUT_F16>();
         hipLaunchKernelGGL((gemm_i8_streamk_kernel<C, W8A8_OUT_F16>), dim3(s.blocks),
-                           dim3(C::kThreads), C::kLdsBytes, stream, p, vec_ok, t0, s, sync, part,
+                           dim3(C::kThreads), C::kLdsBytes, stream, p, t0, s, sync, part,
                            watch);
     }
     return hipGetLastError();

@@ -887,17 +887,17 @@ uint32_t device_cus()
 } // namespace
 
 hipError_t launch_grouped_gemm(const w8a8_group_desc* groups_dev, uint32_t ngroups,
-                               uint32_t total_tiles, int cfg, int out_type, int vec_ok,
+                               uint32_t total_tiles, int cfg, int out_type,
                                hipStream_t stream)
 {
     const auto* g = reinterpret_cast<const gemm::KArgs*>(groups_dev);
     if(cfg == 1)
-        return gemm::launch_grouped<GemmGroupedMid>(g, ngroups, total_tiles, out_type, vec_ok,
+        return gemm::launch_grouped<GemmGroupedMid>(g, ngroups, total_tiles, out_type,
                                                     stream);
     if(cfg == 2)
-        return gemm::launch_grouped<GemmGroupedSmall>(g, ngroups, total_tiles, out_type, vec_ok,
+        return gemm::launch_grouped<GemmGroupedSmall>(g, ngroups, total_tiles, out_type,
                                                       stream);
-    return gemm::launch_grouped<GemmGrouped>(g, ngroups, total_tiles, out_type, vec_ok, stream);
+    return gemm::launch_grouped<GemmGrouped>(g, ngroups, total_tiles, out_type, stream);
 }
 
 uint32_t grouped_gemm_tiles(uint32_t m, uint32_t n, int cfg)
@@ -944,14 +944,10 @@ hipError_t launch_moe_gemm(const MoeGemmArgs& a, hipStream_t stream)
     const bool split = a.ws != nullptr && a.ws_bytes >= moe_gemm_workspace_bytes();
     q.ws           = split ? static_cast<int32_t*>(a.ws) : nullptr;
     q.cus          = split ? device_cus() : 0;
-    const size_t esz    = a.out_type == W8A8_OUT_I32 ? 4 : 2;
-    const int    vec_ok = reinterpret_cast<uintptr_t>(a.c) % (4 * esz) == 0 && a.ldc % 4 == 0
-                       && (a.scale_w == nullptr
-                           || (reinterpret_cast<uintptr_t>(a.scale_w) % 16 == 0 && a.n % 4 == 0));
     // rows (the sort's padded capacity) / experts stands for the rows per expert
     if(moe_tile_rows_128(a.rows, a.experts))
-        return gemm::launch_moe<GemmGroupedMid>(q, a.out_type, vec_ok, stream);
-    return gemm::launch_moe<GemmGrouped, GemmGroupedWide>(q, a.out_type, vec_ok, stream);
+        return gemm::launch_moe<GemmGroupedMid>(q, a.out_type, stream);
+    return gemm::launch_moe<GemmGrouped, GemmGroupedWide>(q, a.out_type, stream);
 }
 
 // The SiLU epilogue's tiles: wave tiles 128 columns wide (64 outputs, one
@@ -1008,10 +1004,9 @@ hipError_t launch_moe_gate_up_silu(const MoeSiluArgs& a, hipStream_t stream)
     q.cus          = device_cus();
     // pmax group-major: row stride ldp = rows
     const gemm::SiluOut so{h, pmax, a.s2, a.inter, a.rows, a.inter};
-    const int vec_ok = a.scale_w == nullptr || reinterpret_cast<uintptr_t>(a.scale_w) % 16 == 0;
     hipError_t e = moe_tile_rows_128(a.rows, a.experts)
-                       ? gemm::launch_moe_silu<GemmSiluMid>(q, so, vec_ok, stream)
-                       : gemm::launch_moe_silu<GemmSilu, GemmSiluWide>(q, so, vec_ok, stream);
+                       ? gemm::launch_moe_silu<GemmSiluMid>(q, so, stream)
+                       : gemm::launch_moe_silu<GemmSilu, GemmSiluWide>(q, so, stream);
     if(e != hipSuccess) return e;
 
     const uint64_t h_bytes  = (uint64_t)a.rows * a.inter * 2;

@@ -182,7 +182,7 @@ uint32_t   grouped_gemm_tiles(uint32_t m, uint32_t n, int cfg);
 // the CUs (tiles[c] = total tiles of configuration c), else 128 x 128.
 int        grouped_gemm_cfg(const uint64_t tiles[3]);
 hipError_t launch_grouped_gemm(const w8a8_group_desc* groups_dev, uint32_t ngroups,
-                               uint32_t total_tiles, int cfg, int out_type, int vec_ok,
+                               uint32_t total_tiles, int cfg, int out_type,
                                hipStream_t stream);
 
 struct MoeGemmArgs {

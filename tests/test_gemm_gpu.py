@@ -151,6 +151,33 @@ def test_k_split_exact(w8a8, gpu, m, n, k):
     assert_f16_bitexact(cf[rows], O.dequant_f16(acc, sa[rows], sb))
 
 
+# Outputs at odd rows and addresses: 16-byte stores of interior tiles, and the
+# elements around the matrix untouched, for each tile and the decode kernels.
+@pytest.mark.parametrize("m,n,k", [(4100, 3001, 160), (1500, 4001, 272), (513, 4099, 272),
+                                   (100, 1003, 1040), (40, 515, 400), (3, 77, 64)])
+def test_unaligned_outputs_exact(w8a8, gpu, m, n, k):
+    import torch
+    a, b, sa, sb = inputs(m, n, k, m + 2 * n + k)
+    ad, bd = dev(a, gpu), dev(b, gpu)
+    sbd = torch.empty(n + 1, dtype=torch.float32, device=gpu)[1:].copy_(dev(sb, gpu))
+    pw = w8a8.pack_weights(bd)
+    acc = O.gemm_i32(a, b)
+    want = O.dequant_f16(acc, sa, sb)
+    for packed in (False, True):
+        for dt in (torch.float16, torch.int32):
+            buf = torch.full((m * (n + 2) + 1,), 7, dtype=dt, device=gpu)
+            out = buf[1:].view(m, n + 2)[:, :n]
+            sc = (dev(sa, gpu), sbd) if dt == torch.float16 else (None, None)
+            if packed:
+                w8a8.gemm_packed(ad, pw, *sc, out=out)
+            else:
+                w8a8.gemm(ad, bd, *sc, out=out)
+            got = host(buf)
+            assert got[0] == 7 and (got[1:].reshape(m, n + 2)[:, n:] == 7).all()
+            got = np.ascontiguousarray(got[1:].reshape(m, n + 2)[:, :n])
+            assert_f16_bitexact(got, want) if dt == torch.float16 else assert_i32_equal(got, acc)
+
+
 # The direct kernel (any pointer, row stride and K): tails of 1, 15 and 16 bytes
 # either side of a k-tile, single rows and columns, K below 16, each tile size
 # (64, 128 and 256 rows), operands 1-7 bytes off alignment.
