@@ -524,48 +524,57 @@ struct SiluRequant {
     uint32_t        h_bytes, p_bytes, q_bytes, s2_bytes; // buffer extents (< 2 GiB)
 };
 
-// A block of kSqThreads threads takes kRqRows consecutive rows.  Phase 1:
-// the rows' maxima over all groups (thread t reads row t % kRqRows of groups
-// t / kRqRows, + kRqSlots, ...: kRqRows consecutive floats per group, one
-// segment per wave instruction), reduced through LDS, and the rows' experts.
-// Phase 2: each wave quantizes kRqRows / kSqWaves rows, kRqBatch 8-column
-// chunks per lane in flight (h and s2 loads issued before any store).
-// 8 rows per block: cfg5's 8448 rows make 1056 blocks, 4.1 per CU; with 16
-// rows (528 blocks, 2.06 per CU) the CUs holding a third block finished alone
-// (cfg5 layer 1535-1547 -> 1526-1528 us, same box, alternating).
+// A block of kSqThreads threads takes ROWS consecutive rows.  Phase 1:
+// the rows' maxima over all groups (thread t reads row t % ROWS of groups
+// t / ROWS, + kSlots, ...: ROWS consecutive floats per group, one segment per
+// wave instruction), reduced through LDS, and the rows' experts.
+// Phase 2: kRqBatch 8-column chunks per lane in flight (h and s2 loads issued
+// before any store), each wave over ROWS / kSqWaves whole rows or, with one
+// row per block, over its share of the row's columns.
+// 8 rows per block where they make two blocks a CU: cfg5's 8448 rows make
+// 1056, 4.1 per CU; with 16 rows (528 blocks, 2.06 per CU) the CUs holding a
+// third block finished alone (cfg5 layer 1535-1547 -> 1526-1528 us, same box,
+// alternating).  Fewer rows take a block each, or most CUs idle while a few
+// stream 8 rows one after another: 288 rows of 14336 17.1 -> 5.2 us.
 constexpr int kRqRows  = 8;
-constexpr int kRqSlots = kSqThreads / kRqRows;
 constexpr int kRqBatch = 7;
 
-template <bool S2>
+template <bool S2, int ROWS>
 __global__ void __launch_bounds__(kSqThreads) silu_requant_kernel(SiluRequant p)
 {
-    constexpr uint32_t kOob = gemm::kOob;
-    __shared__ float   red[kRqSlots][kRqRows];
-    __shared__ float   rowmax[kRqRows];
-    __shared__ int     rowexp[kRqRows];
+    constexpr uint32_t kOob   = gemm::kOob;
+    constexpr int      kSlots = kSqThreads / ROWS;
+    constexpr int      kRed   = ROWS == 1 ? kSqWaves : kSlots;
+    __shared__ float   red[kRed][ROWS];
+    __shared__ float   rowmax[ROWS];
+    __shared__ int     rowexp[ROWS];
     const int          t    = threadIdx.x;
     const int          wave = t / kWave;
     const int          lane = t % kWave;
-    const uint32_t     r0   = blockIdx.x * kRqRows;
+    const uint32_t     r0   = blockIdx.x * ROWS;
 
     const __amdgpu_buffer_rsrc_t rp = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<float*>(p.pmax), 0, (int)p.p_bytes, gemm::kBufferFlags);
     {
-        const uint32_t row = r0 + t % kRqRows;
+        const uint32_t row = r0 + t % ROWS;
         float          mx  = 0.f;
-        for(uint32_t g = t / kRqRows; g < p.groups; g += kRqSlots) {
+        for(uint32_t g = t / ROWS; g < p.groups; g += kSlots) {
             const uint32_t o = row < p.rows ? (g * p.ldp + row) * 4 : kOob;
             mx = fmaxf(mx, __int_as_float(__builtin_amdgcn_raw_buffer_load_b32(rp, o, 0, 0)));
         }
-        red[t / kRqRows][t % kRqRows] = mx;
-        if(t < kRqRows) rowexp[t] = r0 + t < p.rows ? row_expert(p, r0 + t) : -1;
+        if constexpr(ROWS == 1) {
+            mx = wave_max(mx);
+            if(lane == 0) red[wave][0] = mx;
+        } else {
+            red[t / ROWS][t % ROWS] = mx;
+        }
+        if(t < ROWS) rowexp[t] = r0 + t < p.rows ? row_expert(p, r0 + t) : -1;
     }
     __syncthreads();
-    if(t < kRqRows) {
+    if(t < ROWS) {
         float mx = 0.f;
 #pragma unroll
-        for(int sl = 0; sl < kRqSlots; ++sl) mx = fmaxf(mx, red[sl][t]);
+        for(int sl = 0; sl < kRed; ++sl) mx = fmaxf(mx, red[sl][t]);
         rowmax[t] = mx;
     }
     __syncthreads();
@@ -578,14 +587,16 @@ __global__ void __launch_bounds__(kSqThreads) silu_requant_kernel(SiluRequant p)
     const __amdgpu_buffer_rsrc_t rq = __builtin_amdgcn_make_buffer_rsrc(p.q, 0, (int)p.q_bytes,
                                                                         gemm::kBufferFlags);
     const float qmax = p.qmax;
-    for(int rr = wave; rr < kRqRows; rr += kSqWaves) {
+    constexpr uint32_t kSpan  = kRqBatch * 8 * kWave; // columns of one batch of a wave
+    constexpr uint32_t kStep  = ROWS == 1 ? kSqWaves * kSpan : kSpan;
+    for(int rr = ROWS == 1 ? 0 : wave; rr < ROWS; rr += ROWS == 1 ? 1 : kSqWaves) {
         const uint32_t row   = r0 + rr;
         const int      e     = rowexp[rr];
         if(e < 0) continue; // wave-uniform: padding rows and rows past the end
         const float    rsc   = rowmax[rr] / qmax;
         const float    inv   = rsc > 0.f ? 1.f / rsc : 0.f;
-        if(lane == 0) p.r[row] = rsc;
-        for(uint32_t c0 = 0; c0 < n; c0 += kRqBatch * 8 * kWave) {
+        if(lane == 0 && (ROWS > 1 || wave == 0)) p.r[row] = rsc;
+        for(uint32_t c0 = ROWS == 1 ? wave * kSpan : 0; c0 < n; c0 += kStep) {
             v4i      hv[kRqBatch], s0[kRqBatch], s1[kRqBatch];
             uint32_t col[kRqBatch];
 #pragma unroll
@@ -629,14 +640,32 @@ __global__ void __launch_bounds__(kSqThreads) silu_requant_kernel(SiluRequant p)
     }
 }
 
+uint32_t device_cus()
+{
+    static const uint32_t cus = [] {
+        int dev = 0, c = 256;
+        if(hipGetDevice(&dev) == hipSuccess)
+            (void)hipDeviceGetAttribute(&c, hipDeviceAttributeMultiprocessorCount, dev);
+        return (uint32_t)c;
+    }();
+    return cus;
+}
+
+template <int ROWS>
+hipError_t launch_requant_rows(const SiluRequant& p, hipStream_t stream)
+{
+    const dim3 grid((p.rows + ROWS - 1) / ROWS);
+    if(p.s2 != nullptr)
+        hipLaunchKernelGGL((silu_requant_kernel<true, ROWS>), grid, dim3(kSqThreads), 0, stream, p);
+    else
+        hipLaunchKernelGGL((silu_requant_kernel<false, ROWS>), grid, dim3(kSqThreads), 0, stream, p);
+    return hipGetLastError();
+}
+
 hipError_t launch_requant(const SiluRequant& p, hipStream_t stream)
 {
-    const dim3 grid((p.rows + kRqRows - 1) / kRqRows);
-    if(p.s2 != nullptr)
-        hipLaunchKernelGGL(silu_requant_kernel<true>, grid, dim3(kSqThreads), 0, stream, p);
-    else
-        hipLaunchKernelGGL(silu_requant_kernel<false>, grid, dim3(kSqThreads), 0, stream, p);
-    return hipGetLastError();
+    return p.rows < 2u * kRqRows * device_cus() ? launch_requant_rows<1>(p, stream)
+                                                : launch_requant_rows<kRqRows>(p, stream);
 }
 
 // Gate_up weights interleaved for the SiLU epilogue: output row r of expert
@@ -731,20 +760,43 @@ using GemmGrouped = gemm::Cfg<256, 256, 128, 2, 2, 4, 4, 16>;
 // 128 x 512 tiles (8 waves of 128 x 64, as GemmGrouped; 2 stages of 80 KiB).
 using GemmGroupedWide = gemm::Cfg<128, 512, 128, 2, 1, 8, 4, 16>;
 // MoE GEMM over experts of a few hundred rows: 128-row tiles waste less of
-// each expert's last tile row (moe_tile_rows_128).
+// each expert's last tile row (moe_tile).
 using GemmGroupedMid = gemm::Cfg<128, 256, 128, 3, 2, 4, 4, 16>;
+using GemmGroupedSmall = gemm::Cfg<128, 128, 128, 3, 2, 4, 4, 16>;
+// Decode batches (a few dozen rows per expert): the launch streams every
+// expert's weights, and two blocks a CU keep more of them in flight than one
+// 128-row block, with no MFMA work on 100 rows of padding.
+using GemmMoeFew = gemm::Cfg<64, 128, 128, 3, 2, 4, 4, 16>; // 8 waves of 32 x 32, 72 KiB LDS
 
-// 128-row tiles when the fraction of tile rows an expert of average size
-// fills, times their per-op rate relative to 256-row tiles (about 0.8,
-// measured on the fused-MoE CLI shapes), beats that of 256-row tiles: ~340
-// rows per expert (64 experts, top-6 of 3328 tokens) 1004 -> 1057 TOPS;
-// ~550 rows (32 experts, top-5) stay on 256 rows (1516 vs 1400 TOPS).
-bool moe_tile_rows_128(uint32_t rows, uint32_t experts)
+// Tiles of a MoE GEMM from the rows per expert, rows / experts (the sort's
+// capacity: with the default unit of 32 about 32 more than are routed there).
+// Same outputs from each.  gate_up (with its requantization) / down, us,
+// hidden 4096, inter 14336, 8 experts unless said:
+//   rows per expert       36        64        96       126 (a)    168       331
+//   64 x 128           199 / 85  207 / 87  240 / 124  122 / 62  332 / 167  624 / 301
+//   128 x 128          232 / 86  238 / 88  227 /  91  105 / 63  327 / 158  466 / 215
+//   128 or 256 x 256   232 / 103 245 / 106 239 / 110  113 / 59  291 / 167  459 / 210
+//   (a) 64 experts, hidden 2048, inter 1408
+// 64 rows up to 80: the weights' stream bounds it.  128 x 128 up to 140 for
+// gate_up, and up to 200 for a GEMM whose 256-wide tiles, one row of them per
+// expert, would fill at most half of the CUs (they need the tail split and
+// its partials).  Then 128-row tiles when the fraction of tile rows an expert
+// of average size fills, times their per-op rate relative to 256-row tiles
+// (about 0.8), beats that of 256-row tiles: ~340 rows per expert (64 experts,
+// top-6 of 3328 tokens) 1004 -> 1057 TOPS; ~550 rows (32 experts, top-5)
+// stay on 256 rows (1516 vs 1400 TOPS).
+enum class MoeTile { kFew, kSmall, kMid, kMain };
+
+MoeTile moe_tile(uint32_t rows, uint32_t experts, uint32_t n, bool silu = false)
 {
-    const double avg  = (double)rows / experts;
+    const double avg = (double)rows / experts;
+    if(avg <= 80) return MoeTile::kFew;
+    if(silu ? avg <= 140
+            : avg <= 200 && (uint64_t)experts * ((n + 255) / 256) * 2 <= device_cus())
+        return MoeTile::kSmall;
     const double u256 = avg / (std::ceil(avg / 256.0) * 256.0);
     const double u128 = avg / (std::ceil(avg / 128.0) * 128.0);
-    return u128 * 0.8 > u256;
+    return u128 * 0.8 > u256 ? MoeTile::kMid : MoeTile::kMain;
 }
 
 } // namespace
@@ -871,21 +923,6 @@ hipError_t launch_moe_combine(const uint16_t* y, uint32_t ldy, uint32_t rows_y, 
     return hipGetLastError();
 }
 
-using GemmGroupedSmall = gemm::Cfg<128, 128, 128, 3, 2, 4, 4, 16>;
-
-namespace {
-uint32_t device_cus()
-{
-    static const uint32_t cus = [] {
-        int dev = 0, c = 256;
-        if(hipGetDevice(&dev) == hipSuccess)
-            (void)hipDeviceGetAttribute(&c, hipDeviceAttributeMultiprocessorCount, dev);
-        return (uint32_t)c;
-    }();
-    return cus;
-}
-} // namespace
-
 hipError_t launch_grouped_gemm(const w8a8_group_desc* groups_dev, uint32_t ngroups,
                                uint32_t total_tiles, int cfg, int out_type,
                                hipStream_t stream)
@@ -944,10 +981,16 @@ hipError_t launch_moe_gemm(const MoeGemmArgs& a, hipStream_t stream)
     const bool split = a.ws != nullptr && a.ws_bytes >= moe_gemm_workspace_bytes();
     q.ws           = split ? static_cast<int32_t*>(a.ws) : nullptr;
     q.cus          = split ? device_cus() : 0;
-    // rows (the sort's padded capacity) / experts stands for the rows per expert
-    if(moe_tile_rows_128(a.rows, a.experts))
-        return gemm::launch_moe<GemmGroupedMid>(q, a.out_type, stream);
-    return gemm::launch_moe<GemmGrouped, GemmGroupedWide>(q, a.out_type, stream);
+    switch(moe_tile(a.rows, a.experts, a.n)) {
+    case MoeTile::kFew:
+        q.ws = nullptr, q.cus = 0;
+        return gemm::launch_moe<GemmMoeFew>(q, a.out_type, stream);
+    case MoeTile::kSmall:
+        q.ws = nullptr, q.cus = 0;
+        return gemm::launch_moe<GemmGroupedSmall>(q, a.out_type, stream);
+    case MoeTile::kMid: return gemm::launch_moe<GemmGroupedMid>(q, a.out_type, stream);
+    default: return gemm::launch_moe<GemmGrouped, GemmGroupedWide>(q, a.out_type, stream);
+    }
 }
 
 // The SiLU epilogue's tiles: wave tiles 128 columns wide (64 outputs, one
@@ -957,7 +1000,12 @@ hipError_t launch_moe_gemm(const MoeGemmArgs& a, hipStream_t stream)
 using GemmSilu     = gemm::Cfg<256, 256, 128, 2, 4, 2, 4, 16>;
 using GemmSiluMid  = gemm::Cfg<128, 256, 128, 3, 4, 2, 4, 16>;
 using GemmSiluWide = gemm::Cfg<128, 512, 128, 2, 2, 4, 4, 16>; // GemmSilu's wide partner
-static_assert(GemmSilu::kWaveN == GemmSiluMid::kWaveN, "one pmax layout for both tiles");
+// The same short tiles as the plain GEMM's, in wave tiles 64 columns wide.
+using GemmSiluSmall = gemm::Cfg<128, 128, 128, 2, 4, 2, 4, 16>; // 8 waves of 32 x 64, 64 KiB LDS
+using GemmSiluFew   = gemm::Cfg<64, 128, 128, 3, 2, 2, 4, 16>;  // 4 waves of 32 x 64, 72 KiB LDS
+static_assert(GemmSilu::kWaveN == GemmSiluMid::kWaveN
+                  && GemmSiluSmall::kWaveN == GemmSiluFew::kWaveN,
+              "two pmax layouts");
 static_assert(gemm::Partial<GemmSilu>::kBytes == gemm::Partial<GemmGrouped>::kBytes
                   && gemm::Partial<GemmSiluMid>::kBytes == gemm::Partial<GemmGroupedMid>::kBytes,
               "the SiLU tiles' partials fit moe_gemm_workspace_bytes");
@@ -975,12 +1023,20 @@ size_t moe_gate_up_silu_workspace_bytes(uint32_t rows, uint32_t inter)
 hipError_t launch_moe_gate_up_silu(const MoeSiluArgs& a, hipStream_t stream)
 {
     if(a.rows == 0) return hipSuccess;
-    const uint32_t groups = (2 * a.inter + kSiluGroupCols - 1) / kSiluGroupCols;
+    const MoeTile tile = moe_tile(a.rows, a.experts, 2 * a.inter, true);
+    // The short tiles' waves are half as wide, so pmax has twice the groups: it
+    // lies where the other tiles' K-split partials do, which these do not write.
+    const uint32_t narrow = (2 * a.inter + GemmSiluFew::kWaveN - 1) / GemmSiluFew::kWaveN;
+    const bool     few    = (tile == MoeTile::kFew || tile == MoeTile::kSmall)
+                     && (uint64_t)a.rows * narrow * 4 <= moe_gemm_workspace_bytes();
+    const uint32_t wide   = (2 * a.inter + kSiluGroupCols - 1) / kSiluGroupCols;
+    const uint32_t groups = few ? narrow : wide;
     int8_t*        ws     = static_cast<int8_t*>(a.ws);
     uint16_t*      h      = reinterpret_cast<uint16_t*>(ws);
     float*         pmax   = reinterpret_cast<float*>(ws + align256((size_t)a.rows * a.inter * 2));
     int32_t*       part   = reinterpret_cast<int32_t*>(
-        ws + align256((size_t)a.rows * a.inter * 2) + align256((size_t)a.rows * groups * 4));
+        ws + align256((size_t)a.rows * a.inter * 2) + align256((size_t)a.rows * wide * 4));
+    if(few) pmax = reinterpret_cast<float*>(part);
 
     gemm::MoeArgs q;
     q.a            = a.a;
@@ -1000,13 +1056,19 @@ hipError_t launch_moe_gate_up_silu(const MoeSiluArgs& a, hipStream_t stream)
     q.w_stride     = 2ull * a.inter * a.k;
     q.tsa          = a.tsa;
     q.tsb          = a.tsb;
-    q.ws           = part;
-    q.cus          = device_cus();
+    q.ws           = few ? nullptr : part;
+    q.cus          = few ? 0 : device_cus();
     // pmax group-major: row stride ldp = rows
     const gemm::SiluOut so{h, pmax, a.s2, a.inter, a.rows, a.inter};
-    hipError_t e = moe_tile_rows_128(a.rows, a.experts)
-                       ? gemm::launch_moe_silu<GemmSiluMid>(q, so, stream)
-                       : gemm::launch_moe_silu<GemmSilu, GemmSiluWide>(q, so, stream);
+    // (rows beyond the pmax room keep the 128-row rule)
+    hipError_t e;
+    if(few)
+        e = tile == MoeTile::kFew ? gemm::launch_moe_silu<GemmSiluFew>(q, so, stream)
+                                  : gemm::launch_moe_silu<GemmSiluSmall>(q, so, stream);
+    else if(tile != MoeTile::kMain)
+        e = gemm::launch_moe_silu<GemmSiluMid>(q, so, stream);
+    else
+        e = gemm::launch_moe_silu<GemmSilu, GemmSiluWide>(q, so, stream);
     if(e != hipSuccess) return e;
 
     const uint64_t h_bytes  = (uint64_t)a.rows * a.inter * 2;

@@ -620,6 +620,22 @@ def test_moe_gate_up_silu(w8a8, gpu, t, k, e, h, inter, unit, with_s2):
     assert exact >= total - max(2, total // 100), f"{total - exact} row scales differ"
 
 
+# The short tiles of few rows per expert: 64-row tiles (partial last N tile, two
+# tile rows for the busiest expert), 128 x 128 tiles, and more rows than the
+# one-row-per-block requantization takes.
+@pytest.mark.parametrize("t,k,e,h,inter,unit,with_s2", [
+    (40, 2, 8, 512, 400, 32, True), (1, 2, 8, 256, 48, 32, True), (130, 1, 1, 256, 144, 1, False),
+    (400, 2, 8, 4096, 512, 1, True), (4200, 2, 128, 128, 64, 1, True)])
+def test_moe_gate_up_silu_short_tiles(w8a8, gpu, t, k, e, h, inter, unit, with_s2):
+    test_moe_gate_up_silu(w8a8, gpu, t, k, e, h, inter, unit, with_s2)
+
+
+@pytest.mark.parametrize("t,k,e,h,n,unit", [(40, 2, 8, 4112, 1000, 32), (1, 2, 8, 256, 130, 32),
+                                            (400, 2, 8, 2064, 520, 1), (720, 2, 8, 256, 1100, 1)])
+def test_moe_gemm_short_tiles(w8a8, gpu, t, k, e, h, n, unit):
+    test_moe_gemm_exact(w8a8, gpu, t, k, e, h, n, unit)
+
+
 # Explicit expert row counts for the 256-row SiLU tile: rests of 1-128 rows
 # (300, 40, 1100, 128) take rows of 128 x 512 tiles, a rest of 129 rows and
 # 1000 rows take 256-row tiles, and one expert is empty.  inter = 512 (1024
