@@ -162,6 +162,14 @@ def check(fn: str, status: int) -> None:
         raise W8A8Error(fn, status, msg)
 
 
+_calls: dict[str, object] = {}  # bound entry points of the loaded library, by name
+
+
 def call(name: str, *args) -> None:
     """Call a status-returning entry point and raise W8A8Error on failure."""
-    check(name, getattr(load(), name)(*args))
+    fn = _calls.get(name)
+    if fn is None:
+        fn = _calls[name] = getattr(load(), name)
+    status = fn(*args)
+    if status != SUCCESS:
+        check(name, status)
