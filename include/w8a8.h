@@ -358,16 +358,20 @@ size_t w8a8_grouped_gemm_workspace_size(uint32_t num_groups);
 /*
  * Runs every group's w8a8_gemm in one launch.  Replaces grouped_gemm_kernel
  * (rocwmma_grouped_gemm.cpp:104-178), whose host code uploads the descriptor
- * array with a tile_offset prefix in it (:180-226): here `groups` is a HOST array,
- * validated, then copied into `workspace` by one hipMemcpyAsync on `stream`.
- * The call returns before that copy runs: the host array must stay valid and
+ * array with a tile_offset prefix in it (:180-226): here `groups` is a HOST array.
+ * Up to W8A8_GROUPED_INLINE_GROUPS validated descriptors travel as the launch's
+ * own arguments, and the array is not read again after the call returns.  More
+ * are copied into `workspace` by one hipMemcpyAsync on `stream`, and the call
+ * returns before that copy runs: the host array must then stay valid and
  * unchanged until the stream has reached it (synchronize the stream, or an
- * event recorded after the call, before reusing it).  A HIP graph that
+ * event recorded after the call, before reusing it), and a HIP graph that
  * captures the call records the copy, so every replay reads the host array
- * again: keep it alive and unchanged for as long as the graph may run.  Every group needs the
- * fast-path layout (16-byte aligned a/b, lda, ldb, k multiples of 16) and
+ * again: keep it alive and unchanged for as long as the graph may run.
+ * `workspace` is required and checked for any group count.  Every group needs
+ * the fast-path layout (16-byte aligned a/b, lda, ldb, k multiples of 16) and
  * m*lda, n*ldb < 2^31 (W8A8_ERROR_NOT_SUPPORTED otherwise).
  */
+#define W8A8_GROUPED_INLINE_GROUPS 48
 int w8a8_grouped_gemm(const w8a8_group_desc* groups, uint32_t num_groups, int out_type,
                       void* workspace, size_t workspace_bytes, hipStream_t stream);
 

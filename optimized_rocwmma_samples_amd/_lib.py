@@ -24,6 +24,8 @@ OUT_F16 = 1
 
 STREAMK_WAIT_EXPIRED = 1
 
+GROUPED_INLINE_GROUPS = 48  # W8A8_GROUPED_INLINE_GROUPS
+
 FOLD_MULTIPLY = 0
 FOLD_DIVIDE = 1
 

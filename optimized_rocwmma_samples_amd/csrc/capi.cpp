@@ -546,7 +546,7 @@ int w8a8_grouped_gemm(const w8a8_group_desc* groups, uint32_t num_groups, int ou
                     workspace_bytes, w8a8_grouped_gemm_workspace_size(num_groups));
     if(reinterpret_cast<uintptr_t>(workspace) % 64 != 0)
         return fail(W8A8_ERROR_INVALID_VALUE, "%s: workspace must be 64-byte aligned", fn);
-    uint64_t tiles[3] = {0, 0, 0}; // per tile configuration
+    uint64_t tiles = 0; // of 128 x 128
     for(uint32_t i = 0; i < num_groups; ++i) {
         const w8a8_group_desc& d = groups[i];
         if(d.m == 0) continue;
@@ -564,16 +564,17 @@ int w8a8_grouped_gemm(const w8a8_group_desc* groups, uint32_t num_groups, int ou
                         "%s: group %u: needs 16-byte aligned a/b and lda, ldb, k %% 16 == 0", fn, i);
         if((uint64_t)d.m * d.lda > 0x7FFFFFFFull || (uint64_t)d.n * d.ldb > 0x7FFFFFFFull)
             return fail(W8A8_ERROR_NOT_SUPPORTED, "%s: group %u: operand over 2 GiB", fn, i);
-        for(int c = 0; c < 3; ++c) tiles[c] += w8a8::grouped_gemm_tiles(d.m, d.n, c);
+        tiles += (uint64_t)((d.m + 127) / 128) * ((d.n + 127) / 128);
     }
-    if(tiles[2] > 0x7FFFFFFFull) return fail(W8A8_ERROR_NOT_SUPPORTED, "%s: too many tiles", fn);
-    if(tiles[0] == 0) return hip_status(hipSuccess, fn);
-    const int cfg = w8a8::grouped_gemm_cfg(tiles);
-    hipError_t e = hipMemcpyAsync(workspace, groups, (size_t)num_groups * sizeof(w8a8_group_desc),
-                                  hipMemcpyHostToDevice, stream);
+    if(tiles > 0x7FFFFFFFull) return fail(W8A8_ERROR_NOT_SUPPORTED, "%s: too many tiles", fn);
+    if(tiles == 0) return hip_status(hipSuccess, fn);
+    hipError_t e = hipSuccess;
+    if(num_groups > w8a8::kGroupedInline)
+        e = hipMemcpyAsync(workspace, groups, (size_t)num_groups * sizeof(w8a8_group_desc),
+                           hipMemcpyHostToDevice, stream);
     if(e == hipSuccess)
-        e = w8a8::launch_grouped_gemm(static_cast<const w8a8_group_desc*>(workspace), num_groups,
-                                      (uint32_t)tiles[cfg], cfg, out_type, stream);
+        e = w8a8::launch_grouped_gemm(groups, workspace, num_groups,
+                                      w8a8::grouped_gemm_tile(groups, num_groups), out_type, stream);
     return hip_status(e, fn);
 }
 

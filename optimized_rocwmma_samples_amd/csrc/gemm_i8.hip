@@ -366,6 +366,49 @@ TilePlan plan_tiles(uint32_t m, uint32_t n, uint32_t k, size_t ws_bytes, bool de
     return e.plan;
 }
 
+} // namespace
+
+// One tile for a grouped launch: the plan's costs over the groups' tiles, each
+// CU's blocks at the tiles' mean k-tiles (the longest group's where no CU has
+// two blocks).  Against the tallest tile that fills 3/4 of the CUs: 13 groups
+// of 1-901 rows, 3584 x 3776, 116 -> 82 us a call; 7 and 67 rows, 1280 x 576,
+// kernel 7.4 -> 5.2 us; 256 / 512 / 128 / 768 rows, 4096^2, stays on 208 tiles
+// of 128 x 256 (35 -> 34 us).
+GroupedTile grouped_gemm_tile(const w8a8_group_desc* groups, uint32_t ngroups)
+{
+    GroupedTile best{0, 0, 0};
+    double      cost = 1e300;
+    for(const CfgCost& c : kCosts) {
+        if(c.cfg == TileCfg::kRow) continue;
+        uint64_t tiles = 0, steps = 0, most = 0;
+        double   out = 0, w = 0;
+        for(uint32_t i = 0; i < ngroups; ++i) {
+            const w8a8_group_desc& g = groups[i];
+            if(g.m == 0) continue;
+            const uint64_t t = (uint64_t)ceil_div(g.m, c.bm) * ceil_div(g.n, c.bn);
+            const uint64_t k = ceil_div(g.k, 128);
+            tiles += t;
+            steps += t * k;
+            most = std::max(most, k);
+            out += 2e-6 * g.m * g.n;
+            w += 1e-6 * g.n * (double)g.k;
+        }
+        if(tiles == 0 || tiles > 0x7FFFFFFFull) continue;
+        const uint64_t per_cu = (tiles + device_cus() - 1) / device_cus();
+        const double   nk     = per_cu == 1 ? (double)most : (double)steps / tiles;
+        const double   t      = c.fixed + out * c.out_mb + w * c.w_mb
+                         + nk * (per_cu / c.resident * c.step[c.resident - 1]
+                                 + (per_cu % c.resident ? c.step[per_cu % c.resident - 1] : 0.0));
+        if(t < cost) {
+            cost = t;
+            best = GroupedTile{c.bm, c.bn, (uint32_t)tiles};
+        }
+    }
+    return best;
+}
+
+namespace {
+
 // Bytes reported to callers at the least where a K split may run: the pieces
 // of 128-row tiles (64 x 128 below 65 rows) on the CUs that half a round of
 // them leaves idle.  A bound from the sizes alone, so that a workspace sized

@@ -99,6 +99,34 @@ __global__ void __launch_bounds__(C::kThreads, 1)
     gemm_tile<C, OUT>(p, m0, n0, lds);
 }
 
+// The same launch with its descriptors as kernel arguments, for up to
+// kInlineGroups groups: no copy to the device ahead of it (the copy and the
+// gap behind it were 4 us of a 38 us call), nothing of the caller's read after
+// the call returns.  first[i]: tiles of the groups before i, so a block's group
+// is the last whose first tile is not past it: one compare per lane and a
+// ballot.  The grid is the exact tile count.
+constexpr uint32_t kInlineGroups = W8A8_GROUPED_INLINE_GROUPS; // a launch's arguments: 4 KB
+struct GroupTable {
+    uint32_t first[kInlineGroups];
+    KArgs    g[kInlineGroups];
+};
+static_assert(kInlineGroups <= kWave && sizeof(GroupTable) <= 4000, "one wave, one argument block");
+
+template <class C, int OUT>
+__global__ void __launch_bounds__(C::kThreads, 1) gemm_i8_grouped_inline_kernel(GroupTable t, uint32_t ngroups)
+{
+    extern __shared__ __attribute__((aligned(1024))) int8_t lds[];
+    const uint32_t lane = threadIdx.x % kWave;
+    const uint32_t lid  = xcd_remap(blockIdx.x, gridDim.x);
+    const uint32_t mine = t.first[min(lane, ngroups - 1)];
+    const uint64_t at   = __ballot(lane < ngroups && mine <= lid); // lane 0: first[0] = 0
+    const uint32_t g    = __builtin_amdgcn_readfirstlane(__popcll(at) - 1);
+    const KArgs    p    = t.g[g];
+    uint32_t       m0, n0;
+    local_tile<C>(lid - t.first[g], p.m, p.n, m0, n0);
+    gemm_tile<C, OUT>(p, m0, n0, lds);
+}
+
 struct MoeArgs {
     const int8_t*  a;            // [rows, lda] expert-sorted activations
     const int8_t*  w;            // expert e at w + e * w_stride: [n, ldw]
@@ -510,21 +538,40 @@ void raise_lds_once(const void* kern)
     });
 }
 
+// groups_host: the validated descriptors.  Up to kInlineGroups travel in the
+// launch; more are read from groups_dev, the caller's workspace they were
+// copied to.
+template <class C, int OUT>
+hipError_t launch_grouped_out(const KArgs* groups_host, const KArgs* groups_dev, uint32_t ngroups,
+                              uint32_t total_tiles, hipStream_t stream)
+{
+    if(ngroups > kInlineGroups) {
+        raise_lds_once<C, OUT, 0>(reinterpret_cast<const void*>(gemm_i8_grouped_kernel<C, OUT>));
+        hipLaunchKernelGGL((gemm_i8_grouped_kernel<C, OUT>), dim3(total_tiles), dim3(C::kThreads),
+                           C::kLdsBytes, stream, groups_dev, ngroups);
+        return hipGetLastError();
+    }
+    GroupTable t{};
+    uint32_t   tiles = 0;
+    for(uint32_t i = 0; i < ngroups; ++i) {
+        const KArgs& g = t.g[i] = groups_host[i];
+        t.first[i]     = tiles;
+        tiles += ((g.m + C::kBM - 1) / C::kBM) * ((g.n + C::kBN - 1) / C::kBN);
+    }
+    raise_lds_once<C, OUT, 3>(reinterpret_cast<const void*>(gemm_i8_grouped_inline_kernel<C, OUT>));
+    hipLaunchKernelGGL((gemm_i8_grouped_inline_kernel<C, OUT>), dim3(tiles), dim3(C::kThreads),
+                       C::kLdsBytes, stream, t, ngroups);
+    return hipGetLastError();
+}
+
 template <class C>
-hipError_t launch_grouped(const KArgs* groups_dev, uint32_t ngroups, uint32_t total_tiles,
-                          int out_type, hipStream_t stream)
+hipError_t launch_grouped(const KArgs* groups_host, const KArgs* groups_dev, uint32_t ngroups,
+                          uint32_t total_tiles, int out_type, hipStream_t stream)
 {
     if(total_tiles == 0) return hipSuccess;
-    if(out_type == W8A8_OUT_I32) {
-        raise_lds_once<C, W8A8_OUT_I32, 0>(reinterpret_cast<const void*>(gemm_i8_grouped_kernel<C, W8A8_OUT_I32>));
-        hipLaunchKernelGGL((gemm_i8_grouped_kernel<C, W8A8_OUT_I32>), dim3(total_tiles),
-                           dim3(C::kThreads), C::kLdsBytes, stream, groups_dev, ngroups);
-    } else {
-        raise_lds_once<C, W8A8_OUT_F16, 0>(reinterpret_cast<const void*>(gemm_i8_grouped_kernel<C, W8A8_OUT_F16>));
-        hipLaunchKernelGGL((gemm_i8_grouped_kernel<C, W8A8_OUT_F16>), dim3(total_tiles),
-                           dim3(C::kThreads), C::kLdsBytes, stream, groups_dev, ngroups);
-    }
-    return hipGetLastError();
+    return out_type == W8A8_OUT_I32
+               ? launch_grouped_out<C, W8A8_OUT_I32>(groups_host, groups_dev, ngroups, total_tiles, stream)
+               : launch_grouped_out<C, W8A8_OUT_F16>(groups_host, groups_dev, ngroups, total_tiles, stream);
 }
 
 // Grid bound: every expert's last m tile may be partial, so at most

@@ -767,6 +767,7 @@ using GemmGroupedSmall = gemm::Cfg<128, 128, 128, 3, 2, 4, 4, 16>;
 // expert's weights, and two blocks a CU keep more of them in flight than one
 // 128-row block, with no MFMA work on 100 rows of padding.
 using GemmMoeFew = gemm::Cfg<64, 128, 128, 3, 2, 4, 4, 16>; // 8 waves of 32 x 32, 72 KiB LDS
+using GemmGroupedTiny = gemm::Cfg<64, 64, 128, 4, 2, 2, 4, 16>; // 4 waves of 32 x 32, 64 KiB LDS
 
 // Tiles of a MoE GEMM from the rows per expert, rows / experts (the sort's
 // capacity: with the default unit of 32 about 32 more than are routed there).
@@ -923,34 +924,26 @@ hipError_t launch_moe_combine(const uint16_t* y, uint32_t ldy, uint32_t rows_y, 
     return hipGetLastError();
 }
 
-hipError_t launch_grouped_gemm(const w8a8_group_desc* groups_dev, uint32_t ngroups,
-                               uint32_t total_tiles, int cfg, int out_type,
+// The tile of a grouped launch and its total tile count (grouped_gemm_tile).
+hipError_t launch_grouped_gemm(const w8a8_group_desc* groups, const void* groups_dev,
+                               uint32_t ngroups, const GroupedTile& tile, int out_type,
                                hipStream_t stream)
 {
-    const auto* g = reinterpret_cast<const gemm::KArgs*>(groups_dev);
-    if(cfg == 1)
-        return gemm::launch_grouped<GemmGroupedMid>(g, ngroups, total_tiles, out_type,
-                                                    stream);
-    if(cfg == 2)
-        return gemm::launch_grouped<GemmGroupedSmall>(g, ngroups, total_tiles, out_type,
-                                                      stream);
-    return gemm::launch_grouped<GemmGrouped>(g, ngroups, total_tiles, out_type, stream);
+    const auto* h = reinterpret_cast<const gemm::KArgs*>(groups);
+    const auto* d = static_cast<const gemm::KArgs*>(groups_dev);
+    switch(tile.bm * 1000 + tile.bn) {
+    case 256256:
+        return gemm::launch_grouped<GemmGrouped>(h, d, ngroups, tile.tiles, out_type, stream);
+    case 128256:
+        return gemm::launch_grouped<GemmGroupedMid>(h, d, ngroups, tile.tiles, out_type, stream);
+    case 128128:
+        return gemm::launch_grouped<GemmGroupedSmall>(h, d, ngroups, tile.tiles, out_type, stream);
+    case 64128:
+        return gemm::launch_grouped<GemmMoeFew>(h, d, ngroups, tile.tiles, out_type, stream);
+    default:
+        return gemm::launch_grouped<GemmGroupedTiny>(h, d, ngroups, tile.tiles, out_type, stream);
+    }
 }
-
-uint32_t grouped_gemm_tiles(uint32_t m, uint32_t n, int cfg)
-{
-    const uint32_t bm = cfg == 0 ? 256 : 128, bn = cfg == 2 ? 128 : 256;
-    return ((m + bm - 1) / bm) * ((n + bn - 1) / bn);
-}
-
-int grouped_gemm_cfg(const uint64_t tiles[3])
-{
-    const uint64_t enough = (uint64_t)device_cus() * 3 / 4;
-    if(tiles[0] >= enough) return 0;
-    if(tiles[1] >= enough) return 1;
-    return 2;
-}
-
 
 size_t moe_gemm_workspace_bytes()
 {

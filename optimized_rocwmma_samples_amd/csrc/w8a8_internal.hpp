@@ -174,16 +174,18 @@ hipError_t launch_moe_combine(const uint16_t* y, uint32_t ldy, uint32_t rows_y, 
                               const int32_t* dst_row, uint32_t tokens, uint32_t topk, uint32_t n,
                               uint16_t* out, uint32_t ldo, hipStream_t stream);
 
-// Grouped GEMM over device descriptors (validated by the caller: fast-path
-// alignment, every operand under 2 GiB).
-// Grouped GEMM tile configurations: 0 = 256 x 256, 1 = 128 x 256, 2 = 128 x 128.
-uint32_t   grouped_gemm_tiles(uint32_t m, uint32_t n, int cfg);
-// The tallest configuration whose tile total is at least 3/4 of a round of
-// the CUs (tiles[c] = total tiles of configuration c), else 128 x 128.
-int        grouped_gemm_cfg(const uint64_t tiles[3]);
-hipError_t launch_grouped_gemm(const w8a8_group_desc* groups_dev, uint32_t ngroups,
-                               uint32_t total_tiles, int cfg, int out_type,
-                               hipStream_t stream);
+// Grouped GEMM (moe.hip).  grouped_gemm_tile: one tile for all groups, of the
+// least estimated time (gemm_i8.hip), and the total tile count with it; tiles =
+// 0 for empty groups only.  groups: the validated host descriptors; groups_dev:
+// their copy, read only for more than kGroupedInline groups.
+constexpr uint32_t kGroupedInline = W8A8_GROUPED_INLINE_GROUPS;
+struct GroupedTile {
+    uint32_t bm, bn, tiles;
+};
+GroupedTile grouped_gemm_tile(const w8a8_group_desc* groups, uint32_t ngroups);
+hipError_t  launch_grouped_gemm(const w8a8_group_desc* groups, const void* groups_dev,
+                                uint32_t ngroups, const GroupedTile& tile, int out_type,
+                                hipStream_t stream);
 
 struct MoeGemmArgs {
     const int8_t*  a;

@@ -159,6 +159,27 @@ def test_grouped_gemm_int32_and_f16(w8a8, gpu):
         assert_f16_bitexact(host(o), e)
 
 
+# Each tile of a grouped launch (64 x 64 ... 256 x 256, ragged), empty groups at
+# both ends, and one group more than travels in the launch's arguments.
+@pytest.mark.parametrize("ms,n,k", [([7, 0, 67], 200, 80), ([0, 300, 5, 90, 700, 0], 1300, 144),
+                                    ([1000, 1, 513], 2100, 272), ([2100, 2000, 900], 3000, 160),
+                                    ([3] * 48, 130, 64), ([5, 0, 70] * 17, 130, 64)])
+def test_grouped_gemm_tiles_and_counts(w8a8, gpu, ms, n, k):
+    import torch
+    a = G.int8(5, G.TID_A, (max(ms), k))
+    b = G.int8(6, G.TID_B, (n, k))
+    sa = G.uniform(7, G.TID_SA, (max(ms),), 1e-3, 1e-2)
+    sb = G.uniform(8, G.TID_SB, (n,), 1e-3, 1e-2)
+    ad, bd, sad, sbd = dev(a, gpu), dev(b, gpu), dev(sa, gpu), dev(sb, gpu)
+    acc = O.gemm_i32(a, b)
+    want = O.dequant_f16(acc, sa, sb)
+    for got, m in zip(w8a8.grouped_gemm([(ad[:m], bd, None, None) for m in ms],
+                                        out_dtype=torch.int32), ms):
+        assert_i32_equal(host(got), acc[:m])
+    for got, m in zip(w8a8.grouped_gemm([(ad[:m], bd, sad[:m], sbd) for m in ms]), ms):
+        assert_f16_bitexact(host(got), want[:m])
+
+
 def _sorted_problem(t, k, e, h, n, unit, seed):
     ids = routing_ids(t, e, k, seed)
     count, start, padded, sorted_ids, dst = O.moe_sort(ids, e, unit)
