@@ -15,11 +15,17 @@
 //
 // sq_rows_kernel (HBM-bound: 3 bytes moved per element):
 //   * One wavefront owns a row segment of CPL*512 elements; WPR wavefronts
-//     share a row.  Each lane issues CPL 16-byte loads (8 fp16) so a wave
-//     instruction reads 1 KiB contiguous, and the whole segment is in flight
-//     at once.
-//   * The smoothed row stays in VGPRs: x is read from HBM exactly once
-//     (the reference re-reads it in its second pass, :101-117).
+//     share a row.  Each lane issues CPL 16-byte loads (8 fp16) at whatever
+//     address the row has (the hardware takes unaligned global accesses), so a
+//     wave instruction reads 1 KiB contiguous and the whole segment is in
+//     flight at once; only the chunk that straddles N goes element by element.
+//     15238 x 1337, odd rows: 71 -> 17 us with 16-byte accesses.
+//   * x stays in VGPRs: it is read from HBM exactly once (the reference
+//     re-reads it in its second pass, :101-117), and once for all of a token's
+//     experts where the MoE form gives tokens to groups of waves: per expert
+//     only its smooth scale is read (2916 x 7168, top 6 92 -> 58 us).  With few
+//     pairs or experts a token a group takes one pair (PAIRS; dispatch says
+//     where).
 //   * absmax: DPP quad/mirror steps inside each 16-lane row + 4 readlanes;
 //     rows spread over several waves merge through 16 bytes of LDS.
 //   * Output: each lane packs 8 int8 and stores 8 bytes (a wave writes 512
@@ -68,84 +74,104 @@ __device__ __forceinline__ RowSrc resolve_row(const QuantRows& p, uint32_t row)
     return rs;
 }
 
-// CPL: 16-byte chunks per lane; WPR: waves per row; VEC: aligned vector I/O.
-template <int CPL, int WPR, bool MOE, bool VEC>
+// CPL: 16-byte chunks per lane; WPR: waves per row.  MOE: a group of WPR waves
+// takes a token and writes its topk rows one after another, or (PAIRS) one
+// (token, slot) pair.
+template <int CPL, int WPR, bool MOE, bool PAIRS>
 __global__ void __launch_bounds__(kSqThreads) sq_rows_kernel(QuantRows p)
 {
     constexpr int kRowsPerBlock = kSqWaves / WPR;
     constexpr int kSpan         = CPL * 8 * kWave;
+    constexpr bool kTokens      = MOE && !PAIRS;
+    __shared__ float red[2][kSqWaves];
 
     const int      wave = threadIdx.x / kWave;
     const int      lane = threadIdx.x % kWave;
     const int      rib  = wave / WPR; // row in block
     const int      part = wave % WPR; // segment of the row
-    const uint32_t row  = blockIdx.x * kRowsPerBlock + rib;
+    const uint32_t unit = blockIdx.x * kRowsPerBlock + rib; // token, pair or row
+    const uint32_t slots = kTokens ? p.topk : 1;
+    const uint32_t row0  = unit * slots;
+    const uint32_t n     = p.n;
+    const uint32_t base  = part * kSpan + lane * 8;
 
-    RowSrc src = resolve_row<MOE>(p, row);
-
-    float    pv[CPL * 8];
-    float    amax = 0.f;
-    const uint32_t n    = p.n;
-    const uint32_t base = part * kSpan + lane * 8;
-
-    if(src.valid) {
+    v4i raw[CPL]; // zeros past N and for units past the last
+    if(row0 < p.rows) {
+        const uint16_t* x = p.x + (size_t)(MOE ? row0 / p.topk : row0) * p.ldx;
 #pragma unroll
         for(int j = 0; j < CPL; ++j) {
             const uint32_t c = base + j * (8 * kWave);
-            if(VEC && c + 8 <= n) {
-                const uint4 raw = *reinterpret_cast<const uint4*>(src.x + c);
-                const float4 s0 = *reinterpret_cast<const float4*>(src.s + c);
-                const float4 s1 = *reinterpret_cast<const float4*>(src.s + c + 4);
-                pv[j * 8 + 0] = mul_h16_f32<false>(raw.x, s0.x);
-                pv[j * 8 + 1] = mul_h16_f32<true>(raw.x, s0.y);
-                pv[j * 8 + 2] = mul_h16_f32<false>(raw.y, s0.z);
-                pv[j * 8 + 3] = mul_h16_f32<true>(raw.y, s0.w);
-                pv[j * 8 + 4] = mul_h16_f32<false>(raw.z, s1.x);
-                pv[j * 8 + 5] = mul_h16_f32<true>(raw.z, s1.y);
-                pv[j * 8 + 6] = mul_h16_f32<false>(raw.w, s1.z);
-                pv[j * 8 + 7] = mul_h16_f32<true>(raw.w, s1.w);
-            } else {
+            raw[j]           = v4i{0};
+            if(c + 8 <= n) {
+                __builtin_memcpy(&raw[j], x + c, 16);
+            } else if(c < n) {
+                uint32_t w[4] = {0, 0, 0, 0};
 #pragma unroll
-                for(int e = 0; e < 8; ++e)
-                    pv[j * 8 + e] = (c + e < n) ? half_bits_to_float(src.x[c + e]) * src.s[c + e]
-                                                : 0.f;
+                for(int e = 0; e < 7; ++e)
+                    if(c + e < n) w[e / 2] |= (uint32_t)x[c + e] << (16 * (e % 2));
+                raw[j] = v4i{(int)w[0], (int)w[1], (int)w[2], (int)w[3]};
             }
-#pragma unroll
-            for(int e = 0; e < 8; ++e) amax = fmaxf(amax, fabsf(pv[j * 8 + e]));
         }
     }
-
-    amax = wave_max(amax);
-    if constexpr(WPR > 1) {
-        __shared__ float red[kSqWaves];
-        if(lane == 0) red[wave] = amax;
-        __syncthreads();
-#pragma unroll
-        for(int w = 0; w < WPR; ++w) amax = fmaxf(amax, red[rib * WPR + w]);
-    }
-    if(!src.valid) return;
-
     const float qmax = p.qmax;
-    const float rs   = amax / qmax; // correctly rounded fp32 division
-    if(part == 0 && lane == 0) p.r[src.dst] = rs;
-    const float inv = (rs > 0.f) ? (1.f / rs) : 0.f;
+    for(uint32_t slot = 0; slot < slots; ++slot) { // the same count in every wave
+        const RowSrc src = resolve_row<MOE>(p, row0 + slot);
+        float        pv[CPL * 8];
+        float        amax = 0.f;
+        if(src.valid) {
+#pragma unroll
+            for(int j = 0; j < CPL; ++j) {
+                const uint32_t c     = base + j * (8 * kWave);
+                float          sv[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+                if(c + 8 <= n) {
+                    __builtin_memcpy(sv, src.s + c, 16);
+                    __builtin_memcpy(sv + 4, src.s + c + 4, 16);
+                } else if(c < n) {
+#pragma unroll
+                    for(int e = 0; e < 7; ++e)
+                        if(c + e < n) sv[e] = src.s[c + e];
+                }
+                const uint32_t w[4] = {(uint32_t)raw[j].x, (uint32_t)raw[j].y, (uint32_t)raw[j].z,
+                                       (uint32_t)raw[j].w};
+#pragma unroll
+                for(int e = 0; e < 4; ++e) {
+                    pv[j * 8 + 2 * e]     = mul_h16_f32<false>(w[e], sv[2 * e]);
+                    pv[j * 8 + 2 * e + 1] = mul_h16_f32<true>(w[e], sv[2 * e + 1]);
+                }
+#pragma unroll
+                for(int e = 0; e < 8; ++e) amax = fmaxf(amax, fabsf(pv[j * 8 + e]));
+            }
+        }
+        amax = wave_max(amax);
+        if constexpr(WPR > 1) {
+            float* r = red[slot % 2]; // the other half may still be read from the slot before
+            if(lane == 0) r[wave] = amax;
+            __syncthreads();
+#pragma unroll
+            for(int w = 0; w < WPR; ++w) amax = fmaxf(amax, r[rib * WPR + w]);
+        }
+        if(!src.valid) continue;
+        const float rs = amax / qmax; // correctly rounded fp32 division
+        if(part == 0 && lane == 0) p.r[src.dst] = rs;
+        const float inv = (rs > 0.f) ? (1.f / rs) : 0.f;
 
-    int8_t* qrow = p.q + (size_t)src.dst * p.ldq;
+        int8_t* qrow = p.q + (size_t)src.dst * p.ldq;
 #pragma unroll
-    for(int j = 0; j < CPL; ++j) {
-        const uint32_t c = base + j * (8 * kWave);
-        const float*   v = pv + j * 8;
-        if(VEC && c + 8 <= n) {
-            uint2 packed;
-            packed.x = cvt_pack4_i8(quant_f(v[0], inv, qmax), quant_f(v[1], inv, qmax),
-                                    quant_f(v[2], inv, qmax), quant_f(v[3], inv, qmax));
-            packed.y = cvt_pack4_i8(quant_f(v[4], inv, qmax), quant_f(v[5], inv, qmax),
-                                    quant_f(v[6], inv, qmax), quant_f(v[7], inv, qmax));
-            *reinterpret_cast<uint2*>(qrow + c) = packed;
-        } else {
+        for(int j = 0; j < CPL; ++j) {
+            const uint32_t c = base + j * (8 * kWave);
+            const float*   v = pv + j * 8;
+            uint32_t       packed[2];
+            packed[0] = cvt_pack4_i8(quant_f(v[0], inv, qmax), quant_f(v[1], inv, qmax),
+                                     quant_f(v[2], inv, qmax), quant_f(v[3], inv, qmax));
+            packed[1] = cvt_pack4_i8(quant_f(v[4], inv, qmax), quant_f(v[5], inv, qmax),
+                                     quant_f(v[6], inv, qmax), quant_f(v[7], inv, qmax));
+            if(c + 8 <= n) {
+                __builtin_memcpy(qrow + c, packed, 8);
+            } else {
 #pragma unroll
-            for(int e = 0; e < 8; ++e)
-                if(c + e < n) qrow[c + e] = (int8_t)quant_i8(v[e], inv, qmax);
+                for(int e = 0; e < 7; ++e)
+                    if(c + e < n) qrow[c + e] = (int8_t)(packed[e / 4] >> (8 * (e % 4)));
+            }
         }
     }
 }
@@ -401,29 +427,26 @@ hipError_t launch_stream(const QuantRows& p, hipStream_t stream)
     return hipSuccess;
 }
 
-template <int CPL, int WPR, bool MOE>
-hipError_t launch_rows(const QuantRows& p, bool vec, hipStream_t stream)
+template <int CPL, int WPR, bool MOE, bool PAIRS = false>
+hipError_t launch_rows(const QuantRows& p, hipStream_t stream)
 {
-    constexpr int kRowsPerBlock = kSqWaves / WPR;
-    dim3          grid((p.rows + kRowsPerBlock - 1) / kRowsPerBlock);
-    if(vec)
-        hipLaunchKernelGGL((sq_rows_kernel<CPL, WPR, MOE, true>), grid, dim3(kSqThreads), 0,
-                           stream, p);
-    else
-        hipLaunchKernelGGL((sq_rows_kernel<CPL, WPR, MOE, false>), grid, dim3(kSqThreads), 0,
-                           stream, p);
+    constexpr int  kRowsPerBlock = kSqWaves / WPR;
+    const uint32_t units         = MOE && !PAIRS ? p.rows / p.topk : p.rows;
+    hipLaunchKernelGGL((sq_rows_kernel<CPL, WPR, MOE, PAIRS>),
+                       dim3((units + kRowsPerBlock - 1) / kRowsPerBlock), dim3(kSqThreads), 0,
+                       stream, p);
     return hipGetLastError();
 }
 
 template <bool MOE>
 hipError_t dispatch(const QuantRows& p, hipStream_t stream)
 {
-    // 16-byte x loads, 32-byte aligned s loads, 8-byte q stores.
-    const bool vec = (reinterpret_cast<uintptr_t>(p.x) % 16 == 0) && (p.ldx % 8 == 0)
-                     && (reinterpret_cast<uintptr_t>(p.s) % 16 == 0) && (!MOE || p.n % 4 == 0)
-                     && (reinterpret_cast<uintptr_t>(p.q) % 8 == 0) && (p.ldq % 8 == 0);
     const uint32_t n = p.n;
     if constexpr(!MOE) {
+        // 16-byte x loads, 32-byte aligned s loads, 8-byte q stores
+        const bool vec = (reinterpret_cast<uintptr_t>(p.x) % 16 == 0) && (p.ldx % 8 == 0)
+                         && (reinterpret_cast<uintptr_t>(p.s) % 16 == 0)
+                         && (reinterpret_cast<uintptr_t>(p.q) % 8 == 0) && (p.ldq % 8 == 0);
         // aligned dense rows: the streaming kernel (s in LDS, rows double-buffered)
         if(vec && n % 8 == 0) {
             // (configurations chosen by a sweep on MI355X over CPL, WPR,
@@ -461,13 +484,31 @@ hipError_t dispatch(const QuantRows& p, hipStream_t stream)
             if(n <= 32768) return launch_stream<4, 16, 1024>(p, stream);
         }
     }
-    if(n <= 512) return launch_rows<1, 1, MOE>(p, vec, stream);
-    if(n <= 1024) return launch_rows<2, 1, MOE>(p, vec, stream);
-    if(n <= 2048) return launch_rows<4, 1, MOE>(p, vec, stream);
-    if(n <= 4096) return launch_rows<8, 1, MOE>(p, vec, stream);
-    if(n <= 8192) return launch_rows<16, 1, MOE>(p, vec, stream);
-    if(n <= 16384) return launch_rows<16, 2, MOE>(p, vec, stream);
-    if(n <= 32768) return launch_rows<16, 4, MOE>(p, vec, stream);
+    if constexpr(MOE) {
+        // fewer pairs than two blocks a CU: a block for each (32 pairs of 4096:
+        // 7.3 -> 4.1 us)
+        if(p.rows <= 512 && n <= 4096)
+            return n <= 2048 ? launch_rows<1, 4, MOE, true>(p, stream)
+                             : launch_rows<2, 4, MOE, true>(p, stream);
+        // Pairs up to 3072 of them and for one or two experts a token, where
+        // reading x once saves less than the serial slots cost: 768 / 2400 /
+        // 6000 / 17496 pairs of 7168, top 6, 8.2 / 16.0 / 32 / 81 us by pairs,
+        // 17.1 / 17.7 / 23 / 58 by tokens; 600 / 2000 / 8192 pairs of 4096,
+        // top 2, 6.0 / 8.3 / 20.5 against 7.4 / 9.2 / 21.4.
+        if(n > 2048 && n <= 32768 && (p.rows <= 3072 || p.topk <= 2)) {
+            if(n <= 4096) return launch_rows<4, 2, MOE, true>(p, stream);
+            if(n <= 8192) return launch_rows<4, 4, MOE, true>(p, stream);
+            if(n <= 16384) return launch_rows<8, 4, MOE, true>(p, stream);
+            return launch_rows<16, 4, MOE, true>(p, stream);
+        }
+    }
+    if(n <= 512) return launch_rows<1, 1, MOE>(p, stream);
+    if(n <= 1024) return launch_rows<2, 1, MOE>(p, stream);
+    if(n <= 2048) return launch_rows<4, 1, MOE>(p, stream);
+    if(n <= 4096) return launch_rows<4, 2, MOE>(p, stream);
+    if(n <= 8192) return launch_rows<4, 4, MOE>(p, stream);
+    if(n <= 16384) return launch_rows<8, 4, MOE>(p, stream);
+    if(n <= 32768) return launch_rows<16, 4, MOE>(p, stream);
     hipLaunchKernelGGL((sq_twopass_kernel<MOE>), dim3(p.rows), dim3(kSqThreads), 0, stream, p);
     return hipGetLastError();
 }

@@ -193,6 +193,30 @@ def test_moe_token_major(w8a8, gpu, tokens, hidden, experts, topk):
     check_exact(host(q), host(r), qo, ro)
 
 
+# By pairs and by tokens, each count of waves a row, odd lengths (rows at odd
+# addresses, a last chunk of 1-7 elements); ids outside the experts skipped.
+@pytest.mark.parametrize("tokens,hidden,experts,topk", [
+    (9, 513, 8, 6), (85, 2049, 8, 6), (40, 8191, 8, 6), (300, 4097, 4, 2), (1300, 1001, 8, 6),
+    (530, 2055, 8, 6), (530, 4103, 16, 6), (3, 16001, 4, 3), (1040, 8199, 4, 3), (700, 257, 8, 6)])
+def test_moe_pairs_and_tokens(w8a8, gpu, tokens, hidden, experts, topk):
+    test_moe_token_major(w8a8, gpu, tokens, hidden, experts, topk)
+
+
+@pytest.mark.parametrize("m,n", [(37, 9), (37, 513), (700, 1337), (37, 2047), (33, 4095), (5, 8001),
+                                 (3, 16390), (3, 32767)])
+def test_odd_rows_at_odd_addresses(w8a8, gpu, m, n):
+    import torch
+    x = G.activations(n, m, n)
+    s = G.uniform(n, G.TID_S, (n + 1,), 0.5, 2.0)
+    buf = torch.zeros(m * n + 1, dtype=torch.float16, device=gpu)
+    xd = buf[1:].view(m, n).copy_(dev(x, gpu))
+    qbuf = torch.full((m * (n + 3) + 1,), -99, dtype=torch.int8, device=gpu)
+    q, r = w8a8.smoothquant(xd, dev(s, gpu)[1:], out=qbuf[1:].view(m, n + 3)[:, :n])
+    check_exact(host(q), host(r), *O.smoothquant(x, s[1:]))
+    got = host(qbuf)
+    assert got[0] == -99 and (got[1:].reshape(m, n + 3)[:, n:] == -99).all()
+
+
 def test_moe_sorted_destinations(w8a8, gpu):
     import torch
     tokens, hidden, experts, topk = 50, 4096, 8, 2
