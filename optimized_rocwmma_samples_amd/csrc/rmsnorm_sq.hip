@@ -25,7 +25,10 @@
 // every access a buffer instruction with an out-of-range offset for masked
 // lanes (no branches, exact vmcnt waits).  Two reductions per row (sum of
 // squares, then absmax) go through DPP within a wave and LDS across waves.
-// rmsq_generic_kernel: any stride, alignment or length; one block per row.
+// rmsq_rows_kernel (any stride and alignment, N <= 32768): 16-byte accesses at
+// whatever address a row has, the row held in registers and once, in fp32, in
+// LDS.
+// rmsq_generic_kernel: longer rows; one block per row, three passes.
 #include "w8a8_device.hpp"
 #include "w8a8_internal.hpp"
 
@@ -257,10 +260,207 @@ rmsq_stream_kernel(NormRows p, uint32_t iters)
     }
 }
 
-// Any stride, alignment and length: one block per row, three passes over the
-// row (the later passes re-read it, mostly from L2).
+// 16 bytes (cnt >= 8) or the cnt < 8 fp16 values left in a row, zeros after them.
+__device__ __forceinline__ v4i load_chunk(const uint16_t* x, int cnt)
+{
+    v4i v{0};
+    if(cnt >= 8) {
+        __builtin_memcpy(&v, x, 16);
+    } else if(cnt > 0) {
+        uint32_t w[4] = {0, 0, 0, 0};
+#pragma unroll
+        for(int e = 0; e < 7; ++e)
+            if(e < cnt) w[e / 2] |= (uint32_t)x[e] << (16 * (e % 2));
+        v = v4i{(int)w[0], (int)w[1], (int)w[2], (int)w[3]};
+    }
+    return v;
+}
+
+__device__ __forceinline__ void load_chunk(float (&d)[8], const float* v, int cnt)
+{
+    if(cnt >= 8) {
+        __builtin_memcpy(d, v, 16);
+        __builtin_memcpy(d + 4, v + 4, 16);
+    } else {
+#pragma unroll
+        for(int e = 0; e < 8; ++e) d[e] = e < cnt ? v[e] : 0.f;
+    }
+}
+
+__device__ __forceinline__ void store_chunk(uint16_t* x, const uint32_t (&w)[4], int cnt)
+{
+    if(cnt >= 8) {
+        __builtin_memcpy(x, w, 16);
+    } else {
+#pragma unroll
+        for(int e = 0; e < 7; ++e)
+            if(e < cnt) x[e] = (uint16_t)(w[e / 2] >> (16 * (e % 2)));
+    }
+}
+
 constexpr int kGenThreads = 256;
 
+// Any stride and alignment: WPR waves per row, CPL 16-byte chunks per lane.
+// A row is read once and stays in registers.  Its squares are added in the
+// order of rmsq_generic_kernel (256 sums of every 256th column, then the
+// waves' totals left to right), for which the row passes through LDS in fp32:
+// rows of a length have the same bits whichever of the two kernels they take.
+// What the generic kernel spends its time on is a chain of 2-byte loads, each
+// waiting for the one before, in three passes.  WPR = 1 needs no barrier and
+// keeps up to 20 rows per CU in flight; longer rows take 4 or 16 waves so that
+// a single long row is not one wave's work.  Bound by vector instructions (23
+// an element, 45% of the time) and by each row's chain of load, sum, maximum
+// and store; loading gamma and s ahead of the sum, or more waves of fewer
+// chunks, gave nothing.
+template <int CPL, int WPR, bool RES>
+__global__ void __launch_bounds__(WPR > 4 ? WPR * kWave : kGenThreads)
+rmsq_rows_kernel(NormRows p, uint32_t row_floats)
+{
+    constexpr int kSums = kGenThreads / kWave; // waves' worth of partial sums
+    extern __shared__ __attribute__((aligned(16))) float lds[];
+    __shared__ float red[2][WPR];
+
+    const int      wave = threadIdx.x / kWave;
+    const int      lane = threadIdx.x % kWave;
+    const int      part = wave % WPR;
+    const uint32_t row  = WPR == 1 ? blockIdx.x * (blockDim.x / kWave) + wave : blockIdx.x;
+    if(row >= p.rows) return; // WPR > 1: a row is a block
+    const uint32_t  n    = p.n;
+    const uint32_t  base = (part * CPL * kWave + lane) * 8;
+    float*          v_l  = lds + (WPR == 1 ? wave * row_floats : 0);
+    const uint16_t* xr   = p.x + (size_t)row * p.ldx;
+    const uint16_t* rr   = RES ? p.res + (size_t)row * p.ldx : nullptr;
+    uint16_t*       xo   = p.x_out ? p.x_out + (size_t)row * p.ldx : nullptr;
+    auto left = [&](int j) { return (int)n - (int)(base + j * (8 * kWave)); };
+
+    // 1. v = x (+ res) to LDS; u = half(v) in registers and to x_out
+    v4i x[CPL], res[CPL];
+#pragma unroll
+    for(int j = 0; j < CPL; ++j) {
+        x[j] = load_chunk(xr + base + j * (8 * kWave), left(j));
+        if constexpr(RES) res[j] = load_chunk(rr + base + j * (8 * kWave), left(j));
+    }
+#pragma unroll
+    for(int j = 0; j < CPL; ++j) {
+        if(left(j) <= 0) continue;
+        float v[8];
+#pragma unroll
+        for(int e = 0; e < 8; ++e) {
+            v[e] = half_bits_to_float(((uint32_t)x[j][e / 2] >> (16 * (e % 2))) & 0xFFFFu);
+            if constexpr(RES)
+                v[e] += half_bits_to_float(((uint32_t)res[j][e / 2] >> (16 * (e % 2))) & 0xFFFFu);
+        }
+        float4* d = reinterpret_cast<float4*>(v_l + base + j * (8 * kWave));
+        d[0]      = float4{v[0], v[1], v[2], v[3]};
+        d[1]      = float4{v[4], v[5], v[6], v[7]};
+        if constexpr(RES) {
+#pragma unroll
+            for(int e = 0; e < 4; ++e) x[j][e] = (int)pack_half2(v[2 * e], v[2 * e + 1]);
+        }
+        if(xo) {
+            const uint32_t w[4] = {(uint32_t)x[j].x, (uint32_t)x[j].y, (uint32_t)x[j].z,
+                                   (uint32_t)x[j].w};
+            store_chunk(xo + base + j * (8 * kWave), w, left(j));
+        }
+    }
+
+    // 2. sum of squares, rstd
+    float ss;
+    if constexpr(WPR == 1) {
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        float t[kSums] = {};
+        for(uint32_t c0 = 0; c0 < n; c0 += kGenThreads)
+#pragma unroll
+            for(int w = 0; w < kSums; ++w) {
+                const uint32_t c = c0 + w * kWave + lane;
+                const float    v = c < n ? v_l[c] : 0.f;
+                t[w] += v * v;
+            }
+        ss = wave_sum(t[0]);
+#pragma unroll
+        for(int w = 1; w < kSums; ++w) ss = ss + wave_sum(t[w]);
+    } else {
+        __syncthreads();
+        if(wave < kSums) {
+            float t = 0.f;
+#pragma unroll 8
+            for(uint32_t c = threadIdx.x; c < n; c += kGenThreads) t += v_l[c] * v_l[c];
+            t = wave_sum(t);
+            if(lane == 0) red[0][wave] = t;
+        }
+        __syncthreads();
+        ss = red[0][0];
+#pragma unroll
+        for(int w = 1; w < kSums; ++w) ss = ss + red[0][w];
+    }
+    const float rstd = rsqrtf(ss / (float)n + p.eps);
+
+    // 3. y and the products to quantize
+    uint16_t* yr   = p.y ? p.y + (size_t)row * p.ldy : nullptr;
+    float     amax = 0.f;
+    float     pv[CPL * 8];
+#pragma unroll
+    for(int j = 0; j < CPL; ++j) {
+        if(left(j) <= 0) continue;
+        const uint32_t c = base + j * (8 * kWave);
+        float          g[8];
+        load_chunk(g, p.gamma + c, left(j));
+        uint32_t yh[4];
+#pragma unroll
+        for(int e = 0; e < 4; ++e) {
+            const uint32_t w = (uint32_t)x[j][e];
+            yh[e] = pack_half2((half_bits_to_float(w & 0xFFFFu) * rstd) * g[2 * e],
+                               (half_bits_to_float(w >> 16) * rstd) * g[2 * e + 1]);
+        }
+        if(yr) store_chunk(yr + c, yh, left(j));
+        if(p.q) {
+            float s[8];
+            load_chunk(s, p.s + c, left(j));
+#pragma unroll
+            for(int e = 0; e < 8; e += 2) {
+                pv[j * 8 + e]     = mul_h16_f32<false>(yh[e / 2], s[e]);
+                pv[j * 8 + e + 1] = mul_h16_f32<true>(yh[e / 2], s[e + 1]);
+                amax = fmaxf(fmaxf(amax, fabsf(pv[j * 8 + e])), fabsf(pv[j * 8 + e + 1]));
+            }
+        }
+    }
+    if(!p.q) return; // the same in every lane
+
+    // 4. quantize
+    amax = wave_max(amax);
+    if constexpr(WPR > 1) {
+        if(lane == 0) red[1][wave] = amax;
+        __syncthreads();
+#pragma unroll
+        for(int w = 0; w < WPR; ++w) amax = fmaxf(amax, red[1][w]);
+    }
+    const float qmax = p.qmax;
+    const float rs   = amax / qmax;
+    if(part == 0 && lane == 0) p.r[row] = rs;
+    const float inv = rs > 0.f ? 1.f / rs : 0.f;
+    int8_t*     qr  = p.q + (size_t)row * p.ldq;
+#pragma unroll
+    for(int j = 0; j < CPL; ++j) {
+        if(left(j) <= 0) continue;
+        const float* v     = pv + j * 8;
+        uint32_t     pk[2] = {cvt_pack4_i8(quant_f(v[0], inv, qmax), quant_f(v[1], inv, qmax),
+                                           quant_f(v[2], inv, qmax), quant_f(v[3], inv, qmax)),
+                              cvt_pack4_i8(quant_f(v[4], inv, qmax), quant_f(v[5], inv, qmax),
+                                           quant_f(v[6], inv, qmax), quant_f(v[7], inv, qmax))};
+        int8_t* d = qr + base + j * (8 * kWave);
+        if(left(j) >= 8) {
+            __builtin_memcpy(d, pk, 8);
+        } else {
+#pragma unroll
+            for(int e = 0; e < 7; ++e)
+                if(e < left(j)) d[e] = (int8_t)(pk[e / 4] >> (8 * (e % 4)));
+        }
+    }
+}
+
+// Rows longer than the register-resident path covers: one block per row, three
+// passes over the row (the later passes re-read it, mostly from L2).
 template <bool RES>
 __global__ void __launch_bounds__(kGenThreads) rmsq_generic_kernel(NormRows p)
 {
@@ -372,6 +572,31 @@ hipError_t launch_stream_norm(const NormRows& p, hipStream_t stream)
     return hipSuccess;
 }
 
+template <int CPL, int WPR>
+hipError_t launch_rows_norm(const NormRows& p, hipStream_t stream)
+{
+    constexpr int  kThreads = WPR > 4 ? WPR * kWave : kGenThreads;
+    constexpr int  kRows    = WPR == 1 ? kThreads / kWave : 1;
+    const uint32_t floats   = (p.n + 7) / 8 * 8; // one row's share of LDS
+    const size_t   lds      = (size_t)kRows * floats * sizeof(float);
+    const dim3     grid((p.rows + kRows - 1) / kRows);
+    if constexpr((size_t)CPL * WPR * 512 * kRows * sizeof(float) >= 65536) { // red is in LDS too
+        static std::once_flag once;
+        std::call_once(once, [] {
+            for(const void* k : {reinterpret_cast<const void*>(rmsq_rows_kernel<CPL, WPR, true>),
+                                 reinterpret_cast<const void*>(rmsq_rows_kernel<CPL, WPR, false>)})
+                (void)hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                          CPL * WPR * 512 * kRows * sizeof(float));
+            (void)hipGetLastError();
+        });
+    }
+    if(p.res)
+        hipLaunchKernelGGL((rmsq_rows_kernel<CPL, WPR, true>), grid, dim3(kThreads), lds, stream, p, floats);
+    else
+        hipLaunchKernelGGL((rmsq_rows_kernel<CPL, WPR, false>), grid, dim3(kThreads), lds, stream, p, floats);
+    return hipGetLastError();
+}
+
 template <int CPL, int WPR, int THREADS, int BPC>
 hipError_t launch_by_outputs(const NormRows& p, hipStream_t stream)
 {
@@ -397,7 +622,7 @@ hipError_t launch_rmsnorm_sq(const NormRows& p, hipStream_t stream)
     const bool vec = n % 8 == 0 && p.ldx % 8 == 0 && p.ldy % 8 == 0 && p.ldq % 8 == 0
                      && al(p.x, 16) && al(p.res, 16) && al(p.x_out, 16) && al(p.y, 16)
                      && al(p.q, 8) && al(p.gamma, 16) && al(p.s, 16);
-    // x_out without a residual is a plain copy: the generic kernel does it
+    // x_out without a residual is a plain copy: the rows kernel does it
     if(vec && !(p.x_out && !p.res)) {
         // two 16-byte chunks per lane and tensor: x and residual double-buffered
         // fit 128 VGPRs, i.e. two 512-thread blocks per CU
@@ -407,6 +632,20 @@ hipError_t launch_rmsnorm_sq(const NormRows& p, hipStream_t stream)
         if(n <= 8192) return launch_by_outputs<2, 8, 512, 2>(p, stream);
         if(n <= 16384) return launch_by_outputs<2, 16, 1024, 1>(p, stream);
     }
+    // Other rows by length, kernel times against the generic kernel's: 12633 x 881
+    // with residual 43 -> 22.6 us, 3000 x 4095 45 -> 28, 3000 x 8191 71 -> 36 (without),
+    // 500 x 16383 73 -> 20.4, 1 x 14716 36 -> 7.4.
+    if(n <= 512) return launch_rows_norm<1, 1>(p, stream);
+    // up to 8 rows a CU, all resident: a block a row (1 x 2047 4.4 us against 9.5 by
+    // one wave, 1000 x 881 5.6 against 6.7); past that a wave a row, which waits at
+    // no barrier (30000 x 2047 146 us against 173)
+    if(n <= 2048 && p.rows <= 2048) return launch_rows_norm<1, 4>(p, stream);
+    if(n <= 1024) return launch_rows_norm<2, 1>(p, stream);
+    if(n <= 2048) return launch_rows_norm<4, 1>(p, stream);
+    if(n <= 4096) return launch_rows_norm<2, 4>(p, stream);
+    if(n <= 8192) return launch_rows_norm<4, 4>(p, stream);
+    if(n <= 16384) return launch_rows_norm<2, 16>(p, stream);
+    if(n <= 32768) return launch_rows_norm<4, 16>(p, stream);
     if(p.res)
         hipLaunchKernelGGL(rmsq_generic_kernel<true>, dim3(p.rows), dim3(kGenThreads), 0, stream, p);
     else

@@ -54,7 +54,7 @@ def inputs(m, n, seed):
 
 
 # rows of whole 16-byte chunks take the streaming kernel (N <= 16384 per
-# configuration); the others (N % 8 != 0, N > 16384) take the generic kernel
+# configuration); the others (N % 8 != 0, N > 16384) the rows kernel, N > 32768 the generic one
 SHAPES = [(64, 4096), (256, 2048), (1, 512), (17, 8192), (5, 16384), (100, 4104), (33, 1000),
           (9, 1024), (3, 20000), (7, 24), (2, 7)]
 
@@ -134,6 +134,42 @@ def test_strided_rows(w8a8, gpu):
     assert (host(xo.as_strided((m, pad), (n + pad, 1), n)) == 3.0).all()
     assert (host(y.as_strided((m, 8), (n + 8, 1), n)) == 5.0).all()
     assert (host(q.as_strided((m, 16), (n + 16, 1), n)) == 9).all()
+
+
+# Rows at odd addresses and of odd lengths: each count of waves a row and of
+# chunks a lane, full and ragged, and a row past the last that they cover.
+@pytest.mark.parametrize("m,n", [(5, 1), (37, 9), (3, 512), (37, 1023), (9, 2041), (2049, 1001), (2049, 1025),
+                                 (5, 4095), (3, 8191), (3, 8200), (2, 16384), (2, 32767), (2, 32769)])
+@pytest.mark.parametrize("with_res", [True, False])
+def test_odd_rows_at_odd_addresses(w8a8, gpu, m, n, with_res):
+    import torch
+    x, res, gamma, s = inputs(m, n, 300 + n)
+
+    def at_odd(a, fill, pad=3):
+        """a's rows, pad elements apart, from the second element of a buffer on"""
+        buf = torch.full((m * (n + pad) + 1,), fill, dtype=a.dtype, device=gpu)
+        rows = buf[1:].view(m, n + pad)
+        rows[:, :n] = a
+        return buf, rows[:, :n]
+
+    def padding(buf):
+        return np.append(host(buf)[1:].reshape(m, n + 3)[:, n:], host(buf)[0])
+
+    gd = torch.cat([torch.zeros(1), torch.from_numpy(gamma)]).to(gpu)[1:]
+    sd = torch.cat([torch.zeros(1), torch.from_numpy(s)]).to(gpu)[1:]
+    _, xd = at_odd(dev(x, gpu), 1)
+    _, rd = at_odd(dev(res, gpu), 1) if with_res else (None, None)
+    xbuf, xo = at_odd(torch.zeros_like(xd), 3) if with_res else (None, None)
+    ybuf, y = at_odd(torch.zeros_like(xd), 5)
+    qbuf, q = at_odd(torch.zeros((m, n), dtype=torch.int8, device=gpu), 9)
+    _, _, _, r = w8a8.add_rmsnorm_smoothquant(xd, gd, sd, residual=rd, x_out=xo, y=y, q=q)
+    xo_o, y_o, q_o, r_o = O.rmsnorm_smoothquant(x, gamma, s, res=res if with_res else None)
+    if with_res:
+        assert np.array_equal(host(xo).view(np.uint16), xo_o.view(np.uint16))
+        assert (padding(xbuf) == 3).all()
+    check_y(host(y), y_o)
+    check_quant(host(q), host(r), host(y), s, q_o, r_o)
+    assert (padding(ybuf) == 5).all() and (padding(qbuf) == 9).all()
 
 
 def test_zero_rows_and_default_fill(w8a8, gpu):
