@@ -122,10 +122,11 @@ int w8a8_add_rmsnorm_smoothquant(const void* x, const void* residual, const floa
 
 /*
  * Bytes of device workspace w8a8_gemm can use for this problem.  Sample
- * layout: A and B are repacked K-contiguous into it.  Primary layout: int32
- * K-split partials when the problem's tiles would fill at most half of the
- * CUs (0 otherwise); the rocWMMA split-K sample likewise takes a
- * caller-allocated workspace (rocwmma_gemm_splitk.cpp:214).
+ * layout: A and B are repacked K-contiguous into it (plus the K split of the
+ * GEMM over them).  Primary layout: int32 K-split partials of problems with
+ * few tiles or a last round that is nearly empty (0 otherwise); the rocWMMA
+ * split-K sample likewise takes a caller-allocated workspace
+ * (rocwmma_gemm_splitk.cpp:214).
  */
 size_t w8a8_gemm_workspace_size(uint32_t m, uint32_t n, uint32_t k, int layout);
 
@@ -142,17 +143,20 @@ size_t w8a8_gemm_workspace_size(uint32_t m, uint32_t n, uint32_t k, int layout);
  *           half((float(acc) * sa) * sb),  sa = scale_a ? scale_a[m] : tensor_scale_a,
  *                                          sb = scale_b ? scale_b[n] : tensor_scale_b
  * Argument order follows gemm_quant_tensor_scale (m, n, k, a, b, c, lda, ldb, ldc, scales).
- * Decode shapes (m <= 64) run a weight-streaming kernel that splits K across
- * the waves of each block and reduces the int32 partials in LDS: the role of
- * gemm_splitk_stage1/gemm_splitk_reduce (rocwmma_gemm_splitk.cpp:104-201) and
- * streamk_gemm_kernel (rocwmma_streamk_gemm.cpp:86-211), in one launch with no
- * workspace, bit-identical to the full GEMM.
- * Primary layout with a workspace (16-byte aligned, at least
- * w8a8_gemm_workspace_size bytes; NULL or smaller: not used): a problem
- * whose tiles fill at most half of the CUs runs each tile as K pieces on the
- * idle CUs, the pieces' int32 partials go to the workspace and a second
- * launch sums them, again bit-identical.  Calls sharing a workspace must be
- * ordered on one stream.
+ * Decode shapes (m <= 64) run tiles of 32 or 64 rows or, where the whole
+ * launch is a few k-tiles per wave, a weight-streaming kernel that splits K
+ * across the waves of each block and reduces the int32 partials in LDS: the
+ * role of gemm_splitk_stage1/gemm_splitk_reduce
+ * (rocwmma_gemm_splitk.cpp:104-201) and streamk_gemm_kernel
+ * (rocwmma_streamk_gemm.cpp:86-211), bit-identical to the full GEMM.
+ * Primary layout with a workspace (16-byte aligned): where it is estimated to
+ * be faster, each tile runs as K pieces on otherwise idle CUs, the pieces'
+ * int32 partials go to the workspace and a second launch sums them, again
+ * bit-identical.  w8a8_gemm_workspace_size bytes allow every such plan; with
+ * less (or NULL) the plans that fit remain.  Calls sharing a workspace must
+ * be ordered on one stream.
+ * The sample layout without room to repack (and small problems with it) is
+ * computed in place.
  */
 int w8a8_gemm(uint32_t m, uint32_t n, uint32_t k, const int8_t* a, const int8_t* b, void* c,
               uint32_t lda, uint32_t ldb, uint32_t ldc, const float* scale_a,
@@ -226,9 +230,10 @@ int w8a8_debug_streamk_wait(uint32_t spin_limit, uint32_t phantom_pieces);
  * workspace w8a8_gemm would take (K-split partials, the sample layout's
  * repack) is a scratch array the library holds on each GPU it runs on, of
  * W8A8_NOALLOC_SCRATCH_BYTES, kept until the process ends.  Results are
- * bit-identical to w8a8_gemm given a workspace of that size.  Shapes whose
- * w8a8_gemm_workspace_size exceeds it return W8A8_ERROR_INVALID_VALUE
- * before any HIP call.  The entry point calls no allocating routine (no
+ * bit-identical to w8a8_gemm given a workspace of that size.  Sample-layout
+ * shapes whose repacked operands (K rounded up to 16) exceed it return
+ * W8A8_ERROR_INVALID_VALUE before any HIP call; a K split takes a plan that
+ * fits.  The entry point calls no allocating routine (no
  * hipMalloc / hipFree), for callers that cannot allocate: code under HIP
  * graph capture, tight serving loops, harnesses that forbid allocation.
  * Every call on one GPU shares that GPU's array, and nothing in it needs
@@ -301,8 +306,9 @@ int w8a8_quantize_weights(const void* w, uint32_t n, uint32_t k, uint32_t ldw,
 /*
  * Bytes of device workspace w8a8_gemm_packed / w8a8_fused_sq_gemm_packed can
  * use for an m x n x k problem: the int32 split-K partials of decode shapes
- * with 32 < m <= 64 (the caller-allocated workspace of the reference's
- * split-K, rocwmma_gemm_splitk.cpp:214); 0 when the shape takes no workspace.
+ * with 32 < m <= 64 and of larger m whose tiles are few (the caller-allocated
+ * workspace of the reference's split-K, rocwmma_gemm_splitk.cpp:214); 0 when
+ * the shape takes no workspace.
  */
 size_t w8a8_gemm_packed_workspace_size(uint32_t m, uint32_t n, uint32_t k);
 
@@ -312,8 +318,8 @@ size_t w8a8_gemm_packed_workspace_size(uint32_t m, uint32_t n, uint32_t k);
  * A with lda % 16 == 0 and k % 16 == 0 (W8A8_ERROR_NOT_SUPPORTED otherwise).
  * Decode shapes (m <= 64) stream the packed weights at close to HBM rate.
  * workspace (16-byte aligned, ws_bytes >= w8a8_gemm_packed_workspace_size)
- * lets 32 < m <= 64 split K across blocks; NULL runs the unsplit kernel
- * (same results).
+ * lets m > 32 split K across blocks; NULL runs the unsplit kernel (same
+ * results).
  */
 int w8a8_gemm_packed(uint32_t m, uint32_t n, uint32_t k, const int8_t* a,
                      const int8_t* w_packed, void* c, uint32_t lda, uint32_t ldc,

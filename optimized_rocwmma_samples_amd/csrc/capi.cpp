@@ -234,7 +234,7 @@ static size_t repack_bytes(uint32_t m, uint32_t n, uint32_t k, uint32_t step)
 size_t w8a8_gemm_workspace_size(uint32_t m, uint32_t n, uint32_t k, int layout)
 {
     if(layout == W8A8_LAYOUT_A_ROW_B_NK) {
-        // K-split partials for launches that fill at most half the CUs
+        // K-split partials
         w8a8::GemmArgs g{m, n, k, nullptr, nullptr, nullptr, k, k, n, nullptr, nullptr, 1.f, 1.f,
                          W8A8_OUT_F16};
         return w8a8::gemm_nk_workspace_bytes(g);

@@ -1,9 +1,8 @@
 // gemm_i8.hip -- launchers of the int8 GEMM: the gfx950 MFMA tile kernel
 // (gemm_i8_kernel.hpp) over row-major or packed weights (gemm_i8_pack.hpp), the
-// decode kernels for m <= 64 (gemm_i8_decode_kernel.hpp), a generic strided
-// kernel for shapes the tile kernels do not take (k % 16 != 0, unaligned
-// operands) and the repack used for the reference sample's A col-major /
-// B [K,N] layout.
+// decode kernels for m <= 64 (gemm_i8_decode_kernel.hpp), the tile kernel for
+// operands those do not take (k % 16 != 0, unaligned: gemm_i8_direct_kernel.hpp)
+// and the repack used for the reference sample's A col-major / B [K,N] layout.
 #include "gemm_i8_decode_kernel.hpp"
 #include "gemm_i8_decode_wide_kernel.hpp"
 #include "gemm_i8_direct_kernel.hpp"
@@ -25,7 +24,7 @@ namespace {
 using gemm::KArgs;
 
 // Production tile configuration, and the smaller tiles of launches that
-// would leave most CUs idle with it (pick_tile_cfg).  All on the
+// would leave most CUs idle with it (plan_tiles).  All on the
 // 16 x 16 x 64 MFMA (gemm::Cfg): against the 32 x 32 x 32 form, GEMM-only,
 // cold weights, cfg3 projections: M = 8192 1448 -> 1389 µs, M = 2048 411 ->
 // 398 µs, M = 512 144 -> 132 µs (sum of the four).

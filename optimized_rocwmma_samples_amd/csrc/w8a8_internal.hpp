@@ -64,8 +64,8 @@ struct GemmArgs {
 // k % 16 == 0.
 // Small m (decode) is routed to the decode kernel inside launch_gemm_nk.
 bool       gemm_fast_path_ok(const GemmArgs& g);
-// ws (optional): int32 partials of a K split, used when the launch's tiles
-// fill at most half the CUs and ws_bytes >= gemm_nk_workspace_bytes(g).
+// ws (optional): int32 partials of a K split, where a plan whose partials fit
+// ws_bytes is estimated to be faster; gemm_nk_workspace_bytes allows them all.
 hipError_t launch_gemm_nk(const GemmArgs& g, void* ws, size_t ws_bytes, hipStream_t stream);
 size_t     gemm_nk_workspace_bytes(const GemmArgs& g);
 // Explicit stream-K over every tile (w8a8_gemm_streamk): `blocks` blocks (0:
@@ -129,9 +129,9 @@ hipError_t launch_quantize_weights(const WeightQuant& p, bool divide, bool packe
 // A, lda % 16 == 0, k % 16 == 0 and every A panel addressable (< 2 GiB).
 bool       gemm_packed_ok(const GemmArgs& g);
 hipError_t launch_gemm_packed(const GemmArgs& g, void* ws, size_t ws_bytes, hipStream_t stream);
-// Split-K workspace the packed path can use for this problem (decode shapes
-// 32 < m <= 64); 0 when none is used.  A smaller (or no) workspace falls back
-// to the unsplit decode kernel.
+// Split-K workspace the packed path can use for this problem (m > 32); 0 when
+// none is used.  A smaller (or no) workspace falls back to the unsplit decode
+// kernel (m <= 64) or to a plan whose partials fit.
 size_t     packed_workspace_bytes(const GemmArgs& g);
 
 // Tile GEMM over any pointers, strides and K (gemm_i8_direct_kernel.hpp): the
