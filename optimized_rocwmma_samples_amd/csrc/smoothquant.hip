@@ -74,16 +74,19 @@ __device__ __forceinline__ RowSrc resolve_row(const QuantRows& p, uint32_t row)
     return rs;
 }
 
+constexpr int sq_rows_threads(int wpr) { return wpr * kWave > kSqThreads ? wpr * kWave : kSqThreads; }
+
 // CPL: 16-byte chunks per lane; WPR: waves per row.  MOE: a group of WPR waves
 // takes a token and writes its topk rows one after another, or (PAIRS) one
 // (token, slot) pair.
 template <int CPL, int WPR, bool MOE, bool PAIRS>
-__global__ void __launch_bounds__(kSqThreads) sq_rows_kernel(QuantRows p)
+__global__ void __launch_bounds__(sq_rows_threads(WPR)) sq_rows_kernel(QuantRows p)
 {
-    constexpr int kRowsPerBlock = kSqWaves / WPR;
+    constexpr int kWaves        = sq_rows_threads(WPR) / kWave;
+    constexpr int kRowsPerBlock = kWaves / WPR;
     constexpr int kSpan         = CPL * 8 * kWave;
     constexpr bool kTokens      = MOE && !PAIRS;
-    __shared__ float red[2][kSqWaves];
+    __shared__ float red[2][kWaves];
 
     const int      wave = threadIdx.x / kWave;
     const int      lane = threadIdx.x % kWave;
@@ -430,10 +433,11 @@ hipError_t launch_stream(const QuantRows& p, hipStream_t stream)
 template <int CPL, int WPR, bool MOE, bool PAIRS = false>
 hipError_t launch_rows(const QuantRows& p, hipStream_t stream)
 {
-    constexpr int  kRowsPerBlock = kSqWaves / WPR;
+    constexpr int  kThreads      = sq_rows_threads(WPR);
+    constexpr int  kRowsPerBlock = kThreads / kWave / WPR;
     const uint32_t units         = MOE && !PAIRS ? p.rows / p.topk : p.rows;
     hipLaunchKernelGGL((sq_rows_kernel<CPL, WPR, MOE, PAIRS>),
-                       dim3((units + kRowsPerBlock - 1) / kRowsPerBlock), dim3(kSqThreads), 0,
+                       dim3((units + kRowsPerBlock - 1) / kRowsPerBlock), dim3(kThreads), 0,
                        stream, p);
     return hipGetLastError();
 }
@@ -498,8 +502,8 @@ hipError_t dispatch(const QuantRows& p, hipStream_t stream)
         if(n > 2048 && n <= 32768 && (p.rows <= 3072 || p.topk <= 2)) {
             if(n <= 4096) return launch_rows<4, 2, MOE, true>(p, stream);
             if(n <= 8192) return launch_rows<4, 4, MOE, true>(p, stream);
-            if(n <= 16384) return launch_rows<8, 4, MOE, true>(p, stream);
-            return launch_rows<16, 4, MOE, true>(p, stream);
+            if(n <= 16384) return launch_rows<2, 16, MOE, true>(p, stream);
+            return launch_rows<4, 16, MOE, true>(p, stream);
         }
     }
     if(n <= 512) return launch_rows<1, 1, MOE>(p, stream);
@@ -507,8 +511,15 @@ hipError_t dispatch(const QuantRows& p, hipStream_t stream)
     if(n <= 2048) return launch_rows<4, 1, MOE>(p, stream);
     if(n <= 4096) return launch_rows<4, 2, MOE>(p, stream);
     if(n <= 8192) return launch_rows<4, 4, MOE>(p, stream);
-    if(n <= 16384) return launch_rows<8, 4, MOE>(p, stream);
-    if(n <= 32768) return launch_rows<16, 4, MOE>(p, stream);
+    // Rows of more than 8192: 16 waves, but 4 for more dense rows than fill the
+    // chip (1 / 512 / 8000 rows of 8199: 3.4 / 7.0 / 80 us by 16 waves, 5.5 / 8.2 /
+    // 68 by 4; 1 / 8000 of 28671 5.0 / 192 against 8.0 / 230; 1024 tokens of
+    // 14336, top 4, 28.6 against 35.3).
+    if constexpr(!MOE) {
+        if(n <= 16384 && p.rows > 1024) return launch_rows<8, 4, MOE>(p, stream);
+    }
+    if(n <= 16384) return launch_rows<2, 16, MOE>(p, stream);
+    if(n <= 32768) return launch_rows<4, 16, MOE>(p, stream);
     hipLaunchKernelGGL((sq_twopass_kernel<MOE>), dim3(p.rows), dim3(kSqThreads), 0, stream, p);
     return hipGetLastError();
 }

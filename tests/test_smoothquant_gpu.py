@@ -197,13 +197,14 @@ def test_moe_token_major(w8a8, gpu, tokens, hidden, experts, topk):
 # addresses, a last chunk of 1-7 elements); ids outside the experts skipped.
 @pytest.mark.parametrize("tokens,hidden,experts,topk", [
     (9, 513, 8, 6), (85, 2049, 8, 6), (40, 8191, 8, 6), (300, 4097, 4, 2), (1300, 1001, 8, 6),
-    (530, 2055, 8, 6), (530, 4103, 16, 6), (3, 16001, 4, 3), (1040, 8199, 4, 3), (700, 257, 8, 6)])
+    (530, 2055, 8, 6), (530, 4103, 16, 6), (3, 16001, 4, 3), (1040, 8199, 4, 3), (700, 257, 8, 6),
+    (3, 16399, 4, 2), (1040, 16399, 4, 3)])
 def test_moe_pairs_and_tokens(w8a8, gpu, tokens, hidden, experts, topk):
     test_moe_token_major(w8a8, gpu, tokens, hidden, experts, topk)
 
 
 @pytest.mark.parametrize("m,n", [(37, 9), (37, 513), (700, 1337), (37, 2047), (33, 4095), (5, 8001),
-                                 (3, 16390), (3, 32767)])
+                                 (3, 8201), (1030, 8201), (3, 16390), (3, 32767)])
 def test_odd_rows_at_odd_addresses(w8a8, gpu, m, n):
     import torch
     x = G.activations(n, m, n)
