@@ -191,6 +191,8 @@ def test_zero_rows_and_default_fill(w8a8, gpu):
 def test_add_rmsnorm_vs_reference_kernel(w8a8, gpu, m, n):
     # the reference's own kernel_add_rmsnorm2d_fwd on the same device buffers
     # (N % 8 == 0: the reference has no tail loop for the last N % 8 columns)
+    if O.ref() is None:
+        pytest.skip("oracle/_ref (reference kernels) not built")
     x, res, gamma, _ = inputs(m, n, 300 + n)
     xd, rd, gd = dev(x, gpu), dev(res, gpu), dev(gamma, gpu)
     xo_ref, y_ref = O.ref_rmsnorm2d_gpu(xd, gd, residual=rd)
@@ -202,6 +204,8 @@ def test_add_rmsnorm_vs_reference_kernel(w8a8, gpu, m, n):
 @pytest.mark.parametrize("m,n", [(64, 4096), (16, 8192), (32, 2048)])
 def test_rmsnorm_vs_reference_kernel(w8a8, gpu, m, n):
     # N a multiple of 2048: the reference's tail loop adds nothing twice there
+    if O.ref() is None:
+        pytest.skip("oracle/_ref (reference kernels) not built")
     x, _, gamma, _ = inputs(m, n, 400 + n)
     xd, gd = dev(x, gpu), dev(gamma, gpu)
     _, y_ref = O.ref_rmsnorm2d_gpu(xd, gd)
