@@ -221,6 +221,18 @@ int w8a8_gemm_streamk_status(uint32_t* flags, int clear);
 int w8a8_debug_streamk_wait(uint32_t spin_limit, uint32_t phantom_pieces);
 
 /*
+ * Test hook: the kernel a call of the given sizes takes, so that tests can
+ * say which one they run.  Host arithmetic only (without a GPU: of 256 CUs).
+ * sizes and plan hold 4 and 3 values:
+ *   W8A8_PLAN_MOE_QUANT  tokens * topk, hidden, topk
+ *                        -> 16-byte chunks per lane, waves per row (0: two
+ *                           passes over a row), 1 where a group of waves takes
+ *                           a token, 0 where it takes a (token, slot) pair
+ */
+#define W8A8_PLAN_MOE_QUANT 0
+int w8a8_debug_plan(int kind, const uint32_t* sizes, uint32_t* plan);
+
+/*
  * Bytes of the per-GPU scratch array w8a8_gemm_noalloc uses (32 MiB).
  */
 #define W8A8_NOALLOC_SCRATCH_BYTES (32u << 20)

@@ -24,6 +24,8 @@ OUT_F16 = 1
 
 STREAMK_WAIT_EXPIRED = 1
 
+PLAN_MOE_QUANT = 0  # w8a8_debug_plan kinds
+
 GROUPED_INLINE_GROUPS = 48  # W8A8_GROUPED_INLINE_GROUPS
 
 FOLD_MULTIPLY = 0
@@ -68,6 +70,8 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
     "w8a8_gemm_streamk_blocks": (_u32, [_u32, _u32, _u32, _u32]),
     "w8a8_gemm_streamk_status": (_i32, [ctypes.POINTER(ctypes.c_uint32), _i32]),
     "w8a8_debug_streamk_wait": (_i32, [_u32, _u32]),
+    "w8a8_debug_plan": (_i32, [_i32, ctypes.POINTER(ctypes.c_uint32),
+                               ctypes.POINTER(ctypes.c_uint32)]),
     "w8a8_fused_sq_gemm": (_i32, [_ptr, _ptr, _ptr, _ptr, _ptr, _u32, _u32, _u32, _u32, _u32,
                                   _u32, _ptr, _ptr, _ptr, _size, _ptr]),
     "w8a8_pack_weights_size": (_size, [_u32, _u32]),

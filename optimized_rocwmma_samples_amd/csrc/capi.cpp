@@ -406,6 +406,23 @@ int w8a8_debug_streamk_wait(uint32_t spin_limit, uint32_t phantom_pieces)
     return W8A8_SUCCESS;
 }
 
+int w8a8_debug_plan(int kind, const uint32_t* sizes, uint32_t* plan)
+{
+    const char* fn = "w8a8_debug_plan";
+    if(!sizes || !plan) return fail(W8A8_ERROR_INVALID_VALUE, "%s: null pointer argument", fn);
+    auto set = [&](uint32_t a, uint32_t b, uint32_t c) {
+        plan[0] = a, plan[1] = b, plan[2] = c;
+        return W8A8_SUCCESS;
+    };
+    switch(kind) {
+    case W8A8_PLAN_MOE_QUANT: {
+        const w8a8::QuantPlan d = w8a8::moe_quant_plan(sizes[0], sizes[1], sizes[2]);
+        return set(d.chunks, d.waves, d.tokens);
+    }
+    default: return fail(W8A8_ERROR_INVALID_VALUE, "%s: unknown kind %d", fn, kind);
+    }
+}
+
 int w8a8_fused_sq_gemm(const void* x, const float* smooth_scale, const int8_t* w,
                        const float* scale_w, void* c, uint32_t m, uint32_t n, uint32_t k,
                        uint32_t ldx, uint32_t ldw, uint32_t ldc, int8_t* q, float* row_scale,

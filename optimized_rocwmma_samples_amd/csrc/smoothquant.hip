@@ -5,13 +5,16 @@
 //   p = float(x[row, n]) * s[n];  r = max|p| / qmax;  inv = r > 0 ? 1/r : 0
 //   q[row, n] = int8(clamp(rint(p * inv), -qmax, qmax))
 //
-// Two kernels, the same per-element operations (bit-identical results):
+// The kernels, all with the same per-element operations (bit-identical results):
 //   * sq_stream_kernel (dense rows, 16-byte aligned, N % 8 == 0, N <= 32768):
 //     s staged once per block in LDS, one block per CU walking the rows with
 //     a grid stride and double-buffering them in registers (described at the
 //     kernel);
-//   * sq_rows_kernel / sq_twopass_kernel: everything else (the MoE gather,
-//     unaligned or odd-length rows, very long rows).
+//   * sq_rows_kernel: a dense row, or one (token, slot) pair of the MoE form, of
+//     any alignment and length to 32768;
+//   * sq_tokens_kernel: the MoE form where reading a token once for all of its
+//     experts pays (moe_quant_plan says where);
+//   * sq_twopass_kernel: longer rows.
 //
 // sq_rows_kernel (HBM-bound: 3 bytes moved per element):
 //   * One wavefront owns a row segment of CPL*512 elements; WPR wavefronts
@@ -19,13 +22,9 @@
 //     address the row has (the hardware takes unaligned global accesses), so a
 //     wave instruction reads 1 KiB contiguous and the whole segment is in
 //     flight at once; only the chunk that straddles N goes element by element.
-//     15238 x 1337, odd rows: 71 -> 17 us with 16-byte accesses.
-//   * x stays in VGPRs: it is read from HBM exactly once (the reference
-//     re-reads it in its second pass, :101-117), and once for all of a token's
-//     experts where the MoE form gives tokens to groups of waves: per expert
-//     only its smooth scale is read (2916 x 7168, top 6 92 -> 58 us).  With few
-//     pairs or experts a token a group takes one pair (PAIRS; dispatch says
-//     where).
+//     15000 x 1337, odd rows: 71 -> 15 us.
+//   * The products stay in VGPRs: x is read from HBM exactly once (the
+//     reference re-reads it in its second pass, :101-117).
 //   * absmax: DPP quad/mirror steps inside each 16-lane row + 4 readlanes;
 //     rows spread over several waves merge through 16 bytes of LDS.
 //   * Output: each lane packs 8 int8 and stores 8 bytes (a wave writes 512
@@ -75,32 +74,122 @@ __device__ __forceinline__ RowSrc resolve_row(const QuantRows& p, uint32_t row)
 }
 
 constexpr int sq_rows_threads(int wpr) { return wpr * kWave > kSqThreads ? wpr * kWave : kSqThreads; }
+// Waves per SIMD that a lane's products leave room for; without it the compiler
+// takes 82 VGPRs for CPL = 8 and a wave fewer fits.
+constexpr int sq_rows_waves(int cpl) { return cpl == 4 ? 8 : cpl == 8 ? 6 : 1; }
 
-// CPL: 16-byte chunks per lane; WPR: waves per row.  MOE: a group of WPR waves
-// takes a token and writes its topk rows one after another, or (PAIRS) one
-// (token, slot) pair.
-template <int CPL, int WPR, bool MOE, bool PAIRS>
-__global__ void __launch_bounds__(sq_rows_threads(WPR)) sq_rows_kernel(QuantRows p)
+// CPL: 16-byte chunks per lane; WPR: waves per row.  A chunk's x and s are
+// loaded and multiplied together, and both tails are computed in their own
+// branch: x ahead of s, or the packing ahead of the branch, costs 12-34 VGPRs and
+// with them two waves a SIMD (8192 pairs of 4096, top 1: 22.4 us, 18.7 as it is).
+template <int CPL, int WPR, bool MOE>
+__global__ void __launch_bounds__(sq_rows_threads(WPR), sq_rows_waves(CPL)) sq_rows_kernel(QuantRows p)
 {
     constexpr int kWaves        = sq_rows_threads(WPR) / kWave;
     constexpr int kRowsPerBlock = kWaves / WPR;
     constexpr int kSpan         = CPL * 8 * kWave;
-    constexpr bool kTokens      = MOE && !PAIRS;
-    __shared__ float red[2][kWaves];
 
     const int      wave = threadIdx.x / kWave;
     const int      lane = threadIdx.x % kWave;
     const int      rib  = wave / WPR; // row in block
     const int      part = wave % WPR; // segment of the row
-    const uint32_t unit = blockIdx.x * kRowsPerBlock + rib; // token, pair or row
-    const uint32_t slots = kTokens ? p.topk : 1;
-    const uint32_t row0  = unit * slots;
-    const uint32_t n     = p.n;
-    const uint32_t base  = part * kSpan + lane * 8;
+    const RowSrc   src  = resolve_row<MOE>(p, blockIdx.x * kRowsPerBlock + rib);
+    const uint32_t n    = p.n;
+    const uint32_t base = part * kSpan + lane * 8;
 
-    v4i raw[CPL]; // zeros past N and for units past the last
+    float pv[CPL * 8];
+    float amax = 0.f;
+    if(src.valid) {
+#pragma unroll
+        for(int j = 0; j < CPL; ++j) {
+            const uint32_t c = base + j * (8 * kWave);
+            if(c + 8 <= n) {
+                uint32_t w[4];
+                float    sv[8];
+                __builtin_memcpy(w, src.x + c, 16);
+                __builtin_memcpy(sv, src.s + c, 16);
+                __builtin_memcpy(sv + 4, src.s + c + 4, 16);
+#pragma unroll
+                for(int e = 0; e < 4; ++e) {
+                    pv[j * 8 + 2 * e]     = mul_h16_f32<false>(w[e], sv[2 * e]);
+                    pv[j * 8 + 2 * e + 1] = mul_h16_f32<true>(w[e], sv[2 * e + 1]);
+                }
+            } else {
+#pragma unroll
+                for(int e = 0; e < 8; ++e)
+                    pv[j * 8 + e] = e < 7 && c + e < n
+                                        ? half_bits_to_float(src.x[c + e]) * src.s[c + e]
+                                        : 0.f;
+            }
+#pragma unroll
+            for(int e = 0; e < 8; ++e) amax = fmaxf(amax, fabsf(pv[j * 8 + e]));
+        }
+    }
+
+    amax = wave_max(amax);
+    if constexpr(WPR > 1) {
+        __shared__ float red[kWaves];
+        if(lane == 0) red[wave] = amax;
+        __syncthreads();
+#pragma unroll
+        for(int w = 0; w < WPR; ++w) amax = fmaxf(amax, red[rib * WPR + w]);
+    }
+    if(!src.valid) return;
+
+    const float qmax = p.qmax;
+    const float rs   = amax / qmax; // correctly rounded fp32 division
+    if(part == 0 && lane == 0) p.r[src.dst] = rs;
+    const float inv = (rs > 0.f) ? (1.f / rs) : 0.f;
+
+    int8_t* qrow = p.q + (size_t)src.dst * p.ldq;
+#pragma unroll
+    for(int j = 0; j < CPL; ++j) {
+        const uint32_t c = base + j * (8 * kWave);
+        const float*   v = pv + j * 8;
+        auto           pack = [&](uint32_t(&o)[2]) {
+            o[0] = cvt_pack4_i8(quant_f(v[0], inv, qmax), quant_f(v[1], inv, qmax),
+                                quant_f(v[2], inv, qmax), quant_f(v[3], inv, qmax));
+            o[1] = cvt_pack4_i8(quant_f(v[4], inv, qmax), quant_f(v[5], inv, qmax),
+                                quant_f(v[6], inv, qmax), quant_f(v[7], inv, qmax));
+        };
+        uint32_t packed[2];
+        if constexpr(CPL == 1) pack(packed); // short rows are mostly their tail
+        if(c + 8 <= n) {
+            if constexpr(CPL > 1) pack(packed);
+            __builtin_memcpy(qrow + c, packed, 8);
+        } else {
+#pragma unroll
+            for(int e = 0; e < 7; ++e)
+                if(c + e < n)
+                    qrow[c + e] = CPL == 1 ? (int8_t)(packed[e / 4] >> (8 * (e % 4)))
+                                           : (int8_t)quant_i8(v[e], inv, qmax);
+        }
+    }
+}
+
+// The MoE form with x read once for all of a token's experts: a group of WPR
+// waves holds the token's x in VGPRs and writes its topk rows one after another,
+// reading only each expert's smooth scale (2916 x 7168, top 6 92 -> 58 us).
+template <int CPL, int WPR>
+__global__ void __launch_bounds__(sq_rows_threads(WPR)) sq_tokens_kernel(QuantRows p)
+{
+    constexpr int kWaves          = sq_rows_threads(WPR) / kWave;
+    constexpr int kTokensPerBlock = kWaves / WPR;
+    constexpr int kSpan           = CPL * 8 * kWave;
+    __shared__ float red[2][kWaves];
+
+    const int      wave = threadIdx.x / kWave;
+    const int      lane = threadIdx.x % kWave;
+    const int      tib  = wave / WPR; // token in block
+    const int      part = wave % WPR; // segment of the row
+    const uint32_t tok  = blockIdx.x * kTokensPerBlock + tib;
+    const uint32_t row0 = tok * p.topk;
+    const uint32_t n    = p.n;
+    const uint32_t base = part * kSpan + lane * 8;
+
+    v4i raw[CPL]; // zeros past N and for tokens past the last
     if(row0 < p.rows) {
-        const uint16_t* x = p.x + (size_t)(MOE ? row0 / p.topk : row0) * p.ldx;
+        const uint16_t* x = p.x + (size_t)tok * p.ldx;
 #pragma unroll
         for(int j = 0; j < CPL; ++j) {
             const uint32_t c = base + j * (8 * kWave);
@@ -117,8 +206,8 @@ __global__ void __launch_bounds__(sq_rows_threads(WPR)) sq_rows_kernel(QuantRows
         }
     }
     const float qmax = p.qmax;
-    for(uint32_t slot = 0; slot < slots; ++slot) { // the same count in every wave
-        const RowSrc src = resolve_row<MOE>(p, row0 + slot);
+    for(uint32_t slot = 0; slot < p.topk; ++slot) { // the same count in every wave
+        const RowSrc src = resolve_row<true>(p, row0 + slot);
         float        pv[CPL * 8];
         float        amax = 0.f;
         if(src.valid) {
@@ -151,7 +240,7 @@ __global__ void __launch_bounds__(sq_rows_threads(WPR)) sq_rows_kernel(QuantRows
             if(lane == 0) r[wave] = amax;
             __syncthreads();
 #pragma unroll
-            for(int w = 0; w < WPR; ++w) amax = fmaxf(amax, r[rib * WPR + w]);
+            for(int w = 0; w < WPR; ++w) amax = fmaxf(amax, r[tib * WPR + w]);
         }
         if(!src.valid) continue;
         const float rs = amax / qmax; // correctly rounded fp32 division
@@ -430,23 +519,40 @@ hipError_t launch_stream(const QuantRows& p, hipStream_t stream)
     return hipSuccess;
 }
 
-template <int CPL, int WPR, bool MOE, bool PAIRS = false>
+template <int CPL, int WPR, bool MOE>
 hipError_t launch_rows(const QuantRows& p, hipStream_t stream)
 {
-    constexpr int  kThreads      = sq_rows_threads(WPR);
-    constexpr int  kRowsPerBlock = kThreads / kWave / WPR;
-    const uint32_t units         = MOE && !PAIRS ? p.rows / p.topk : p.rows;
-    hipLaunchKernelGGL((sq_rows_kernel<CPL, WPR, MOE, PAIRS>),
-                       dim3((units + kRowsPerBlock - 1) / kRowsPerBlock), dim3(kThreads), 0,
+    constexpr int kThreads      = sq_rows_threads(WPR);
+    constexpr int kRowsPerBlock = kThreads / kWave / WPR;
+    hipLaunchKernelGGL((sq_rows_kernel<CPL, WPR, MOE>),
+                       dim3((p.rows + kRowsPerBlock - 1) / kRowsPerBlock), dim3(kThreads), 0,
+                       stream, p);
+    return hipGetLastError();
+}
+
+template <int CPL, int WPR>
+hipError_t launch_tokens(const QuantRows& p, hipStream_t stream)
+{
+    constexpr int  kThreads        = sq_rows_threads(WPR);
+    constexpr int  kTokensPerBlock = kThreads / kWave / WPR;
+    const uint32_t tokens          = p.rows / p.topk;
+    hipLaunchKernelGGL((sq_tokens_kernel<CPL, WPR>),
+                       dim3((tokens + kTokensPerBlock - 1) / kTokensPerBlock), dim3(kThreads), 0,
                        stream, p);
     return hipGetLastError();
 }
 
 template <bool MOE>
-hipError_t dispatch(const QuantRows& p, hipStream_t stream)
+hipError_t launch_twopass(const QuantRows& p, hipStream_t stream)
+{
+    hipLaunchKernelGGL((sq_twopass_kernel<MOE>), dim3(p.rows), dim3(kSqThreads), 0, stream, p);
+    return hipGetLastError();
+}
+
+hipError_t launch_dense(const QuantRows& p, hipStream_t stream)
 {
     const uint32_t n = p.n;
-    if constexpr(!MOE) {
+    {
         // 16-byte x loads, 32-byte aligned s loads, 8-byte q stores
         const bool vec = (reinterpret_cast<uintptr_t>(p.x) % 16 == 0) && (p.ldx % 8 == 0)
                          && (reinterpret_cast<uintptr_t>(p.s) % 16 == 0)
@@ -488,48 +594,78 @@ hipError_t dispatch(const QuantRows& p, hipStream_t stream)
             if(n <= 32768) return launch_stream<4, 16, 1024>(p, stream);
         }
     }
-    if constexpr(MOE) {
-        // fewer pairs than two blocks a CU: a block for each (32 pairs of 4096:
-        // 7.3 -> 4.1 us)
-        if(p.rows <= 512 && n <= 4096)
-            return n <= 2048 ? launch_rows<1, 4, MOE, true>(p, stream)
-                             : launch_rows<2, 4, MOE, true>(p, stream);
-        // Pairs up to 3072 of them and for one or two experts a token, where
-        // reading x once saves less than the serial slots cost: 768 / 2400 /
-        // 6000 / 17496 pairs of 7168, top 6, 8.2 / 16.0 / 32 / 81 us by pairs,
-        // 17.1 / 17.7 / 23 / 58 by tokens; 600 / 2000 / 8192 pairs of 4096,
-        // top 2, 6.0 / 8.3 / 20.5 against 7.4 / 9.2 / 21.4.
-        if(n > 2048 && n <= 32768 && (p.rows <= 3072 || p.topk <= 2)) {
-            if(n <= 4096) return launch_rows<4, 2, MOE, true>(p, stream);
-            if(n <= 8192) return launch_rows<4, 4, MOE, true>(p, stream);
-            if(n <= 16384) return launch_rows<2, 16, MOE, true>(p, stream);
-            return launch_rows<4, 16, MOE, true>(p, stream);
-        }
+    if(n <= 512) return launch_rows<1, 1, false>(p, stream);
+    if(n <= 1024) return launch_rows<2, 1, false>(p, stream);
+    if(n <= 2048) return launch_rows<4, 1, false>(p, stream);
+    if(n <= 4096) return launch_rows<4, 2, false>(p, stream);
+    if(n <= 8192) return launch_rows<4, 4, false>(p, stream);
+    // Rows of more than 8192: 16 waves, but 4 for more rows than fill the chip
+    // (1 / 512 / 8000 rows of 8199: 3.4 / 7.0 / 80 us by 16 waves, 5.5 / 8.2 /
+    // 68 by 4; 1 / 8000 of 28671 5.0 / 192 against 8.0 / 230).
+    if(n <= 16384 && p.rows > 1024) return launch_rows<8, 4, false>(p, stream);
+    if(n <= 16384) return launch_rows<2, 16, false>(p, stream);
+    if(n <= 32768) return launch_rows<4, 16, false>(p, stream);
+    return launch_twopass<false>(p, stream);
+}
+
+hipError_t launch_moe(const QuantRows& p, hipStream_t stream)
+{
+    const QuantPlan d  = moe_quant_plan(p.rows, p.n, p.topk);
+    auto            is = [&](uint32_t chunks, uint32_t waves) { return d.chunks == chunks && d.waves == waves; };
+    if(d.tokens) {
+        if(is(1, 1)) return launch_tokens<1, 1>(p, stream);
+        if(is(2, 1)) return launch_tokens<2, 1>(p, stream);
+        if(is(4, 4)) return launch_tokens<4, 4>(p, stream);
+        if(is(2, 16)) return launch_tokens<2, 16>(p, stream);
+        return launch_tokens<4, 16>(p, stream);
     }
-    if(n <= 512) return launch_rows<1, 1, MOE>(p, stream);
-    if(n <= 1024) return launch_rows<2, 1, MOE>(p, stream);
-    if(n <= 2048) return launch_rows<4, 1, MOE>(p, stream);
-    if(n <= 4096) return launch_rows<4, 2, MOE>(p, stream);
-    if(n <= 8192) return launch_rows<4, 4, MOE>(p, stream);
-    // Rows of more than 8192: 16 waves, but 4 for more dense rows than fill the
-    // chip (1 / 512 / 8000 rows of 8199: 3.4 / 7.0 / 80 us by 16 waves, 5.5 / 8.2 /
-    // 68 by 4; 1 / 8000 of 28671 5.0 / 192 against 8.0 / 230; 1024 tokens of
-    // 14336, top 4, 28.6 against 35.3).
-    if constexpr(!MOE) {
-        if(n <= 16384 && p.rows > 1024) return launch_rows<8, 4, MOE>(p, stream);
-    }
-    if(n <= 16384) return launch_rows<2, 16, MOE>(p, stream);
-    if(n <= 32768) return launch_rows<4, 16, MOE>(p, stream);
-    hipLaunchKernelGGL((sq_twopass_kernel<MOE>), dim3(p.rows), dim3(kSqThreads), 0, stream, p);
-    return hipGetLastError();
+    if(is(1, 1)) return launch_rows<1, 1, true>(p, stream);
+    if(is(1, 2)) return launch_rows<1, 2, true>(p, stream);
+    if(is(2, 1)) return launch_rows<2, 1, true>(p, stream);
+    if(is(1, 4)) return launch_rows<1, 4, true>(p, stream);
+    if(is(4, 1)) return launch_rows<4, 1, true>(p, stream);
+    if(is(2, 4)) return launch_rows<2, 4, true>(p, stream);
+    if(is(4, 2)) return launch_rows<4, 2, true>(p, stream);
+    if(is(8, 1)) return launch_rows<8, 1, true>(p, stream);
+    if(is(4, 4)) return launch_rows<4, 4, true>(p, stream);
+    if(is(2, 16)) return launch_rows<2, 16, true>(p, stream);
+    if(is(4, 16)) return launch_rows<4, 16, true>(p, stream);
+    return launch_twopass<true>(p, stream);
 }
 
 } // namespace
 
+// By pairs each row is on its own, in as few waves as keep the chip full; by
+// tokens x is read once but a token's slots run one after another, which pays
+// only where many pairs share few tokens and x is most of the traffic.  Measured
+// over 40-8192 tokens, top 1-8, hidden 512-28672 (us by pairs / by tokens):
+//   512: 32000 pairs 11.5 / 12.9, 49152 17.0 / 16.4
+//   1024 (881): 2400 pairs 4.7 / 10.7, 12000 9.9 / 13.7, 16000 12.3 / 12.1
+//   2048: 600 pairs, top 6 3.7 / 7.1, 12000 12.3 / 16.1, 65536 47.1 / 47.6
+//   4096: 4200 pairs, top 6 10.7 / 12.3, 16000 25.6 / 29.1, 49152 68.3 / 71.0
+//   7168: 2400 pairs, top 8 13.1 / 18.8, 4200 19.6 / 19.0, 24000 87 / 66;
+//         top 2 8000 28.5 / 30.0
+//   14336: 800 pairs, top 8 13.0 / 18.1, 1400, top 2 15.1 / 13.3, 9000 87 / 61
+//   20000: 2800 pairs, top 4 38 / 39, 6000 69 / 74; 28672: 47 / 42, 95 / 81; top 2
+//         3000 44 / 50
+QuantPlan moe_quant_plan(uint32_t pairs, uint32_t n, uint32_t topk)
+{
+    if(n <= 512) return {1, 1, pairs > 36000};
+    if(n <= 1024 && pairs <= 1536) return {1, 2, false};
+    if(n <= 1024) return {2, 1, pairs > 12288};
+    if(n <= 2048) return pairs <= 1536 ? QuantPlan{1, 4, false} : QuantPlan{4, 1, false};
+    if(n <= 4096 && pairs <= 1024) return {2, 4, false};
+    if(n <= 4096) return pairs <= 10240 ? QuantPlan{4, 2, false} : QuantPlan{8, 1, false};
+    if(n <= 8192) return {4, 4, pairs > 3584 && topk > 2};
+    if(n <= 16384) return {2, 16, pairs > 1280};
+    if(n <= 32768) return {4, 16, pairs > 2048 && topk > 2};
+    return {0, 0, false};
+}
+
 hipError_t launch_smoothquant(const QuantRows& p, hipStream_t stream)
 {
     if(p.rows == 0) return hipSuccess;
-    return p.topk_ids ? dispatch<true>(p, stream) : dispatch<false>(p, stream);
+    return p.topk_ids ? launch_moe(p, stream) : launch_dense(p, stream);
 }
 
 } // namespace w8a8

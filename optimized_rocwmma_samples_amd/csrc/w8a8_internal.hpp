@@ -29,6 +29,13 @@ struct QuantRows {
 };
 
 hipError_t launch_smoothquant(const QuantRows& p, hipStream_t stream);
+// How the MoE form runs: 16-byte chunks per lane, waves per row (0: two passes),
+// and whether a group of waves takes a token with all its slots or one pair.
+struct QuantPlan {
+    uint32_t chunks, waves;
+    bool     tokens;
+};
+QuantPlan moe_quant_plan(uint32_t pairs, uint32_t n, uint32_t topk);
 
 // RMSNorm (+ residual add) fused with the quantizer (rmsnorm_sq.hip).  x,
 // residual and x_out share the row stride ldx; residual, x_out, y, s, q and r

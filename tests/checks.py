@@ -41,3 +41,12 @@ def ulp_diff(a, b):
     a = np.ascontiguousarray(a, np.float32).view(np.int32).astype(np.int64)
     b = np.ascontiguousarray(b, np.float32).view(np.int32).astype(np.int64)
     return np.abs(a - b)
+
+
+def plan(w8a8, kind, *sizes):
+    """w8a8_debug_plan: the kernel that a call of these sizes takes."""
+    import ctypes
+    given = (ctypes.c_uint32 * 4)(*sizes)
+    got = (ctypes.c_uint32 * 3)()
+    assert w8a8.library().w8a8_debug_plan(kind, given, got) == 0
+    return tuple(got)
