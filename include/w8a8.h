@@ -224,12 +224,19 @@ int w8a8_debug_streamk_wait(uint32_t spin_limit, uint32_t phantom_pieces);
  * Test hook: the kernel a call of the given sizes takes, so that tests can
  * say which one they run.  Host arithmetic only (without a GPU: of 256 CUs).
  * sizes and plan hold 4 and 3 values:
- *   W8A8_PLAN_MOE_QUANT  tokens * topk, hidden, topk
+ *   W8A8_PLAN_MOE_QUANT    tokens * topk, hidden, topk
  *                        -> 16-byte chunks per lane, waves per row (0: two
  *                           passes over a row), 1 where a group of waves takes
  *                           a token, 0 where it takes a (token, slot) pair
+ *   W8A8_PLAN_GEMM         m, n, k, workspace bytes (16-byte aligned operands,
+ *                          lda, ldb, k multiples of 16)
+ *   W8A8_PLAN_GEMM_PACKED  the same, m > 64
+ *                        -> tile rows, tile columns, K pieces (0, 32, 1: the
+ *                           decode kernel)
  */
 #define W8A8_PLAN_MOE_QUANT 0
+#define W8A8_PLAN_GEMM 1
+#define W8A8_PLAN_GEMM_PACKED 2
 int w8a8_debug_plan(int kind, const uint32_t* sizes, uint32_t* plan);
 
 /*

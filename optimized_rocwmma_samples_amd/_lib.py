@@ -25,6 +25,8 @@ OUT_F16 = 1
 STREAMK_WAIT_EXPIRED = 1
 
 PLAN_MOE_QUANT = 0  # w8a8_debug_plan kinds
+PLAN_GEMM = 1
+PLAN_GEMM_PACKED = 2
 
 GROUPED_INLINE_GROUPS = 48  # W8A8_GROUPED_INLINE_GROUPS
 

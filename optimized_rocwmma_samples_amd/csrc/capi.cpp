@@ -419,6 +419,12 @@ int w8a8_debug_plan(int kind, const uint32_t* sizes, uint32_t* plan)
         const w8a8::QuantPlan d = w8a8::moe_quant_plan(sizes[0], sizes[1], sizes[2]);
         return set(d.chunks, d.waves, d.tokens);
     }
+    case W8A8_PLAN_GEMM:
+    case W8A8_PLAN_GEMM_PACKED:
+        if(sizes[0] == 0 || sizes[1] == 0 || sizes[2] == 0)
+            return fail(W8A8_ERROR_INVALID_VALUE, "%s: m, n, k must be > 0", fn);
+        w8a8::gemm_plan(sizes, kind == W8A8_PLAN_GEMM_PACKED, plan);
+        return W8A8_SUCCESS;
     default: return fail(W8A8_ERROR_INVALID_VALUE, "%s: unknown kind %d", fn, kind);
     }
 }

@@ -308,7 +308,10 @@ double decode_cost(uint32_t m, uint32_t n, uint32_t k)
 
 // The plan of least estimated time among those whose partials fit ws_bytes.
 // 256 x 256 tiles where the persistent kernel may run them (two whole rounds,
-// K <= 4096) and from four rounds on; below that, what the launch lacks
+// K <= 4096) and from four rounds on, unless 128-row tiles would save half a
+// tile row: 151936 columns of K = 4096 1 / 64 / 100 / 300 rows 159 / 172 /
+// 179 / 267 us in 256 x 256 tiles, 113 / 129 / 157 / 252 in the searched ones (64 x
+// 64, 64 x 128, 128 x 128, 128 x 256).  Otherwise what the launch lacks
 // decides: blocks, k-tiles per block or both.  m <= 64: row-major weights also have
 // the decode kernel.  Against the fixed rules this replaced (largest tile
 // that fills 3/4 of the CUs, K split when half of them idle): 128 x 4096 x
@@ -318,7 +321,8 @@ double decode_cost(uint32_t m, uint32_t n, uint32_t k)
 TilePlan search_plan(uint32_t m, uint32_t n, uint32_t k, size_t ws_bytes, bool decode, bool packed)
 {
     TilePlan best{TileCfg::kMain, 1, 0};
-    if((uint64_t)ceil_div(m, 256) * ceil_div(n, 256) >= (k <= 4096 ? 2ull : 4ull) * device_cus())
+    if((uint64_t)ceil_div(m, 256) * ceil_div(n, 256) >= (k <= 4096 ? 2ull : 4ull) * device_cus()
+       && ceil_div(m, 128) % 2 == 0)
         return best;
     double         cost = decode ? decode_cost(m, n, k) : 1e300;
     const uint32_t most = std::min(gemm::kMaxParts, ceil_div(k, 128) / kMinKtPlan);
@@ -404,6 +408,18 @@ GroupedTile grouped_gemm_tile(const w8a8_group_desc* groups, uint32_t ngroups)
         }
     }
     return best;
+}
+
+// The plan of a GEMM over row-major (with at least 16-byte aligned operands) or
+// packed weights, for tests: tile rows and columns, K pieces; the decode kernel
+// as 0 x 32.
+void gemm_plan(const uint32_t* sizes, bool packed, uint32_t* plan)
+{
+    const TilePlan p = plan_tiles(sizes[0], sizes[1], sizes[2], sizes[3],
+                                  !packed && sizes[0] <= kDecodeMaxM, packed);
+    plan[0] = 0, plan[1] = 32, plan[2] = p.parts;
+    for(const CfgCost& c : kCosts)
+        if(c.cfg == p.cfg) plan[0] = c.bm, plan[1] = c.bn;
 }
 
 namespace {

@@ -75,6 +75,9 @@ bool       gemm_fast_path_ok(const GemmArgs& g);
 // ws_bytes is estimated to be faster; gemm_nk_workspace_bytes allows them all.
 hipError_t launch_gemm_nk(const GemmArgs& g, void* ws, size_t ws_bytes, hipStream_t stream);
 size_t     gemm_nk_workspace_bytes(const GemmArgs& g);
+// sizes: m, n, k, workspace bytes -> plan: tile rows, tile columns, K pieces
+// (0 x 32: the decode kernel).  Packed weights: m > 64.
+void       gemm_plan(const uint32_t* sizes, bool packed, uint32_t* plan);
 // Explicit stream-K over every tile (w8a8_gemm_streamk): `blocks` blocks (0:
 // one per CU, never more than the problem's k-tiles); ws: 16-byte aligned,
 // streamk_workspace_bytes.  Needs gemm_fast_path_ok and A, B under 2 GiB

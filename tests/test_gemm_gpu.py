@@ -9,7 +9,8 @@ import numpy as np
 import pytest
 
 import oracle_lib as O
-from checks import assert_f16_bitexact, assert_i32_equal, dev, host
+from checks import assert_f16_bitexact, assert_i32_equal, dev, host, plan
+from optimized_rocwmma_samples_amd import _lib as L
 from optimized_rocwmma_samples_amd import datagen as G
 
 pytestmark = pytest.mark.gpu
@@ -251,6 +252,22 @@ def test_short_tiles_exact(w8a8, gpu, m, n, k):
     assert_i32_equal(host(w8a8.gemm_packed(ad, pw, out_dtype=torch.int32)), acc)
     assert_f16_bitexact(host(w8a8.gemm(ad, bd, sad, sbd)), want)
     assert_f16_bitexact(host(w8a8.gemm_packed(ad, pw, sad, sbd)), want)
+
+
+# Few rows of many columns (more than two rounds of 256 x 256 tiles): short tiles.
+@pytest.mark.parametrize("m,n,k,rows", [(3, 131100, 160, 32), (100, 131100, 144, 64),
+                                        (300, 70001, 160, 64)])
+def test_few_rows_of_many_columns_exact(w8a8, gpu, m, n, k, rows):
+    import torch
+    a, b, sa, sb = inputs(m, n, k, m + n + k)
+    ad, bd = dev(a, gpu), dev(b, gpu)
+    acc = O.gemm_i32(a, b)
+    assert plan(w8a8, L.PLAN_GEMM, m, n, k, w8a8.gemm_workspace_size(m, n, k))[0] == rows
+    assert_i32_equal(host(w8a8.gemm(ad, bd, out_dtype=torch.int32)), acc)
+    if m > 64:
+        assert plan(w8a8, L.PLAN_GEMM_PACKED, m, n, k, 0)[0] == rows
+        c = w8a8.gemm_packed(ad, w8a8.pack_weights(bd), dev(sa, gpu), dev(sb, gpu))
+        assert_f16_bitexact(host(c), O.dequant_f16(acc, sa, sb))
 
 
 def test_k_split_strided(w8a8, gpu):
