@@ -270,13 +270,21 @@ constexpr CfgCost kCosts[] = {
 constexpr uint32_t kMinKtPlan    = 6;        // k-tiles of a K piece, at least
 constexpr size_t   kMaxPlanBytes = 64 << 20; // partials of a plan, at most
 // A split call launches twice, and the host needs about 3.5 µs a launch and
-// 4 µs around it: a GPU time below that is not seen (25 x 784 x 2944, split
-// 15.0 -> 19.8 µs a layer although its kernels take 2 µs less).
+// 4 µs around it: an eager caller does not see a GPU time below that (25 x 784 x
+// 2944, split 15.0 -> 19.8 µs a layer although its kernels take 2 µs less).
 constexpr double kSplitHostUs = 11.0;
 
 uint32_t ceil_div(uint32_t a, uint32_t b) { return (a + b - 1) / b; }
 
-double plan_cost(const CfgCost& c, uint32_t m, uint32_t n, uint32_t k, uint32_t parts, bool packed)
+// seen: what the caller waits for, at least the host's time of a split call; gpu
+// decides between plans that are alike in it (a replayed graph or a caller with
+// other work in flight sees the GPU's time).
+struct PlanTime {
+    double seen, gpu;
+    bool   operator<(const PlanTime& o) const { return seen != o.seen ? seen < o.seen : gpu < o.gpu; }
+};
+
+PlanTime plan_cost(const CfgCost& c, uint32_t m, uint32_t n, uint32_t k, uint32_t parts, bool packed)
 {
     const uint32_t cus    = device_cus();
     const uint32_t tm     = ceil_div(m, c.bm);
@@ -292,8 +300,9 @@ double plan_cost(const CfgCost& c, uint32_t m, uint32_t n, uint32_t k, uint32_t 
     }
     t += steps * (per_cu / c.resident * c.step[c.resident - 1]
                   + (per_cu % c.resident ? c.step[per_cu % c.resident - 1] : 0.0));
-    if(parts == 1) return t;
-    return std::max(t + c.split + 4e-6 * blocks * c.bm * c.bn * c.split_mb, kSplitHostUs);
+    if(parts == 1) return {t, t};
+    t += c.split + 4e-6 * blocks * c.bm * c.bn * c.split_mb;
+    return {std::max(t, kSplitHostUs), t};
 }
 
 // The row-major decode kernel (32 weight rows a block, its waves splitting K
@@ -324,7 +333,8 @@ TilePlan search_plan(uint32_t m, uint32_t n, uint32_t k, size_t ws_bytes, bool d
     if((uint64_t)ceil_div(m, 256) * ceil_div(n, 256) >= (k <= 4096 ? 2ull : 4ull) * device_cus()
        && ceil_div(m, 128) % 2 == 0)
         return best;
-    double         cost = decode ? decode_cost(m, n, k) : 1e300;
+    const double   dec  = decode ? decode_cost(m, n, k) : 1e300;
+    PlanTime       cost{dec, dec};
     const uint32_t most = std::min(gemm::kMaxParts, ceil_div(k, 128) / kMinKtPlan);
     if(decode) best.cfg = TileCfg::kDecode;
     for(const CfgCost& c : kCosts) {
@@ -336,7 +346,7 @@ TilePlan search_plan(uint32_t m, uint32_t n, uint32_t k, size_t ws_bytes, bool d
             if(bytes > std::min(ws_bytes, kMaxPlanBytes)
                || (p > 1 && tiles * p > (uint64_t)device_cus() * c.resident))
                 break;
-            const double t = plan_cost(c, m, n, k, p, packed);
+            const PlanTime t = plan_cost(c, m, n, k, p, packed);
             if(t < cost) {
                 cost = t;
                 best = TilePlan{c.cfg, p, (size_t)bytes};
