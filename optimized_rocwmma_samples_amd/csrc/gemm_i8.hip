@@ -293,7 +293,7 @@ PlanTime plan_cost(const CfgCost& c, uint32_t m, uint32_t n, uint32_t k, uint32_
     uint64_t       per_cu = (blocks + cus - 1) / cus;
     double         t      = c.fixed + 2e-6 * m * n * c.out_mb + 1e-6 * n * (double)k * c.w_mb;
     // launch_main runs a last round of at most half the CUs as smaller tiles
-    if(c.cfg == TileCfg::kMain && per_cu > 1 && blocks % cus * 2 <= cus
+    if(c.cfg == TileCfg::kMain && per_cu > 1 && blocks % cus != 0 && blocks % cus * 2 <= cus
        && blocks / cus * cus % tm == 0) {
         t += steps * kCosts[1].step[0];
         --per_cu;
