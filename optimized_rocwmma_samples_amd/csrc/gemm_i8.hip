@@ -15,6 +15,7 @@
 #include <atomic>
 #include <map>
 #include <mutex>
+#include <numeric>
 #include <tuple>
 
 namespace w8a8 {
@@ -253,19 +254,25 @@ struct TilePlan {
 //   + out_mb x output MB + w_mb x weight MB
 //   + (pieces > 1) (split + split_mb x partial MB)
 // with step x cross where row-major operands' rows cross 128-byte lines (K no
-// multiple of 128: every 128-byte row piece of a k-tile is then two requests).
+// multiple of 128: a 128-byte row piece off a line is two requests).  The
+// shortest tiles make the most requests for their sums, and with the chip full
+// of them the requests are what their k-steps wait for: there the factor rises
+// to 1 + full x share of the rows off a line, from `from` blocks a CU to `to`
+// (181 x 19016 x 9488: 64 x 64 tiles, 3.5 blocks a CU, 122 us against 99 in 128 x
+// 256 ones; one factor for every load had said 81 against 88).  Fitted on 193
+// sizes with such K, every configuration and 1-8 pieces measured.
 struct CfgCost {
     TileCfg  cfg;
     uint32_t bm, bn, resident; // resident: blocks a CU holds (LDS)
-    double   fixed, step[3], split, split_mb, out_mb, w_mb, cross;
+    double   fixed, step[3], split, split_mb, out_mb, w_mb, cross, full, from, to;
 };
 constexpr CfgCost kCosts[] = {
-    {TileCfg::kMain, 256, 256, 1, 6.2, {1.19}, 6.5, 0.45, 0.27, 0.044, 1.06},
-    {TileCfg::kMidM, 128, 256, 1, 4.9, {0.71}, 4.7, 0.38, 0.34, 0.043, 1.25},
-    {TileCfg::kSmall, 128, 128, 1, 3.6, {0.42}, 3.8, 0.40, 0.40, 0.023, 1.25},
-    {TileCfg::kNarrow, 64, 128, 2, 3.2, {0.30, 0.63}, 3.7, 0.32, 0.23, 0.061, 1.40},
-    {TileCfg::kTiny, 64, 64, 2, 3.3, {0.24, 0.42}, 3.3, 0.47, 0.37, 0.030, 1.10},
-    {TileCfg::kRow, 32, 64, 3, 3.4, {0.23, 0.36, 0.59}, 3.0, 0.41, 0.0, 0.048, 1.02},
+    {TileCfg::kMain, 256, 256, 1, 6.2, {1.19}, 6.5, 0.45, 0.27, 0.044, 1.06, 0.0, 0.0, 1.0},
+    {TileCfg::kMidM, 128, 256, 1, 4.9, {0.71}, 4.7, 0.38, 0.34, 0.043, 1.25, 0.0, 0.0, 1.0},
+    {TileCfg::kSmall, 128, 128, 1, 3.6, {0.42}, 3.8, 0.40, 0.40, 0.023, 1.25, 0.0, 0.0, 1.0},
+    {TileCfg::kNarrow, 64, 128, 2, 3.2, {0.30, 0.63}, 3.7, 0.32, 0.23, 0.061, 1.40, 0.0, 0.0, 1.0},
+    {TileCfg::kTiny, 64, 64, 2, 3.3, {0.24, 0.42}, 3.3, 0.47, 0.37, 0.030, 1.10, 0.8, 0.8, 2.0},
+    {TileCfg::kRow, 32, 64, 3, 3.4, {0.23, 0.36, 0.59}, 3.0, 0.41, 0.0, 0.048, 1.02, 0.6, 0.9, 1.5},
 };
 constexpr uint32_t kMinKtPlan    = 6;        // k-tiles of a K piece, at least
 constexpr size_t   kMaxPlanBytes = 64 << 20; // partials of a plan, at most
@@ -289,7 +296,13 @@ PlanTime plan_cost(const CfgCost& c, uint32_t m, uint32_t n, uint32_t k, uint32_
     const uint32_t cus    = device_cus();
     const uint32_t tm     = ceil_div(m, c.bm);
     const uint64_t blocks = (uint64_t)tm * ceil_div(n, c.bn) * parts;
-    const double   steps  = ceil_div(ceil_div(k, 128), parts) * (packed || k % 128 == 0 ? 1.0 : c.cross);
+    double         factor = 1.0;
+    if(!packed && k % 128 != 0) {
+        const double ramp = std::clamp(((double)blocks / cus - c.from) / (c.to - c.from), 0.0, 1.0);
+        const double off  = 1.0 - std::gcd(k, 128u) / 128.0; // rows off a line
+        factor            = std::max(c.cross, 1.0 + c.full * off * ramp);
+    }
+    const double   steps  = ceil_div(ceil_div(k, 128), parts) * factor;
     uint64_t       per_cu = (blocks + cus - 1) / cus;
     double         t      = c.fixed + 2e-6 * m * n * c.out_mb + 1e-6 * n * (double)k * c.w_mb;
     // launch_main runs a last round of at most half the CUs as smaller tiles

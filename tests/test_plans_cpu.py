@@ -66,3 +66,14 @@ def test_few_rows_of_many_columns_take_short_tiles(w8a8, kind, m, n, k, rows):
 def test_plans_alike_to_the_host_are_told_apart_by_gpu_time(w8a8, m, n, k, rows):
     got = plan(w8a8, L.PLAN_GEMM, m, n, k, WS)
     assert got[0] == rows and got[1] == 64 and got[2] > 1
+
+
+# K no multiple of 128 and the chip full of short tiles, whose k-steps then wait for
+# twice the requests (181 x 19016 x 9488 in 64 x 64 tiles 122 us, others 99).
+@pytest.mark.parametrize("m,n,k,slower", [
+    (181, 19016, 9488, (64, 64, 1)), (43, 14272, 28576, (64, 64, 2)),
+    (41, 10880, 22384, (64, 64, 3)), (55, 26616, 3616, (64, 64, 1)),
+    (34, 7928, 18624, (64, 64, 4)), (48, 8920, 9888, (64, 64, 3)),
+    (31, 21128, 6608, (32, 64, 1))])
+def test_short_tiles_of_rows_off_a_line_cost_a_full_chip_more(w8a8, m, n, k, slower):
+    assert plan(w8a8, L.PLAN_GEMM, m, n, k, WS) != slower
