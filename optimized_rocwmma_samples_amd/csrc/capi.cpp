@@ -425,6 +425,11 @@ int w8a8_debug_plan(int kind, const uint32_t* sizes, uint32_t* plan)
             return fail(W8A8_ERROR_INVALID_VALUE, "%s: m, n, k must be > 0", fn);
         w8a8::gemm_plan(sizes, kind == W8A8_PLAN_GEMM_PACKED, plan);
         return W8A8_SUCCESS;
+    case W8A8_PLAN_MOE_GEMM:
+        if(sizes[0] == 0 || sizes[1] == 0)
+            return fail(W8A8_ERROR_INVALID_VALUE, "%s: experts and rows must be > 0", fn);
+        w8a8::moe_gemm_plan(sizes, plan);
+        return W8A8_SUCCESS;
     default: return fail(W8A8_ERROR_INVALID_VALUE, "%s: unknown kind %d", fn, kind);
     }
 }

@@ -800,6 +800,23 @@ MoeTile moe_tile(uint32_t rows, uint32_t experts, uint32_t n, bool silu = false)
     return u128 * 0.8 > u256 ? MoeTile::kMid : MoeTile::kMain;
 }
 
+// Whether a launch of 64 x 128 or 128 x 128 tiles is cut along K (TailSplit): where
+// the experts that can have rows make tiles for at most half of the CUs and a
+// tile has two pieces' k-tiles.  How many have rows is the router's: at most the
+// pairs, which at the default unit are the rows past 32 an expert.  One token of
+// the 8-expert Mixtral layer (2 experts, 64 tiles of 112 k-tiles) 52.9 -> 30.6 us,
+// two 56 -> 42; one expert of 1-48 rows 52 -> 23, of 100 rows (128 x 128) 65 -> 28.
+// Launches that fill the CUs go without the second launch (16 tokens 79.0 us, 81.2
+// with it).
+bool moe_short_split(uint32_t rows, uint32_t experts, uint32_t n, uint32_t k)
+{
+    const uint64_t pad    = 32ull * experts;
+    const uint64_t pairs  = rows > pad ? rows - pad : rows;
+    const uint64_t active = std::min<uint64_t>(experts, pairs);
+    return active * ((n + 127) / 128) * 2 <= device_cus()
+           && (k + 127) / 128 >= 2 * gemm::kMinKtPerPart;
+}
+
 } // namespace
 
 static_assert(sizeof(gemm::KArgs) == sizeof(w8a8_group_desc)
@@ -945,6 +962,7 @@ hipError_t launch_grouped_gemm(const w8a8_group_desc* groups, const void* groups
     }
 }
 
+// (the shorter tiles' partials are smaller)
 size_t moe_gemm_workspace_bytes()
 {
     return std::max(gemm::moe_workspace_bytes<GemmGrouped>(device_cus()),
@@ -974,16 +992,26 @@ hipError_t launch_moe_gemm(const MoeGemmArgs& a, hipStream_t stream)
     const bool split = a.ws != nullptr && a.ws_bytes >= moe_gemm_workspace_bytes();
     q.ws           = split ? static_cast<int32_t*>(a.ws) : nullptr;
     q.cus          = split ? device_cus() : 0;
-    switch(moe_tile(a.rows, a.experts, a.n)) {
-    case MoeTile::kFew:
+    const MoeTile tile = moe_tile(a.rows, a.experts, a.n);
+    if((tile == MoeTile::kFew || tile == MoeTile::kSmall)
+       && !moe_short_split(a.rows, a.experts, a.n, a.k))
         q.ws = nullptr, q.cus = 0;
-        return gemm::launch_moe<GemmMoeFew>(q, a.out_type, stream);
-    case MoeTile::kSmall:
-        q.ws = nullptr, q.cus = 0;
-        return gemm::launch_moe<GemmGroupedSmall>(q, a.out_type, stream);
+    switch(tile) {
+    case MoeTile::kFew: return gemm::launch_moe<GemmMoeFew>(q, a.out_type, stream);
+    case MoeTile::kSmall: return gemm::launch_moe<GemmGroupedSmall>(q, a.out_type, stream);
     case MoeTile::kMid: return gemm::launch_moe<GemmGroupedMid>(q, a.out_type, stream);
     default: return gemm::launch_moe<GemmGrouped, GemmGroupedWide>(q, a.out_type, stream);
     }
+}
+
+void moe_gemm_plan(const uint32_t* sizes, uint32_t* plan)
+{
+    const uint32_t experts = sizes[0], rows = sizes[1], n = sizes[2], k = sizes[3];
+    const MoeTile  tile    = moe_tile(rows, experts, n);
+    const bool     tall    = tile == MoeTile::kMid || tile == MoeTile::kMain;
+    plan[0]                = tile == MoeTile::kMain ? 256 : tile == MoeTile::kFew ? 64 : 128;
+    plan[1]                = tall ? 256 : 128;
+    plan[2]                = tall || moe_short_split(rows, experts, n, k);
 }
 
 // The SiLU epilogue's tiles: wave tiles 128 columns wide (64 outputs, one

@@ -77,3 +77,23 @@ def test_plans_alike_to_the_host_are_told_apart_by_gpu_time(w8a8, m, n, k, rows)
     (31, 21128, 6608, (32, 64, 1))])
 def test_short_tiles_of_rows_off_a_line_cost_a_full_chip_more(w8a8, m, n, k, slower):
     assert plan(w8a8, L.PLAN_GEMM, m, n, k, WS) != slower
+
+
+def capacity(tokens, topk, experts, unit=32):
+    return tokens * topk + experts * unit  # w8a8_moe_sort_capacity
+
+
+# Few experts with rows: 64-row tiles had run whole, 112 k-tiles one after another on a
+# quarter of the CUs (one token, K = 14336: 53 us; cut along K 31).
+@pytest.mark.parametrize("tokens,topk,experts,n,k,tile", [
+    (1, 2, 8, 4096, 14336, (64, 128, 1)), (2, 2, 8, 4096, 14336, (64, 128, 1)),
+    (1, 2, 16, 4096, 6400, (64, 128, 1)), (1, 1, 1, 4096, 14336, (64, 128, 1)),
+    (48, 1, 1, 4096, 14336, (64, 128, 1)), (48, 2, 2, 4096, 14336, (64, 128, 1)),
+    (100, 1, 1, 4096, 14336, (128, 128, 1)), (100, 2, 2, 4096, 14336, (128, 128, 1)),
+    # the CUs full, or nothing to cut: no second launch
+    (16, 2, 8, 4096, 14336, (64, 128, 0)), (4, 2, 8, 4096, 14336, (64, 128, 0)),
+    (400, 2, 8, 4096, 14336, (128, 128, 0)), (1, 6, 64, 7168, 2048, (64, 128, 0)),
+    (1, 2, 8, 4096, 4000, (64, 128, 1)), (1, 2, 8, 4096, 3968, (64, 128, 0))])
+def test_expert_gemm_of_few_tiles_is_cut_along_k(w8a8, tokens, topk, experts, n, k, tile):
+    rows = capacity(tokens, topk, experts)
+    assert plan(w8a8, L.PLAN_MOE_GEMM, experts, rows, n, k) == tile
