@@ -330,8 +330,8 @@ double decode_cost(uint32_t m, uint32_t n, uint32_t k)
 
 // The plan of least estimated time among those whose partials fit ws_bytes.
 // 256 x 256 tiles where the persistent kernel may run them (two whole rounds,
-// K <= 4096) and from four rounds on, unless 128-row tiles would save half a
-// tile row: 151936 columns of K = 4096 1 / 64 / 100 / 300 rows 159 / 172 /
+// K <= 4096) and from four rounds on, unless a quarter of their rows or more would
+// be padding: 151936 columns of K = 4096 1 / 64 / 100 / 300 rows 159 / 172 /
 // 179 / 267 us in 256 x 256 tiles, 113 / 129 / 157 / 252 in the searched ones (64 x
 // 64, 64 x 128, 128 x 128, 128 x 256).  Otherwise what the launch lacks
 // decides: blocks, k-tiles per block or both.  m <= 64: row-major weights also have
@@ -344,7 +344,7 @@ TilePlan search_plan(uint32_t m, uint32_t n, uint32_t k, size_t ws_bytes, bool d
 {
     TilePlan best{TileCfg::kMain, 1, 0};
     if((uint64_t)ceil_div(m, 256) * ceil_div(n, 256) >= (k <= 4096 ? 2ull : 4ull) * device_cus()
-       && ceil_div(m, 128) % 2 == 0)
+       && m * 4ull > ceil_div(m, 256) * 768ull)
         return best;
     const double   dec  = decode ? decode_cost(m, n, k) : 1e300;
     PlanTime       cost{dec, dec};

@@ -45,13 +45,14 @@ WS = 64 << 20  # workspace of every plan
 
 # A vocabulary-wide projection makes many 256 x 256 tiles however few rows it has:
 # 1-64 rows of 151936 columns had gone to them (159 us against 113 at one row),
-# and so had rows that fill at most half of the last tile row.
+# and so had other row counts that leave a quarter or more of the tiles empty.
 @pytest.mark.parametrize("kind", [L.PLAN_GEMM, L.PLAN_GEMM_PACKED])
 @pytest.mark.parametrize("m,n,k,rows", [
     (1, 151936, 4096, 64), (16, 131072, 4096, 64), (64, 151936, 4096, 64),
     (65, 151936, 4096, 128), (100, 151936, 4096, 128), (128, 262144, 8192, 128),
     (300, 151936, 4096, 128), (200, 151936, 4096, 256), (256, 151936, 2048, 256),
-    (8192, 28672, 4096, 256), (8100, 28672, 14336, 256)])
+    (8192, 28672, 4096, 256), (8100, 28672, 14336, 256), (4100, 8200, 160, 256),
+    (640, 151936, 1024, 256)])
 def test_few_rows_of_many_columns_take_short_tiles(w8a8, kind, m, n, k, rows):
     if kind == L.PLAN_GEMM or m > 64:
         assert plan(w8a8, kind, m, n, k, WS)[0] == rows
