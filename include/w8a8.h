@@ -123,10 +123,12 @@ int w8a8_add_rmsnorm_smoothquant(const void* x, const void* residual, const floa
 /*
  * Bytes of device workspace w8a8_gemm can use for this problem.  Sample
  * layout: A and B are repacked K-contiguous into it (plus the K split of the
- * GEMM over them).  Primary layout: int32 K-split partials of problems with
- * few tiles or a last round that is nearly empty (0 otherwise); the rocWMMA
- * split-K sample likewise takes a caller-allocated workspace
- * (rocwmma_gemm_splitk.cpp:214).
+ * GEMM over them).  Primary layout: the int32 partials of a K split, for
+ * problems whose tiles leave CUs idle and whose K is long enough that the
+ * pieces are estimated to repay their traffic (0 otherwise); the rocWMMA split-K
+ * sample likewise takes a caller-allocated workspace
+ * (rocwmma_gemm_splitk.cpp:214).  Not monotone in m, n or k: a workspace for
+ * several shapes takes the largest of their sizes.
  */
 size_t w8a8_gemm_workspace_size(uint32_t m, uint32_t n, uint32_t k, int layout);
 
@@ -331,7 +333,8 @@ int w8a8_quantize_weights(const void* w, uint32_t n, uint32_t k, uint32_t ldw,
  * use for an m x n x k problem: the int32 split-K partials of decode shapes
  * with 32 < m <= 64 and of larger m whose tiles are few (the caller-allocated
  * workspace of the reference's split-K, rocwmma_gemm_splitk.cpp:214); 0 when
- * the shape takes no workspace.
+ * the shape takes no workspace.  Not monotone in m (few tiles take more than
+ * many): a workspace for several m takes the largest of their sizes.
  */
 size_t w8a8_gemm_packed_workspace_size(uint32_t m, uint32_t n, uint32_t k);
 

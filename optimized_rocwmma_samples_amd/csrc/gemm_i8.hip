@@ -447,27 +447,6 @@ void gemm_plan(const uint32_t* sizes, bool packed, uint32_t* plan)
 
 namespace {
 
-// Bytes reported to callers at the least where a K split may run: the pieces
-// of 128-row tiles (64 x 128 below 65 rows) on the CUs that half a round of
-// them leaves idle.  A bound from the sizes alone, so that a workspace sized
-// once does not depend on the plan's fitted constants.
-size_t half_round_bytes(uint32_t m, uint32_t n, uint32_t k)
-{
-    const uint32_t cus = device_cus();
-    uint32_t       bm = 64, bn = 128;
-    if(m > kDecodeMaxM) {
-        auto few = [&] { return (uint64_t)ceil_div(m, bm) * ceil_div(n, bn) < cus * 3ull / 4; };
-        bm = bn = 256;
-        if(few()) bm = 128;
-        if(few()) bn = 128;
-    }
-    const uint64_t tiles = (uint64_t)ceil_div(m, bm) * ceil_div(n, bn);
-    if(tiles * 2 > cus) return 0;
-    const uint32_t parts = std::min({cus / (uint32_t)tiles,
-                                     ceil_div(k, 128) / gemm::kMinKtPerPart, gemm::kMaxParts});
-    return parts < 2 ? 0 : (size_t)tiles * parts * bm * bn * 4;
-}
-
 // K splits of the wide decode kernel for one weight panel: the count that
 // minimises the weight bytes of the busiest CU, ceil(blocks / CUs) / splits
 // (the fewest splits among equals), at least 8 k-tiles per split; 1 = no
@@ -640,8 +619,7 @@ bool persist_pays(const KArgs& p, int out_type)
 size_t gemm_nk_workspace_bytes(const GemmArgs& g)
 {
     if(g.m == 0 || g.n == 0 || g.k == 0) return 0;
-    const TilePlan p = plan_tiles(g.m, g.n, g.k, kMaxPlanBytes, g.m <= kDecodeMaxM, false);
-    return std::max(p.bytes, half_round_bytes(g.m, g.n, g.k));
+    return plan_tiles(g.m, g.n, g.k, kMaxPlanBytes, g.m <= kDecodeMaxM, false).bytes;
 }
 
 // The weights of rows [n0, ...) of a panel (packed: n0 a multiple of the slab).

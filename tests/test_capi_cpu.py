@@ -11,6 +11,7 @@ from pathlib import Path
 import pytest
 
 import optimized_rocwmma_samples_amd as W
+from checks import plan
 from optimized_rocwmma_samples_amd import _lib
 
 ROOT = Path(__file__).resolve().parents[1]
@@ -112,18 +113,25 @@ def test_gemm_validation(w8a8, kw, needle):
 def test_gemm_workspace_size(w8a8):
     ws = W.gemm_workspace_size(100, 200, 300, W.LAYOUT_A_COL_B_KN)
     assert ws >= (100 + 200) * 304 and ws % 256 == 0
-    # primary layout: K-split partials (64 KiB per 128 x 128 tile piece) only
-    # when the tiles fill at most half of the 256 CUs and K allows 2 pieces
-    # of 16 k-tiles
-    assert W.gemm_workspace_size(100, 200, 300) == 0          # K too short
-    assert W.gemm_workspace_size(512, 4096, 4096) == 128 * 2 * 65536
-    assert W.gemm_workspace_size(512, 512, 16384) == 16 * 8 * 65536
-    assert W.gemm_workspace_size(8192, 4096, 4096) == 0       # fills the chip
-    # m <= 64: 64 x 128 tiles (32 KiB per piece) when they fill the chip or can split
-    assert W.gemm_workspace_size(32, 4096, 16384) == 32 * 8 * 32768
-    assert W.gemm_workspace_size(1, 8192, 28672) == 64 * 4 * 32768
-    assert W.gemm_workspace_size(16, 28672, 8192) == 0        # 224 tiles fill the chip
-    assert W.gemm_workspace_size(8, 1000, 512) == 0           # K too short: decode kernel
+
+
+# Primary layout and packed weights above 64 rows: the int32 partials of the plan's K
+# pieces, 0 where it has none (small K, or tiles that fill the chip).
+@pytest.mark.parametrize("m,n,k,split", [
+    (100, 200, 300, False), (512, 4096, 4096, False), (512, 4096, 14336, True),
+    (512, 512, 16384, True), (8192, 4096, 4096, False), (32, 4096, 16384, True),
+    (1, 8192, 28672, True), (16, 28672, 8192, False), (8, 1000, 512, False),
+    (1000, 1500, 4112, False), (300, 600, 8192, True), (128, 4096, 4096, False),
+    (1020, 5824, 18752, True), (2291, 1008, 20480, True), (71, 9072, 11200, True)])
+def test_gemm_workspace_is_what_the_plan_uses(w8a8, m, n, k, split):
+    sizes = [(_lib.PLAN_GEMM, W.gemm_workspace_size(m, n, k))]
+    if m > 64:
+        sizes.append((_lib.PLAN_GEMM_PACKED, W.gemm_packed_workspace_size(m, n, k)))
+    for kind, size in sizes:
+        bm, bn, pieces = plan(w8a8, kind, m, n, k, 64 << 20)
+        tiles = -(-m // bm) * -(-n // bn) if bm else 0
+        assert size == (tiles * pieces * bm * bn * 4 if pieces > 1 else 0)
+    assert (sizes[0][1] > 0) == split
 
 
 def test_fused_validation(w8a8):
