@@ -235,6 +235,9 @@ int w8a8_debug_streamk_wait(uint32_t spin_limit, uint32_t phantom_pieces);
  *   W8A8_PLAN_GEMM_PACKED  the same, m > 64
  *                        -> tile rows, tile columns, K pieces (0, 32, 1: the
  *                           decode kernel)
+ *   W8A8_PLAN_GEMM_ANY     m, n, k (operands of any other alignment or K)
+ *                        -> tile rows, tile columns, 1 (0, 0, 1: one output
+ *                           per thread)
  *   W8A8_PLAN_MOE_GEMM     experts, rows, n, k
  *                        -> tile rows, tile columns, 1 where tiles that leave
  *                           CUs idle are cut along K (with the workspace)
@@ -243,6 +246,7 @@ int w8a8_debug_streamk_wait(uint32_t spin_limit, uint32_t phantom_pieces);
 #define W8A8_PLAN_GEMM 1
 #define W8A8_PLAN_GEMM_PACKED 2
 #define W8A8_PLAN_MOE_GEMM 3
+#define W8A8_PLAN_GEMM_ANY 4
 int w8a8_debug_plan(int kind, const uint32_t* sizes, uint32_t* plan);
 
 /*

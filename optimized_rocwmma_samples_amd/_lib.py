@@ -28,6 +28,7 @@ PLAN_MOE_QUANT = 0  # w8a8_debug_plan kinds
 PLAN_GEMM = 1
 PLAN_GEMM_PACKED = 2
 PLAN_MOE_GEMM = 3
+PLAN_GEMM_ANY = 4
 
 GROUPED_INLINE_GROUPS = 48  # W8A8_GROUPED_INLINE_GROUPS
 

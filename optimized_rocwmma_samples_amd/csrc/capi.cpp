@@ -313,7 +313,10 @@ static int gemm_entry(const char* fn, uint32_t m, uint32_t n, uint32_t k, const 
     if(workspace && reinterpret_cast<uintptr_t>(workspace) % 16 != 0)
         return fail(W8A8_ERROR_INVALID_VALUE, "%s: workspace must be 16-byte aligned", fn);
     if(!w8a8::gemm_fast_path_ok(g))
-        return hip_status(w8a8::launch_gemm_direct(g, false, stream), fn);
+        return hip_status(w8a8::generic_pays(g)
+                              ? w8a8::launch_gemm_generic(g, lda, 1, ldb, 1, stream)
+                              : w8a8::launch_gemm_direct(g, false, stream),
+                          fn);
     return hip_status(w8a8::launch_gemm_nk(g, workspace, workspace ? workspace_bytes : 0, stream),
                       fn);
 }
@@ -424,6 +427,9 @@ int w8a8_debug_plan(int kind, const uint32_t* sizes, uint32_t* plan)
         if(sizes[0] == 0 || sizes[1] == 0 || sizes[2] == 0)
             return fail(W8A8_ERROR_INVALID_VALUE, "%s: m, n, k must be > 0", fn);
         w8a8::gemm_plan(sizes, kind == W8A8_PLAN_GEMM_PACKED, plan);
+        return W8A8_SUCCESS;
+    case W8A8_PLAN_GEMM_ANY:
+        w8a8::gemm_any_plan(sizes, plan);
         return W8A8_SUCCESS;
     case W8A8_PLAN_MOE_GEMM:
         if(sizes[0] == 0 || sizes[1] == 0)

@@ -187,11 +187,15 @@ def test_unaligned_outputs_exact(w8a8, gpu, m, n, k):
             assert_f16_bitexact(got, want) if dt == torch.float16 else assert_i32_equal(got, acc)
 
 
-# The direct kernel (any pointer, row stride and K): tails of 1, 15 and 16 bytes
-# either side of a k-tile, single rows and columns, K below 16, each tile size
-# (64, 128 and 256 rows), operands 1-7 bytes off alignment.
-DIRECT_SHAPES = [(1, 1, 1), (3, 5, 15), (65, 63, 17), (64, 129, 127), (130, 66, 129), (200, 100, 255),
-                 (1, 300, 1001), (1700, 1650, 100), (3400, 3330, 33)]
+# Any pointer, row stride and K: tails of 1, 15 and 16 bytes either side of a
+# k-tile, single rows and columns, K below 16, operands 1-7 bytes off alignment, in
+# the generic kernel (tile 0) and each tile of the direct kernel (64, 128 and 256
+# rows), one k-tile and several (the register ring's refills and both LDS stages).
+DIRECT_SHAPES = [(1, 1, 1, 0), (3, 5, 15, 0), (65, 63, 17, 0), (900, 1050, 11, 64),
+                 (300, 290, 31, 64), (64, 129, 127, 64), (130, 66, 129, 64), (200, 100, 255, 64),
+                 (1, 300, 1001, 64), (300, 200, 641, 64), (1700, 1650, 100, 128),
+                 (1700, 1650, 257, 128), (1650, 1700, 529, 128), (3400, 3330, 33, 256),
+                 (3400, 3330, 385, 256), (3330, 3400, 527, 256)]
 
 
 def _at_offset(a, ld, off, gpu):
@@ -203,9 +207,10 @@ def _at_offset(a, ld, off, gpu):
 
 
 @pytest.mark.parametrize("pad,off", [(0, 0), (1, 3), (16, 8)])
-@pytest.mark.parametrize("m,n,k", DIRECT_SHAPES)
-def test_any_alignment_exact(w8a8, gpu, m, n, k, pad, off):
+@pytest.mark.parametrize("m,n,k,tile", DIRECT_SHAPES)
+def test_any_alignment_exact(w8a8, gpu, m, n, k, tile, pad, off):
     import torch
+    assert plan(w8a8, L.PLAN_GEMM_ANY, m, n, k) == (tile, tile, 1)
     a, b, sa, sb = inputs(m, n, k, 3 * m + 5 * n + k)
     ad, bd = _at_offset(a, k + pad, off, gpu), _at_offset(b, k + pad, off + 4, gpu)
     acc = O.gemm_i32(a, b)

@@ -98,3 +98,13 @@ def capacity(tokens, topk, experts, unit=32):
 def test_expert_gemm_of_few_tiles_is_cut_along_k(w8a8, tokens, topk, experts, n, k, tile):
     rows = capacity(tokens, topk, experts)
     assert plan(w8a8, L.PLAN_MOE_GEMM, experts, rows, n, k) == tile
+
+
+# Few products of a short K: a tile's k-step is mostly zeros (300 x 300 x 9 7.4 us,
+# one output per thread 3.3).
+@pytest.mark.parametrize("m,n,k,tile", [
+    (8, 1021, 9, 0), (300, 300, 9, 0), (55, 1307, 17, 0), (40, 304, 27, 0), (500, 1001, 9, 0),
+    (640, 640, 13, 0), (1000, 1000, 9, 64), (1500, 900, 3, 64), (500, 1001, 17, 64), (100, 1000, 25, 64), (4, 60, 33, 64),
+    (1000, 1000, 1000, 64), (1700, 1650, 100, 128), (3400, 3330, 33, 256)])
+def test_few_products_of_a_short_k_run_one_per_thread(w8a8, m, n, k, tile):
+    assert plan(w8a8, L.PLAN_GEMM_ANY, m, n, k) == (tile, tile, 1)
