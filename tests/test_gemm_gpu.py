@@ -46,20 +46,27 @@ def test_f16_dequant_mode2(w8a8, gpu, m, n, k):
     assert_f16_bitexact(host(c), O.dequant_f16(O.gemm_i32(a, b), sa, sb))
 
 
-# The launch picks its tile by how many 256 x 256 tiles there are (256 CUs):
-#   >= 192 of them: 256 x 256; else >= 192 tiles of 128 x 256: 128 x 256;
-#   else 128 x 128.  Each with partial tiles on both edges.
+# Every tile of the plan (rows x columns; 0 x 32: the decode kernel), unsplit, with
+# partial tiles on both edges and a K tail; the last seven with odd rows of C.
 TILE_CFG_SHAPES = [
-    (4100, 3000, 160),   # 17 x 12 = 204 tiles of 256 x 256
-    (2048, 4096, 512),   # 128 of 256 x 256 -> 256 of 128 x 256
-    (1500, 4000, 272),   # 96 of 256 x 256 -> 192 of 128 x 256, ragged edges
-    (700, 1100, 400),    # 15 of 256 x 256 -> 128 x 128, ragged edges
+    (4100, 3000, 160, (64, 128)), (2048, 4096, 512, (64, 128)), (1500, 4000, 272, (64, 128)),
+    (700, 1100, 400, (64, 64)), (2, 107, 144, (0, 32)), (3, 107, 3680, (32, 64)),
+    (90, 123, 144, (64, 64)), (771, 1051, 144, (64, 128)), (713, 2883, 656, (128, 128)),
+    (1746, 4227, 688, (128, 256)), (1497, 8675, 400, (256, 256)),
 ]
 
 
-@pytest.mark.parametrize("m,n,k", TILE_CFG_SHAPES)
-def test_tile_configs_exact(w8a8, gpu, m, n, k):
+def unsplit_tile(w8a8, m, n, k, packed=False):
+    kind = L.PLAN_GEMM_PACKED if packed else L.PLAN_GEMM
+    rows, cols, pieces = plan(w8a8, kind, m, n, k, 64 << 20)
+    assert pieces == 1
+    return rows, cols
+
+
+@pytest.mark.parametrize("m,n,k,tile", TILE_CFG_SHAPES)
+def test_tile_configs_exact(w8a8, gpu, m, n, k, tile):
     import torch
+    assert unsplit_tile(w8a8, m, n, k) == tile
     a, b, sa, sb = inputs(m, n, k, m + 3 * n + 5 * k)
     ad, bd = dev(a, gpu), dev(b, gpu)
     acc = O.gemm_i32(a, b)
@@ -160,11 +167,16 @@ def test_k_split_exact(w8a8, gpu, m, n, k, tile):
         assert_f16_bitexact(host(w8a8.gemm_packed(ad, pw, sad, sbd, workspace=ws)), cf)
 
 
-# Outputs at odd rows and addresses: 16-byte stores of interior tiles, and the
-# elements around the matrix untouched, for each tile and the decode kernels.
-@pytest.mark.parametrize("m,n,k", [(4100, 3001, 160), (1500, 4001, 272), (513, 4099, 272),
-                                   (100, 1003, 1040), (40, 515, 400), (3, 77, 64)])
-def test_unaligned_outputs_exact(w8a8, gpu, m, n, k):
+# Outputs at odd rows and addresses, channel scales 4 bytes off: 16-byte accesses of
+# interior tiles, and the elements around the matrix untouched, for each tile over
+# row-major and packed weights and the decode kernels.
+@pytest.mark.parametrize("m,n,k,tile", [
+    (4100, 3001, 160, (64, 128)), (1500, 4001, 272, (64, 128)), (100, 1003, 1040, (64, 64)),
+    (40, 515, 400, (0, 32)), (3, 77, 64, (0, 32)), (3, 107, 3680, (32, 64)),
+    (713, 2883, 656, (128, 128)), (1746, 4227, 688, (128, 256)), (1497, 8675, 400, (256, 256))])
+def test_unaligned_outputs_exact(w8a8, gpu, m, n, k, tile):
+    assert unsplit_tile(w8a8, m, n, k) == tile
+    assert m <= 64 or unsplit_tile(w8a8, m, n, k, packed=True) == tile
     import torch
     a, b, sa, sb = inputs(m, n, k, m + 2 * n + k)
     ad, bd = dev(a, gpu), dev(b, gpu)
@@ -220,10 +232,12 @@ def test_any_alignment_exact(w8a8, gpu, m, n, k, tile, pad, off):
 
 
 # The sample layout: in place (few tiles, short K), repacked (with and without
-# the room for 128-byte rows), in place for want of a workspace, and 1-3 rows
-# or columns, each with ragged sizes and leading dimensions.
+# the room for 128-byte rows), in place for want of a workspace (each tile size,
+# several k-tiles and a tail), and 1-3 rows or columns, each with ragged sizes and
+# leading dimensions.
 @pytest.mark.parametrize("m,n,k", [(4, 4, 1), (130, 767, 996), (186, 1044, 1394), (2, 300, 200),
-                                   (300, 3, 77), (700, 900, 2051), (1, 1, 5)])
+                                   (300, 3, 77), (700, 900, 2051), (1, 1, 5), (1700, 1650, 403),
+                                   (3330, 3400, 527)])
 def test_sample_layout_routes_exact(w8a8, gpu, m, n, k):
     import torch
     a, b, _, _ = inputs(m, n, k, m + 7 * n + 3 * k)
@@ -243,17 +257,18 @@ def test_sample_layout_routes_exact(w8a8, gpu, m, n, k):
 # The short tiles (several blocks a CU) and their K pieces, row-major and packed
 # weights: edges of 32 / 64 rows and 64 / 128 columns, K tails, one k-tile.
 SHORT_TILE_SHAPES = [
-    (1, 5000, 4096), (33, 4104, 2064),          # 32 x 64 tiles
-    (31, 520, 17152), (64, 1000, 8208),         # ... in K pieces
-    (65, 4096, 16), (191, 1001, 1040),          # 64 x 64
-    (70, 512, 17072), (226, 380, 12224),        # ... in K pieces
-    (513, 4100, 272), (512, 4096, 2048),        # 64 x 128
+    (1, 5000, 4096, (32, 64, 3)), (33, 4104, 2064, (32, 64, 1)),
+    (31, 520, 17152, (32, 64, 8)), (64, 1000, 8208, (32, 64, 7)),
+    (65, 4096, 16, (64, 128, 1)), (191, 1001, 1040, (64, 64, 1)),
+    (70, 512, 17072, (64, 64, 8)), (226, 380, 12224, (64, 64, 8)),
+    (513, 4100, 272, (64, 128, 1)), (512, 4096, 2048, (64, 128, 1)),
 ]
 
 
-@pytest.mark.parametrize("m,n,k", SHORT_TILE_SHAPES)
-def test_short_tiles_exact(w8a8, gpu, m, n, k):
+@pytest.mark.parametrize("m,n,k,kernel", SHORT_TILE_SHAPES)
+def test_short_tiles_exact(w8a8, gpu, m, n, k, kernel):
     import torch
+    assert plan(w8a8, L.PLAN_GEMM, m, n, k, w8a8.gemm_workspace_size(m, n, k)) == kernel
     a, b, sa, sb = inputs(m, n, k, 11 * m + n + k)
     ad, bd, sad, sbd = dev(a, gpu), dev(b, gpu), dev(sa, gpu), dev(sb, gpu)
     pw = w8a8.pack_weights(bd)
@@ -410,7 +425,7 @@ def test_fused_sq_gemm(w8a8, gpu):
 # projections at M in {512, 2048, 8192}.  These are the headline launches:
 # at M = 8192 qkv / o_proj / gate_up (K = 4096, 32 k-tiles) run the persistent
 # kernel and down (K = 14336) the one-tile-per-block kernel; at M = 512 the
-# small tiles with the K split (workspace allocated as the bench does).
+# smaller tiles, down split along K (workspace allocated as the bench does).
 # q and r are checked in full; c is checked bit-exact on the first and last
 # tile rows (256 rows each) plus 256 seeded random rows.
 CFG3_PROJECTIONS = [("qkv", 4096, 6144), ("o_proj", 4096, 4096), ("gate_up", 4096, 28672),
