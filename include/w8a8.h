@@ -241,12 +241,17 @@ int w8a8_debug_streamk_wait(uint32_t spin_limit, uint32_t phantom_pieces);
  *   W8A8_PLAN_MOE_GEMM     experts, rows, n, k
  *                        -> tile rows, tile columns, 1 where tiles that leave
  *                           CUs idle are cut along K (with the workspace)
+ *   W8A8_PLAN_NORM_ANY     M, N (RMSNorm of rows off the 16-byte alignment or
+ *                          with N no multiple of 8)
+ *                        -> 16-byte chunks per lane, waves per row (0: three
+ *                           passes over a row), 0
  */
 #define W8A8_PLAN_MOE_QUANT 0
 #define W8A8_PLAN_GEMM 1
 #define W8A8_PLAN_GEMM_PACKED 2
 #define W8A8_PLAN_MOE_GEMM 3
 #define W8A8_PLAN_GEMM_ANY 4
+#define W8A8_PLAN_NORM_ANY 5
 int w8a8_debug_plan(int kind, const uint32_t* sizes, uint32_t* plan);
 
 /*

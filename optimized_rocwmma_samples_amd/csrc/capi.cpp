@@ -428,6 +428,10 @@ int w8a8_debug_plan(int kind, const uint32_t* sizes, uint32_t* plan)
             return fail(W8A8_ERROR_INVALID_VALUE, "%s: m, n, k must be > 0", fn);
         w8a8::gemm_plan(sizes, kind == W8A8_PLAN_GEMM_PACKED, plan);
         return W8A8_SUCCESS;
+    case W8A8_PLAN_NORM_ANY: {
+        const w8a8::NormPlan d = w8a8::norm_rows_plan(sizes[0], sizes[1]);
+        return set(d.chunks, d.waves, 0);
+    }
     case W8A8_PLAN_GEMM_ANY:
         w8a8::gemm_any_plan(sizes, plan);
         return W8A8_SUCCESS;

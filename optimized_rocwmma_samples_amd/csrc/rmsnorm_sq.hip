@@ -28,7 +28,8 @@
 // rmsq_rows_kernel (any stride and alignment, N <= 32768): 16-byte accesses at
 // whatever address a row has, the row held in registers and once, in fp32, in
 // LDS.
-// rmsq_generic_kernel: longer rows; one block per row, three passes.
+// rmsq_generic_kernel: longer rows, and few short ones (norm_rows_plan); one block
+// per row, three passes.
 #include "w8a8_device.hpp"
 #include "w8a8_internal.hpp"
 
@@ -459,8 +460,9 @@ rmsq_rows_kernel(NormRows p, uint32_t row_floats)
     }
 }
 
-// Rows longer than the register-resident path covers: one block per row, three
-// passes over the row (the later passes re-read it, mostly from L2).
+// Rows longer than the register-resident path covers, and few short ones: one
+// block per row, three passes over the row (the later passes re-read it, mostly
+// from L2).
 template <bool RES>
 __global__ void __launch_bounds__(kGenThreads) rmsq_generic_kernel(NormRows p)
 {
@@ -613,6 +615,30 @@ hipError_t launch_by_outputs(const NormRows& p, hipStream_t stream)
 
 } // namespace
 
+// Rows that the stream kernel does not take, by length.  Kernel times against the
+// generic kernel's: 12633 x 881 with residual 43 -> 22.6 us, 3000 x 4095 45 -> 28,
+// 3000 x 8191 71 -> 36 (without), 500 x 16383 73 -> 20.4, 1 x 14716 36 -> 7.4.
+NormPlan norm_rows_plan(uint32_t rows, uint32_t n)
+{
+    // Short rows, few of them: an element or two a thread, where the rows kernel's
+    // way through LDS takes longer than the generic kernel's three passes (with
+    // residual, rows / generic: 64 x 110 4.7 / 3.7 us, 512 x 255 4.8 / 3.9, 64 x 510 4.8 /
+    // 4.4; 2000 x 50 4.6 / 4.5, 2000 x 510 5.5 / 6.1, 32768 x 255 33 / 41)
+    if(n <= 512 && rows <= (n <= 256 ? 2304u : 768u)) return {0, 0};
+    if(n <= 512) return {1, 1};
+    // up to 8 rows a CU, all resident: a block a row (1 x 2047 4.4 us against 9.5 by
+    // one wave, 1000 x 881 5.6 against 6.7); past that a wave a row, which waits at
+    // no barrier (30000 x 2047 146 us against 173)
+    if(n <= 2048 && rows <= 2048) return {1, 4};
+    if(n <= 1024) return {2, 1};
+    if(n <= 2048) return {4, 1};
+    if(n <= 4096) return {2, 4};
+    if(n <= 8192) return {4, 4};
+    if(n <= 16384) return {2, 16};
+    if(n <= 32768) return {4, 16};
+    return {0, 0};
+}
+
 hipError_t launch_rmsnorm_sq(const NormRows& p, hipStream_t stream)
 {
     if(p.rows == 0) return hipSuccess;
@@ -632,20 +658,16 @@ hipError_t launch_rmsnorm_sq(const NormRows& p, hipStream_t stream)
         if(n <= 8192) return launch_by_outputs<2, 8, 512, 2>(p, stream);
         if(n <= 16384) return launch_by_outputs<2, 16, 1024, 1>(p, stream);
     }
-    // Other rows by length, kernel times against the generic kernel's: 12633 x 881
-    // with residual 43 -> 22.6 us, 3000 x 4095 45 -> 28, 3000 x 8191 71 -> 36 (without),
-    // 500 x 16383 73 -> 20.4, 1 x 14716 36 -> 7.4.
-    if(n <= 512) return launch_rows_norm<1, 1>(p, stream);
-    // up to 8 rows a CU, all resident: a block a row (1 x 2047 4.4 us against 9.5 by
-    // one wave, 1000 x 881 5.6 against 6.7); past that a wave a row, which waits at
-    // no barrier (30000 x 2047 146 us against 173)
-    if(n <= 2048 && p.rows <= 2048) return launch_rows_norm<1, 4>(p, stream);
-    if(n <= 1024) return launch_rows_norm<2, 1>(p, stream);
-    if(n <= 2048) return launch_rows_norm<4, 1>(p, stream);
-    if(n <= 4096) return launch_rows_norm<2, 4>(p, stream);
-    if(n <= 8192) return launch_rows_norm<4, 4>(p, stream);
-    if(n <= 16384) return launch_rows_norm<2, 16>(p, stream);
-    if(n <= 32768) return launch_rows_norm<4, 16>(p, stream);
+    const NormPlan d  = norm_rows_plan(p.rows, n);
+    auto           is = [&](uint32_t chunks, uint32_t waves) { return d.chunks == chunks && d.waves == waves; };
+    if(is(1, 1)) return launch_rows_norm<1, 1>(p, stream);
+    if(is(1, 4)) return launch_rows_norm<1, 4>(p, stream);
+    if(is(2, 1)) return launch_rows_norm<2, 1>(p, stream);
+    if(is(4, 1)) return launch_rows_norm<4, 1>(p, stream);
+    if(is(2, 4)) return launch_rows_norm<2, 4>(p, stream);
+    if(is(4, 4)) return launch_rows_norm<4, 4>(p, stream);
+    if(is(2, 16)) return launch_rows_norm<2, 16>(p, stream);
+    if(is(4, 16)) return launch_rows_norm<4, 16>(p, stream);
     if(p.res)
         hipLaunchKernelGGL(rmsq_generic_kernel<true>, dim3(p.rows), dim3(kGenThreads), 0, stream, p);
     else

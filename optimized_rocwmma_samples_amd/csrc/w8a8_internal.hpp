@@ -53,6 +53,12 @@ struct NormRows {
     float           eps, qmax;
 };
 hipError_t launch_rmsnorm_sq(const NormRows& p, hipStream_t stream);
+// Rows of any alignment and length: 16-byte chunks per lane and waves per row (0: the
+// generic kernel).
+struct NormPlan {
+    uint32_t chunks, waves;
+};
+NormPlan norm_rows_plan(uint32_t rows, uint32_t n);
 
 struct GemmArgs {
     uint32_t       m, n, k;
