@@ -235,7 +235,8 @@ int w8a8_debug_streamk_wait(uint32_t spin_limit, uint32_t phantom_pieces);
  *   W8A8_PLAN_GEMM_PACKED  the same, m > 64
  *                        -> tile rows, tile columns, K pieces (0, 32, 1: the
  *                           decode kernel)
- *   W8A8_PLAN_GEMM_ANY     m, n, k (operands of any other alignment or K)
+ *   W8A8_PLAN_GEMM_ANY     m, n, k, 0 (operands of any other alignment or K) or
+ *                          1 (the sample layout computed in place)
  *                        -> tile rows, tile columns, 1 (0, 0, 1: one output
  *                           per thread)
  *   W8A8_PLAN_MOE_GEMM     experts, rows, n, k

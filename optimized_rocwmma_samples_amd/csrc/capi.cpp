@@ -290,6 +290,8 @@ static int gemm_entry(const char* fn, uint32_t m, uint32_t n, uint32_t k, const 
                           && workspace_bytes >= repack_bytes(m, n, k, kRepackStepLeast);
         if(room && reinterpret_cast<uintptr_t>(workspace) % 256 != 0)
             return fail(W8A8_ERROR_INVALID_VALUE, "%s: workspace must be 256-byte aligned", fn);
+        if(w8a8::generic_pays(g, true))
+            return hip_status(w8a8::launch_gemm_generic(g, 1, lda, 1, ldb, stream), fn);
         if(w8a8::direct_kn_pays(g) || (!room && w8a8::gemm_direct_kn_ok(g)))
             return hip_status(w8a8::launch_gemm_direct(g, true, stream), fn);
         if(!room) return hip_status(w8a8::launch_gemm_generic(g, 1, lda, 1, ldb, stream), fn);
@@ -313,7 +315,7 @@ static int gemm_entry(const char* fn, uint32_t m, uint32_t n, uint32_t k, const 
     if(workspace && reinterpret_cast<uintptr_t>(workspace) % 16 != 0)
         return fail(W8A8_ERROR_INVALID_VALUE, "%s: workspace must be 16-byte aligned", fn);
     if(!w8a8::gemm_fast_path_ok(g))
-        return hip_status(w8a8::generic_pays(g)
+        return hip_status(w8a8::generic_pays(g, false)
                               ? w8a8::launch_gemm_generic(g, lda, 1, ldb, 1, stream)
                               : w8a8::launch_gemm_direct(g, false, stream),
                           fn);

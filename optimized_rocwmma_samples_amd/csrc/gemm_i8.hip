@@ -447,13 +447,14 @@ void gemm_plan(const uint32_t* sizes, bool packed, uint32_t* plan)
         if(c.cfg == p.cfg) plan[0] = c.bm, plan[1] = c.bn;
 }
 
-// The same for operands of any alignment and K: the direct kernel's tile, or 0 x 0
-// for the generic kernel.
+// The same for operands of any alignment and K (sizes[3] = 0) or the sample layout
+// in place (1): the direct kernel's tile, or 0 x 0 for the generic kernel.
 void gemm_any_plan(const uint32_t* sizes, uint32_t* plan)
 {
     GemmArgs g{};
     g.m = sizes[0], g.n = sizes[1], g.k = sizes[2];
-    plan[0] = plan[1] = generic_pays(g) ? 0 : direct_tile(g.m, g.n);
+    const bool kn = sizes[3] != 0, one = generic_pays(g, kn) || (kn && !gemm_direct_kn_ok(g));
+    plan[0] = plan[1] = one ? 0 : direct_tile(g.m, g.n);
     plan[2]           = 1;
 }
 
@@ -1039,12 +1040,15 @@ hipError_t launch_gemm_direct(const GemmArgs& g, bool kn, hipStream_t stream)
 // below 16, and one output per thread is done sooner while there are few products.
 // Microseconds of either, fitted to 110 sizes: 300 x 300 x 9 3.3 against 7.4, 640 x 640
 // x 13 6.4 / 8.4, 1000 x 1000 x 9 8.7 / 7.5, 1500 x 900 x 3 6.5 / 5.7, 55 x 1307 x 17
-// 3.8 / 4.6, 100 x 1000 x 25 5.2 / 4.5.
-bool generic_pays(const GemmArgs& g)
+// 3.8 / 4.6, 100 x 1000 x 25 5.2 / 4.5.  The sample layout in place, whose tiles load
+// quads of either operand: 120 sizes, 218 x 252 x 1 3.1 / 4.4, 123 x 75 x 14 3.9 / 4.3,
+// 557 x 1018 x 12 5.8 / 4.5, 12 x 755 x 30 5.3 / 4.2.
+bool generic_pays(const GemmArgs& g, bool kn)
 {
     const double k = g.k, outputs = (double)g.m * g.n;
-    return g.k < 32
-           && 2.6 + 0.05 * k + 1e-6 * outputs * (1.7 + 0.47 * k) < 4.4 + (g.k < 16 ? 0.33 * k : 0.0);
+    if(g.k >= 32) return false;
+    if(kn) return 2.8 + 0.07 * k + 1e-6 * outputs * (1.0 + 0.15 * k) < 4.25;
+    return 2.6 + 0.05 * k + 1e-6 * outputs * (1.7 + 0.47 * k) < 4.4 + (g.k < 16 ? 0.33 * k : 0.0);
 }
 
 bool gemm_direct_kn_ok(const GemmArgs& g) { return g.m >= 4 && g.n >= 4; }

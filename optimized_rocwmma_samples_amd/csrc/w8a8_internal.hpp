@@ -84,7 +84,7 @@ size_t     gemm_nk_workspace_bytes(const GemmArgs& g);
 // sizes: m, n, k, workspace bytes -> plan: tile rows, tile columns, K pieces
 // (0 x 32: the decode kernel).  Packed weights: m > 64.
 void       gemm_plan(const uint32_t* sizes, bool packed, uint32_t* plan);
-void       gemm_any_plan(const uint32_t* sizes, uint32_t* plan); // m, n, k: any alignment
+void       gemm_any_plan(const uint32_t* sizes, uint32_t* plan); // m, n, k, sample layout
 // Explicit stream-K over every tile (w8a8_gemm_streamk): `blocks` blocks (0:
 // one per CU, never more than the problem's k-tiles); ws: 16-byte aligned,
 // streamk_workspace_bytes.  Needs gemm_fast_path_ok and A, B under 2 GiB
@@ -159,9 +159,9 @@ bool       gemm_direct_kn_ok(const GemmArgs& g);
 bool       direct_kn_pays(const GemmArgs& g);
 
 // Generic strided GEMM: A(m,k) = a[m*sam + k*sak], B(n,k) = b[n*sbn + k*sbk].
-// One output per thread: where generic_pays (primary layout, few products of
-// short K), and the sample layout with m < 4 or n < 4 and no workspace.
-bool       generic_pays(const GemmArgs& g);
+// One output per thread: where generic_pays (few products of short K; kn: the
+// sample layout), and the sample layout with m < 4 or n < 4 and no workspace.
+bool       generic_pays(const GemmArgs& g, bool kn);
 hipError_t launch_gemm_generic(const GemmArgs& g, size_t sam, size_t sak, size_t sbn,
                                size_t sbk, hipStream_t stream);
 

@@ -231,13 +231,14 @@ def test_any_alignment_exact(w8a8, gpu, m, n, k, tile, pad, off):
                         O.dequant_f16(acc, sa, sb))
 
 
-# The sample layout: in place (few tiles, short K), repacked (with and without
+# The sample layout: in place (few products of a short K one per thread; few tiles,
+# short K), repacked (with and without
 # the room for 128-byte rows), in place for want of a workspace (each tile size,
 # several k-tiles and a tail), and 1-3 rows or columns, each with ragged sizes and
 # leading dimensions.
 @pytest.mark.parametrize("m,n,k", [(4, 4, 1), (130, 767, 996), (186, 1044, 1394), (2, 300, 200),
                                    (300, 3, 77), (700, 900, 2051), (1, 1, 5), (1700, 1650, 403),
-                                   (3330, 3400, 527)])
+                                   (3330, 3400, 527), (123, 75, 14), (5, 6, 31)])
 def test_sample_layout_routes_exact(w8a8, gpu, m, n, k):
     import torch
     a, b, _, _ = inputs(m, n, k, m + 7 * n + 3 * k)

@@ -110,6 +110,15 @@ def test_few_products_of_a_short_k_run_one_per_thread(w8a8, m, n, k, tile):
     assert plan(w8a8, L.PLAN_GEMM_ANY, m, n, k) == (tile, tile, 1)
 
 
+# The sample layout in place likewise (218 x 252 x 1 4.4 us in tiles, 3.1 one per thread).
+@pytest.mark.parametrize("m,n,k,tile", [
+    (4, 4, 1, 0), (218, 252, 1, 0), (280, 832, 4, 0), (123, 75, 14, 0), (1345, 8, 2, 0),
+    (12, 755, 30, 64), (557, 1018, 12, 64), (1513, 1544, 8, 64), (4, 60, 33, 64),
+    (1700, 1650, 403, 128), (3330, 3400, 527, 256), (3, 300, 77, 0)])
+def test_few_products_of_the_sample_layout_run_one_per_thread(w8a8, m, n, k, tile):
+    assert plan(w8a8, L.PLAN_GEMM_ANY, m, n, k, 1) == (tile, tile, 1)
+
+
 # Few short rows of RMSNorm: the generic kernel is done sooner (64 x 110 with residual
 # 3.7 us, a wave a row 4.7).
 @pytest.mark.parametrize("m,n,chunks,waves", [
