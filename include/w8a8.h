@@ -246,6 +246,9 @@ int w8a8_debug_streamk_wait(uint32_t spin_limit, uint32_t phantom_pieces);
  *                          with N no multiple of 8)
  *                        -> 16-byte chunks per lane, waves per row (0: three
  *                           passes over a row), 0
+ *   W8A8_PLAN_MOE_REQUANT  rows, inter, block
+ *                        -> rows per block of the requantization behind the
+ *                           SiLU epilogue, the block's first row, 0
  */
 #define W8A8_PLAN_MOE_QUANT 0
 #define W8A8_PLAN_GEMM 1
@@ -253,6 +256,7 @@ int w8a8_debug_streamk_wait(uint32_t spin_limit, uint32_t phantom_pieces);
 #define W8A8_PLAN_MOE_GEMM 3
 #define W8A8_PLAN_GEMM_ANY 4
 #define W8A8_PLAN_NORM_ANY 5
+#define W8A8_PLAN_MOE_REQUANT 6
 int w8a8_debug_plan(int kind, const uint32_t* sizes, uint32_t* plan);
 
 /*

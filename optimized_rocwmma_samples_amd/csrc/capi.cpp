@@ -442,6 +442,10 @@ int w8a8_debug_plan(int kind, const uint32_t* sizes, uint32_t* plan)
             return fail(W8A8_ERROR_INVALID_VALUE, "%s: experts and rows must be > 0", fn);
         w8a8::moe_gemm_plan(sizes, plan);
         return W8A8_SUCCESS;
+    case W8A8_PLAN_MOE_REQUANT:
+        if(sizes[0] == 0) return fail(W8A8_ERROR_INVALID_VALUE, "%s: rows must be > 0", fn);
+        w8a8::moe_requant_plan(sizes, plan);
+        return W8A8_SUCCESS;
     default: return fail(W8A8_ERROR_INVALID_VALUE, "%s: unknown kind %d", fn, kind);
     }
 }

@@ -348,6 +348,25 @@ __device__ __forceinline__ int row_expert(const P& p, uint32_t row)
     return e;
 }
 
+// row_expert of one row by a whole wave, a load for 64 experts instead of one after
+// another for each halving of the range.
+template <class P>
+__device__ __forceinline__ int wave_row_expert(const P& p, uint32_t row)
+{
+    const int lane = threadIdx.x % kWave;
+    int       e = -1, end = 0;
+    for(int base = 0; base < (int)p.experts; base += kWave) {
+        const int      i     = min(base + lane, (int)p.experts - 1);
+        const int      start = p.expert_start[i], count = p.expert_count[i];
+        const uint64_t in    = __ballot(base + lane < (int)p.experts && start <= (int32_t)row);
+        if(in == 0) break; // starts ascend
+        const int last = 63 - __builtin_clzll(in);
+        e              = base + last;
+        end            = __builtin_amdgcn_readlane(start, last) + __builtin_amdgcn_readlane(count, last);
+    }
+    return (int32_t)row < end ? e : -1;
+}
+
 // Generic form (any inter, alignment and size): element loads and stores.
 template <int CPL, int WPR>
 __global__ void __launch_bounds__(kSqThreads) silu_quant_kernel(SiluRows p)
@@ -530,14 +549,25 @@ struct SiluRequant {
 // wave instruction), reduced through LDS, and the rows' experts.
 // Phase 2: kRqBatch 8-column chunks per lane in flight (h and s2 loads issued
 // before any store), each wave over ROWS / kSqWaves whole rows or, with one
-// row per block, over its share of the row's columns.
+// row per block, the block over its row.
 // 8 rows per block where they make two blocks a CU: cfg5's 8448 rows make
 // 1056, 4.1 per CU; with 16 rows (528 blocks, 2.06 per CU) the CUs holding a
 // third block finished alone (cfg5 layer 1535-1547 -> 1526-1528 us, same box,
 // alternating).  Fewer rows take a block each, or most CUs idle while a few
-// stream 8 rows one after another: 288 rows of 14336 17.1 -> 5.2 us.
+// stream 8 rows one after another: 288 rows of 14336 17.1 -> 4.8 us.  Rows of one
+// batch a wave take one from 10 rows a CU on (2048 columns: 2304 rows 7.7 us by
+// eights, 6.4 by ones; 3072 7.9 / 7.8; 3584 8.8 / 9.8).  Blocks of a row follow
+// gemm::xcd_remap: the rows that an expert has are the first of its 32, so that
+// one or two an expert in block order would all be on one XCD (64 experts
+// of one row, 14336 columns 19.2 -> 9.6 us; 8 rows a block 11.1).
 constexpr int kRqRows  = 8;
 constexpr int kRqBatch = 7;
+
+// The first row of a block.
+__host__ __device__ inline uint32_t requant_row(uint32_t rows_a_block, uint32_t block, uint32_t blocks)
+{
+    return rows_a_block == 1 ? gemm::xcd_remap(block, blocks) : block * rows_a_block;
+}
 
 template <bool S2, int ROWS>
 __global__ void __launch_bounds__(kSqThreads) silu_requant_kernel(SiluRequant p)
@@ -551,8 +581,13 @@ __global__ void __launch_bounds__(kSqThreads) silu_requant_kernel(SiluRequant p)
     const int          t    = threadIdx.x;
     const int          wave = t / kWave;
     const int          lane = t % kWave;
-    const uint32_t     r0   = blockIdx.x * ROWS;
+    const uint32_t     r0   = requant_row(ROWS, blockIdx.x, gridDim.x);
 
+    int expert = -1; // of the only row
+    if constexpr(ROWS == 1) {
+        expert = wave_row_expert(p, r0);
+        if(expert < 0) return; // padding
+    }
     const __amdgpu_buffer_rsrc_t rp = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<float*>(p.pmax), 0, (int)p.p_bytes, gemm::kBufferFlags);
     {
@@ -567,8 +602,8 @@ __global__ void __launch_bounds__(kSqThreads) silu_requant_kernel(SiluRequant p)
             if(lane == 0) red[wave][0] = mx;
         } else {
             red[t / ROWS][t % ROWS] = mx;
+            if(t < ROWS) rowexp[t] = r0 + t < p.rows ? row_expert(p, r0 + t) : -1;
         }
-        if(t < ROWS) rowexp[t] = r0 + t < p.rows ? row_expert(p, r0 + t) : -1;
     }
     __syncthreads();
     if(t < ROWS) {
@@ -587,22 +622,24 @@ __global__ void __launch_bounds__(kSqThreads) silu_requant_kernel(SiluRequant p)
     const __amdgpu_buffer_rsrc_t rq = __builtin_amdgcn_make_buffer_rsrc(p.q, 0, (int)p.q_bytes,
                                                                         gemm::kBufferFlags);
     const float qmax = p.qmax;
-    constexpr uint32_t kSpan  = kRqBatch * 8 * kWave; // columns of one batch of a wave
-    constexpr uint32_t kStep  = ROWS == 1 ? kSqWaves * kSpan : kSpan;
+    // columns of one batch's load: of a wave, or of the block on its only row
+    constexpr int kLanes = ROWS == 1 ? kSqThreads : kWave;
+    const int     chunk  = ROWS == 1 ? t : lane;
     for(int rr = ROWS == 1 ? 0 : wave; rr < ROWS; rr += ROWS == 1 ? 1 : kSqWaves) {
         const uint32_t row   = r0 + rr;
-        const int      e     = rowexp[rr];
+        const int      e     = ROWS == 1 ? expert : rowexp[rr];
         if(e < 0) continue; // wave-uniform: padding rows and rows past the end
         const float    rsc   = rowmax[rr] / qmax;
         const float    inv   = rsc > 0.f ? 1.f / rsc : 0.f;
-        if(lane == 0 && (ROWS > 1 || wave == 0)) p.r[row] = rsc;
-        for(uint32_t c0 = ROWS == 1 ? wave * kSpan : 0; c0 < n; c0 += kStep) {
+        if(chunk == 0) p.r[row] = rsc;
+        for(uint32_t c0 = 0; c0 < n; c0 += kRqBatch * 8 * kLanes) {
             v4i      hv[kRqBatch], s0[kRqBatch], s1[kRqBatch];
             uint32_t col[kRqBatch];
 #pragma unroll
             for(int j = 0; j < kRqBatch; ++j) {
-                const uint32_t c = c0 + (j * kWave + lane) * 8;
+                const uint32_t c = c0 + (j * kLanes + chunk) * 8;
                 col[j]           = c < n ? c : kOob;
+                if(ROWS == 1 && c0 + j * kLanes * 8 >= n) continue; // uniform
                 hv[j] = __builtin_amdgcn_raw_buffer_load_b128(
                     rh, col[j] != kOob ? (row * p.ldh + c) * 2 : kOob, 0, 0);
                 if constexpr(S2) {
@@ -613,6 +650,7 @@ __global__ void __launch_bounds__(kSqThreads) silu_requant_kernel(SiluRequant p)
             }
 #pragma unroll
             for(int j = 0; j < kRqBatch; ++j) {
+                if(ROWS == 1 && c0 + j * kLanes * 8 >= n) break; // uniform
                 const uint32_t hw[4] = {(uint32_t)hv[j].x, (uint32_t)hv[j].y, (uint32_t)hv[j].z,
                                         (uint32_t)hv[j].w};
                 float          sv[8] = {1.f, 1.f, 1.f, 1.f, 1.f, 1.f, 1.f, 1.f};
@@ -662,10 +700,16 @@ hipError_t launch_requant_rows(const SiluRequant& p, hipStream_t stream)
     return hipGetLastError();
 }
 
+uint32_t requant_rows_a_block(uint32_t rows, uint32_t inter)
+{
+    const uint32_t line = (inter <= kRqBatch * 8 * kWave ? 10u : 2u * kRqRows) * device_cus();
+    return rows < line ? 1 : kRqRows;
+}
+
 hipError_t launch_requant(const SiluRequant& p, hipStream_t stream)
 {
-    return p.rows < 2u * kRqRows * device_cus() ? launch_requant_rows<1>(p, stream)
-                                                : launch_requant_rows<kRqRows>(p, stream);
+    return requant_rows_a_block(p.rows, p.inter) == 1 ? launch_requant_rows<1>(p, stream)
+                                                      : launch_requant_rows<kRqRows>(p, stream);
 }
 
 // Gate_up weights interleaved for the SiLU epilogue: output row r of expert
@@ -1002,6 +1046,13 @@ hipError_t launch_moe_gemm(const MoeGemmArgs& a, hipStream_t stream)
     case MoeTile::kMid: return gemm::launch_moe<GemmGroupedMid>(q, a.out_type, stream);
     default: return gemm::launch_moe<GemmGrouped, GemmGroupedWide>(q, a.out_type, stream);
     }
+}
+
+void moe_requant_plan(const uint32_t* sizes, uint32_t* plan)
+{
+    plan[0] = requant_rows_a_block(sizes[0], sizes[1]);
+    plan[1] = requant_row(plan[0], sizes[2], (sizes[0] + plan[0] - 1) / plan[0]);
+    plan[2] = 0;
 }
 
 void moe_gemm_plan(const uint32_t* sizes, uint32_t* plan)

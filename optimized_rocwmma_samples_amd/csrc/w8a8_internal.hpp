@@ -225,6 +225,8 @@ hipError_t launch_moe_gemm(const MoeGemmArgs& a, hipStream_t stream);
 // sizes: experts, rows, n, k -> plan: tile rows, tile columns, whether a tail that
 // fills few CUs is cut along K (given the workspace).
 void       moe_gemm_plan(const uint32_t* sizes, uint32_t* plan);
+// sizes: rows, inter, block -> plan: rows a block, the block's first row
+void       moe_requant_plan(const uint32_t* sizes, uint32_t* plan);
 // Workspace that lets launch_moe_gemm split its last partial round of tiles
 // along K (one int32 tile partial per CU of the current device).
 size_t moe_gemm_workspace_bytes();

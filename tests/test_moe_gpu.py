@@ -644,10 +644,13 @@ def test_moe_gate_up_silu(w8a8, gpu, t, k, e, h, inter, unit, with_s2):
 
 # The short tiles of few rows per expert: 64-row tiles (partial last N tile, two
 # tile rows for the busiest expert), 128 x 128 tiles, and more rows than the
-# one-row-per-block requantization takes.
+# one-row-per-block requantization takes, of either length; that one with columns past
+# a batch of the block's loads and more experts than a wave has lanes.
 @pytest.mark.parametrize("t,k,e,h,inter,unit,with_s2", [
     (40, 2, 8, 512, 400, 32, True), (1, 2, 8, 256, 48, 32, True), (130, 1, 1, 256, 144, 1, False),
-    (400, 2, 8, 4096, 512, 1, True), (4200, 2, 128, 128, 64, 1, True)])
+    (400, 2, 8, 4096, 512, 1, True), (4200, 2, 128, 128, 64, 1, True),
+    (1300, 2, 8, 128, 512, 32, True), (2, 2, 8, 64, 14352, 32, True),
+    (60, 2, 130, 64, 2064, 1, True), (3, 1, 130, 64, 2048, 32, False)])
 def test_moe_gate_up_silu_short_tiles(w8a8, gpu, t, k, e, h, inter, unit, with_s2):
     test_moe_gate_up_silu(w8a8, gpu, t, k, e, h, inter, unit, with_s2)
 

@@ -140,3 +140,24 @@ def test_few_products_of_the_sample_layout_run_one_per_thread(w8a8, m, n, k, til
     (9, 32769, 0, 0)])
 def test_few_short_norm_rows_take_the_generic_kernel(w8a8, m, n, chunks, waves):
     assert plan(w8a8, L.PLAN_NORM_ANY, m, n) == (chunks, waves, 0)
+
+
+# The requantization of expert rows.  A row a block where eight a block would be
+# few blocks; with rows of one batch a wave that ends earlier (2048 columns, 3584 rows
+# 8.8 us by eights, 9.8 by ones).
+@pytest.mark.parametrize("rows,inter,per_block", [
+    (256, 14336, 1), (4095, 14336, 1), (4096, 14336, 8), (8448, 14336, 8), (4095, 3600, 1),
+    (2559, 3584, 1), (2560, 3584, 8), (3840, 2048, 8), (3328, 512, 8), (2048, 1408, 1)])
+def test_requantized_rows_a_block(w8a8, rows, inter, per_block):
+    assert plan(w8a8, L.PLAN_MOE_REQUANT, rows, inter, 0)[0] == per_block
+
+
+# The rows that decoding gives an expert are the first of its 32: they are spread over
+# the eight XCDs (64 experts of one row, 14336 columns, all on one: 19.2 us, spread 9.6).
+@pytest.mark.parametrize("experts", [8, 16, 64, 100])
+def test_first_rows_of_experts_are_spread_over_the_xcds(w8a8, experts):
+    rows = 32 * experts
+    first = [plan(w8a8, L.PLAN_MOE_REQUANT, rows, 14336, b)[1] for b in range(rows)]
+    assert sorted(first) == list(range(rows))
+    on = [sum(b % 8 == x and r % 32 == 0 for b, r in enumerate(first)) for x in range(8)]
+    assert max(on) <= -(-experts // 8) + 1
