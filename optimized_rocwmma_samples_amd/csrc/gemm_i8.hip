@@ -247,10 +247,10 @@ struct TilePlan {
     size_t   bytes; // int32 partials of the pieces
 };
 
-// Time of a launch in µs, fitted per configuration to 1000-odd launches of
-// random sizes (m 1-4096, n 64-28672, k 512-28672, weights cold or in the
-// MALL; median error 3-6%):
+// Time of a launch in µs, fitted per configuration to launches of random sizes
+// (m 1-4096, n 64-28672, k 512-28672) with weights cold and in the MALL:
 //   fixed + sum over a CU's blocks of k-tiles x step[blocks resident together]
+//   + round x rounds of resident blocks after the first
 //   + out_mb x output MB + w_mb x weight MB
 //   + (pieces > 1) (split + split_mb x partial MB)
 // with step x cross where row-major operands' rows cross 128-byte lines (K no
@@ -261,19 +261,32 @@ struct TilePlan {
 // (181 x 19016 x 9488: 64 x 64 tiles, 3.5 blocks a CU, 122 us against 99 in 128 x
 // 256 ones; one factor for every load had said 81 against 88).  Fitted on 193
 // sizes with such K, every configuration and 1-8 pieces measured.
+// m <= 64 (kDecodeMaxM) never fills taller tiles, larger m never needs shorter
+// ones.  64 x 128 tiles in more rows than one have costs of their own: each
+// weight panel is read by several blocks, and cold weights keep a k-step waiting
+// longer (529 x 1984 x 8192: 32.6 us in one round of them, 24 estimated with the
+// one row's costs; 22.9 in 128 x 128 tiles).  Their and the 128 x 128 tiles' step and
+// all `round`s: every plan of 1600 sizes of 65-3000 rows measured, row-major and
+// packed, cold and in the MALL; the plan is on average 0.75% slower than the best and
+// for 2% of the sizes by more than 10% (1.6 and 6% with one row's costs and no
+// round).  500 more of K 64-1024 and up to 70000 columns: 1.3% against 4.1%.
 struct CfgCost {
     TileCfg  cfg;
     uint32_t bm, bn, resident; // resident: blocks a CU holds (LDS)
-    double   fixed, step[3], split, split_mb, out_mb, w_mb, cross, full, from, to;
+    uint32_t least, most;      // the m it serves
+    double   fixed, step[3], round, split, split_mb, out_mb, w_mb, cross, full, from, to;
 };
-constexpr CfgCost kCosts[] = {
-    {TileCfg::kMain, 256, 256, 1, 6.2, {1.19}, 6.5, 0.45, 0.27, 0.044, 1.06, 0.0, 0.0, 1.0},
-    {TileCfg::kMidM, 128, 256, 1, 4.9, {0.71}, 4.7, 0.38, 0.34, 0.043, 1.25, 0.0, 0.0, 1.0},
-    {TileCfg::kSmall, 128, 128, 1, 3.6, {0.42}, 3.8, 0.40, 0.40, 0.023, 1.25, 0.0, 0.0, 1.0},
-    {TileCfg::kNarrow, 64, 128, 2, 3.2, {0.30, 0.63}, 3.7, 0.32, 0.23, 0.061, 1.40, 0.0, 0.0, 1.0},
-    {TileCfg::kTiny, 64, 64, 2, 3.3, {0.24, 0.42}, 3.3, 0.47, 0.37, 0.030, 1.10, 0.8, 0.8, 2.0},
-    {TileCfg::kRow, 32, 64, 3, 3.4, {0.23, 0.36, 0.59}, 3.0, 0.41, 0.0, 0.048, 1.02, 0.6, 0.9, 1.5},
+constexpr uint32_t kAnyM    = 0xFFFFFFFFu;
+constexpr CfgCost  kCosts[] = {
+    {TileCfg::kMain, 256, 256, 1, 65, kAnyM, 6.2, {1.19}, 1.0, 6.5, 0.45, 0.27, 0.044, 1.06, 0.0, 0.0, 1.0},
+    {TileCfg::kMidM, 128, 256, 1, 65, kAnyM, 4.9, {0.71}, 0.0, 4.7, 0.38, 0.34, 0.043, 1.25, 0.0, 0.0, 1.0},
+    {TileCfg::kSmall, 128, 128, 1, 65, kAnyM, 3.6, {0.45}, 0.7, 3.8, 0.40, 0.40, 0.023, 1.25, 0.0, 0.0, 1.0},
+    {TileCfg::kNarrow, 64, 128, 2, 1, 64, 3.2, {0.30, 0.63}, 0.0, 3.7, 0.32, 0.23, 0.061, 1.40, 0.0, 0.0, 1.0},
+    {TileCfg::kNarrow, 64, 128, 2, 65, kAnyM, 3.2, {0.375, 0.745}, 0.7, 3.7, 0.32, 0.30, 0.061, 1.40, 0.0, 0.0, 1.0},
+    {TileCfg::kTiny, 64, 64, 2, 1, kAnyM, 3.3, {0.24, 0.42}, 0.3, 3.3, 0.47, 0.37, 0.030, 1.10, 0.8, 0.8, 2.0},
+    {TileCfg::kRow, 32, 64, 3, 1, 64, 3.4, {0.23, 0.36, 0.59}, 0.0, 3.0, 0.41, 0.0, 0.048, 1.02, 0.6, 0.9, 1.5},
 };
+static_assert(kDecodeMaxM == 64, "the rows that kCosts' entries serve");
 constexpr uint32_t kMinKtPlan    = 6;        // k-tiles of a K piece, at least
 constexpr size_t   kMaxPlanBytes = 64 << 20; // partials of a plan, at most
 // A split call launches twice, and the host needs about 3.5 µs a launch and
@@ -291,18 +304,22 @@ struct PlanTime {
     bool   operator<(const PlanTime& o) const { return seen != o.seen ? seen < o.seen : gpu < o.gpu; }
 };
 
+// What a k-step of row-major operands takes against one of whole 128-byte lines.
+double line_factor(const CfgCost& c, uint32_t k, uint64_t blocks)
+{
+    if(k % 128 == 0) return 1.0;
+    const double ramp
+        = std::clamp(((double)blocks / device_cus() - c.from) / (c.to - c.from), 0.0, 1.0);
+    const double off = 1.0 - std::gcd(k, 128u) / 128.0; // rows off a line
+    return std::max(c.cross, 1.0 + c.full * off * ramp);
+}
+
 PlanTime plan_cost(const CfgCost& c, uint32_t m, uint32_t n, uint32_t k, uint32_t parts, bool packed)
 {
     const uint32_t cus    = device_cus();
     const uint32_t tm     = ceil_div(m, c.bm);
     const uint64_t blocks = (uint64_t)tm * ceil_div(n, c.bn) * parts;
-    double         factor = 1.0;
-    if(!packed && k % 128 != 0) {
-        const double ramp = std::clamp(((double)blocks / cus - c.from) / (c.to - c.from), 0.0, 1.0);
-        const double off  = 1.0 - std::gcd(k, 128u) / 128.0; // rows off a line
-        factor            = std::max(c.cross, 1.0 + c.full * off * ramp);
-    }
-    const double   steps  = ceil_div(ceil_div(k, 128), parts) * factor;
+    const double   steps  = ceil_div(ceil_div(k, 128), parts) * (packed ? 1.0 : line_factor(c, k, blocks));
     uint64_t       per_cu = (blocks + cus - 1) / cus;
     double         t      = c.fixed + 2e-6 * m * n * c.out_mb + 1e-6 * n * (double)k * c.w_mb;
     // launch_main runs a last round of at most half the CUs as smaller tiles
@@ -312,7 +329,8 @@ PlanTime plan_cost(const CfgCost& c, uint32_t m, uint32_t n, uint32_t k, uint32_
         --per_cu;
     }
     t += steps * (per_cu / c.resident * c.step[c.resident - 1]
-                  + (per_cu % c.resident ? c.step[per_cu % c.resident - 1] : 0.0));
+                  + (per_cu % c.resident ? c.step[per_cu % c.resident - 1] : 0.0))
+         + c.round * ((per_cu - 1) / c.resident);
     if(parts == 1) return {t, t};
     t += c.split + 4e-6 * blocks * c.bm * c.bn * c.split_mb;
     return {std::max(t, kSplitHostUs), t};
@@ -351,8 +369,7 @@ TilePlan search_plan(uint32_t m, uint32_t n, uint32_t k, size_t ws_bytes, bool d
     const uint32_t most = std::min(gemm::kMaxParts, ceil_div(k, 128) / kMinKtPlan);
     if(decode) best.cfg = TileCfg::kDecode;
     for(const CfgCost& c : kCosts) {
-        // m <= 64 never fills taller tiles, larger m never needs shorter ones
-        if(m <= kDecodeMaxM ? c.bm > 64 : c.bm < 64) continue;
+        if(m < c.least || m > c.most) continue;
         const uint64_t tiles = (uint64_t)ceil_div(m, c.bm) * ceil_div(n, c.bn);
         for(uint32_t p = 1; p <= std::max(1u, most); ++p) {
             const uint64_t bytes = p == 1 ? 0 : tiles * p * c.bm * c.bn * 4;
@@ -412,26 +429,29 @@ GroupedTile grouped_gemm_tile(const w8a8_group_desc* groups, uint32_t ngroups)
     GroupedTile best{0, 0, 0};
     double      cost = 1e300;
     for(const CfgCost& c : kCosts) {
-        if(c.cfg == TileCfg::kRow) continue;
-        uint64_t tiles = 0, steps = 0, most = 0;
-        double   out = 0, w = 0;
+        if(c.most != kAnyM) continue;
+        auto     count = [&](const w8a8_group_desc& g) {
+            return (uint64_t)ceil_div(g.m, c.bm) * ceil_div(g.n, c.bn);
+        };
+        uint64_t tiles = 0;
+        for(uint32_t i = 0; i < ngroups; ++i) tiles += count(groups[i]);
+        if(tiles == 0 || tiles > 0x7FFFFFFFull) continue;
+        double steps = 0, most = 0, out = 0, w = 0;
         for(uint32_t i = 0; i < ngroups; ++i) {
             const w8a8_group_desc& g = groups[i];
             if(g.m == 0) continue;
-            const uint64_t t = (uint64_t)ceil_div(g.m, c.bm) * ceil_div(g.n, c.bn);
-            const uint64_t k = ceil_div(g.k, 128);
-            tiles += t;
-            steps += t * k;
+            const double k = ceil_div(g.k, 128);
+            steps += count(g) * k;
             most = std::max(most, k);
             out += 2e-6 * g.m * g.n;
             w += 1e-6 * g.n * (double)g.k;
         }
-        if(tiles == 0 || tiles > 0x7FFFFFFFull) continue;
         const uint64_t per_cu = (tiles + device_cus() - 1) / device_cus();
-        const double   nk     = per_cu == 1 ? (double)most : (double)steps / tiles;
+        const double   nk     = per_cu == 1 ? most : steps / tiles;
         const double   t      = c.fixed + out * c.out_mb + w * c.w_mb
                          + nk * (per_cu / c.resident * c.step[c.resident - 1]
-                                 + (per_cu % c.resident ? c.step[per_cu % c.resident - 1] : 0.0));
+                                 + (per_cu % c.resident ? c.step[per_cu % c.resident - 1] : 0.0))
+                         + c.round * ((per_cu - 1) / c.resident);
         if(t < cost) {
             cost = t;
             best = GroupedTile{c.bm, c.bn, (uint32_t)tiles};

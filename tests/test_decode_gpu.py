@@ -91,7 +91,7 @@ def test_packed_int32_exact(w8a8, gpu, m, n, k):
 # Packed weights above the decode sizes: every tile of the plan (rows x columns), with
 # partial tiles, partial slabs and a K tail.
 @pytest.mark.parametrize("m,n,k,tile", [
-    (3072, 4096, 256, (64, 128)), (1500, 4000, 272, (64, 128)), (700, 1100, 400, (64, 128)),
+    (3072, 4096, 256, (256, 256)), (1500, 4000, 272, (64, 128)), (700, 1100, 400, (64, 64)),
     (90, 123, 144, (64, 64)), (713, 2883, 656, (128, 128)), (1746, 4227, 688, (128, 256)),
     (1497, 8675, 400, (256, 256))])
 def test_packed_block_heights_exact(w8a8, gpu, m, n, k, tile):
@@ -112,7 +112,7 @@ def test_packed_block_heights_exact(w8a8, gpu, m, n, k, tile):
 # the K split with a partial last slab and K tail.
 @pytest.mark.parametrize("m,n,k,kernel", [
     (4100, 8200, 160, (256, 256, 1)), (4100, 8200, 16, (256, 256, 1)),
-    (2000, 17000, 272, (256, 256, 1)), (2048, 5000, 144, (64, 128, 1)),
+    (2000, 17000, 272, (256, 256, 1)), (1564, 3351, 224, (64, 128, 1)),
     (300, 600, 8208, (64, 64, 5))])
 def test_packed_tile_kernels_match_row_major(w8a8, gpu, m, n, k, kernel):
     assert plan(w8a8, L.PLAN_GEMM_PACKED, m, n, k, 64 << 20) == kernel

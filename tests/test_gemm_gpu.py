@@ -47,12 +47,12 @@ def test_f16_dequant_mode2(w8a8, gpu, m, n, k):
 
 
 # Every tile of the plan (rows x columns; 0 x 32: the decode kernel), unsplit, with
-# partial tiles on both edges and a K tail; the last seven with odd rows of C.
+# partial tiles on both edges and a K tail; the last eight with odd rows of C.
 TILE_CFG_SHAPES = [
-    (4100, 3000, 160, (64, 128)), (2048, 4096, 512, (64, 128)), (1500, 4000, 272, (64, 128)),
+    (4100, 3000, 160, (256, 256)), (2048, 4096, 512, (128, 256)), (1500, 4000, 272, (128, 256)),
     (700, 1100, 400, (64, 64)), (2, 107, 144, (0, 32)), (3, 107, 3680, (32, 64)),
-    (90, 123, 144, (64, 64)), (771, 1051, 144, (64, 128)), (713, 2883, 656, (128, 128)),
-    (1746, 4227, 688, (128, 256)), (1497, 8675, 400, (256, 256)),
+    (90, 123, 144, (64, 64)), (771, 1051, 144, (64, 64)), (549, 2785, 240, (64, 128)),
+    (713, 2883, 656, (128, 128)), (1746, 4227, 688, (128, 256)), (1497, 8675, 400, (256, 256)),
 ]
 
 
@@ -135,7 +135,8 @@ def test_persistent_tiles_strided_output(w8a8, gpu):
 # rows of C, a K tail in the last piece.
 SPLIT_SHAPES = [
     (10, 107, 4128, (32, 64)), (64, 1000, 8208, (32, 64)), (83, 107, 4176, (64, 64)),
-    (257, 851, 7104, (64, 128)), (300, 600, 8192, (64, 128)), (512, 512, 16384, (64, 128)),
+    (257, 851, 7104, (64, 64)), (300, 600, 8192, (64, 64)), (512, 512, 16384, (64, 128)),
+    (305, 1097, 9744, (64, 128)),
     (204, 2739, 8512, (128, 128)), (512, 4096, 14336, (128, 128)),
     (1200, 1067, 21200, (128, 256)), (2062, 2099, 15296, (256, 256)),
 ]
@@ -171,7 +172,7 @@ def test_k_split_exact(w8a8, gpu, m, n, k, tile):
 # interior tiles, and the elements around the matrix untouched, for each tile over
 # row-major and packed weights and the decode kernels.
 @pytest.mark.parametrize("m,n,k,tile", [
-    (4100, 3001, 160, (64, 128)), (1500, 4001, 272, (64, 128)), (100, 1003, 1040, (64, 64)),
+    (4100, 3001, 160, (256, 256)), (990, 1621, 368, (64, 128)), (100, 1003, 1040, (64, 64)),
     (40, 515, 400, (0, 32)), (3, 77, 64, (0, 32)), (3, 107, 3680, (32, 64)),
     (713, 2883, 656, (128, 128)), (1746, 4227, 688, (128, 256)), (1497, 8675, 400, (256, 256))])
 def test_unaligned_outputs_exact(w8a8, gpu, m, n, k, tile):
@@ -260,9 +261,9 @@ def test_sample_layout_routes_exact(w8a8, gpu, m, n, k):
 SHORT_TILE_SHAPES = [
     (1, 5000, 4096, (32, 64, 3)), (33, 4104, 2064, (32, 64, 1)),
     (31, 520, 17152, (32, 64, 8)), (64, 1000, 8208, (32, 64, 7)),
-    (65, 4096, 16, (64, 128, 1)), (191, 1001, 1040, (64, 64, 1)),
+    (65, 4096, 16, (64, 64, 1)), (191, 1001, 1040, (64, 64, 1)),
     (70, 512, 17072, (64, 64, 8)), (226, 380, 12224, (64, 64, 8)),
-    (513, 4100, 272, (64, 128, 1)), (512, 4096, 2048, (64, 128, 1)),
+    (549, 2785, 240, (64, 128, 1)), (418, 885, 9152, (64, 128, 5)), (512, 4096, 2048, (64, 128, 1)),
 ]
 
 
@@ -284,7 +285,7 @@ def test_short_tiles_exact(w8a8, gpu, m, n, k, kernel):
 
 
 # Few rows of many columns (more than two rounds of 256 x 256 tiles): short tiles.
-@pytest.mark.parametrize("m,n,k", [(3, 131100, 160), (100, 131100, 144), (300, 70001, 160)])
+@pytest.mark.parametrize("m,n,k", [(3, 131100, 160), (100, 131100, 144), (257, 66001, 512)])
 def test_few_rows_of_many_columns_exact(w8a8, gpu, m, n, k):
     import torch
     a, b, sa, sb = inputs(m, n, k, m + n + k)

@@ -81,6 +81,18 @@ def test_few_rows_leave_the_decode_kernel_for_a_tenth(w8a8, m, n, k, kernel):
     assert plan(w8a8, L.PLAN_GEMM, m, n, k, WS) == kernel
 
 
+# More than 64 rows: 64 x 128 tiles in one round of the CUs with cold weights and a long
+# K (529 x 1984 x 8192 32.6 us, 128 x 128 tiles in three pieces 22.9), and several
+# rounds of short tiles at a short K (918 x 24832 x 384 34 us, 256 x 256 tiles 27).
+@pytest.mark.parametrize("kind", [L.PLAN_GEMM, L.PLAN_GEMM_PACKED])
+@pytest.mark.parametrize("m,n,k,tile", [
+    (529, 1984, 8192, (128, 128)), (1304, 784, 7936, (128, 128)), (688, 2176, 11136, (128, 128)),
+    (735, 1792, 6912, (128, 128)), (876, 2208, 11648, (128, 128)), (918, 24832, 384, (256, 256)),
+    (332, 17152, 512, (128, 256)), (512, 4096, 4096, (64, 128)), (300, 6144, 4096, (64, 128))])
+def test_short_tiles_of_several_rows_cost_what_they_take(w8a8, kind, m, n, k, tile):
+    assert plan(w8a8, kind, m, n, k, WS)[:2] == tile
+
+
 # K no multiple of 128 and the chip full of short tiles, whose k-steps then wait for
 # twice the requests (181 x 19016 x 9488 in 64 x 64 tiles 122 us, others 99).
 @pytest.mark.parametrize("m,n,k,slower", [

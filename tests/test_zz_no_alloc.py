@@ -58,7 +58,7 @@ def test_noalloc_refuses_oversized_shapes_before_hip(w8a8):
 
 # (m, n, k), K pieces: two large and a smaller split (the scratch holds the partials),
 # then two shapes with no split, one a decode kernel's, and split decode tiles
-SHAPES = [(512, 4096, 14336, 2), (1200, 1067, 21200, 5), (300, 600, 8192, 8),
+SHAPES = [(512, 4096, 14336, 2), (1200, 1067, 21200, 5), (300, 600, 8192, 5),
           (1000, 1000, 1008, 1), (512, 4096, 4096, 1), (8, 1000, 512, 1), (16, 4096, 4096, 4),
           (32, 4096, 16384, 8)]
 
