@@ -246,6 +246,8 @@ int w8a8_debug_streamk_wait(uint32_t spin_limit, uint32_t phantom_pieces);
  *                          with N no multiple of 8)
  *                        -> 16-byte chunks per lane, waves per row (0: three
  *                           passes over a row), 0
+ *   W8A8_PLAN_GROUPED      groups (1 to 64) and the m, n, k of each
+ *                        -> tile rows, tile columns, 1
  *   W8A8_PLAN_MOE_REQUANT  rows, inter, block
  *                        -> rows per block of the requantization behind the
  *                           SiLU epilogue, the block's first row, 0
@@ -257,6 +259,7 @@ int w8a8_debug_streamk_wait(uint32_t spin_limit, uint32_t phantom_pieces);
 #define W8A8_PLAN_GEMM_ANY 4
 #define W8A8_PLAN_NORM_ANY 5
 #define W8A8_PLAN_MOE_REQUANT 6
+#define W8A8_PLAN_GROUPED 7
 int w8a8_debug_plan(int kind, const uint32_t* sizes, uint32_t* plan);
 
 /*

@@ -31,6 +31,7 @@ PLAN_MOE_GEMM = 3
 PLAN_GEMM_ANY = 4
 PLAN_NORM_ANY = 5
 PLAN_MOE_REQUANT = 6
+PLAN_GROUPED = 7
 
 GROUPED_INLINE_GROUPS = 48  # W8A8_GROUPED_INLINE_GROUPS
 

@@ -442,6 +442,11 @@ int w8a8_debug_plan(int kind, const uint32_t* sizes, uint32_t* plan)
             return fail(W8A8_ERROR_INVALID_VALUE, "%s: experts and rows must be > 0", fn);
         w8a8::moe_gemm_plan(sizes, plan);
         return W8A8_SUCCESS;
+    case W8A8_PLAN_GROUPED:
+        if(sizes[0] == 0 || sizes[0] > 64 || sizes[1] == 0 || sizes[2] == 0 || sizes[3] == 0)
+            return fail(W8A8_ERROR_INVALID_VALUE, "%s: 1 to 64 groups, m, n, k > 0", fn);
+        w8a8::grouped_plan(sizes, plan);
+        return W8A8_SUCCESS;
     case W8A8_PLAN_MOE_REQUANT:
         if(sizes[0] == 0) return fail(W8A8_ERROR_INVALID_VALUE, "%s: rows must be > 0", fn);
         w8a8::moe_requant_plan(sizes, plan);

@@ -423,7 +423,8 @@ TilePlan plan_tiles(uint32_t m, uint32_t n, uint32_t k, size_t ws_bytes, bool de
 // two blocks).  Against the tallest tile that fills 3/4 of the CUs: 13 groups
 // of 1-901 rows, 3584 x 3776, 116 -> 82 us a call; 7 and 67 rows, 1280 x 576,
 // kernel 7.4 -> 5.2 us; 256 / 512 / 128 / 768 rows, 4096^2, stays on 208 tiles
-// of 128 x 256 (35 -> 34 us).
+// of 128 x 256 (35 -> 34 us).  Rows off a 128-byte line count as in plan_cost: 60 groups of
+// 622 rows, 3968 x 3568, 875 -> 746 us, 16 of 288, 5600 x 4448, 224 -> 199.
 GroupedTile grouped_gemm_tile(const w8a8_group_desc* groups, uint32_t ngroups)
 {
     GroupedTile best{0, 0, 0};
@@ -440,7 +441,7 @@ GroupedTile grouped_gemm_tile(const w8a8_group_desc* groups, uint32_t ngroups)
         for(uint32_t i = 0; i < ngroups; ++i) {
             const w8a8_group_desc& g = groups[i];
             if(g.m == 0) continue;
-            const double k = ceil_div(g.k, 128);
+            const double k = ceil_div(g.k, 128) * line_factor(c, g.k, tiles);
             steps += count(g) * k;
             most = std::max(most, k);
             out += 2e-6 * g.m * g.n;
@@ -458,6 +459,15 @@ GroupedTile grouped_gemm_tile(const w8a8_group_desc* groups, uint32_t ngroups)
         }
     }
     return best;
+}
+
+// sizes: groups alike (up to 64), their m, n, k.
+void grouped_plan(const uint32_t* sizes, uint32_t* plan)
+{
+    w8a8_group_desc groups[64] = {};
+    for(auto& g : groups) g.m = sizes[1], g.n = sizes[2], g.k = sizes[3];
+    const GroupedTile t = grouped_gemm_tile(groups, std::min(sizes[0], 64u));
+    plan[0] = t.bm, plan[1] = t.bn, plan[2] = 1;
 }
 
 uint32_t direct_tile(uint32_t m, uint32_t n);

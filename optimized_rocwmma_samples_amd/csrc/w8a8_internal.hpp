@@ -84,6 +84,7 @@ size_t     gemm_nk_workspace_bytes(const GemmArgs& g);
 // sizes: m, n, k, workspace bytes -> plan: tile rows, tile columns, K pieces
 // (0 x 32: the decode kernel).  Packed weights: m > 64.
 void       gemm_plan(const uint32_t* sizes, bool packed, uint32_t* plan);
+void       grouped_plan(const uint32_t* sizes, uint32_t* plan); // groups, their m, n, k
 void       gemm_any_plan(const uint32_t* sizes, uint32_t* plan); // m, n, k, sample layout
 // Explicit stream-K over every tile (w8a8_gemm_streamk): `blocks` blocks (0:
 // one per CU, never more than the problem's k-tiles); ws: 16-byte aligned,

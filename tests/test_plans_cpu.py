@@ -173,3 +173,14 @@ def test_first_rows_of_experts_are_spread_over_the_xcds(w8a8, experts):
     assert sorted(first) == list(range(rows))
     on = [sum(b % 8 == x and r % 32 == 0 for b, r in enumerate(first)) for x in range(8)]
     assert max(on) <= -(-experts // 8) + 1
+
+
+# Groups with K no multiple of 128: each 128-byte row piece is two requests, which short
+# tiles wait for most (60 groups of 622 rows, 3968 x 3568, 875 us in 128 x 256 tiles, 746
+# in 256 x 256).
+@pytest.mark.parametrize("groups,m,n,k,tile", [
+    (60, 622, 3968, 3568, (256, 256)), (16, 568, 5888, 4128, (256, 256)),
+    (16, 288, 5600, 4448, (256, 256)), (60, 534, 5392, 3648, (256, 256)),
+    (4, 416, 4096, 4096, (128, 256)), (1, 67, 576, 1280, (64, 64))])
+def test_groups_of_rows_off_a_line_take_tall_tiles(w8a8, groups, m, n, k, tile):
+    assert plan(w8a8, L.PLAN_GROUPED, groups, m, n, k)[:2] == tile
