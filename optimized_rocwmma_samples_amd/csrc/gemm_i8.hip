@@ -123,12 +123,15 @@ __global__ void __launch_bounds__(256) repack_i8_kernel(Repack a, Repack b, uint
         const uint32_t in  = p.rows < 4 ? 0 : min(r0 + row, p.rows - 4); // a quad past the end moves inside
         const uint32_t sh  = min(r0 + row - in, 3u) * 8;
         uint32_t       x[16];
-        if(p.rows < 4) { // uniform: 1-3 source columns, byte by byte
+        if(p.rows < 4) { // uniform: 1-3 source columns, byte by byte, all in flight
+#pragma unroll
             for(int j = 0; j < 16; ++j) {
                 const uint32_t c = c0 + ch * 16 + j;
-                x[j]             = 0;
-                for(uint32_t e = 0; e < p.rows && c < cols; ++e)
-                    x[j] |= (uint32_t)(uint8_t)p.src[(size_t)c * p.ld + e] << (8 * e);
+                uint32_t       e[3];
+#pragma unroll
+                for(uint32_t i = 0; i < 3; ++i) // past the end: the last row or column
+                    e[i] = (uint8_t)p.src[(size_t)min(c, cols - 1) * p.ld + min(i, p.rows - 1)];
+                x[j] = c < cols ? e[0] | e[1] << 8 | e[2] << 16 : 0;
             }
         } else if(c0 + 128 <= cols) { // uniform
             const int8_t* s = p.src + (size_t)(c0 + ch * 16) * p.ld + in;

@@ -239,7 +239,8 @@ def test_any_alignment_exact(w8a8, gpu, m, n, k, tile, pad, off):
 # leading dimensions.
 @pytest.mark.parametrize("m,n,k", [(4, 4, 1), (130, 767, 996), (186, 1044, 1394), (2, 300, 200),
                                    (300, 3, 77), (700, 900, 2051), (1, 1, 5), (1700, 1650, 403),
-                                   (3330, 3400, 527), (123, 75, 14), (5, 6, 31)])
+                                   (3330, 3400, 527), (123, 75, 14), (5, 6, 31),
+                                   (3, 2, 1466)])
 def test_sample_layout_routes_exact(w8a8, gpu, m, n, k):
     import torch
     a, b, _, _ = inputs(m, n, k, m + 7 * n + 3 * k)
