@@ -304,7 +304,6 @@ __device__ __forceinline__ void epilogue_silu(const KArgs& p, uint32_t m0, uint3
                                               const float* s2, uint32_t ldh, uint32_t ldp,
                                               uint32_t inter)
 {
-    static_assert(C::kMfma == 16, "SiLU epilogue: 16 x 16 MFMA layout");
     using A                  = Acc<C>;
     constexpr int kPairs     = A::kQuadsN / 2;
     constexpr int kOutCols   = C::kWaveN / 2;

@@ -9,7 +9,7 @@
 //
 // Tile hierarchy (Cfg): block BM x BN x BK, WAVES_M x WAVES_N waves, each wave
 // owning a (BM/WAVES_M) x (BN/WAVES_N) tile of 16 x 16 v_mfma_i32_16x16x64_i8
-// blocks (or 32 x 32 v_mfma_i32_32x32x32_i8 ones, Cfg's MFMA_ parameter).
+// blocks.
 // The MFMA is issued with srcA = B fragment (rows n) and srcB = A fragment
 // (rows m): D[i=n][j=m], so each lane owns one m and runs of 4 consecutive n
 // (Acc<C>'s quads) and the epilogue writes 4 fp16 (8 B) or 4 int32 (16 B)
@@ -51,20 +51,18 @@ namespace w8a8 {
 
 namespace gemm {
 
-// MFMA_: the matrix instruction of the tile body, 32 for v_mfma_i32_32x32x32_i8
-// or 16 for v_mfma_i32_16x16x64_i8.  Both retire the same int8 ops per cycle
-// and read the same LDS bytes per op for a given wave tile; on MI355X under
-// the power limit the 16 x 16 x 64 form sustains ~14% more ops on random
-// operands (3.60 against 3.16 POP/s in a loop fed from LDS like the tile
-// body; plausibly because it reads and writes half the accumulator bytes per
-// op).
+// The matrix instruction is v_mfma_i32_16x16x64_i8: the 32 x 32 x 32 form retires
+// the same int8 ops per cycle and reads the same LDS bytes per op, but under the
+// power limit this one sustains ~14% more ops on random operands (3.60 against
+// 3.16 POP/s in a loop fed from LDS like the tile body; plausibly because it reads
+// and writes half the accumulator bytes per op).
 // PACKB_: B is the packed weight buffer (gemm_i8_pack.hpp; KArgs::ldb unused)
 // instead of rows of K bytes.  Its 8 KiB (slab, k-tile) blocks go to LDS as
 // they are, 1 KiB contiguous per wave-load, and the fragments are read from
 // that order (FragReader); everything else of the tile is the same, and so
 // are the sums.
 template <int BM_, int BN_, int BK_, int STAGES_, int WAVES_M_, int WAVES_N_, int GROUP_M_ = 8,
-          int MFMA_ = 32, bool PACKB_ = false>
+          bool PACKB_ = false>
 struct Cfg {
     static constexpr int kBM      = BM_;
     static constexpr int kBN      = BN_;
@@ -77,7 +75,7 @@ struct Cfg {
     static constexpr int kThreads = kWaves * kWave;
     static constexpr int kWaveM   = kBM / kWavesM;
     static constexpr int kWaveN   = kBN / kWavesN;
-    static constexpr int kMfma    = MFMA_;
+    static constexpr int kMfma    = 16;                  // rows and columns of one MFMA
     static constexpr bool kPackB  = PACKB_;
     static constexpr int kTilesM  = kWaveM / kMfma;      // MFMA blocks per wave tile
     static constexpr int kTilesN  = kWaveN / kMfma;
@@ -91,7 +89,7 @@ struct Cfg {
     static constexpr int kLoadsA  = kABytes / 1024 / kWaves; // wave-loads per wave per stage
     static constexpr int kLoadsB  = kBBytes / 1024 / kWaves;
     static constexpr int kLoads   = kLoadsA + kLoadsB;
-    static constexpr int kMfmaK   = kMfma == 32 ? 32 : 64; // depth of one MFMA
+    static constexpr int kMfmaK   = 64;                  // depth of one MFMA
     static constexpr int kSubK    = kBK / kMfmaK;        // MFMA k-groups per tile
 
     static_assert(kChunks == 2 || kChunks == 4 || kChunks == 8, "BK in {32, 64, 128}");
@@ -100,9 +98,8 @@ struct Cfg {
     static_assert(kSubK % 2 == 0, "fragment ping-pong needs an even k-group count per k-tile");
     static_assert(kLoadsA * kWaves * 1024 == kABytes && kLoadsB * kWaves * 1024 == kBBytes,
                   "tile bytes must split evenly into 1 KiB wave-loads");
-    static_assert(kMfma == 32 || kMfma == 16, "32x32x32 or 16x16x64 MFMA");
-    static_assert(!kPackB || (kMfma == 16 && kBK == kPackK && kBN % kSlab == 0),
-                  "packed B: the 16x16x64 form over whole slabs and packed k-tiles");
+    static_assert(!kPackB || (kBK == kPackK && kBN % kSlab == 0),
+                  "packed B: whole slabs and packed k-tiles");
     static_assert(kBK % kMfmaK == 0, "whole MFMA k-groups per tile");
     static_assert(kWaveM % 32 == 0 && kWaveN % 32 == 0, "wave tile of whole 32-row passes");
     static_assert(kStages >= 2, "at least double buffering");
@@ -169,24 +166,6 @@ __device__ __forceinline__ void block_barrier()
     asm volatile("" ::: "memory");
 }
 
-// One MFMA k-group (32 x 32 x 32 form): MFMAs and the DS reads of the next
-// fragments alternate, then the remaining MFMAs follow.  The first MFMA stays
-// ahead of the reads so it waits only on fragments read one group earlier.
-template <int NMFMA, int NDS, int ID>
-__device__ __forceinline__ void interleave_mfma_ds()
-{
-    constexpr int kPairs = NDS < NMFMA ? NDS : NMFMA;
-#pragma unroll
-    for(int i = 0; i < kPairs; ++i) {
-        __builtin_amdgcn_sched_group_barrier(kSchedMfma, 1, ID);
-        __builtin_amdgcn_sched_group_barrier(kSchedDsRead, 1, ID);
-    }
-    if constexpr(NMFMA > kPairs)
-        __builtin_amdgcn_sched_group_barrier(kSchedMfma, NMFMA - kPairs, ID);
-    if constexpr(NDS > kPairs)
-        __builtin_amdgcn_sched_group_barrier(kSchedDsRead, NDS - kPairs, ID);
-}
-
 // The group after the barrier also issues the refill of the freed stage:
 // steps of (one MFMA, its share of global->LDS loads, its share of DS reads),
 // then the remaining MFMAs.
@@ -228,70 +207,27 @@ __device__ __forceinline__ void interleave_rows16()
 // The int32 accumulators of one wave tile, in the lane layout of the tile's
 // MFMA (srcA = B fragment, srcB = A fragment, so D[n][m]).  Epilogues see
 // them as quads: 4 outputs of one row m at 4 consecutive columns n, quad
-// (qm, qn) at wave-tile row row(qm) and first column col(qn):
-//   MFMA 32: r[i][j] is the 32 x 32 block (i, j); quad (qm, qn) is
-//     r[qm][qn / 4][4 (qn % 4) ...], m = 32 qm + lane % 32,
-//     n = 32 (qn / 4) + 8 (qn % 4) + 4 (lane / 32);
-//   MFMA 16: r[i][j] is the 16 x 16 block (i, j) and quad (i, j) itself,
-//     m = 16 qm + lane % 16, n = 16 qn + 4 (lane / 16).
+// (qm, qn) at wave-tile row row(qm) and first column col(qn): the 16 x 16 block
+// (qm, qn), m = 16 qm + lane % 16, n = 16 qn + 4 (lane / 16).
 // Quads are numbered q = qm * kQuadsN + qn (the K-split partial layout).
 template <class C>
 struct Acc {
-    static constexpr bool kBig    = C::kMfma == 32;
-    static constexpr int  kQuadsM = C::kTilesM;
-    static constexpr int  kQuadsN = kBig ? C::kTilesN * 4 : C::kTilesN;
-    static constexpr int  kQuads  = kQuadsM * kQuadsN;
-    using Block                   = std::conditional_t<kBig, v16i, v4i>;
-    Block r[C::kTilesM][C::kTilesN];
+    static constexpr int kQuadsM = C::kTilesM;
+    static constexpr int kQuadsN = C::kTilesN;
+    static constexpr int kQuads  = kQuadsM * kQuadsN;
+    v4i r[C::kTilesM][C::kTilesN];
 
-    __device__ static __forceinline__ int row(int qm, int lane)
-    {
-        return kBig ? qm * 32 + (lane & 31) : qm * 16 + (lane & 15);
-    }
-    __device__ static __forceinline__ int col(int qn, int lane)
-    {
-        return kBig ? (qn >> 2) * 32 + (qn & 3) * 8 + (lane >> 5) * 4 : qn * 16 + (lane >> 4) * 4;
-    }
+    __device__ static __forceinline__ int row(int qm, int lane) { return qm * 16 + (lane & 15); }
+    __device__ static __forceinline__ int col(int qn, int lane) { return qn * 16 + (lane >> 4) * 4; }
     __device__ __forceinline__ void zero()
     {
 #pragma unroll
         for(int i = 0; i < C::kTilesM; ++i)
 #pragma unroll
-            for(int j = 0; j < C::kTilesN; ++j) r[i][j] = Block{0};
+            for(int j = 0; j < C::kTilesN; ++j) r[i][j] = v4i{0};
     }
-    __device__ __forceinline__ v4i quad(int qm, int qn) const
-    {
-        if constexpr(kBig) {
-            const v16i& b = r[qm][qn >> 2];
-            const int   o = (qn & 3) * 4;
-            return v4i{b[o], b[o + 1], b[o + 2], b[o + 3]};
-        } else {
-            return r[qm][qn];
-        }
-    }
-    __device__ __forceinline__ void add(int qm, int qn, const v4i& v)
-    {
-        if constexpr(kBig) {
-            v16i&     b = r[qm][qn >> 2];
-            const int o = (qn & 3) * 4;
-            b[o] += v.x, b[o + 1] += v.y, b[o + 2] += v.z, b[o + 3] += v.w;
-        } else {
-            r[qm][qn] += v;
-        }
-    }
-    // r += the products of one k-group's fragments
-    __device__ __forceinline__ void mfma(const v4i (&af)[C::kTilesM], const v4i (&bf)[C::kTilesN])
-    {
-#pragma unroll
-        for(int i = 0; i < C::kTilesM; ++i)
-#pragma unroll
-            for(int j = 0; j < C::kTilesN; ++j) {
-                if constexpr(kBig)
-                    r[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(bf[j], af[i], r[i][j], 0, 0, 0);
-                else
-                    r[i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(bf[j], af[i], r[i][j], 0, 0, 0);
-            }
-    }
+    __device__ __forceinline__ v4i quad(int qm, int qn) const { return r[qm][qn]; }
+    __device__ __forceinline__ void add(int qm, int qn, const v4i& v) { r[qm][qn] += v; }
 };
 
 // The global -> LDS loads of the packed B operand: wave-load j of a tile's B
@@ -322,8 +258,6 @@ __device__ __forceinline__ int b_bytes(const KArgs& p)
 // below bit 4, so they come from the lane alone.
 template <class C>
 struct FragReader {
-    using FragA = v4i[C::kTilesM];
-    using FragB = v4i[C::kTilesN];
     int offa, offb;       // byte offsets of fragment 0 within a stage
     int cofs[C::kSubK];   // byte offset of each k-group's chunk
     int cofb;             // packed B: byte offset of k-group 0's chunk
@@ -353,43 +287,29 @@ struct FragReader {
                                                  + g * (C::kMfmaK / 16 * 512) + cofb);
         return *reinterpret_cast<const v4i*>(sbase + offb + t * C::kMfma * C::kBK + cofs[g]);
     }
-    __device__ __forceinline__ void load(const int8_t* sbase, int g, FragA& af, FragB& bf) const
-    {
-#pragma unroll
-        for(int t = 0; t < C::kTilesM; ++t) af[t] = a(sbase, g, t);
-#pragma unroll
-        for(int t = 0; t < C::kTilesN; ++t) bf[t] = b(sbase, g, t);
-    }
 };
 
 // The k-loop's fragment registers, and one k-group of MFMAs with the reads of
 // the next k-group's fragments interleaved.  Slot s = k-group parity (even
 // kSubK, so k-group g of every k-tile uses slot g & 1).
-//   MFMA 32: two full fragment sets; a group reads the next into the other.
-//   MFMA 16: the operand with more fragments per wave tile is the outer one
-//     (A unless the wave tile is wider than tall): one register set, the next
-//     group's outer fragment t read into fragment t's registers right after
-//     its MFMAs have issued, (outer - 1) x inner MFMAs before its first use;
-//     the inner fragments ping-pong, next inner fragment t read after outer
-//     fragment t (the earliest slots, so they have the most time to land
-//     before the next group starts).  A 128 x 64 wave tile holds 64 fragment
-//     VGPRs instead of 96, which keeps its loop within 256 VGPRs.
+// The operand with more fragments per wave tile is the outer one (A unless the
+// wave tile is wider than tall): one register set, the next group's outer
+// fragment t read into fragment t's registers right after its MFMAs have
+// issued, (outer - 1) x inner MFMAs before its first use; the inner fragments
+// ping-pong, next inner fragment t read after outer fragment t (the earliest
+// slots, so they have the most time to land before the next group starts).  A
+// 128 x 64 wave tile holds 64 fragment VGPRs instead of 96, which keeps its
+// loop within 256 VGPRs.
 // NVMEM: global -> LDS loads issued just before, spread over the group.
 template <class C>
 struct FragPipe {
-    static constexpr bool kBig       = C::kMfma == 32;
     static constexpr bool kRowsOuter = C::kTilesM >= C::kTilesN;
     static constexpr int  kOuter     = kRowsOuter ? C::kTilesM : C::kTilesN;
     static constexpr int  kInner     = kRowsOuter ? C::kTilesN : C::kTilesM;
     static constexpr int  kMfmaN     = C::kTilesM * C::kTilesN;
-    static constexpr int  kDs        = C::kTilesM + C::kTilesN;
     FragReader<C> fr;
-    // MFMA 32 registers
-    v4i fa[kBig ? 2 : 1][kBig ? C::kTilesM : 1];
-    v4i fb[kBig ? 2 : 1][kBig ? C::kTilesN : 1];
-    // MFMA 16 registers
-    v4i fo[kBig ? 1 : kOuter];
-    v4i fi[kBig ? 1 : 2][kBig ? 1 : kInner];
+    v4i fo[kOuter];
+    v4i fi[2][kInner];
 
     __device__ __forceinline__ FragPipe(int wm, int wn, int lane) : fr(wm, wn, lane) {}
 
@@ -415,47 +335,30 @@ struct FragPipe {
 
     __device__ __forceinline__ void first(const int8_t* sbase)
     {
-        if constexpr(kBig) {
-            fr.load(sbase, 0, fa[0], fb[0]);
-        } else {
 #pragma unroll
-            for(int t = 0; t < kOuter; ++t) fo[t] = outer(sbase, 0, t);
+        for(int t = 0; t < kOuter; ++t) fo[t] = outer(sbase, 0, t);
 #pragma unroll
-            for(int t = 0; t < kInner; ++t) fi[0][t] = inner(sbase, 0, t);
-        }
+        for(int t = 0; t < kInner; ++t) fi[0][t] = inner(sbase, 0, t);
     }
 
     template <int NVMEM>
     __device__ __forceinline__ void step(Acc<C>& acc, int s, const int8_t* sbase_n, int g_n)
     {
-        if constexpr(kBig) {
-            fr.load(sbase_n, g_n, fa[s ^ 1], fb[s ^ 1]);
-            acc.mfma(fa[s], fb[s]);
-            if constexpr(NVMEM > 0)
-                interleave_mfma_vmem_ds<kMfmaN, NVMEM, kDs, 1>();
-            else
-                interleave_mfma_ds<kMfmaN, kDs, 0>();
-        } else {
 #pragma unroll
-            for(int o = 0; o < kOuter; ++o) {
-                mfma_outer(acc, s, o);
-                fo[o] = outer(sbase_n, g_n, o);
-                if(o < kInner) fi[s ^ 1][o] = inner(sbase_n, g_n, o);
-            }
-            interleave_rows16<0, kOuter, kInner, NVMEM, (NVMEM > 0 ? 1 : 0)>();
+        for(int o = 0; o < kOuter; ++o) {
+            mfma_outer(acc, s, o);
+            fo[o] = outer(sbase_n, g_n, o);
+            if(o < kInner) fi[s ^ 1][o] = inner(sbase_n, g_n, o);
         }
+        interleave_rows16<0, kOuter, kInner, NVMEM, (NVMEM > 0 ? 1 : 0)>();
     }
     // a k-group with no fragments to read next: MFMAs only, with the NVMEM
     // global -> LDS loads issued just before spread over them
     template <int NVMEM = 0>
     __device__ __forceinline__ void last(Acc<C>& acc, int s)
     {
-        if constexpr(kBig) {
-            acc.mfma(fa[s], fb[s]);
-        } else {
 #pragma unroll
-            for(int o = 0; o < kOuter; ++o) mfma_outer(acc, s, o);
-        }
+        for(int o = 0; o < kOuter; ++o) mfma_outer(acc, s, o);
         if constexpr(NVMEM > 0) interleave_mfma_vmem_ds<kMfmaN, NVMEM, 0, 1>();
     }
 };
