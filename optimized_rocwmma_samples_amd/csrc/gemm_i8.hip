@@ -39,12 +39,12 @@ using gemm::KArgs;
 // (plan_tiles says where each wins).
 template <bool PB>
 struct Tiles {
-    using Main   = gemm::Cfg<256, 256, 128, 2, 2, 4, 4, PB>;
-    using MidM   = gemm::Cfg<128, 256, 128, 3, 2, 4, 4, PB>; // 8 waves of 64 x 64, 144 KiB LDS
-    using Small  = gemm::Cfg<128, 128, 128, 3, 2, 4, 4, PB>; // 8 waves of 64 x 32, 96 KiB LDS
-    using Narrow = gemm::Cfg<64, 128, 128, 3, 2, 4, 4, PB>;  // 8 waves of 32 x 32, 72 KiB LDS
-    using Tiny   = gemm::Cfg<64, 64, 128, 4, 2, 2, 4, PB>;   // 4 waves of 32 x 32, 64 KiB LDS
-    using Row    = gemm::Cfg<32, 64, 128, 4, 1, 2, 4, PB>;   // 2 waves of 32 x 32, 48 KiB LDS
+    using Main   = gemm::Cfg<256, 256, 128, 2, 2, 4, 4, 16, PB>;
+    using MidM   = gemm::Cfg<128, 256, 128, 3, 2, 4, 4, 16, PB>; // 8 waves of 64 x 64, 144 KiB LDS
+    using Small  = gemm::Cfg<128, 128, 128, 3, 2, 4, 4, 16, PB>; // 8 waves of 64 x 32, 96 KiB LDS
+    using Narrow = gemm::Cfg<64, 128, 128, 3, 2, 4, 4, 16, PB>;  // 8 waves of 32 x 32, 72 KiB LDS
+    using Tiny   = gemm::Cfg<64, 64, 128, 4, 2, 2, 4, 16, PB>;   // 4 waves of 32 x 32, 64 KiB LDS
+    using Row    = gemm::Cfg<32, 64, 128, 4, 1, 2, 4, 16, PB>;   // 2 waves of 32 x 32, 48 KiB LDS
 };
 using GemmMain    = Tiles<false>::Main;
 using GemmMidM    = Tiles<false>::MidM;
@@ -1058,9 +1058,9 @@ template <bool COLS>
 hipError_t launch_direct_tiles(const GemmArgs& g, hipStream_t stream)
 {
     if(g.m == 0 || g.n == 0) return hipSuccess;
-    using Big    = gemm::Cfg<256, 256, 128, 2, 2, 4, 4>;
-    using Middle = gemm::Cfg<128, 128, 128, 2, 2, 4, 4>;
-    using Little = gemm::Cfg<64, 64, 128, 2, 2, 2, 4>;
+    using Big    = gemm::Cfg<256, 256, 128, 2, 2, 4, 4, 16>;
+    using Middle = gemm::Cfg<128, 128, 128, 2, 2, 4, 4, 16>;
+    using Little = gemm::Cfg<64, 64, 128, 2, 2, 2, 4, 16>;
     constexpr int  kAhead = COLS ? 1 : 2; // k-tiles in registers (a quad unit is 16 VGPRs)
     const KArgs    p      = make_kargs(g);
     if((uint64_t)ceil_div(g.m, 64) * ceil_div(g.n, 64) > 0x7FFFFFFFull) return hipErrorInvalidValue;

@@ -51,7 +51,7 @@ namespace w8a8 {
 
 namespace gemm {
 
-// The matrix instruction is v_mfma_i32_16x16x64_i8: the 32 x 32 x 32 form retires
+// MFMA_: the matrix instruction, v_mfma_i32_16x16x64_i8 (16): the 32 x 32 x 32 form retires
 // the same int8 ops per cycle and reads the same LDS bytes per op, but under the
 // power limit this one sustains ~14% more ops on random operands (3.60 against
 // 3.16 POP/s in a loop fed from LDS like the tile body; plausibly because it reads
@@ -62,7 +62,7 @@ namespace gemm {
 // that order (FragReader); everything else of the tile is the same, and so
 // are the sums.
 template <int BM_, int BN_, int BK_, int STAGES_, int WAVES_M_, int WAVES_N_, int GROUP_M_ = 8,
-          bool PACKB_ = false>
+          int MFMA_ = 16, bool PACKB_ = false>
 struct Cfg {
     static constexpr int kBM      = BM_;
     static constexpr int kBN      = BN_;
@@ -75,7 +75,7 @@ struct Cfg {
     static constexpr int kThreads = kWaves * kWave;
     static constexpr int kWaveM   = kBM / kWavesM;
     static constexpr int kWaveN   = kBN / kWavesN;
-    static constexpr int kMfma    = 16;                  // rows and columns of one MFMA
+    static constexpr int kMfma    = MFMA_;
     static constexpr bool kPackB  = PACKB_;
     static constexpr int kTilesM  = kWaveM / kMfma;      // MFMA blocks per wave tile
     static constexpr int kTilesN  = kWaveN / kMfma;
@@ -98,6 +98,7 @@ struct Cfg {
     static_assert(kSubK % 2 == 0, "fragment ping-pong needs an even k-group count per k-tile");
     static_assert(kLoadsA * kWaves * 1024 == kABytes && kLoadsB * kWaves * 1024 == kBBytes,
                   "tile bytes must split evenly into 1 KiB wave-loads");
+    static_assert(kMfma == 16, "the 16x16x64 MFMA");
     static_assert(!kPackB || (kBK == kPackK && kBN % kSlab == 0),
                   "packed B: whole slabs and packed k-tiles");
     static_assert(kBK % kMfmaK == 0, "whole MFMA k-groups per tile");

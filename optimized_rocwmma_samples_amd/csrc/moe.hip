@@ -799,19 +799,19 @@ __global__ void __launch_bounds__(256)
     }
 }
 
-using GemmGrouped = gemm::Cfg<256, 256, 128, 2, 2, 4, 4>;
+using GemmGrouped = gemm::Cfg<256, 256, 128, 2, 2, 4, 4, 16>;
 // GemmGrouped's wide partner: an expert's rest of at most 128 rows runs as
 // 128 x 512 tiles (8 waves of 128 x 64, as GemmGrouped; 2 stages of 80 KiB).
-using GemmGroupedWide = gemm::Cfg<128, 512, 128, 2, 1, 8, 4>;
+using GemmGroupedWide = gemm::Cfg<128, 512, 128, 2, 1, 8, 4, 16>;
 // MoE GEMM over experts of a few hundred rows: 128-row tiles waste less of
 // each expert's last tile row (moe_tile).
-using GemmGroupedMid = gemm::Cfg<128, 256, 128, 3, 2, 4, 4>;
-using GemmGroupedSmall = gemm::Cfg<128, 128, 128, 3, 2, 4, 4>;
+using GemmGroupedMid = gemm::Cfg<128, 256, 128, 3, 2, 4, 4, 16>;
+using GemmGroupedSmall = gemm::Cfg<128, 128, 128, 3, 2, 4, 4, 16>;
 // Decode batches (a few dozen rows per expert): the launch streams every
 // expert's weights, and two blocks a CU keep more of them in flight than one
 // 128-row block, with no MFMA work on 100 rows of padding.
-using GemmMoeFew = gemm::Cfg<64, 128, 128, 3, 2, 4, 4>; // 8 waves of 32 x 32, 72 KiB LDS
-using GemmGroupedTiny = gemm::Cfg<64, 64, 128, 4, 2, 2, 4>; // 4 waves of 32 x 32, 64 KiB LDS
+using GemmMoeFew = gemm::Cfg<64, 128, 128, 3, 2, 4, 4, 16>; // 8 waves of 32 x 32, 72 KiB LDS
+using GemmGroupedTiny = gemm::Cfg<64, 64, 128, 4, 2, 2, 4, 16>; // 4 waves of 32 x 32, 64 KiB LDS
 
 // Tiles of a MoE GEMM from the rows per expert, rows / experts (the sort's
 // capacity: with the default unit of 32 about 32 more than are routed there).
@@ -1069,12 +1069,12 @@ void moe_gemm_plan(const uint32_t* sizes, uint32_t* plan)
 // 128-byte line of h per row and wave), otherwise as GemmGrouped /
 // GemmGroupedMid (16 x 16 x 64 MFMA, whose lane layout the 32-row gate/up
 // interleave matches).
-using GemmSilu     = gemm::Cfg<256, 256, 128, 2, 4, 2, 4>;
-using GemmSiluMid  = gemm::Cfg<128, 256, 128, 3, 4, 2, 4>;
-using GemmSiluWide = gemm::Cfg<128, 512, 128, 2, 2, 4, 4>; // GemmSilu's wide partner
+using GemmSilu     = gemm::Cfg<256, 256, 128, 2, 4, 2, 4, 16>;
+using GemmSiluMid  = gemm::Cfg<128, 256, 128, 3, 4, 2, 4, 16>;
+using GemmSiluWide = gemm::Cfg<128, 512, 128, 2, 2, 4, 4, 16>; // GemmSilu's wide partner
 // The same short tiles as the plain GEMM's, in wave tiles 64 columns wide.
-using GemmSiluSmall = gemm::Cfg<128, 128, 128, 2, 4, 2, 4>; // 8 waves of 32 x 64, 64 KiB LDS
-using GemmSiluFew   = gemm::Cfg<64, 128, 128, 3, 2, 2, 4>;  // 4 waves of 32 x 64, 72 KiB LDS
+using GemmSiluSmall = gemm::Cfg<128, 128, 128, 2, 4, 2, 4, 16>; // 8 waves of 32 x 64, 64 KiB LDS
+using GemmSiluFew   = gemm::Cfg<64, 128, 128, 3, 2, 2, 4, 16>;  // 4 waves of 32 x 64, 72 KiB LDS
 static_assert(GemmSilu::kWaveN == GemmSiluMid::kWaveN
                   && GemmSiluSmall::kWaveN == GemmSiluFew::kWaveN,
               "two pmax layouts");
