@@ -596,8 +596,9 @@ struct Partial {
     static_assert(C::kWaves % kFixupWaves == 0, "whole fixup blocks");
 };
 
-// K pieces of a split tile: at most kMaxParts, each at least kMinKtPerPart
-// k-tiles (shorter pieces do not repay the partial traffic).
+// K pieces of a split tile: at most kMaxParts.  The expert GEMM's tail split, decided
+// on the device, keeps each at kMinKtPerPart k-tiles or more (shorter pieces do not
+// repay the partial traffic there); the host's plan has its own least.
 constexpr uint32_t kMaxParts     = 8;
 constexpr uint32_t kMinKtPerPart = 16;
 
@@ -834,7 +835,7 @@ __global__ void __launch_bounds__(C::kThreads, 1) gemm_i8_tile_kernel(KArgs p)
     gemm_tile<C, OUT>(p, tm * C::kBM, tn * C::kBN, lds);
 }
 
-// K split of a launch whose tiles fill at most half of the CUs: logical
+// K split of a launch, all its blocks resident together (the plan's): logical
 // block b runs piece b % parts of tile b / parts (k-tiles [part * nk / parts,
 // (part + 1) * nk / parts)) and stores its int32 accumulators to
 // ws + b * Partial<C>::kInts; gemm_i8_split_fixup_kernel then sums each
