@@ -1086,7 +1086,7 @@ hipError_t launch_gemm_direct(const GemmArgs& g, bool kn, hipStream_t stream)
 bool generic_pays(const GemmArgs& g, bool kn)
 {
     const double k = g.k, outputs = (double)g.m * g.n;
-    if(g.k >= 32) return false;
+    if(g.k >= 32 || ceil_div(g.m, 16) > 65535) return false; // its grid's rows
     if(kn) return 2.8 + 0.07 * k + 1e-6 * outputs * (1.0 + 0.15 * k) < 4.25;
     return 2.6 + 0.05 * k + 1e-6 * outputs * (1.7 + 0.47 * k) < 4.4 + (g.k < 16 ? 0.33 * k : 0.0);
 }

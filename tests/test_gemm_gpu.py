@@ -257,6 +257,20 @@ def test_sample_layout_routes_exact(w8a8, gpu, m, n, k):
         assert_i32_equal(host(c), acc)
 
 
+# More rows than one output per thread has a grid for, with and without the room to
+# repack: K below 32 and few products all the same.
+@pytest.mark.parametrize("m,n", [(1100000, 1), (1048560, 1)])
+def test_sample_layout_of_very_many_rows(w8a8, gpu, m, n):
+    import torch
+    a, b, _, _ = inputs(m, n, 1, 5)
+    at = _at_offset(np.ascontiguousarray(a.T), m + 1, 0, gpu)
+    bt = _at_offset(np.ascontiguousarray(b.T), n + 1, 0, gpu)
+    c = w8a8.gemm(at, bt, layout=w8a8.LAYOUT_A_COL_B_KN, out_dtype=torch.int32)
+    assert_i32_equal(host(c), O.gemm_i32(a, b))
+    prim = w8a8.gemm(_at_offset(a, 1, 0, gpu), _at_offset(b, 1, 0, gpu), out_dtype=torch.int32)
+    assert_i32_equal(host(prim), O.gemm_i32(a, b))
+
+
 # The short tiles (several blocks a CU) and their K pieces, row-major and packed
 # weights: edges of 32 / 64 rows and 64 / 128 columns, K tails, one k-tile.
 SHORT_TILE_SHAPES = [
