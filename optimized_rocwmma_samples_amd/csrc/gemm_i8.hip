@@ -390,8 +390,11 @@ TilePlan search_plan(uint32_t m, uint32_t n, uint32_t k, size_t ws_bytes, bool d
     // tiles neither cut along K nor are estimated 10% faster for: 231 sizes within that
     // run through it 15% faster with weights in L2, 3.5% in the MALL, 1.5% cold (1 x 752
     // x 2816 5.7 us warm, 8.4 in 32 x 64 tiles).  Off the lines it is 18% faster warm but
-    // 3-4% slower elsewhere (37 sizes), and below 1536 slower in all three.
-    if(m <= 16 && k >= 1536 && k % 128 == 0 && best.parts == 1 && dec < 1.1 * cost.seen)
+    // 3-4% slower elsewhere (37 sizes), and below 1536 slower in all three.  Weights of
+    // fewer than 256 rows, a megabyte or less, it always keeps: 1 x 21 x 3856 5.5 us,
+    // 11.2 in 32 x 64 tiles; 19 sizes 1.85 times as fast in L2, 1.5 in the MALL, 2% slower cold.
+    if(m <= 16 && k >= 1536 && best.parts == 1
+       && decode && (n < 256 || (k % 128 == 0 && dec < 1.1 * cost.seen)))
         best.cfg = TileCfg::kDecode;
     return best;
 }

@@ -50,7 +50,7 @@ def test_f16_dequant_mode2(w8a8, gpu, m, n, k):
 # partial tiles on both edges and a K tail; the last eight with odd rows of C.
 TILE_CFG_SHAPES = [
     (4100, 3000, 160, (256, 256)), (2048, 4096, 512, (128, 256)), (1500, 4000, 272, (128, 256)),
-    (700, 1100, 400, (64, 64)), (2, 107, 144, (0, 32)), (3, 107, 3680, (32, 64)),
+    (700, 1100, 400, (64, 64)), (2, 107, 144, (0, 32)), (3, 373, 3520, (32, 64)),
     (90, 123, 144, (64, 64)), (771, 1051, 144, (64, 64)), (549, 2785, 240, (64, 128)),
     (713, 2883, 656, (128, 128)), (1746, 4227, 688, (128, 256)), (1497, 8675, 400, (256, 256)),
 ]
@@ -173,7 +173,7 @@ def test_k_split_exact(w8a8, gpu, m, n, k, tile):
 # row-major and packed weights and the decode kernels.
 @pytest.mark.parametrize("m,n,k,tile", [
     (4100, 3001, 160, (256, 256)), (990, 1621, 368, (64, 128)), (100, 1003, 1040, (64, 64)),
-    (40, 515, 400, (0, 32)), (3, 77, 64, (0, 32)), (3, 107, 3680, (32, 64)),
+    (40, 515, 400, (0, 32)), (3, 77, 64, (0, 32)), (3, 373, 3520, (32, 64)),
     (713, 2883, 656, (128, 128)), (1746, 4227, 688, (128, 256)), (1497, 8675, 400, (256, 256))])
 def test_unaligned_outputs_exact(w8a8, gpu, m, n, k, tile):
     assert unsplit_tile(w8a8, m, n, k) == tile

@@ -71,10 +71,12 @@ def test_plans_alike_to_the_host_are_told_apart_by_gpu_time(w8a8, m, n, k, rows)
 
 # Up to 16 rows of whole 128-byte lines where the decode kernel and unsplit tiles are
 # within a tenth of each other by the estimate: weights in L2 run up to twice as fast
-# through the decode kernel (5 x 2464 x 2176 7.1 us in 64 x 64 tiles, 4.9).
+# through the decode kernel (5 x 2464 x 2176 7.1 us in 64 x 64 tiles, 4.9); fewer than
+# 256 columns at any K.
 @pytest.mark.parametrize("m,n,k,kernel", [
     (1, 752, 2816, (0, 32, 1)), (5, 2464, 2176, (0, 32, 1)), (2, 3807, 1920, (0, 32, 1)),
     (8, 3712, 2816, (0, 32, 1)), (16, 3584, 2304, (0, 32, 1)), (3, 320, 3840, (0, 32, 1)),
+    (1, 21, 3856, (0, 32, 1)), (16, 255, 3920, (0, 32, 1)), (17, 21, 3856, (32, 64, 1)),
     (15, 2816, 3248, (32, 64, 1)), (1, 17664, 256, (64, 128, 1)), (6, 6912, 4096, (64, 64, 1)), (1, 28672, 8192, (64, 128, 1)), (4, 662, 4032, (32, 64, 5)),
     (23, 497, 3168, (32, 64, 1)), (37, 928, 3072, (32, 64, 1))])
 def test_few_rows_leave_the_decode_kernel_for_a_tenth(w8a8, m, n, k, kernel):
