@@ -847,7 +847,8 @@ MoeTile moe_tile(uint32_t rows, uint32_t experts, uint32_t n, bool silu = false)
 // Whether a launch of 64 x 128 or 128 x 128 tiles is cut along K (TailSplit): where
 // the experts that can have rows make tiles for at most half of the CUs and a
 // tile has two pieces' k-tiles.  How many have rows is the router's: at most the
-// pairs, which at the default unit are the rows past 32 an expert.  One token of
+// pairs, which at the default unit are the rows past 32 an expert and at a unit of 1
+// (too few rows for the other) those past one.  One token of
 // the 8-expert Mixtral layer (2 experts, 64 tiles of 112 k-tiles) 52.9 -> 30.6 us,
 // two 56 -> 42; one expert of 1-48 rows 52 -> 23, of 100 rows (128 x 128) 65 -> 28.
 // Launches that fill the CUs go without the second launch (16 tokens 79.0 us, 81.2
@@ -855,7 +856,7 @@ MoeTile moe_tile(uint32_t rows, uint32_t experts, uint32_t n, bool silu = false)
 bool moe_short_split(uint32_t rows, uint32_t experts, uint32_t n, uint32_t k)
 {
     const uint64_t pad    = 32ull * experts;
-    const uint64_t pairs  = rows > pad ? rows - pad : rows;
+    const uint64_t pairs  = rows > pad ? rows - pad : rows > experts ? rows - experts : rows;
     const uint64_t active = std::min<uint64_t>(experts, pairs);
     return active * ((n + 127) / 128) * 2 <= device_cus()
            && (k + 127) / 128 >= 2 * gemm::kMinKtPerPart;

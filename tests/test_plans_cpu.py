@@ -126,6 +126,15 @@ def test_expert_gemm_of_few_tiles_is_cut_along_k(w8a8, tokens, topk, experts, n,
     assert plan(w8a8, L.PLAN_MOE_GEMM, experts, rows, n, k) == tile
 
 
+# The same with the sort's unit at 1, whose capacity is a row an expert more than pairs.
+@pytest.mark.parametrize("tokens,topk,experts,n,k,split", [
+    (1, 2, 8, 4096, 14336, 1), (2, 2, 8, 4096, 14336, 1), (1, 6, 64, 1024, 8192, 1),
+    (16, 2, 8, 4096, 14336, 0), (100, 2, 8, 4096, 14336, 0)])
+def test_few_experts_at_a_unit_of_one(w8a8, tokens, topk, experts, n, k, split):
+    rows = capacity(tokens, topk, experts, unit=1)
+    assert plan(w8a8, L.PLAN_MOE_GEMM, experts, rows, n, k) == (64, 128, split)
+
+
 # Few products of a short K: a tile's k-step is mostly zeros (300 x 300 x 9 7.4 us,
 # one output per thread 3.3).
 @pytest.mark.parametrize("m,n,k,tile", [
