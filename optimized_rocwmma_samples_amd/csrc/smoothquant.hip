@@ -640,24 +640,26 @@ hipError_t launch_moe(const QuantRows& p, hipStream_t stream)
 // only where many pairs share few tokens and x is most of the traffic.  Measured
 // over 40-8192 tokens, top 1-8, hidden 512-28672 (us by pairs / by tokens):
 //   512: 32000 pairs 11.5 / 12.9, 49152 17.0 / 16.4
-//   1024 (881): 2400 pairs 4.7 / 10.7, 12000 9.9 / 13.7, 16000 12.3 / 12.1
+//   881: 2400 pairs 4.7 / 10.7, 12000 9.9 / 13.7, 19800 16.0 / 17.3, 32000 23.4 / 21.3;
+//   1024 (whole 16 bytes): 19800 13.4 / 15.6, 48000 24.1 / 25.8
 //   2048: 600 pairs, top 6 3.7 / 7.1, 12000 12.3 / 16.1, 65536 47.1 / 47.6
 //   4096: 4200 pairs, top 6 10.7 / 12.3, 16000 25.6 / 29.1, 49152 68.3 / 71.0
 //   7168: 2400 pairs, top 8 13.1 / 18.8, 4200 19.6 / 19.0, 24000 87 / 66;
 //         top 2 8000 28.5 / 30.0
-//   14336: 800 pairs, top 8 13.0 / 18.1, 1400, top 2 15.1 / 13.3, 9000 87 / 61
+//   14336: 800 pairs, top 8 13.0 / 18.1, 1400, top 2 15.1 / 13.3, 9000 87 / 61; 176
+//         tokens, fewer than the CUs, top 8 16.9 / 18.1, 400, top 4 18.6 / 16.6
 //   20000: 2800 pairs, top 4 38 / 39, 6000 69 / 74; 28672: 47 / 42, 95 / 81; top 2
 //         3000 44 / 50
 QuantPlan moe_quant_plan(uint32_t pairs, uint32_t n, uint32_t topk)
 {
     if(n <= 512) return {1, 1, pairs > 36000};
     if(n <= 1024 && pairs <= 1536) return {1, 2, false};
-    if(n <= 1024) return {2, 1, pairs > 12288};
+    if(n <= 1024) return {2, 1, pairs > 24576 && n % 8 != 0};
     if(n <= 2048) return pairs <= 1536 ? QuantPlan{1, 4, false} : QuantPlan{4, 1, false};
     if(n <= 4096 && pairs <= 1024) return {2, 4, false};
     if(n <= 4096) return pairs <= 10240 ? QuantPlan{4, 2, false} : QuantPlan{8, 1, false};
     if(n <= 8192) return {4, 4, pairs > 3584 && topk > 2};
-    if(n <= 16384) return {2, 16, pairs > 1280};
+    if(n <= 16384) return {2, 16, pairs > 1280 && pairs >= 256 * topk};
     if(n <= 32768) return {4, 16, pairs > 2048 && topk > 2};
     return {0, 0, false};
 }

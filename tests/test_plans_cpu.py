@@ -24,7 +24,8 @@ def test_debug_plan_rejects_bad_arguments(w8a8):
 @pytest.mark.parametrize("tokens,hidden,topk", [
     (123, 1408, 6), (300, 2048, 6), (498, 2048, 6), (1225, 1408, 6), (531, 2048, 2),
     (300, 512, 8), (700, 881, 6), (152, 881, 4), (2171, 2048, 4), (8192, 2048, 6),
-    (441, 4096, 8), (4930, 4096, 4), (700, 4096, 6), (300, 7168, 8)])
+    (441, 4096, 8), (4930, 4096, 4), (700, 4096, 6), (300, 7168, 8), (3300, 1024, 6),
+    (8000, 960, 6), (3300, 881, 6), (176, 14336, 8), (176, 12000, 8)])
 def test_moe_quantizer_of_few_or_short_rows_goes_by_pairs(w8a8, tokens, hidden, topk):
     chunks, waves, by_tokens = plan(w8a8, L.PLAN_MOE_QUANT, tokens * topk, hidden, topk)
     assert not by_tokens and chunks * waves * 512 >= hidden
