@@ -437,24 +437,30 @@ GroupedTile grouped_gemm_tile(const w8a8_group_desc* groups, uint32_t ngroups)
     double      cost = 1e300;
     for(const CfgCost& c : kCosts) {
         if(c.most != kAnyM) continue;
-        auto     count = [&](const w8a8_group_desc& g) {
-            return (uint64_t)ceil_div(g.m, c.bm) * ceil_div(g.n, c.bn);
-        };
-        uint64_t tiles = 0;
-        for(uint32_t i = 0; i < ngroups; ++i) tiles += count(groups[i]);
-        if(tiles == 0 || tiles > 0x7FFFFFFFull) continue;
-        double steps = 0, most = 0, out = 0, w = 0;
+        // this runs on each call: shifts for the tile's divisions, and one loop, [1] the
+        // groups with rows off a line, whose factor the last of them gives
+        const int sm = __builtin_ctz(c.bm), sn = __builtin_ctz(c.bn);
+        uint64_t  tiles = 0, steps[2] = {0, 0}, most[2] = {0, 0};
+        uint32_t  off_k = 0;
+        double    out = 0, w = 0;
         for(uint32_t i = 0; i < ngroups; ++i) {
             const w8a8_group_desc& g = groups[i];
             if(g.m == 0) continue;
-            const double k = ceil_div(g.k, 128) * line_factor(c, g.k, tiles);
-            steps += count(g) * k;
-            most = std::max(most, k);
+            const uint64_t t   = (uint64_t)((g.m + c.bm - 1) >> sm) * ((g.n + c.bn - 1) >> sn);
+            const uint64_t k   = ceil_div(g.k, 128);
+            const int      off = g.k % 128 != 0;
+            tiles += t;
+            steps[off] += t * k;
+            most[off] = std::max(most[off], k);
+            if(off) off_k = g.k;
             out += 2e-6 * g.m * g.n;
             w += 1e-6 * g.n * (double)g.k;
         }
+        if(tiles == 0 || tiles > 0x7FFFFFFFull) continue;
+        const double   f      = off_k ? line_factor(c, off_k, tiles) : 1.0;
         const uint64_t per_cu = (tiles + device_cus() - 1) / device_cus();
-        const double   nk     = per_cu == 1 ? most : steps / tiles;
+        const double   nk     = per_cu == 1 ? std::max<double>(most[0], most[1] * f)
+                                            : (steps[0] + steps[1] * f) / tiles;
         const double   t      = c.fixed + out * c.out_mb + w * c.w_mb
                          + nk * (per_cu / c.resident * c.step[c.resident - 1]
                                  + (per_cu % c.resident ? c.step[per_cu % c.resident - 1] : 0.0))
