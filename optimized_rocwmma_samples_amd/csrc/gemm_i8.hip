@@ -304,7 +304,10 @@ uint32_t ceil_div(uint32_t a, uint32_t b) { return (a + b - 1) / b; }
 // other work in flight sees the GPU's time).
 struct PlanTime {
     double seen, gpu;
-    bool   operator<(const PlanTime& o) const { return seen != o.seen ? seen < o.seen : gpu < o.gpu; }
+    bool   operator<(const PlanTime& o) const
+    {
+        return seen != o.seen ? seen < o.seen : gpu < o.gpu;
+    }
 };
 
 // What a k-step of row-major operands takes against one of whole 128-byte lines.
@@ -317,12 +320,14 @@ double line_factor(const CfgCost& c, uint32_t k, uint64_t blocks)
     return std::max(c.cross, 1.0 + c.full * off * ramp);
 }
 
-PlanTime plan_cost(const CfgCost& c, uint32_t m, uint32_t n, uint32_t k, uint32_t parts, bool packed)
+PlanTime plan_cost(const CfgCost& c, uint32_t m, uint32_t n, uint32_t k, uint32_t parts,
+                   bool packed)
 {
     const uint32_t cus    = device_cus();
     const uint32_t tm     = ceil_div(m, c.bm);
     const uint64_t blocks = (uint64_t)tm * ceil_div(n, c.bn) * parts;
-    const double   steps  = ceil_div(ceil_div(k, 128), parts) * (packed ? 1.0 : line_factor(c, k, blocks));
+    const double   factor = packed ? 1.0 : line_factor(c, k, blocks);
+    const double   steps  = ceil_div(ceil_div(k, 128), parts) * factor;
     uint64_t       per_cu = (blocks + cus - 1) / cus;
     double         t      = c.fixed + 2e-6 * m * n * c.out_mb + 1e-6 * n * (double)k * c.w_mb;
     // launch_main runs a last round of at most half the CUs as smaller tiles

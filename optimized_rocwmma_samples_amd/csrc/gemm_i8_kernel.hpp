@@ -219,7 +219,10 @@ struct Acc {
     v4i r[C::kTilesM][C::kTilesN];
 
     __device__ static __forceinline__ int row(int qm, int lane) { return qm * 16 + (lane & 15); }
-    __device__ static __forceinline__ int col(int qn, int lane) { return qn * 16 + (lane >> 4) * 4; }
+    __device__ static __forceinline__ int col(int qn, int lane)
+    {
+        return qn * 16 + (lane >> 4) * 4;
+    }
     __device__ __forceinline__ void zero()
     {
 #pragma unroll

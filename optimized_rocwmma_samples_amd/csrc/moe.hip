@@ -362,7 +362,7 @@ __device__ __forceinline__ int wave_row_expert(const P& p, uint32_t row)
         if(in == 0) break; // starts ascend
         const int last = 63 - __builtin_clzll(in);
         e              = base + last;
-        end            = __builtin_amdgcn_readlane(start, last) + __builtin_amdgcn_readlane(count, last);
+        end = __builtin_amdgcn_readlane(start, last) + __builtin_amdgcn_readlane(count, last);
     }
     return (int32_t)row < end ? e : -1;
 }
@@ -564,7 +564,8 @@ constexpr int kRqRows  = 8;
 constexpr int kRqBatch = 7;
 
 // The first row of a block.
-__host__ __device__ inline uint32_t requant_row(uint32_t rows_a_block, uint32_t block, uint32_t blocks)
+__host__ __device__ inline uint32_t requant_row(uint32_t rows_a_block, uint32_t block,
+                                                uint32_t blocks)
 {
     return rows_a_block == 1 ? gemm::xcd_remap(block, blocks) : block * rows_a_block;
 }

@@ -659,7 +659,9 @@ hipError_t launch_rmsnorm_sq(const NormRows& p, hipStream_t stream)
         if(n <= 16384) return launch_by_outputs<2, 16, 1024, 1>(p, stream);
     }
     const NormPlan d  = norm_rows_plan(p.rows, n);
-    auto           is = [&](uint32_t chunks, uint32_t waves) { return d.chunks == chunks && d.waves == waves; };
+    auto           is = [&](uint32_t chunks, uint32_t waves) {
+        return d.chunks == chunks && d.waves == waves;
+    };
     if(is(1, 1)) return launch_rows_norm<1, 1>(p, stream);
     if(is(1, 4)) return launch_rows_norm<1, 4>(p, stream);
     if(is(2, 1)) return launch_rows_norm<2, 1>(p, stream);

@@ -83,7 +83,8 @@ constexpr int sq_rows_waves(int cpl) { return cpl == 4 ? 8 : cpl == 8 ? 6 : 1; }
 // branch: x ahead of s, or the packing ahead of the branch, costs 12-34 VGPRs and
 // with them two waves a SIMD (8192 pairs of 4096, top 1: 22.4 us, 18.7 as it is).
 template <int CPL, int WPR, bool MOE>
-__global__ void __launch_bounds__(sq_rows_threads(WPR), sq_rows_waves(CPL)) sq_rows_kernel(QuantRows p)
+__global__ void __launch_bounds__(sq_rows_threads(WPR), sq_rows_waves(CPL))
+    sq_rows_kernel(QuantRows p)
 {
     constexpr int kWaves        = sq_rows_threads(WPR) / kWave;
     constexpr int kRowsPerBlock = kWaves / WPR;
@@ -611,7 +612,9 @@ hipError_t launch_dense(const QuantRows& p, hipStream_t stream)
 hipError_t launch_moe(const QuantRows& p, hipStream_t stream)
 {
     const QuantPlan d  = moe_quant_plan(p.rows, p.n, p.topk);
-    auto            is = [&](uint32_t chunks, uint32_t waves) { return d.chunks == chunks && d.waves == waves; };
+    auto            is = [&](uint32_t chunks, uint32_t waves) {
+        return d.chunks == chunks && d.waves == waves;
+    };
     if(d.tokens) {
         if(is(1, 1)) return launch_tokens<1, 1>(p, stream);
         if(is(2, 1)) return launch_tokens<2, 1>(p, stream);

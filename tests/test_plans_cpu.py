@@ -78,7 +78,8 @@ def test_plans_alike_to_the_host_are_told_apart_by_gpu_time(w8a8, m, n, k, rows)
     (1, 752, 2816, (0, 32, 1)), (5, 2464, 2176, (0, 32, 1)), (2, 3807, 1920, (0, 32, 1)),
     (8, 3712, 2816, (0, 32, 1)), (16, 3584, 2304, (0, 32, 1)), (3, 320, 3840, (0, 32, 1)),
     (1, 21, 3856, (0, 32, 1)), (16, 255, 3920, (0, 32, 1)), (17, 21, 3856, (32, 64, 1)),
-    (15, 2816, 3248, (32, 64, 1)), (1, 17664, 256, (64, 128, 1)), (6, 6912, 4096, (64, 64, 1)), (1, 28672, 8192, (64, 128, 1)), (4, 662, 4032, (32, 64, 5)),
+    (15, 2816, 3248, (32, 64, 1)), (1, 17664, 256, (64, 128, 1)),
+    (6, 6912, 4096, (64, 64, 1)), (1, 28672, 8192, (64, 128, 1)), (4, 662, 4032, (32, 64, 5)),
     (23, 497, 3168, (32, 64, 1)), (37, 928, 3072, (32, 64, 1))])
 def test_few_rows_leave_the_decode_kernel_for_a_tenth(w8a8, m, n, k, kernel):
     assert plan(w8a8, L.PLAN_GEMM, m, n, k, WS) == kernel
@@ -140,7 +141,8 @@ def test_few_experts_at_a_unit_of_one(w8a8, tokens, topk, experts, n, k, split):
 # one output per thread 3.3).
 @pytest.mark.parametrize("m,n,k,tile", [
     (8, 1021, 9, 0), (300, 300, 9, 0), (55, 1307, 17, 0), (40, 304, 27, 0), (500, 1001, 9, 0),
-    (640, 640, 13, 0), (1000, 1000, 9, 64), (1500, 900, 3, 64), (500, 1001, 17, 64), (100, 1000, 25, 64), (4, 60, 33, 64),
+    (640, 640, 13, 0), (1000, 1000, 9, 64), (1500, 900, 3, 64), (500, 1001, 17, 64), (100, 1000, 25, 64),
+    (4, 60, 33, 64),
     (1000, 1000, 1000, 64), (1700, 1650, 100, 128), (3400, 3330, 33, 256)])
 def test_few_products_of_a_short_k_run_one_per_thread(w8a8, m, n, k, tile):
     assert plan(w8a8, L.PLAN_GEMM_ANY, m, n, k) == (tile, tile, 1)
